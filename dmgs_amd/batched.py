@@ -15,7 +15,6 @@ every call).  Here:
   from a counting pass and checked after the fact (``overflowed``), so a
   steady-state step has no host synchronisation and can be captured in a
   HIP graph (``BatchedStep``);
-* the blend work-group shape / LDS batch depth is picked by ``autotune``.
 
 Images and gradients equal those of B single-view ``render`` calls followed
 by autograd through the activations (same per-view arithmetic).
@@ -31,9 +30,9 @@ from . import _native as N
 CHANNELS = 59
 XYZ, SCALE, ROT, OPACITY, SH = 0, 3, 6, 10, 11
 STAGE_GEOMETRY, STAGE_BINNING, STAGE_BLEND, STAGES_ALL = 1, 2, 4, 7
-RENDER_VARIANTS = ("16x16 px, 256-deep LDS batch", "16x16 px, 128-deep", "8x8 px, 64-deep", "8x8 px, 128-deep",
-                   "one wave per tile, 64-deep", "one wave per tile, 128-deep",
-                   "16x16 px 256-deep forward, one-wave-per-tile 64-deep backward")
+# Every variant runs the same kernels (the launch picks its shape from its own sizes, see csrc/render.hip);
+# the numbers stay valid for callers that pass one.
+RENDER_VARIANTS = ("four waves per tile forward, one wave per tile or list segment backward",) * 7
 
 
 def pack_params(xyz, log_scale, rotation, opacity_logit, features_dc, features_rest, out=None):
@@ -345,27 +344,22 @@ class BatchedRenderer:
 
     # ---- autotuning -------------------------------------------------------
     def autotune(self, params, dL_dimages=None, reps=3):
-        """Time forward + backward for every blend variant and keep the
-        fastest.  Returns {variant: ms}."""
+        """Time forward + backward.  Returns {variant: ms}; one measurement
+        serves every variant, since they run the same kernels."""
         self._require_plan()
         if dL_dimages is None:
             dL_dimages = torch.full((3 * self.total_pixels,), 1e-3, device=self.device)
         images = self.new_images()
         grads = torch.empty(CHANNELS, self.P, dtype=torch.float32, device=self.device)
-        times = {}
-        for v in range(len(RENDER_VARIANTS)):
-            self.variant = v
+        self.forward(params, images)
+        self.backward(params, dL_dimages, grads)
+        torch.cuda.synchronize(self.device)
+        t0 = time.perf_counter()
+        for _ in range(reps):
             self.forward(params, images)
             self.backward(params, dL_dimages, grads)
-            torch.cuda.synchronize(self.device)
-            t0 = time.perf_counter()
-            for _ in range(reps):
-                self.forward(params, images)
-                self.backward(params, dL_dimages, grads)
-            torch.cuda.synchronize(self.device)
-            times[v] = 1000.0 * (time.perf_counter() - t0) / reps
-        self.variant = min(times, key=times.get)
-        return times
+        torch.cuda.synchronize(self.device)
+        return dict.fromkeys(range(len(RENDER_VARIANTS)), 1000.0 * (time.perf_counter() - t0) / reps)
 
 
 class BatchedLoss:

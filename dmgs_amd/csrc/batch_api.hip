@@ -70,7 +70,9 @@ int bits_for(uint32_t n) {
 // scan, the depth-sort scratch, per-tile ranges and per-pixel blend state.
 struct StateLayout {
   size_t splats, keys_a, keys_b, order_a, order_b, rects, rects_sorted, radii, offsets, gscratch, visible,
-      status, tile_order, tile_bucket, bucket_hist, tile_work, ranges, final_T, n_contrib, total;
+      status, tile_order, tile_bucket, bucket_hist, tile_work, ranges, final_T, n_contrib, tile_last,
+      seg_head, seg_rec, seg_state, total;
+  int seg_cap;  // slots for the list segments a forward keeps for its backward (0: too many tiles for any)
   StateLayout(size_t N, size_t T, size_t X) {
     size_t o = 0;
     splats = o; o += align_up(N * DMGS_SPLAT_F4 * 16);
@@ -92,6 +94,11 @@ struct StateLayout {
     ranges = o; o += align_up(T * 8);
     final_T = o; o += align_up(X * 4);
     n_contrib = o; o += align_up(X * 4);
+    seg_cap = T <= (size_t)dmgs::kSegmentTiles ? (int)std::min<size_t>(16384, std::max<size_t>(1024, N / 16)) : 0;
+    tile_last = o; o += align_up(seg_cap ? T * 4 : 0);
+    seg_head = o; o += align_up(8);
+    seg_rec = o; o += align_up((size_t)seg_cap * 16);
+    seg_state = o; o += (size_t)seg_cap * 256 * 16;
     total = o;
   }
 };
@@ -191,9 +198,15 @@ dmgs::RenderArgs render_args(const dmgs_batch* b, const Ctx& c) {
   r.n_contrib = at<uint32_t>(b->state, c.S.n_contrib);
   r.gacc = static_cast<float*>(b->bwd_ws);
   r.tile_order = at<uint32_t>(b->state, c.S.tile_order);
-  // the strip forward measures each tile's backward list length
-  const bool strips_fwd = b->variant == dmgs::kRenderStrips64 || b->variant == dmgs::kRenderStrips128;
-  r.tile_work = strips_fwd ? at<uint32_t>(b->state, c.S.tile_work) : nullptr;
+  r.tile_work = at<uint32_t>(b->state, c.S.tile_work);  // the forward measures each tile's backward list length
+  r.seg.head = at<uint32_t>(b->state, c.S.seg_head);
+  if (b->bwd_ws && c.S.seg_cap) {
+    r.seg.len = dmgs::kSegmentLength;
+    r.seg.cap = c.S.seg_cap;
+    r.seg.rec = at<uint4>(b->state, c.S.seg_rec);
+    r.seg.state = at<float4>(b->state, c.S.seg_state);
+    r.seg.tile_last = at<uint32_t>(b->state, c.S.tile_last);
+  }
   return r;
 }
 
@@ -386,10 +399,10 @@ int dmgs_batched_forward(const dmgs_batch* b, const float* params, float* images
     if (b->bwd_ws) {  // the blend work-groups also clear the backward accumulator
       r.clear = static_cast<float4*>(b->bwd_ws);
       r.clear_n = (c.N * DMGS_GACC_STRIDE + 3) / 4;  // inside the 256-byte-aligned workspace
-      r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);  // for the backward's tile order
-      r.clear_words_n = 512;
     }
-    dmgs::launch_render_fwd(r, st, b->variant);
+    r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);  // for the backward's tile order
+    r.clear_words_n = 512;
+    dmgs::launch_render_fwd(r, st);
     if ((rc = bcheck("batch render forward", st))) return rc;
   }
   return DMGS_OK;
@@ -411,11 +424,13 @@ int dmgs_batched_backward(const dmgs_batch* b, const float* params, const float*
   if (stages & DMGS_STAGE_BLEND) {  // accumulates into bwd_ws, which holds zeros on entry
     dmgs::RenderArgs r = render_args(b, c);
     r.dL_dpix = dL_dimages;
-    // re-order the tiles by the list lengths the strip forward measured
-    // (the forward blend, which every backward follows, zeroed the histogram)
-    dmgs::launch_tile_order_bwd(r, at<uint32_t>(b->state, c.S.tile_order), at<uint8_t>(b->state, c.S.tile_bucket),
+    // re-order the tiles by the list lengths the forward measured (the
+    // forward blend, and then each backward blend, zero the histogram)
+    r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);
+    r.clear_words_n = 512;
+    if (r.seg.len == 0) dmgs::launch_tile_order_bwd(r, at<uint32_t>(b->state, c.S.tile_order), at<uint8_t>(b->state, c.S.tile_bucket),
                                 at<uint32_t>(b->state, c.S.bucket_hist), st, true);
-    dmgs::launch_render_bwd(r, st, b->variant);
+    dmgs::launch_render_bwd(r, st);
     if ((rc = bcheck("batch render backward", st))) return rc;
   }
   if (stages & DMGS_STAGE_GEOMETRY) {

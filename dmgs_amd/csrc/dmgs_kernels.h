@@ -154,6 +154,22 @@ void launch_gather_rects(const uint2* rects, const uint32_t* order, uint2* rects
 void launch_mv_geometry_bwd(const MVArgs& a, hipStream_t s);
 
 // ---- blend ----
+// List segments that a forward keeps for its backward (render.hip).  At most kSegmentTiles tiles: with 8160
+// tiles (1920x1080) keeping them costs as much as it gives (forward + backward of 1M Gaussians 335 us with,
+// 331 without), with 2500 it saves 60 us of 230.  64 members: shorter ones cost the forward more than the
+// backward gains from 2500 tiles on, 128 lose 15-60 us on the cases with few tiles.
+constexpr int kSegmentTiles = 4096;
+constexpr int kSegmentLength = 64;
+constexpr int kTileSegments = 256;  // kept segments of one tile at most
+constexpr uint32_t kNoSegment = 0xFFFFFFFFu;
+constexpr uint32_t kSegMagic = 0x5E600001u;
+struct Segments {
+  int len, cap;          // members per segment (0: none are kept), slots
+  uint32_t* head;        // [0] slots asked for, [1] kSegMagic once a forward keeps segments
+  uint4* rec;            // per slot: tile, first and one past the last list position
+  float4* state;         // per slot: the tile's 256 pixels' T behind the segment and the colour added behind it
+  uint32_t* tile_last;   // per tile: where its last (not kept) segment begins
+};
 // Single view: W, H, grid_x, grid_y, bg and the image pointers describe the
 // view.  Several views: `views` / `tile_view` map each global tile to its
 // view; images, final_T and n_contrib are packed at each view's pixel_base.
@@ -188,22 +204,9 @@ struct RenderArgs {
   // dispatch order starts from
   uint32_t* clear_words;
   int clear_words_n;
+  Segments seg;
 };
-// Work-group shape / LDS batch depth of the blend kernels (results are the
-// same for every variant; the autotuner picks the fastest).  The strip
-// variants run one wave per tile (four pixels per lane) forward and
-// backward; kRenderMixed pairs the 16x256 forward with the strip backward.
-enum RenderVariant {
-  kRender16x256 = 0,
-  kRender16x128 = 1,
-  kRender8x64 = 2,
-  kRender8x128 = 3,
-  kRenderStrips64 = 4,
-  kRenderStrips128 = 5,
-  kRenderMixed = 6,
-  kRenderVariants = 7
-};
-void launch_render_fwd(const RenderArgs& a, hipStream_t s, int variant = kRender16x256);
+void launch_render_fwd(const RenderArgs& a, hipStream_t s);
 // Multi-view: order the a.num_tiles tiles by decreasing list length (a
 // binned estimate of their cost) so the longest start first.  bucket: one
 // byte per tile, hist: 512 words of scratch.
@@ -213,7 +216,7 @@ void launch_tile_order(const RenderArgs& a, uint32_t* order, uint8_t* bucket, ui
 // cost: the backward's exact list length.
 void launch_tile_order_bwd(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, hipStream_t s,
                            bool hist_zeroed = false);
-void launch_render_bwd(const RenderArgs& a, hipStream_t s, int variant = kRender16x256);
+void launch_render_bwd(const RenderArgs& a, hipStream_t s);
 
 // ---- geometry backward ----
 struct GeometryBwdArgs {

@@ -7,28 +7,32 @@
 // alpha = min(0.99, o exp(power)), skip if alpha < 1/255, stop (without
 // adding) once T (1 - alpha) < 1e-4, C += c alpha T; output C + T bg.
 //
-// Layout: a workgroup covers SUB x SUB pixels of a 16x16 binning tile (SUB =
-// 16: the whole tile with 4 wave64; SUB = 8: one wave64 per quarter tile, four
-// workgroups reading the same list).  Splat records are staged in LDS in
-// batches of BATCH with one 48-byte gather per record.  Every variant
-// evaluates each pixel in the same order, so they give identical images.
+// Forward (render_fwd_quads_kernel): one 256-lane work-group per 16x16 binning tile, each of its four waves
+// owning one 8x8 quadrant, one pixel per lane.  Backward (render_bwd_strips_kernel): one wave per tile, or per
+// kept segment of a tile's list, each lane owning four pixels.
 //
 // Backward: the list is walked from the back, starting at the largest
-// n_contrib of the workgroup (entries behind every pixel's last contributor
+// n_contrib of the tile (entries behind every pixel's last contributor
 // cannot contribute), transmittance is recomputed (times 1 / (1 - alpha), one
-// reciprocal) instead of being stored, and each wave reduces its 9 per-splat
-// partial gradients with DPP row sums into a per-batch LDS accumulator; the
-// workgroup flushes that accumulator with one global atomic per (splat,
-// value) per batch.
+// reciprocal) instead of being stored, and the wave sums its 9 per-splat
+// partial gradients into a per-batch LDS accumulator; the work-group flushes
+// that accumulator with one global atomic per (splat, value) per batch.
 //
 // Several views in one launch: a global tile id indexes the ranges; the view
 // table gives each tile's image size, background and packed output offset.
 //
-// Footprint skip: staging also stores the bounding box of the splat's
-// alpha >= 1/255 region, the ellipse  d^T Q d <= 2 ln(255 o)  (Q the conic),
-// widened by one pixel.  A wave whose 64 pixels all lie outside the box
-// skips the splat: no pixel of it could pass the alpha test, so skipping
-// changes nothing (the splat is still counted in the list positions).
+// Kept segments.  A lone wave takes 400 ns per (tile, splat) in the backward (a chain of dependent
+// operations), so a launch of few tiles with long lists (a 200x200 view: 169 tiles, up to 900 entries
+// walked) used to take as long as its longest list: 375 us.  A forward that will be followed by a backward
+// therefore keeps, every 64 members of a tile's list, the pixels' transmittance and the colour added since
+// the last boundary; at the end of the list it turns those colours into "the colour added behind this
+// boundary" (sums from the back, so that each has its own relative precision; the difference of two
+// running totals would lose it).  That is the whole state of the backward recursion at the boundary, so
+// every 64-member segment is a work-group of its own.  Slots (4 KB) come from a counter; a tile that gets
+// none has a longer last segment.  Launches of more than kSegmentTiles tiles fill the GPU without it.
+// Blend backward of one view, us, before and after (MI355X): 10k Gaussians at 200x200 375 -> 77, 1M at
+// 800x800 225 -> 107, 491k face-bound at 800x800 1385 -> 216, 500k at 333x251 1731 -> 177 (their forwards
+// get 7-45 us longer: the states are written, summed and cleared).
 #include "dmgs_common.h"
 #include "dmgs_kernels.h"
 
@@ -38,21 +42,47 @@ namespace dmgs {
 // from the conic scaled once per staged splat: q = log2(e) (-a/2, -b, -c/2).
 constexpr float kLog2e = 1.44269504088896341f;
 
-// Three 16-byte fields per staged splat, all indexed alike: one address
-// register serves every field of a splat (fixed offsets between them).
-template <int BATCH>
-struct SplatLDS {
-  float4 xym[BATCH];     // x, y, reach mask (bits, reach_mask), list position (bits)
-  float4 qo[BATCH];      // scaled conic q, opacity
-  float4 rgb_id[BATCH];  // r, g, b, id (bits)
+// A staged splat is three 16-byte fields, all indexed alike: one address register serves every field (fixed
+// offsets between them).  The two kernels pair the values differently: the forward reads whole fields (ten
+// values in two 16-byte reads and one of 8), the backward the narrow parts it needs next.
+struct StagedSplat {
+  float x, y;            // pixel position
+  float qx, qy, qz, o;   // scaled conic, opacity
+  float r, g, b;
+  uint32_t pos, mask, id;  // list position, reach mask (reach_mask), splat id
 };
-template <int BATCH>
-__device__ __forceinline__ uint32_t splat_mask(const SplatLDS<BATCH>& L, int j) {
-  return __float_as_uint(L.xym[j].z);
-}
-template <int BATCH>
-__device__ __forceinline__ uint32_t splat_pos(const SplatLDS<BATCH>& L, int j) {
-  return __float_as_uint(L.xym[j].w);
+template <int SLOTS>
+struct FwdSplats {
+  float4 xyq[SLOTS];   // x, y, q.x, q.y
+  float4 qorg[SLOTS];  // q.z, opacity, red, green
+  float4 bpmi[SLOTS];  // blue, position, mask, id
+  __device__ __forceinline__ void put(int j, const StagedSplat& s) {
+    xyq[j] = make_float4(s.x, s.y, s.qx, s.qy);
+    qorg[j] = make_float4(s.qz, s.o, s.r, s.g);
+    bpmi[j] = make_float4(s.b, __uint_as_float(s.pos), __uint_as_float(s.mask), __uint_as_float(s.id));
+  }
+  __device__ __forceinline__ uint32_t mask(int j) const { return __float_as_uint(bpmi[j].z); }
+  __device__ __forceinline__ uint32_t pos(int j) const { return __float_as_uint(bpmi[j].y); }
+};
+template <int SLOTS>
+struct BwdSplats {
+  float4 xym[SLOTS];     // x, y, mask, position
+  float4 qo[SLOTS];      // scaled conic, opacity
+  float4 rgb_id[SLOTS];  // r, g, b, id
+  __device__ __forceinline__ void put(int j, const StagedSplat& s) {
+    xym[j] = make_float4(s.x, s.y, __uint_as_float(s.mask), __uint_as_float(s.pos));
+    qo[j] = make_float4(s.qx, s.qy, s.qz, s.o);
+    rgb_id[j] = make_float4(s.r, s.g, s.b, __uint_as_float(s.id));
+  }
+  __device__ __forceinline__ uint32_t mask(int j) const { return __float_as_uint(xym[j].z); }
+  __device__ __forceinline__ uint32_t pos(int j) const { return __float_as_uint(xym[j].w); }
+  __device__ __forceinline__ uint32_t id(int j) const { return __float_as_uint(rgb_id[j].w); }
+};
+
+// The element of an LDS array at a byte offset.
+template <typename T, int N>
+__device__ __forceinline__ T lds_at(const T (&a)[N], uint32_t byte_offset) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(&a[0]) + byte_offset);
 }
 
 // Which pixel rectangles of the work-group a splat can reach.  A splat passes
@@ -63,9 +93,9 @@ __device__ __forceinline__ uint32_t splat_pos(const SplatLDS<BATCH>& L, int j) {
 // bit is clear: no pixel there could pass the alpha test, so results are
 // unchanged.  Margins (rectangle +0.01 px, tau x 1.001 + 0.001) keep the test
 // conservative against rounding.
-struct RowRects {  // n rectangles [x0, x1] x [y0 + k h, y0 + k h + h - 1]
-  float x0, x1, y0, h;
-  int n;
+struct PixelRects {  // n rectangles of w x h pixels, `cols` (1 or 2) to a row, the first at (x0, y0)
+  float x0, y0, w, h;
+  int cols, n;
 };
 
 // min over the rectangle of q(p - centre) <= tau, q(d) = a dx^2 + 2 b dx dy + c dy^2
@@ -94,15 +124,17 @@ __device__ __forceinline__ bool ellipse_meets_rect(float cx, float cy, float a, 
 }
 
 __device__ __forceinline__ uint32_t reach_mask(float cx, float cy, float a, float b, float c, float o,
-                                               const RowRects& rr) {
+                                               const PixelRects& rr) {
   const float tau = 2.0f * logf(255.0f * o);
   if (!(tau > 0.0f)) return 0u;  // o < 1/255: alpha never reaches the threshold
   if (!(a > 0.0f && c > 0.0f)) return 0xFu;
   const float t = tau * 1.001f + 0.001f, m = 0.01f;
   uint32_t mask = 0;
   for (int k = 0; k < rr.n; ++k) {
-    const float y0 = rr.y0 + (float)k * rr.h;
-    if (ellipse_meets_rect(cx, cy, a, b, c, t, rr.x0 - m, rr.x1 + m, y0 - m, y0 + rr.h - 1.0f + m)) mask |= 1u << k;
+    const int row = rr.cols == 2 ? k >> 1 : k, col = rr.cols == 2 ? k & 1 : 0;
+    const float x0 = rr.x0 + (float)col * rr.w, y0 = rr.y0 + (float)row * rr.h;
+    if (ellipse_meets_rect(cx, cy, a, b, c, t, x0 - m, x0 + rr.w - 1.0f + m, y0 - m, y0 + rr.h - 1.0f + m))
+      mask |= 1u << k;
   }
   return mask;
 }
@@ -116,8 +148,8 @@ __device__ __forceinline__ uint32_t reach_mask(float cx, float cy, float a, floa
 struct PowerDx {
   float xx, xy;  // q.x dx dx, q.y dx
 };
-__device__ __forceinline__ PowerDx power_dx(const float4& q, float dx) {
-  return {__fmul_rn(__fmul_rn(q.x, dx), dx), __fmul_rn(q.y, dx)};
+__device__ __forceinline__ PowerDx power_dx(float qx, float qy, float dx) {
+  return {__fmul_rn(__fmul_rn(qx, dx), dx), __fmul_rn(qy, dx)};
 }
 __device__ __forceinline__ float power_at(const PowerDx& d, float qz, float dy) {
   return fmaf(fmaf(qz, dy, d.xy), dy, d.xx);
@@ -126,41 +158,6 @@ __device__ __forceinline__ float power_at(const PowerDx& d, float qz, float dy) 
 __device__ __forceinline__ float splat_exp2(float p) { return __builtin_amdgcn_exp2f(p); }
 
 #define DMGS_DPP_ADD(v, ctrl) ((v) + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), (ctrl), 0xF, 0xF, true)))
-
-// Wave-uniform test of bit k of a staged mask (read once, scalar branch).
-__device__ __forceinline__ bool reaches(uint32_t mask_lds, int k) {
-  return (__builtin_amdgcn_readfirstlane(mask_lds) >> k) & 1u;
-}
-
-// Row sums of nine per-lane values over each 16-lane DPP row; row lane k < 9
-// returns the sum of value k.  Two reduce-scatter steps over lane bits 0 and
-// 1 (each lane keeps the half of the values its partner gives up: 3 VALU per
-// pair) leave lane m (m = lane & 3) the quad sums of values m and 4 + m;
-// value 8 takes plain butterfly steps; rotating the row by 4 and by 8 then
-// adds the four quads.  28 VALU instead of 54 for nine full row sums.
-__device__ __forceinline__ float row_sums9(const float (&v)[DMGS_GACC_USED], unsigned row_lane) {
-  const bool b0 = (row_lane & 1u) != 0u, b1 = (row_lane & 2u) != 0u;
-  float p[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {  // lanes l, l ^ 1: keep value 2i + b0
-    const float keep = b0 ? v[2 * i + 1] : v[2 * i];
-    const float give = b0 ? v[2 * i] : v[2 * i + 1];
-    p[i] = keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0xB1, 0xF, 0xF, true));
-  }
-  float e = DMGS_DPP_ADD(v[8], 0xB1);
-  float r[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {  // lanes l, l ^ 2: keep value 4i + 2 b1 + b0
-    const float keep = b1 ? p[2 * i + 1] : p[2 * i];
-    const float give = b1 ? p[2 * i] : p[2 * i + 1];
-    r[i] = keep + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(give), 0x4E, 0xF, 0xF, true));
-  }
-  e = DMGS_DPP_ADD(e, 0x4E);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) r[i] = DMGS_DPP_ADD(DMGS_DPP_ADD(r[i], 0x124), 0x128);  // row_ror 4, row_ror 8
-  e = DMGS_DPP_ADD(DMGS_DPP_ADD(e, 0x124), 0x128);
-  return row_lane < 4u ? r[0] : (row_lane < 8u ? r[1] : e);
-}
 
 // Sums over a one-wave work-group of nine per-lane values, through LDS: each
 // lane stores its values 0-7 (red[q][lane]); lane (row r, row position p)
@@ -254,24 +251,24 @@ __device__ __forceinline__ float grad_scale(int k, float ddelx_dx, float ddely_d
 __device__ __forceinline__ float dmean_x(const float4& q, float X, float Y) { return fmaf(q.x, X + X, q.y * Y); }
 __device__ __forceinline__ float dmean_y(const float4& q, float X, float Y) { return fmaf(q.z, Y + Y, q.y * X); }
 
-template <int BATCH>
-__device__ __forceinline__ void stage_splat(SplatLDS<BATCH>& L, int slot, const float4* __restrict__ splats,
-                                            uint32_t id, uint32_t P, const RowRects& rr, uint32_t pos) {
-  if (id >= P) {  // cannot happen for lists built by the binning step; a zero-opacity entry never contributes
-    L.xym[slot] = make_float4(0.f, 0.f, __uint_as_float(0u), __uint_as_float(pos));
-    L.qo[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
-    L.rgb_id[slot] = make_float4(0.f, 0.f, 0.f, __uint_as_float(0u));
-    return;
+// Stages a splat record (s0, s1, s2) of the list position `pos`.
+template <typename L>
+__device__ __forceinline__ void put_splat(L& lds, int slot, float4 s0, float4 s1, float4 s2, uint32_t id, uint32_t P,
+                                          const PixelRects& rr, uint32_t pos) {
+  StagedSplat t{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, pos, 0u, 0u};
+  if (id < P) {  // always, for lists built by the binning step; a zero-opacity splat never contributes
+    constexpr float kHalf = -0.5f * kLog2e;
+    t = {s0.x, s0.y, kHalf * s0.z, -kLog2e * s0.w, kHalf * s1.x, s1.y, s1.z, s1.w, s2.x, pos,
+         reach_mask(s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, rr), id};
   }
-  const float4* sp = splats + (size_t)DMGS_SPLAT_F4 * id;
-  const float4 s0 = sp[0];
-  const float4 s1 = sp[1];
-  const float4 s2 = sp[2];
-  constexpr float kHalf = -0.5f * kLog2e;
-  const uint32_t mask = reach_mask(s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, rr);
-  L.xym[slot] = make_float4(s0.x, s0.y, __uint_as_float(mask), __uint_as_float(pos));
-  L.qo[slot] = make_float4(kHalf * s0.z, -kLog2e * s0.w, kHalf * s1.x, s1.y);
-  L.rgb_id[slot] = make_float4(s1.z, s1.w, s2.x, __uint_as_float(id));
+  lds.put(slot, t);
+}
+
+template <typename L>
+__device__ __forceinline__ void stage_splat(L& lds, int slot, const float4* __restrict__ splats, uint32_t id,
+                                            uint32_t P, const PixelRects& rr, uint32_t pos) {
+  const float4* sp = splats + (size_t)DMGS_SPLAT_F4 * min(id, P - 1);
+  put_splat(lds, slot, sp[0], sp[1], sp[2], id, P, rr, pos);
 }
 
 // Everything a workgroup needs to know about its pixels.
@@ -286,20 +283,24 @@ struct TileCtx {
   float bg0, bg1, bg2;
   uint32_t bit;        // multi-view: this tile's bit in its cell's key masks
   uint2 range;         // single view: the tile's list; multi-view: its cell's list
-  RowRects rows;       // the work-group's pixel rectangles: 16x4 strips (SUB 16) or the 8x8 block
+  PixelRects rows;     // the work-group's pixel rectangles: 8x8 quadrants or 16x4 strips
 };
 
-template <int SUB>
-__device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a) {
-  constexpr int Q = DMGS_BLOCK_X / SUB;  // workgroups per tile edge
-  TileCtx c;
-  const int slot = blockIdx.x / (Q * Q);
-  const int q = blockIdx.x - slot * Q * Q;
-  c.tile = slot;
-  if (a.tile_order) {  // a stale or unset order entry falls back to the identity
+// The tile in dispatch slot `slot`; a stale or unset order entry falls back to the identity.
+__device__ __forceinline__ int ordered_tile(const RenderArgs& a, int slot) {
+  if (a.tile_order) {
     const uint32_t t = a.tile_order[slot];
-    if (t < (uint32_t)a.num_tiles) c.tile = (int)t;
+    if (t < (uint32_t)a.num_tiles) return (int)t;
   }
+  return slot;
+}
+
+// QUADS (256 lanes): wave k covers the 8x8 quadrant k (k & 1: right, k >> 1: lower); otherwise (64 lanes) a
+// lane's first pixel is in the tile's top 16x4 strip.
+template <bool QUADS>
+__device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile) {
+  TileCtx c;
+  c.tile = tile;
   int lt = c.tile, gx = a.grid_x;
   int64_t pbase = 0;
   int list = c.tile;
@@ -326,17 +327,22 @@ __device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a) {
     c.bg2 = a.bg[2];
   }
   const int tx = lt % gx, ty = lt / gx;
-  const int lx = threadIdx.x % SUB, ly = threadIdx.x / SUB;
-  const int ox = tx * DMGS_BLOCK_X + (q % Q) * SUB, oy = ty * DMGS_BLOCK_Y + (q / Q) * SUB;
+  int lx = threadIdx.x % DMGS_BLOCK_X, ly = threadIdx.x / DMGS_BLOCK_X;
+  if constexpr (QUADS) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    lx = (wave & 1) * 8 + (lane & 7);
+    ly = (wave >> 1) * 8 + (lane >> 3);
+  }
+  const int ox = tx * DMGS_BLOCK_X, oy = ty * DMGS_BLOCK_Y;
   c.px = ox + lx;
   c.py = oy + ly;
-  // rectangle k: the rows one wave covers in a 256-lane work-group (= strip k
-  // of a one-wave-per-tile work-group), or the whole 8x8 block
+  // rectangle k: quadrant k, or 16x4 strip k
   c.rows.x0 = (float)ox;
-  c.rows.x1 = (float)(ox + SUB - 1);
   c.rows.y0 = (float)oy;
-  c.rows.h = SUB == 16 ? 4.0f : 8.0f;
-  c.rows.n = SUB == 16 ? 4 : 1;
+  c.rows.w = QUADS ? 8.0f : 16.0f;
+  c.rows.h = QUADS ? 8.0f : 4.0f;
+  c.rows.cols = QUADS ? 2 : 1;
+  c.rows.n = 4;
   c.inside = c.px < c.W && c.py < c.H;
   c.plane = (size_t)c.W * c.H;
   c.pix = (size_t)pbase + (size_t)c.py * c.W + c.px;
@@ -353,6 +359,7 @@ __device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a) {
 // A forward work-group's share of clearing the backward accumulator: run
 // after its blend work, so the stores delay no load of the blend.
 __device__ __forceinline__ void clear_share(const RenderArgs& a) {
+  if (a.seg.head && a.seg.len == 0 && blockIdx.x == 0 && threadIdx.x < 2) a.seg.head[threadIdx.x] = 0u;
   if (a.clear_words && blockIdx.x == 0)
     for (int i = threadIdx.x; i < a.clear_words_n; i += blockDim.x) a.clear_words[i] = 0u;
   if (!a.clear) return;
@@ -361,27 +368,21 @@ __device__ __forceinline__ void clear_share(const RenderArgs& a) {
   for (size_t i = lo + threadIdx.x; i < hi; i += blockDim.x) a.clear[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Stage the next instances of this tile from its cell list (multi-view):
-// visit list positions from `cursor` — forward: cursor, cursor+1, ... below
-// limit; backward: cursor-1, cursor-2, ... down to 0 — min(NT, BATCH) at a
-// time and keep those whose key holds this tile's bit, in visit order, while
-// another chunk surely fits in the BATCH slots; then stage the kept records
-// in one pass, one lane per record (the footprint test then runs once per
-// NT records instead of once per chunk visited).  Advances cursor; returns
-// the number staged (workgroup-uniform); ends with a barrier.  Each staged
-// record carries its list position.
-template <int NT, bool BACKWARD, int BATCH>
-__device__ __forceinline__ int stage_cell_batch(SplatLDS<BATCH>& L, uint32_t* s_wc,
-                                                const RenderArgs& a, const TileCtx& c, int& cursor, int limit) {
-  constexpr int NW = NT / DMGS_WAVE;
-  constexpr int CH = NT < BATCH ? NT : BATCH;  // positions per chunk
-  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// Stage the next instances of this tile from its cell list, back to front (one wave): visit the list
+// positions cursor-1, cursor-2, ... down to lo, 64 at a time, and keep those whose key holds this tile's
+// bit, in visit order, while another chunk surely fits in the BATCH slots; then stage the kept records in
+// one pass, one lane per record (the footprint test then runs once per 64 records instead of once per
+// chunk visited).  Moves cursor down; returns the number staged; ends with a barrier.
+template <int BATCH>
+__device__ __forceinline__ int stage_cell_batch(BwdSplats<BATCH>& L, const RenderArgs& a, const TileCtx& c, int& cursor,
+                                                int lo) {
+  constexpr int CH = DMGS_WAVE < BATCH ? DMGS_WAVE : BATCH;  // positions per chunk
   const uint64_t lt = lanemask_lt();
   int run = 0;
   do {
     const int s = (int)threadIdx.x;
-    const int q = BACKWARD ? cursor - 1 - s : cursor + s;
-    const bool valid = s < CH && (BACKWARD ? q >= 0 : q < limit);
+    const int q = cursor - 1 - s;
+    const bool valid = s < CH && q >= lo;
     // The entry id is requested with the key, both without a branch (lanes
     // past the list read its first entry and ignore it): one memory round
     // trip, not two.
@@ -390,31 +391,16 @@ __device__ __forceinline__ int stage_cell_batch(SplatLDS<BATCH>& L, uint32_t* s_
     const uint32_t id = a.point_list[at];
     const bool member = valid && ((key >> DMGS_CELL_KEY_BITS) & c.bit);
     const uint64_t bal = __ballot(member);
-    int before = run, total;
-    if constexpr (NW == 1) {
-      total = (int)__popcll(bal);
-    } else {
-      if (lane == 0) s_wc[wave] = (uint32_t)__popcll(bal);
-      __syncthreads();
-      total = 0;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) {
-        const int cnt = (int)s_wc[w];
-        before += (w < (int)wave) ? cnt : 0;
-        total += cnt;
-      }
-    }
     if (member) {
-      const int slot = before + (int)__popcll(bal & lt);
+      const int slot = run + (int)__popcll(bal & lt);
       // id and position wait in the record for the staging pass
       L.xym[slot] = make_float4(0.f, 0.f, __uint_as_float(id), __uint_as_float((uint32_t)q));
     }
-    run += total;
-    cursor = BACKWARD ? cursor - CH : cursor + CH;
-    if constexpr (NW > 1) __syncthreads();  // s_wc is rewritten by the next chunk
-  } while (run + CH <= BATCH && (BACKWARD ? cursor > 0 : cursor < limit));
+    run += (int)__popcll(bal);
+    cursor -= CH;
+  } while (run + CH <= BATCH && cursor > lo);
   __syncthreads();
-  for (int s = (int)threadIdx.x; s < run; s += NT) {
+  for (int s = (int)threadIdx.x; s < run; s += DMGS_WAVE) {
     const float4 t = L.xym[s];
     stage_splat(L, s, a.splats, __float_as_uint(t.z), a.P, c.rows, __float_as_uint(t.w));
   }
@@ -422,334 +408,255 @@ __device__ __forceinline__ int stage_cell_batch(SplatLDS<BATCH>& L, uint32_t* s_
   return run;
 }
 
-template <int SUB, int BATCH>
-__global__ __launch_bounds__(SUB* SUB) void render_fwd_kernel(RenderArgs a) {
-  constexpr int NT = SUB * SUB;
-  __shared__ SplatLDS<BATCH> L;
-  const TileCtx c = tile_ctx<SUB>(a);
-  const float pxf = (float)c.px, pyf = (float)c.py;
-  const int todo_total = (int)(c.range.y - c.range.x);
-  const int rounds = (todo_total + BATCH - 1) / BATCH;
+// A group of four staged splats in registers, and the LDS byte offsets of the next group's.
+struct FwdGroup {
+  static constexpr int kN = 4;
+  uint4 at;
+  float4 xyq[kN], qorg[kN];
+};
 
-  bool done = !c.inside;
-  float T = 1.0f;
+// One list position per lane of a 256-lane work-group: the members of the tile (every position of a
+// single view's list; the instances of a cell list whose mask holds the tile's bit) are packed, in list
+// order, into id[] / pos[].
+struct MemberList {
+  uint32_t id[256], pos[256];
+};
+
+// Forward: four waves per 16x16 tile, one pixel per lane, wave k covering the 8x8 quadrant k.  VALU issue
+// bounds it where tiles are many, and one wave's own instruction stream where they are few (a wave issues
+// one instruction in four cycles at best, 190 cycles per splat measured), so the loop is made of as few
+// instructions of any kind as possible: each wave first packs the LDS offsets of the staged splats that reach
+// its quadrant, then takes four at a time, reading the next four while it evaluates the four alphas (whose
+// latencies overlap) and applies them in order with selects instead of branches.  Against one wave per tile
+// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 310 us, 16 uneven views of 3M
+// 5.33 -> 4.21 ms, one 800x800 view 154 -> 53 us, 333x251 of 500k 1377 -> 364 us.  Quadrants because a splat
+// reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on KEEP,
+// CELLS or the launch.
+template <bool CELLS, bool KEEP>
+__global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
+  constexpr int NT = 256, U = FwdGroup::kN;
+  constexpr int G = KEEP ? 64 : NT;  // staged splats blended per round
+  constexpr int kPad = NT * 16;      // offset of the filling splat
+  __shared__ FwdSplats<NT + 1> L;    // slot NT: a splat of zero opacity, which fills up groups
+  __shared__ MemberList M;
+  __shared__ uint32_t s_wc[2][NT / DMGS_WAVE];
+  __shared__ uint32_t s_slot[KEEP ? kTileSegments : 1];
+  __shared__ __align__(16) uint32_t s_reach[NT / DMGS_WAVE][G + 12];
+  const TileCtx c = tile_ctx<true>(a, ordered_tile(a, blockIdx.x));
+  const float pxf = (float)c.px, pyf = (float)c.py;
+  const int len = (int)(c.range.y - c.range.x);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int seg_pixel = ((wave >> 1) * 8 + (lane >> 3)) * 16 + (wave & 1) * 8 + (lane & 7);  // row-major in the tile
+  if (threadIdx.x == 0) L.xyq[NT] = L.qorg[NT] = L.bpmi[NT] = make_float4(0.f, 0.f, 0.f, 0.f);
+  // T > 0 while the pixel blends; a finished pixel (saturated, or outside the image) keeps -T
+  float T = c.inside ? 1.0f : -1.0f;
   float C0 = 0.f, C1 = 0.f, C2 = 0.f;
   uint32_t last_contributor = 0;
-  const int my_rect = SUB == 16 ? (int)(threadIdx.x >> 6) : 0;  // this wave's rectangle in the reach masks
+  // kept segments (see Segments): D is the colour added since the last boundary
+  float D0 = 0.f, D1 = 0.f, D2 = 0.f;
+  int seg_begin = 0, seg_members = 0, segs = 0;
 
-  for (int r = 0; r < rounds; ++r) {
-    if (__syncthreads_count(done) == NT) break;
-    for (int s = threadIdx.x; s < BATCH; s += NT) {
-      const int pos = r * BATCH + s;
-      if (pos < todo_total) stage_splat(L, s, a.splats, a.point_list[c.range.x + pos], a.P, c.rows, (uint32_t)pos);
-    }
+  // The list is taken 256 positions at a time, in three overlapping steps: the keys and ids of one chunk
+  // are on their way while the records of the chunk before it are, and while the one before that is blended.
+  uint32_t key = 0, id = 0;
+  auto request = [&](int at) {  // positions past the list read its first entry and are no members
+    const uint32_t p = c.range.x + (at + (int)threadIdx.x < len ? (uint32_t)(at + (int)threadIdx.x) : 0u);
+    if constexpr (CELLS) key = a.list_keys[p];
+    id = a.point_list[p];
+  };
+  // packs the chunk at `at`; returns the number of members (the barrier that follows is the caller's)
+  int flip = 0;
+  auto pack = [&](int at) {
+    const int q = at + (int)threadIdx.x;
+    const bool member = q < len && (!CELLS || ((key >> DMGS_CELL_KEY_BITS) & c.bit));
+    const uint64_t bal = __ballot(member);
+    if (lane == 0) s_wc[flip][wave] = (uint32_t)__popcll(bal);
     __syncthreads();
-    const int n = min(BATCH, todo_total - r * BATCH);
-    for (int j = 0; !done && j < n; ++j) {
-      if (!reaches(splat_mask(L, j), my_rect)) continue;
-      const uint32_t contributor = (uint32_t)(r * BATCH + j + 1);
-      const float2 xy = make_float2(L.xym[j].x, L.xym[j].y);
-      const float4 q = L.qo[j];
-      const float dx = xy.x - pxf, dy = xy.y - pyf;
-      const float p = power_at(power_dx(q, dx), q.z, dy);
-      if (p > 0.0f) continue;
-      const float alpha = fminf(0.99f, q.w * splat_exp2(p));
-      if (alpha < 1.0f / 255.0f) continue;
-      const float test_T = T * (1.0f - alpha);
-      if (test_T < 0.0001f) {
-        done = true;
-        continue;
+    int before = (int)__popcll(bal & lanemask_lt()), total = 0;
+#pragma unroll
+    for (int w = 0; w < NT / DMGS_WAVE; ++w) {
+      const int cnt = (int)s_wc[flip][w];
+      before += w < wave ? cnt : 0;
+      total += cnt;
+    }
+    flip ^= 1;
+    if (member) {
+      M.id[before] = id;
+      M.pos[before] = (uint32_t)q;
+    }
+    return total;
+  };
+  float4 r0, r1, r2;  // this lane's record of the packed chunk
+  uint32_t my_id = 0, my_pos = 0;
+  auto gather = [&](int n) {
+    const int s = min((int)threadIdx.x, max(n - 1, 0));  // no lane's loads are conditional
+    my_id = M.id[s];
+    my_pos = M.pos[s];
+    const float4* sp = a.splats + (size_t)DMGS_SPLAT_F4 * min(my_id, a.P - 1);
+    r0 = sp[0];
+    r1 = sp[1];
+    r2 = sp[2];
+  };
+  int n_next = 0;  // members of the chunk whose records are on their way
+  if (len > 0) {
+    request(0);
+    n_next = pack(0);
+    __syncthreads();
+    gather(n_next);
+    request(NT);
+  }
+  for (int at = 0; at < len; at += NT) {
+    if (__syncthreads_count(T < 0.f) == NT) break;
+    const int n = n_next;
+    if ((int)threadIdx.x < n) put_splat(L, threadIdx.x, r0, r1, r2, my_id, a.P, c.rows, my_pos + 1);
+    n_next = pack(at + NT);  // its barrier also orders the records; no members past the list
+    __syncthreads();
+    gather(n_next);
+    request(at + 2 * NT);
+    if constexpr (KEEP) {
+      // segment boundaries inside this chunk: before a round, once enough members have passed
+      int want = 0, m = seg_members;
+      for (int h = 0; h < n; h += G) {
+        if (m >= a.seg.len) ++want, m = 0;
+        m += min(G, n - h);
       }
-      const float4 col = L.rgb_id[j];
-      const float w = alpha * T;
-      C0 += col.x * w;
-      C1 += col.y * w;
-      C2 += col.z * w;
-      T = test_T;
-      last_contributor = contributor;
+      want = min(want, kTileSegments - segs);
+      if (want > 0) {
+        if (threadIdx.x == 0) {
+          const uint32_t first = atomicAdd(a.seg.head, (uint32_t)want);
+          for (int k = 0; k < want; ++k) s_slot[segs + k] = first + k < (uint32_t)a.seg.cap ? first + k : kNoSegment;
+        }
+        __syncthreads();
+      }
+    }
+    for (int h = 0; h < NT; h += G) {
+      if (h >= n) break;
+      if constexpr (KEEP) {
+        if (seg_members >= a.seg.len && segs < kTileSegments) {
+          const uint32_t slot = s_slot[segs];
+          const int end = (int)L.pos(h) - 1;
+          if (slot != kNoSegment) {
+            a.seg.state[(size_t)slot * 256 + seg_pixel] = make_float4(fabsf(T), D0, D1, D2);
+            D0 = D1 = D2 = 0.f;
+            if (threadIdx.x == 0) a.seg.rec[slot] = make_uint4((uint32_t)c.tile, (uint32_t)seg_begin, (uint32_t)end, 0u);
+            ++segs;
+            seg_begin = end;
+            seg_members = 0;
+          } else {
+            seg_members = -0x40000000;  // no slots left: the rest of the list is one segment
+          }
+        }
+        seg_members += min(G, n - h);
+      }
+      if (__ballot(T > 0.f) == 0) continue;  // wave-uniform: this quadrant is finished
+      // the round's splats that reach this quadrant, as LDS offsets in list order, filled up for whole groups
+      // and for the two groups read ahead
+      uint32_t* const reach = s_reach[wave];
+      int count = 0;
+#pragma unroll
+      for (int k = 0; k < G; k += 64) {
+        const int s = h + k + lane;
+        const uint64_t bits = __ballot(s < n && ((L.mask(min(s, NT)) >> wave) & 1u));
+        if ((bits >> lane) & 1u) reach[count + (int)__popcll(bits & lanemask_lt())] = (uint32_t)s * 16u;
+        count += (int)__popcll(bits);
+      }
+      if (count == 0) continue;
+      if (lane < 12) reach[count + lane] = kPad;
+      auto fetch = [&](FwdGroup& g, const uint4& at, int next) {
+        const uint32_t o[U] = {at.x, at.y, at.z, at.w};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          g.xyq[u] = lds_at(L.xyq, o[u]);
+          g.qorg[u] = lds_at(L.qorg, o[u]);
+        }
+        g.at = *reinterpret_cast<const uint4*>(reach + next);
+      };
+      // blends `cur` (at the offsets `at`) while `next` is on its way; false when nothing is left to do
+      int done = 0;
+      auto step = [&](FwdGroup& cur, uint4& at, FwdGroup& next) {
+        const uint32_t o[U] = {at.x, at.y, at.z, at.w};
+        float4 bp[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) bp[u] = lds_at(L.bpmi, o[u]);
+        fetch(next, cur.at, done + 2 * U);
+        at = cur.at;
+        float alpha[U];
+        bool ok[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {  // independent of each other: their latencies overlap
+          const float p = power_at(power_dx(cur.xyq[u].z, cur.xyq[u].w, cur.xyq[u].x - pxf), cur.qorg[u].x, cur.xyq[u].y - pyf);
+          const float al = fminf(0.99f, cur.qorg[u].y * splat_exp2(p));
+          ok[u] = (p <= 0.0f) & (al >= 1.0f / 255.0f);
+          alpha[u] = ok[u] ? al : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const float test_T = T * (1.0f - alpha[u]);  // T itself where the splat is skipped
+          const bool take = test_T >= 0.0001f;         // never for a finished pixel
+          const float w = take ? alpha[u] * T : 0.0f;
+          C0 = fmaf(cur.qorg[u].z, w, C0);
+          C1 = fmaf(cur.qorg[u].w, w, C1);
+          C2 = fmaf(bp[u].x, w, C2);
+          if constexpr (KEEP) {
+            D0 = fmaf(cur.qorg[u].z, w, D0);
+            D1 = fmaf(cur.qorg[u].w, w, D1);
+            D2 = fmaf(bp[u].x, w, D2);
+          }
+          T = take ? test_T : -fabsf(T);
+          last_contributor = (take & ok[u]) ? __float_as_uint(bp[u].y) : last_contributor;
+        }
+        done += U;
+        return done < count && __ballot(T > 0.f) != 0;
+      };
+      FwdGroup g0, g1;
+      uint4 at_now = *reinterpret_cast<const uint4*>(reach);
+      fetch(g0, at_now, U);
+      while (step(g0, at_now, g1) && step(g1, at_now, g0)) {
+      }
     }
   }
-  if (c.inside) {
-    const size_t pid = c.pix - c.img / 3;  // pixel index within the view
-    a.final_T[c.pix] = T;
-    a.n_contrib[c.pix] = last_contributor;
-    float* out = a.out_color + c.img;
-    out[pid] = C0 + T * c.bg0;
-    out[c.plane + pid] = C1 + T * c.bg1;
-    out[2 * c.plane + pid] = C2 + T * c.bg2;
-  }
-  clear_share(a);
-}
-
-// Forward over cell lists (multi-view).  Same per-pixel arithmetic and order
-// as render_fwd_kernel; the per-pixel "last contributor" is one past the
-// list position of the last contributing instance.
-template <int SUB, int BATCH>
-__global__ __launch_bounds__(SUB* SUB) void render_fwd_cells_kernel(RenderArgs a) {
-  constexpr int NT = SUB * SUB;
-  __shared__ SplatLDS<BATCH> L;
-  __shared__ uint32_t s_wc[NT / DMGS_WAVE];
-  const TileCtx c = tile_ctx<SUB>(a);
-  const float pxf = (float)c.px, pyf = (float)c.py;
-  const int len = (int)(c.range.y - c.range.x);
-
-  bool done = !c.inside;
-  float T = 1.0f;
-  float C0 = 0.f, C1 = 0.f, C2 = 0.f;
-  uint32_t last_contributor = 0;
-  const int my_rect = SUB == 16 ? (int)(threadIdx.x >> 6) : 0;  // this wave's rectangle in the reach masks
-
-  int cursor = 0;
-  while (cursor < len) {
-    if (__syncthreads_count(done) == NT) break;
-    const int n = stage_cell_batch<NT, false>(L, s_wc, a, c, cursor, len);
-    for (int j = 0; !done && j < n; ++j) {
-      if (!reaches(splat_mask(L, j), my_rect)) continue;
-      const float2 xy = make_float2(L.xym[j].x, L.xym[j].y);
-      const float4 q = L.qo[j];
-      const float dx = xy.x - pxf, dy = xy.y - pyf;
-      const float p = power_at(power_dx(q, dx), q.z, dy);
-      if (p > 0.0f) continue;
-      const float alpha = fminf(0.99f, q.w * splat_exp2(p));
-      if (alpha < 1.0f / 255.0f) continue;
-      const float test_T = T * (1.0f - alpha);
-      if (test_T < 0.0001f) {
-        done = true;
-        continue;
-      }
-      const float4 col = L.rgb_id[j];
-      const float w = alpha * T;
-      C0 += col.x * w;
-      C1 += col.y * w;
-      C2 += col.z * w;
-      T = test_T;
-      last_contributor = splat_pos(L, j) + 1;
-    }
-  }
-  if (c.inside) {
-    const size_t pid = c.pix - c.img / 3;
-    a.final_T[c.pix] = T;
-    a.n_contrib[c.pix] = last_contributor;
-    float* out = a.out_color + c.img;
-    out[pid] = C0 + T * c.bg0;
-    out[c.plane + pid] = C1 + T * c.bg1;
-    out[2 * c.plane + pid] = C2 + T * c.bg2;
-  }
-  clear_share(a);
-}
-
-// Forward with one wave per 16x16 tile (the layout of the strip backward):
-// lane (lx, ly) owns the pixels (lx, ly + 4k), one per 16x4 strip.  Each
-// staged splat is read from LDS once per wave for four pixels; a strip is
-// skipped when the splat's footprint misses it or all its pixels are done.
-// Per pixel the arithmetic and order are render_fwd_kernel's.
-template <int BATCH, bool CELLS>
-__global__ __launch_bounds__(64) void render_fwd_strips_kernel(RenderArgs a) {
-  constexpr int NT = 64;
-  __shared__ SplatLDS<BATCH> L;
-  __shared__ uint32_t s_wc[1];
-  const TileCtx c = tile_ctx<16>(a);
-  const float pxf = (float)c.px;
-  const int len = (int)(c.range.y - c.range.x);
-  float pyf[4];
+  if constexpr (KEEP) {
+    __syncthreads();
+    if (threadIdx.x == 0) a.seg.tile_last[c.tile] = (uint32_t)seg_begin;
+    // a segment's backward starts from the colour behind it: sum the segments' colours from the back
+    for (int i = segs; i > 0; i -= 8) {
+      float4* at[8];
+      float4 e[8];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) pyf[k] = (float)(c.py + 4 * k);
-  // T > 0 while a pixel blends; a finished pixel (saturated, or outside the
-  // image) keeps -T, so one compare tells both
-  float T[4], C0[4], C1[4], C2[4];
-  uint32_t last_contributor[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    T[k] = (c.px < c.W && c.py + 4 * k < c.H) ? 1.0f : -1.0f;
-    C0[k] = C1[k] = C2[k] = 0.f;
-    last_contributor[k] = 0;
-  }
-  int cursor = 0;
-  while (cursor < len) {
-    if (__syncthreads_count(T[0] < 0.f && T[1] < 0.f && T[2] < 0.f && T[3] < 0.f) == NT) break;
-    const int base = cursor;
-    int n;
-    if constexpr (CELLS) {
-      n = stage_cell_batch<NT, false>(L, s_wc, a, c, cursor, len);
-    } else {
-      for (int s = threadIdx.x; s < BATCH; s += NT) {
-        const int pos = base + s;
-        if (pos < len) stage_splat(L, s, a.splats, a.point_list[c.range.x + pos], a.P, c.rows, (uint32_t)pos);
+      for (int k = 0; k < 8; ++k) {  // all loads in flight (past the front: the front's, not used)
+        at[k] = a.seg.state + (size_t)s_slot[max(i - 1 - k, 0)] * 256 + seg_pixel;
+        e[k] = *at[k];
       }
-      __syncthreads();
-      n = min(BATCH, len - base);
-      cursor += n;
-    }
-    uint32_t mask_next = n > 0 ? splat_mask(L, 0) : 0u;  // read one splat ahead
-    for (int j = 0; j < n; ++j) {
-      const uint32_t reach = __builtin_amdgcn_readfirstlane(mask_next);
-      if (j + 1 < n) mask_next = splat_mask(L, j + 1);
-      if (reach == 0u) continue;
-      const float2 xy = make_float2(L.xym[j].x, L.xym[j].y);
-      const float4 q = L.qo[j];
-      uint32_t position;
-      if constexpr (CELLS) {
-        position = splat_pos(L, j);
-      } else {
-        position = (uint32_t)(base + j);
-      }
-      const PowerDx pd = power_dx(q, xy.x - pxf);  // shared by the lane's four pixels (one column)
-      const float4 col = L.rgb_id[j];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (!((reach >> k) & 1u) || __ballot(T[k] > 0.f) == 0) continue;  // wave-uniform
-        // the per-pixel tests become selects: no branch per pixel and splat; a
-        // skipped splat adds colour x 0 (exact) and keeps T
-        const float p = power_at(pd, q.z, xy.y - pyf[k]);
-        const float alpha = fminf(0.99f, q.w * splat_exp2(p));
-        const float test_T = T[k] * (1.0f - alpha);
-        const bool ok = T[k] > 0.f && p <= 0.0f && alpha >= 1.0f / 255.0f;
-        const bool stop = ok && test_T < 0.0001f;
-        const bool take = ok && !stop;
-        const float w = take ? alpha * T[k] : 0.0f;
-        C0[k] = fmaf(col.x, w, C0[k]);
-        C1[k] = fmaf(col.y, w, C1[k]);
-        C2[k] = fmaf(col.z, w, C2[k]);
-        T[k] = take ? test_T : (stop ? -T[k] : T[k]);
-        last_contributor[k] = take ? position + 1 : last_contributor[k];
+      for (int k = 0; k < 8; ++k) {
+        if (k >= i) break;
+        *at[k] = make_float4(e[k].x, D0, D1, D2);
+        D0 += e[k].y;
+        D1 += e[k].z;
+        D2 += e[k].w;
       }
     }
   }
   if (a.tile_work) {  // the backward walks list positions below the tile's largest last contributor
-    uint32_t m = max(max(last_contributor[0], last_contributor[1]), max(last_contributor[2], last_contributor[3]));
+    __shared__ uint32_t s_max[NT / DMGS_WAVE];
+    uint32_t m = last_contributor;
     for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-    if (threadIdx.x == 0) a.tile_work[c.tile] = m;
+    if (lane == 0) s_max[wave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) a.tile_work[c.tile] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
   }
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    if (!(c.px < c.W && c.py + 4 * k < c.H)) continue;
-    const size_t pix = c.pix + (size_t)(4 * k) * c.W;
-    const size_t pid = pix - c.img / 3;
-    const float Tk = fabsf(T[k]);
-    a.final_T[pix] = Tk;
-    a.n_contrib[pix] = last_contributor[k];
+  if (c.inside) {
+    const size_t pid = c.pix - c.img / 3;  // pixel index within the view
+    T = fabsf(T);
+    a.final_T[c.pix] = T;
+    a.n_contrib[c.pix] = last_contributor;
     float* out = a.out_color + c.img;
-    out[pid] = C0[k] + Tk * c.bg0;
-    out[c.plane + pid] = C1[k] + Tk * c.bg1;
-    out[2 * c.plane + pid] = C2[k] + Tk * c.bg2;
+    out[pid] = C0 + T * c.bg0;
+    out[c.plane + pid] = C1 + T * c.bg1;
+    out[2 * c.plane + pid] = C2 + T * c.bg2;
   }
   clear_share(a);
-}
-
-// Backward.  CELLS: the lists are cell lists (multi-view); positions replace
-// the per-tile counter and the staging keeps only this tile's instances.
-template <int SUB, int BATCH, bool CELLS>
-__global__ __launch_bounds__(SUB* SUB) void render_bwd_kernel(RenderArgs a) {
-  constexpr int NT = SUB * SUB;
-  constexpr int NW = NT / DMGS_WAVE;
-  __shared__ SplatLDS<BATCH> L;
-  __shared__ uint32_t s_max[NW];
-  __shared__ float s_acc[BATCH][DMGS_GACC_USED];
-  __shared__ uint32_t s_wc[NW];
-  const TileCtx c = tile_ctx<SUB>(a);
-  const float pxf = (float)c.px, pyf = (float)c.py;
-  const unsigned lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-
-  float T_final = 0.f, g0 = 0.f, g1 = 0.f, g2 = 0.f;
-  uint32_t last_contributor = 0;
-  if (c.inside) {
-    const size_t pid = c.pix - c.img / 3;
-    const float* dp = a.dL_dpix + c.img;
-    T_final = a.final_T[c.pix];
-    last_contributor = a.n_contrib[c.pix];
-    g0 = dp[pid];
-    g1 = dp[c.plane + pid];
-    g2 = dp[2 * c.plane + pid];
-  }
-  const float bg_term = -T_final * (c.bg0 * g0 + c.bg1 * g1 + c.bg2 * g2);  // -T_final <bg, dL/dpixel>
-  const float ddelx_dx = 0.5f * (float)c.W, ddely_dy = 0.5f * (float)c.H;  // d pixel / d NDC
-
-  // Entries at list positions >= max(last contributor) of the workgroup contribute nothing.
-  uint32_t m = last_contributor;
-  for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-  if (lane == 0) s_max[wave] = m;
-  __syncthreads();
-  uint32_t tile_max = 0;
-  for (int w = 0; w < NW; ++w) tile_max = max(tile_max, s_max[w]);
-  const int todo_total = min((int)(c.range.y - c.range.x), (int)tile_max);
-
-  BwdPixel st = bwd_pixel(T_final);
-  const unsigned row_lane = lane & 15;  // lane within its DPP row of 16
-  const int my_rect = SUB == 16 ? (int)(threadIdx.x >> 6) : 0;  // this wave's rectangle in the reach masks
-  int cursor = todo_total;  // list positions below cursor are still to do
-  while (cursor > 0) {
-    __syncthreads();
-    const int top = cursor;
-    int n;
-    if constexpr (CELLS) {
-      for (int s = threadIdx.x; s < BATCH; s += NT) {
-#pragma unroll
-        for (int k = 0; k < DMGS_GACC_USED; ++k) s_acc[s][k] = 0.f;
-      }
-      n = stage_cell_batch<NT, true>(L, s_wc, a, c, cursor, 0);
-    } else {
-      for (int s = threadIdx.x; s < BATCH; s += NT) {
-        const int pos = top - 1 - s;
-        if (pos >= 0) stage_splat(L, s, a.splats, a.point_list[c.range.x + pos], a.P, c.rows, (uint32_t)pos);
-#pragma unroll
-        for (int k = 0; k < DMGS_GACC_USED; ++k) s_acc[s][k] = 0.f;
-      }
-      __syncthreads();
-      n = min(BATCH, top);
-      cursor -= n;
-    }
-    for (int j = 0; j < n; ++j) {
-      if (!reaches(splat_mask(L, j), my_rect)) continue;  // no pixel of this wave can pass the alpha test
-      uint32_t contributor;
-      if constexpr (CELLS) {
-        contributor = splat_pos(L, j);
-      } else {
-        contributor = (uint32_t)(top - 1 - j);
-      }
-      const float2 xy = make_float2(L.xym[j].x, L.xym[j].y);
-      const float4 q = L.qo[j];
-      const float dx = xy.x - pxf, dy = xy.y - pyf;
-      const float p = power_at(power_dx(q, dx), q.z, dy);
-      const float G = splat_exp2(p);
-      const float ga = q.w * G;  // o G: alpha before the 0.99 clamp
-      const float alpha = fminf(0.99f, ga);
-      const bool contrib = contributor < last_contributor && p <= 0.0f && alpha >= 1.0f / 255.0f;
-      if (__ballot(contrib) == 0) continue;  // wave-uniform
-      float v[DMGS_GACC_USED];
-      if (contrib) {
-        float w;
-        const float dL_dalpha = bwd_step(st, alpha, L.rgb_id[j], g0, g1, g2, bg_term, w);
-        const float t = ga * dL_dalpha;
-        const float tdx = t * dx, tdy = t * dy;
-        v[0] = dmean_x(q, tdx, tdy);
-        v[1] = dmean_y(q, tdx, tdy);
-        v[2] = tdx * dx;
-        v[3] = tdx * dy;
-        v[4] = tdy * dy;
-        v[5] = G * dL_dalpha;
-        v[6] = w * g0;
-        v[7] = w * g1;
-        v[8] = w * g2;
-      } else {
-#pragma unroll
-        for (int k = 0; k < DMGS_GACC_USED; ++k) v[k] = 0.f;
-      }
-      // sum over each 16-lane row, then lane k of every row adds value k into
-      // the batch accumulator in LDS (one ds_add with 4 x 9 active lanes)
-      const float mine = row_sums9(v, row_lane);
-      if (row_lane < DMGS_GACC_USED) atomicAdd(&s_acc[j][row_lane], mine);
-    }
-    __syncthreads();
-    // flush the batch: consecutive lanes cover the 9 values of one splat
-    for (int i = threadIdx.x; i < n * DMGS_GACC_USED; i += NT) {
-      const int slot = i / DMGS_GACC_USED, k = i - slot * DMGS_GACC_USED;
-      const float val = s_acc[slot][k] * grad_scale(k, ddelx_dx, ddely_dy);
-      if (val != 0.f) {
-        const uint32_t gid = __float_as_uint(L.rgb_id[slot].w);
-        unsafeAtomicAdd(a.gacc + gacc_index(a.P, gid, k), val);
-      }
-    }
-  }
 }
 
 // Backward with one wave per 16x16 tile: lane (lx, ly) owns the pixels
@@ -758,19 +665,40 @@ __global__ __launch_bounds__(SUB* SUB) void render_bwd_kernel(RenderArgs a) {
 // render_bwd_kernel, and a lane first sums its four pixels' partial
 // gradients, so each (tile, splat) pays for one wave reduction instead of
 // four.
-template <int BATCH, bool CELLS>
+//
+// SEGS: the work-groups below a.seg.cap each take one kept segment of a tile's
+// list (see Segments), the others the rest of a tile's list.
+template <bool CELLS, bool SEGS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void render_bwd_strips_kernel(RenderArgs a) {
-  constexpr int NT = 64;
-  __shared__ SplatLDS<BATCH> L;
+  constexpr int NT = 64, BATCH = 64;
+  int tile, lo = 0, hi = 0x7fffffff;                   // this work-group's list positions [lo, hi)
+  uint32_t seg_end = kNoSegment;                       // the slot of the state at hi (none: the list's end)
+  if constexpr (SEGS) {
+    const bool kept = a.seg.head[1] == kSegMagic;
+    if ((int)blockIdx.x < a.seg.cap) {
+      if (!kept || blockIdx.x >= a.seg.head[0]) return;
+      const uint4 r = a.seg.rec[blockIdx.x];
+      if (r.x >= (uint32_t)a.num_tiles) return;  // never used
+      tile = (int)r.x;
+      lo = (int)r.y;
+      hi = (int)r.z;
+      seg_end = blockIdx.x;
+    } else {
+      tile = (int)blockIdx.x - a.seg.cap;
+      if (kept) lo = (int)a.seg.tile_last[tile];
+    }
+  } else {
+    tile = ordered_tile(a, blockIdx.x);
+  }
+  __shared__ BwdSplats<BATCH> L;
   // Two accumulator sets: a batch's global atomics are issued after the next
   // batch has been staged, so no staging load waits behind them (the memory
   // counter is in order) and they complete while that batch is computed.
   __shared__ __align__(16) float s_acc[2][BATCH][DMGS_GACC_USED];
   __shared__ uint32_t s_gid[2][BATCH];
-  __shared__ uint32_t s_wc[1];
   static_assert(BATCH * DMGS_GACC_USED >= 8 * DMGS_WAVE && (BATCH * DMGS_GACC_USED) % 4 == 0,
                 "one accumulator set holds a splat's 8 x 64 per-lane values");
-  const TileCtx c = tile_ctx<16>(a);  // pixel k = 0 of this lane: (lx, ly), ly in 0..3
+  const TileCtx c = tile_ctx<false>(a, tile);  // pixel k = 0 of this lane: (lx, ly), ly in 0..3
   const unsigned lane = threadIdx.x & 63;
   const WaveSum9 wsum = wave_sum9_lane(lane);
   const float pxf = (float)c.px;
@@ -802,6 +730,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     }
     bg_term[k] = -T_final * (c.bg0 * g0[k] + c.bg1 * g1[k] + c.bg2 * g2[k]);
     st[k] = bwd_pixel(T_final);
+    if constexpr (SEGS) {
+      if (seg_end != kNoSegment) {  // start from the state at hi: T, and the colour behind it
+        const float4 e = a.seg.state[(size_t)seg_end * 256 + threadIdx.x + 64 * k];
+        st[k].T = e.x;
+        st[k].S = (e.y * g0[k] + e.z * g1[k] + e.w * g2[k]) / e.x;
+      }
+    }
   }
   // per strip, the largest last contributor of its 64 pixels (wave-uniform):
   // list positions at or past it cannot contribute to the strip
@@ -813,7 +748,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     strip_max[k] = __builtin_amdgcn_readfirstlane(x);
     m = max(m, strip_max[k]);
   }
-  const int todo_total = min((int)(c.range.y - c.range.x), (int)m);
+  const int todo_total = min(min((int)(c.range.y - c.range.x), (int)m), hi);
 
   // one batch's accumulated sums -> one global atomic per (splat, value)
   auto flush = [&](int buf, int cnt) {
@@ -824,8 +759,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     }
   };
   int buf = 0, prev_n = 0;
-  int cursor = todo_total;  // list positions below cursor are still to do
-  while (cursor > 0) {
+  int cursor = todo_total;  // list positions in [lo, cursor) are still to do
+  while (cursor > lo) {
     __syncthreads();
     const int top = cursor;
     int n;
@@ -834,17 +769,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       for (int k = 0; k < DMGS_GACC_USED; ++k) s_acc[buf][s][k] = 0.f;
     }
     if constexpr (CELLS) {
-      n = stage_cell_batch<NT, true>(L, s_wc, a, c, cursor, 0);
+      n = stage_cell_batch(L, a, c, cursor, lo);
     } else {
       for (int s = threadIdx.x; s < BATCH; s += NT) {
         const int pos = top - 1 - s;
-        if (pos >= 0) stage_splat(L, s, a.splats, a.point_list[c.range.x + pos], a.P, c.rows, (uint32_t)pos);
+        if (pos >= lo) stage_splat(L, s, a.splats, a.point_list[c.range.x + pos], a.P, c.rows, (uint32_t)pos);
       }
       __syncthreads();
-      n = min(BATCH, top);
+      n = min(BATCH, top - lo);
       cursor -= n;
     }
-    for (int s = threadIdx.x; s < n; s += NT) s_gid[buf][s] = __float_as_uint(L.rgb_id[s].w);
+    for (int s = threadIdx.x; s < n; s += NT) s_gid[buf][s] = L.id(s);
     // Every staging load has landed here; saying so keeps the compiler from
     // waiting later (behind the atomics below) for a load it cannot rule out.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -853,14 +788,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     // the flushed set is free until the next batch zeroes it: it holds the
     // per-lane values of the wave sums (wave_sums9) meanwhile
     float(*const s_red)[DMGS_WAVE] = reinterpret_cast<float(*)[DMGS_WAVE]>(&s_acc[buf ^ 1][0][0]);
-    uint32_t mask_next = n > 0 ? splat_mask(L, 0) : 0u;  // read one splat ahead
+    uint32_t mask_next = n > 0 ? L.mask(0) : 0u;  // read one splat ahead
     for (int j = 0; j < n; ++j) {
       const uint32_t reach = __builtin_amdgcn_readfirstlane(mask_next);
-      if (j + 1 < n) mask_next = splat_mask(L, j + 1);
+      if (j + 1 < n) mask_next = L.mask(j + 1);
       if (reach == 0u) continue;
       uint32_t contributor;
       if constexpr (CELLS) {
-        contributor = __builtin_amdgcn_readfirstlane(splat_pos(L, j));
+        contributor = __builtin_amdgcn_readfirstlane(L.pos(j));
       } else {
         contributor = (uint32_t)(top - 1 - j);
       }
@@ -873,7 +808,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       const float4 q = L.qo[j];
       const float4 col = L.rgb_id[j];
       const float dx = xy.x - pxf;
-      const PowerDx pd = power_dx(q, dx);  // shared by the lane's four pixels (one column)
+      const PowerDx pd = power_dx(q.x, q.y, dx);  // shared by the lane's four pixels (one column)
       // per-lane sums over its pixels: sum t, sum t dy, sum t dy^2 (dx is the
       // same for the four pixels, so its powers multiply in once per splat)
       float s_t = 0.f, s_tdy = 0.f, s_tdy2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f;
@@ -910,41 +845,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
   }
   __syncthreads();
   flush(buf ^ 1, prev_n);
-}
-
-template <int SUB, int BATCH>
-static void launch_fwd_t(const RenderArgs& a, hipStream_t s) {
-  constexpr int Q = DMGS_BLOCK_X / SUB;
-  if (a.views)
-    hipLaunchKernelGGL((render_fwd_cells_kernel<SUB, BATCH>), dim3(a.num_tiles * Q * Q), dim3(SUB * SUB), 0, s, a);
-  else
-    hipLaunchKernelGGL((render_fwd_kernel<SUB, BATCH>), dim3(a.num_tiles * Q * Q), dim3(SUB * SUB), 0, s, a);
-}
-
-template <int SUB, int BATCH>
-static void launch_bwd_t(const RenderArgs& a, hipStream_t s) {
-  constexpr int Q = DMGS_BLOCK_X / SUB;
-  if (a.views)
-    hipLaunchKernelGGL((render_bwd_kernel<SUB, BATCH, true>), dim3(a.num_tiles * Q * Q), dim3(SUB * SUB), 0, s, a);
-  else
-    hipLaunchKernelGGL((render_bwd_kernel<SUB, BATCH, false>), dim3(a.num_tiles * Q * Q), dim3(SUB * SUB), 0, s,
-                       a);
-}
-
-template <int BATCH>
-static void launch_fwd_strips_t(const RenderArgs& a, hipStream_t s) {
-  if (a.views)
-    hipLaunchKernelGGL((render_fwd_strips_kernel<BATCH, true>), dim3(a.num_tiles), dim3(64), 0, s, a);
-  else
-    hipLaunchKernelGGL((render_fwd_strips_kernel<BATCH, false>), dim3(a.num_tiles), dim3(64), 0, s, a);
-}
-
-template <int BATCH>
-static void launch_bwd_strips_t(const RenderArgs& a, hipStream_t s) {
-  if (a.views)
-    hipLaunchKernelGGL((render_bwd_strips_kernel<BATCH, true>), dim3(a.num_tiles), dim3(64), 0, s, a);
-  else
-    hipLaunchKernelGGL((render_bwd_strips_kernel<BATCH, false>), dim3(a.num_tiles), dim3(64), 0, s, a);
+  if (a.clear_words && blockIdx.x == 0)  // the tile-order histogram, ready for another backward's
+    for (int i = threadIdx.x; i < a.clear_words_n; i += NT) a.clear_words[i] = 0u;
 }
 
 // Longest-first scheduling of the blend: a tile's cost is about the length
@@ -1003,7 +905,7 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const uint8_t* __restri
   __syncthreads();
   if (cnt[threadIdx.x]) base[threadIdx.x] = start[threadIdx.x] + atomicAdd(&hist[256 + threadIdx.x], cnt[threadIdx.x]);
   __syncthreads();
-  if (t < num_tiles) order[base[b] + rank] = (uint32_t)t;
+  if (t < num_tiles && base[b] + rank < (uint32_t)num_tiles) order[base[b] + rank] = (uint32_t)t;
 }
 
 static void tile_order_impl(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, bool use_work,
@@ -1026,29 +928,32 @@ void launch_tile_order_bwd(const RenderArgs& a, uint32_t* order, uint8_t* bucket
   if (a.tile_work) tile_order_impl(a, order, bucket, hist, true, s, hist_zeroed);
 }
 
-void launch_render_fwd(const RenderArgs& a, hipStream_t s, int variant) {
+// Kept segments: the header is set before each forward that keeps any.
+__global__ void seg_reset_kernel(uint32_t* head) {
+  if (threadIdx.x < 2) head[threadIdx.x] = threadIdx.x == 0 ? 0u : kSegMagic;
+}
+
+void launch_render_fwd(const RenderArgs& a, hipStream_t s) {
   if (a.num_tiles <= 0) return;
-  switch (variant) {
-    case kRender16x128: launch_fwd_t<16, 128>(a, s); break;
-    case kRenderStrips64: launch_fwd_strips_t<64>(a, s); break;
-    case kRenderStrips128: launch_fwd_strips_t<128>(a, s); break;
-    case kRender8x64: launch_fwd_t<8, 64>(a, s); break;
-    case kRender8x128: launch_fwd_t<8, 128>(a, s); break;
-    default: launch_fwd_t<16, 256>(a, s); break;
+  const dim3 grid(a.num_tiles), block(256);
+  if (a.seg.len > 0) {
+    hipLaunchKernelGGL(seg_reset_kernel, dim3(1), dim3(64), 0, s, a.seg.head);
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, true>), grid, block, 0, s, a);
+  } else if (a.views) {
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false>), grid, block, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((render_fwd_quads_kernel<false, false>), grid, block, 0, s, a);
   }
 }
 
-void launch_render_bwd(const RenderArgs& a, hipStream_t s, int variant) {
+void launch_render_bwd(const RenderArgs& a, hipStream_t s) {
   if (a.num_tiles <= 0) return;
-  switch (variant) {
-    case kRenderStrips64:
-    case kRenderMixed: launch_bwd_strips_t<64>(a, s); break;
-    case kRenderStrips128: launch_bwd_strips_t<128>(a, s); break;
-    case kRender16x128: launch_bwd_t<16, 128>(a, s); break;
-    case kRender8x64: launch_bwd_t<8, 64>(a, s); break;
-    case kRender8x128: launch_bwd_t<8, 128>(a, s); break;
-    default: launch_bwd_t<16, 256>(a, s); break;
-  }
+  if (a.seg.len > 0)
+    hipLaunchKernelGGL((render_bwd_strips_kernel<true, true>), dim3(a.seg.cap + a.num_tiles), dim3(64), 0, s, a);
+  else if (a.views)
+    hipLaunchKernelGGL((render_bwd_strips_kernel<true, false>), dim3(a.num_tiles), dim3(64), 0, s, a);
+  else
+    hipLaunchKernelGGL((render_bwd_strips_kernel<false, false>), dim3(a.num_tiles), dim3(64), 0, s, a);
 }
 
 }  // namespace dmgs

@@ -284,14 +284,17 @@ int dmgs_batched_tile_view(const dmgs_view* views, int32_t B, int32_t* tile_view
 
 /* Workspaces of a batch (device memory, caller-owned):
  *   state   K-independent: per (view, Gaussian) splats, keys, radii, scan;
- *           per-tile ranges; per-pixel blend state.  Kept until backward.
+ *           per-tile ranges; per-pixel blend state; up to 4096 tiles, also
+ *           list segments a forward with bwd_ws keeps for its backward.
+ *           Kept until backward.
  *   lists   the (Gaussian, tile) instance lists for up to `capacity`
  *           instances and their sort scratch.  Kept until backward.
  *   bwd_ws  per (view, Gaussian) gradient accumulator (backward only).  A
  *           forward whose BLEND stage runs with bwd_ws set clears it (the
  *           blend work-groups zero it after their blend work, so no clearing
  *           pass runs per step); a backward accumulates into it, so every
- *           backward needs a forward BLEND since the previous backward. */
+ *           backward needs a forward BLEND since the previous backward, or
+ *           zeros in it. */
 size_t dmgs_batched_state_size(int32_t B, int64_t P, int32_t total_tiles, int64_t total_pixels);
 size_t dmgs_batched_lists_size(int64_t capacity);
 size_t dmgs_batched_backward_size(int32_t B, int64_t P);
@@ -312,7 +315,7 @@ typedef struct dmgs_batch {
   int32_t sh_degree;        /* active SH degree (coefficients are always 16 per colour) */
   int64_t num_gaussians;    /* P */
   float scale_modifier;
-  int32_t variant;          /* blend kernel shape 0..6 (same results; picked by an autotuner) */
+  int32_t variant;          /* accepted for callers that set it; the launch picks the blend's shape */
   int32_t total_tiles;
   int32_t total_cells;
   int64_t total_pixels;

@@ -1,0 +1,70 @@
+"""The blend kernels at the edges of their list handling, against the FP64 oracle.
+
+The forward takes a tile's list 256 positions at a time and keeps a segment
+for the backward every 64 members: lists of one entry, around 64 and 256, and
+longer than several chunks; a list cut off by saturation; more segments than
+the workspace has slots for.  Tolerances are those of the other parity tests
+(images 1e-4, gradients 1e-3 norm-relative; 1e-5 between two groupings of the
+same sums)."""
+import math
+
+import pytest
+import torch
+
+from dmgs_amd import batched as BT
+from dmgs_amd import cameras as C
+from dmgs_amd import scenes as S
+from helpers import grad_rel_err
+from oracle import raster as OR
+
+pytestmark = pytest.mark.gpu
+
+
+def _covering(n, logit, seed=0):
+    """n splats that each cover the whole view."""
+    g = torch.Generator().manual_seed(seed)
+    xyz = torch.rand(n, 3, generator=g) - 0.5
+    dc = torch.randn(n, 1, 3, generator=g) * 0.5
+    scale = torch.randn(n, 3, generator=g) * 0.1 + 0.5
+    return S.FreeGaussians(xyz, dc, torch.randn(n, 3, 3, generator=g) * 0.1, scale, torch.randn(n, 4, generator=g),
+                           logit + 0.3 * torch.randn(n, 1, generator=g), 1)
+
+
+@pytest.mark.parametrize("n,logit,size", [
+    (1, -2.0, (16, 16)), (63, -4.0, (17, 16)), (64, -4.0, (16, 33)), (65, -4.0, (33, 17)), (128, -4.0, (16, 16)),
+    (255, -4.5, (20, 20)), (256, -4.5, (20, 20)), (257, -4.5, (20, 20)), (700, -4.5, (48, 40)),
+    (300, 1.0, (40, 40)),       # saturates within the first chunk
+    (600, -4.5, (320, 320))])   # 400 tiles of nine segments, 1024 slots
+def test_list_edges(n, logit, size):
+    print(f"case: list edges n={n} logit={logit} size={size}", flush=True)
+    m = _covering(n, logit)
+    cam = C.camera_at((0.3, -0.2, -4.0), *size, device="cpu")
+    bg = torch.tensor([0.2, 0.5, 0.8])
+    st = OR.settings_for(cam, bg.double(), 1)
+    kw = dict(shs=m.get_features, scales=m.get_scaling, rotations=m.get_rotation)
+    col, _, state = OR.rasterize(m.get_xyz, m.get_opacity, st, **kw)
+    dL = torch.randn(col.shape, generator=torch.Generator().manual_seed(1))
+    dL[:, state["ambiguous"]] = 0.0
+    want = OR.rasterize_backward(state, st, m.get_xyz, dL.double(), **kw)
+    params = BT.pack_model(m.to("cuda"))
+    r = BT.BatchedRenderer([cam], bg, n, sh_degree=1)
+    r.plan(params)
+    images = r.forward(params)
+    grads = r.backward(params, dL.cuda().reshape(-1).contiguous()).clone()
+    ok = ~state["ambiguous"]
+    err = (r.image(images, 0).cpu().double() - col).abs()[:, ok].max().item()
+    assert err < 1e-4, f"image error {err}"
+    got = BT.unpack_grads(grads, 4)
+    o = torch.sigmoid(m._opacity.double())
+    for name, ref in (("_xyz", want[0]), ("_opacity", want[4] * o * (1 - o)),
+                      ("_features_dc", want[2][:, :1])):
+        assert grad_rel_err(got[name], ref) < 1e-3, name
+    # a second backward, and one after a forward that kept no segments
+    twice = r.backward(params, dL.cuda().reshape(-1).contiguous()).clone()
+    ws, r.bwd_ws = r.bwd_ws, None
+    again = r.forward(params)
+    assert torch.equal(again, images)
+    r.bwd_ws, r._acc_clear = ws, False
+    whole = r.backward(params, dL.cuda().reshape(-1).contiguous())
+    assert grad_rel_err(whole, grads) < 1e-5
+    assert grad_rel_err(twice, grads) < 1e-5
