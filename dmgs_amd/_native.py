@@ -46,6 +46,19 @@ class DmgsBatch(ctypes.Structure):
     ]
 
 
+class DmgsGaussians(ctypes.Structure):
+    """struct dmgs_gaussians (include/dmgs.h): one model's tensors."""
+    _fields_ = [("count", c_int64), ("means3D", c_void_p), ("opacities", c_void_p), ("shs", c_void_p),
+                ("shs_rest", c_void_p), ("colors_precomp", c_void_p), ("scales", c_void_p), ("rotations", c_void_p),
+                ("cov3D_precomp", c_void_p), ("raw", c_int32), ("reserved", c_int32)]
+
+
+class DmgsGaussianGrads(ctypes.Structure):
+    """struct dmgs_gaussian_grads (include/dmgs.h)."""
+    _fields_ = [(n, c_void_p) for n in ("means2D", "means3D", "opacities", "shs", "shs_rest", "colors", "cov3D",
+                                        "scales", "rotations")]
+
+
 # name -> (restype, argtypes)
 _SIGNATURES = {
     "dmgs_last_error": (ctypes.c_char_p, []),
@@ -104,6 +117,15 @@ _SIGNATURES = {
     "dmgs_batched_lists_size": (c_size_t, [c_int64]),
     "dmgs_batched_backward_size": (c_size_t, [c_int32, c_int64]),
     "dmgs_batched_offsets": (c_int32, [c_int32, c_int64, c_int32, c_int64, c_int64, ctypes.POINTER(c_size_t)]),
+    "dmgs_view_supported": (c_int32, [c_int32, c_int32]),
+    "dmgs_view_state_size": (c_size_t, [c_int64, c_int32, c_int32, c_int32]),
+    "dmgs_view_geometry": (c_int32, [ctypes.POINTER(DmgsSettings), ctypes.POINTER(DmgsGaussians), c_int32, c_void_p,
+                                     c_void_p, c_void_p, c_void_p]),
+    "dmgs_view_binning": (c_int32, [ctypes.POINTER(DmgsSettings), c_int64, c_int32, c_int64] + [c_void_p] * 3),
+    "dmgs_view_blend": (c_int32, [ctypes.POINTER(DmgsSettings), c_int64, c_int32, c_int64] + [c_void_p] * 5),
+    "dmgs_view_blend_backward": (c_int32, [ctypes.POINTER(DmgsSettings), c_int64, c_int64] + [c_void_p] * 5),
+    "dmgs_view_geometry_backward": (c_int32, [ctypes.POINTER(DmgsSettings), ctypes.POINTER(DmgsGaussians), c_void_p,
+                                              c_void_p, ctypes.POINTER(DmgsGaussianGrads), c_void_p]),
     "dmgs_batched_forward": (c_int32, [ctypes.POINTER(DmgsBatch), c_void_p, c_void_p, c_int32, c_void_p]),
     "dmgs_batched_backward": (c_int32, [ctypes.POINTER(DmgsBatch), c_void_p, c_void_p, c_void_p, c_int32,
                                         c_void_p]),

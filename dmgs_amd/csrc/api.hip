@@ -139,8 +139,13 @@ void fill_geom_common(const dmgs_settings* s, float& fx, float& fy, int& gx, int
 }  // namespace
 
 namespace dmgs {
-// Error reporting for the entry points defined in other translation units.
+// Error reporting and argument checks for the entry points defined in other translation units.
 void set_last_error(const char* msg) { g_last_error = msg; }
+int check_view(const dmgs_settings* s, int64_t P, const float* means3D, const float* opacities, const float* shs,
+               const float* colors_precomp, const float* scales, const float* rotations, const float* cov3D_precomp) {
+  const int rc = check_settings(s);
+  return rc ? rc : check_inputs(s, P, means3D, opacities, shs, colors_precomp, scales, rotations, cov3D_precomp);
+}
 }  // namespace dmgs
 
 extern "C" {

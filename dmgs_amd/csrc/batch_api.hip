@@ -23,7 +23,11 @@
 
 namespace dmgs {
 void set_last_error(const char* msg);
+int check_view(const dmgs_settings* s, int64_t P, const float* means3D, const float* opacities, const float* shs,
+               const float* colors_precomp, const float* scales, const float* rotations, const float* cov3D_precomp);
 }
+static_assert(sizeof(dmgs_gaussians) == 80, "dmgs_gaussians layout");
+static_assert(sizeof(dmgs_gaussian_grads) == 72, "dmgs_gaussian_grads layout");
 
 static_assert(sizeof(dmgs_view) == sizeof(dmgs::ViewDesc), "dmgs_view / ViewDesc layout");
 static_assert(offsetof(dmgs_view, tile_base) == offsetof(dmgs::ViewDesc, tile_base), "dmgs_view layout");
@@ -73,7 +77,7 @@ struct StateLayout {
       status, tile_order, tile_bucket, bucket_hist, tile_work, ranges, final_T, n_contrib, tile_last,
       seg_head, seg_rec, seg_state, total;
   int seg_cap;  // slots for the list segments a forward keeps for its backward (0: too many tiles for any)
-  StateLayout(size_t N, size_t T, size_t X) {
+  StateLayout(size_t N, size_t T, size_t X, bool segments = true) {
     size_t o = 0;
     splats = o; o += align_up(N * DMGS_SPLAT_F4 * 16);
     keys_a = o; o += align_up(N * 4);
@@ -94,7 +98,7 @@ struct StateLayout {
     ranges = o; o += align_up(T * 8);
     final_T = o; o += align_up(X * 4);
     n_contrib = o; o += align_up(X * 4);
-    seg_cap = T <= (size_t)dmgs::kSegmentTiles ? (int)std::min<size_t>(16384, std::max<size_t>(1024, N / 16)) : 0;
+    seg_cap = segments && T <= (size_t)dmgs::kSegmentTiles ? (int)std::min<size_t>(16384, std::max<size_t>(1024, N / 16)) : 0;
     tile_last = o; o += align_up(seg_cap ? T * 4 : 0);
     seg_head = o; o += align_up(8);
     seg_rec = o; o += align_up((size_t)seg_cap * 16);
@@ -145,12 +149,14 @@ struct Ctx {
   size_t N;
   StateLayout S;
   ListLayout L;
-  explicit Ctx(const dmgs_batch* b)
+  explicit Ctx(const dmgs_batch* b, bool segments = true)
       : N((size_t)b->num_views * b->num_gaussians),
-        S(N, (size_t)b->total_tiles, (size_t)b->total_pixels),
+        S(N, (size_t)b->total_tiles, (size_t)b->total_pixels, segments),
         L((size_t)b->capacity), mode(b->cell_mode),
         local_bits(b->cell_mode == 1 ? std::max(1, bits_for((uint32_t)(b->max_view_cells - 1))) : 0),
         global_bits(std::max(1, bits_for((uint32_t)(b->total_cells - 1)))) {}
+  // the depth keys also order by view (with one view plain depth bits do, at any depth)
+  bool view_keys(const dmgs_batch* b) const { return mode == 1 && b->num_views > 1; }
   uint32_t* count(const dmgs_batch* b) const { return at<uint32_t>(b->state, S.offsets) + (N - 1); }
   int mode;
   // key bits of the cell sort: the cell within the view (mode 1) or the
@@ -176,7 +182,7 @@ dmgs::MVArgs mv_args(const dmgs_batch* b, const Ctx& c, const float* params) {
   a.rects = at<uint2>(b->state, c.S.rects);
   a.depth_keys = at<uint32_t>(b->state, c.S.keys_a);  // sorted in place into keys_a / order_a
   a.order = at<uint32_t>(b->state, c.S.order_a);
-  a.view_major = b->cell_mode == 1 ? 1 : 0;
+  a.view_major = c.view_keys(b) ? 1 : 0;
   a.gacc = static_cast<float*>(b->bwd_ws);
   a.dens = b->dens;
   return a;
@@ -208,6 +214,190 @@ dmgs::RenderArgs render_args(const dmgs_batch* b, const Ctx& c) {
     r.seg.tile_last = at<uint32_t>(b->state, c.S.tile_last);
   }
   return r;
+}
+
+// The visible entries, in entry order, sorted by their keys (culled entries drop out in the first pass), and
+// the scan of their cell counts; with_chunks: also the duplicate's chunk table.
+void order_entries(const dmgs_batch* b, const Ctx& c, bool with_chunks, hipStream_t st) {
+  uint32_t* keys = at<uint32_t>(b->state, c.S.keys_a);
+  uint32_t* order = at<uint32_t>(b->state, c.S.order_a);
+  uint32_t* offs = at<uint32_t>(b->state, c.S.offsets);
+  uint32_t* gs = at<uint32_t>(b->state, c.S.gscratch);
+  uint32_t* V_dev = at<uint32_t>(b->state, c.S.visible);
+  dmgs::radix_sort_entry_keys(keys, order, at<uint32_t>(b->state, c.S.keys_b), at<uint32_t>(b->state, c.S.order_b),
+                              c.N, gs, st, V_dev, c.view_keys(b) ? at<uint32_t>(b->state, c.S.status) : nullptr);
+  dmgs::launch_gather_rects(at<uint2>(b->state, c.S.rects), order, at<uint2>(b->state, c.S.rects_sorted), offs, c.N,
+                            st, V_dev);
+  if (with_chunks)
+    dmgs::launch_inclusive_scan_chunks(offs, offs, c.N, gs, at<uint32_t>(b->lists, c.L.chunk), (uint32_t)b->capacity,
+                                       st);
+  else
+    dmgs::launch_inclusive_scan(offs, offs, c.N, gs, st);
+}
+
+// The cell lists, their ranges and the blend's dispatch order.
+int bin_entries(const dmgs_batch* b, const Ctx& c, bool chunks_ready, hipStream_t st) {
+  const uint32_t K = (uint32_t)b->capacity;
+  dmgs::DupArgs d{};
+  d.P = (int)c.N;
+  d.order = at<uint32_t>(b->state, c.S.order_a);
+  d.offsets = at<uint32_t>(b->state, c.S.offsets);
+  d.splats = at<float4>(b->state, c.S.splats);
+  d.rects = at<uint2>(b->state, c.S.rects_sorted);
+  d.views = reinterpret_cast<const dmgs::ViewDesc*>(b->views);
+  d.per_view = (uint32_t)b->num_gaussians;
+  d.tile_keys = at<uint32_t>(b->lists, c.L.tkeys_a);
+  d.values = at<uint32_t>(b->lists, c.L.vals_a);
+  d.K = K;
+  d.K_dev = c.count(b);
+  d.chunk_first = at<uint32_t>(b->lists, c.L.chunk);
+  d.chunk_ready = chunks_ready;
+  d.view_major = b->cell_mode == 1;
+  // the duplicate also zeroes the tile-order histogram and the cell ranges (adjacent)
+  d.zero = at<uint32_t>(b->state, c.S.bucket_hist);
+  d.zero_n = 512 + 2 * (size_t)b->total_cells;
+  // view-major lists: the duplicate also counts the first sort pass's digits
+  const int w0 = d.view_major ? dmgs::radix_min_passes_first_width(K, c.local_bits) : -1;
+  if (w0 > 0) {
+    d.hist = at<uint32_t>(b->lists, c.L.scratch);
+    d.hist_bits = w0;
+  }
+  dmgs::launch_duplicate(d, st);
+  uint32_t* kb = at<uint32_t>(b->lists, c.L.tkeys_b);
+  uint32_t* vb = at<uint32_t>(b->lists, c.L.vals_b);
+  if (d.view_major) {  // sort the cell-within-view bits only; the view order is already there
+    const bool in_b = dmgs::radix_sort_pairs_min_passes(d.tile_keys, d.values, kb, vb, K, c.local_bits,
+                                                        at<uint32_t>(b->lists, c.L.scratch), st, d.K_dev, w0 > 0);
+    if (in_b != c.lists_in_b()) return bfail(DMGS_EHIP, "internal: sorted list buffer mismatch");
+    dmgs::launch_view_cell_ranges(in_b ? kb : d.tile_keys, K, at<uint2>(b->state, c.S.ranges), b->total_cells,
+                                  d.views, st, d.K_dev, true);
+  } else {
+    dmgs::radix_sort_pairs(d.tile_keys, d.values, kb, vb, K, c.global_bits, at<uint32_t>(b->lists, c.L.scratch), st,
+                           d.K_dev);
+    dmgs::launch_tile_ranges(d.tile_keys, K, at<uint2>(b->state, c.S.ranges), b->total_cells, st, d.K_dev,
+                             DMGS_CELL_KEY_MASK);
+  }
+  // blend dispatch order: tiles with the longest lists first
+  dmgs::launch_tile_order(render_args(b, c), at<uint32_t>(b->state, c.S.tile_order),
+                          at<uint8_t>(b->state, c.S.tile_bucket), at<uint32_t>(b->state, c.S.bucket_hist), st, true);
+  return bcheck("batch binning", st);
+}
+
+int blend_views(const dmgs_batch* b, const Ctx& c, float* images, hipStream_t st) {
+  dmgs::RenderArgs r = render_args(b, c);
+  r.out_color = images;
+  if (b->bwd_ws) {  // the blend work-groups also clear the backward accumulator
+    r.clear = static_cast<float4*>(b->bwd_ws);
+    r.clear_n = (c.N * DMGS_GACC_STRIDE + 3) / 4;  // inside the 256-byte-aligned workspace
+  }
+  r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);  // for the backward's tile order
+  r.clear_words_n = 512;
+  dmgs::launch_render_fwd(r, st);
+  return bcheck("batch render forward", st);
+}
+
+// Accumulates into bwd_ws, which holds zeros on entry.
+int blend_views_backward(const dmgs_batch* b, const Ctx& c, const float* dL_dimages, hipStream_t st) {
+  dmgs::RenderArgs r = render_args(b, c);
+  r.dL_dpix = dL_dimages;
+  // re-order the tiles by the list lengths the forward measured (the
+  // forward blend, and then each backward blend, zero the histogram)
+  r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);
+  r.clear_words_n = 512;
+  if (r.seg.len == 0)
+    dmgs::launch_tile_order_bwd(r, at<uint32_t>(b->state, c.S.tile_order), at<uint8_t>(b->state, c.S.tile_bucket),
+                                at<uint32_t>(b->state, c.S.bucket_hist), st, true);
+  dmgs::launch_render_bwd(r, st);
+  return bcheck("batch render backward", st);
+}
+
+// ---- one view over a model's own tensors ----
+// Its state: the batch state of one view, then the view's record and the tile sums.
+struct ViewLayout {
+  int grid_x, grid_y, cells;
+  StateLayout S;
+  size_t record, tile_sums, counts, total;
+  ViewLayout(int64_t P, int W, int H, bool keep)
+      : grid_x((W + DMGS_BLOCK_X - 1) / DMGS_BLOCK_X),
+        grid_y((H + DMGS_BLOCK_Y - 1) / DMGS_BLOCK_Y),
+        cells(cells_along(grid_x) * cells_along(grid_y)),
+        S((size_t)P, (size_t)grid_x * grid_y, (size_t)W * H, keep) {
+    record = S.total;
+    tile_sums = record + align_up(sizeof(dmgs::ViewDesc));
+    counts = tile_sums + align_up(dmgs::kTileSums * 4);
+    total = counts + align_up(8);
+  }
+  static int cells_along(int tiles) { return (tiles + (1 << DMGS_CELL_SHIFT) - 1) >> DMGS_CELL_SHIFT; }
+};
+bool view_has_cells(int32_t W, int32_t H) {
+  if (W <= 0 || H <= 0 || (int64_t)W * H > (int64_t)1 << 30) return false;
+  const int64_t cx = ViewLayout::cells_along((W + DMGS_BLOCK_X - 1) / DMGS_BLOCK_X);
+  const int64_t cy = ViewLayout::cells_along((H + DMGS_BLOCK_Y - 1) / DMGS_BLOCK_Y);
+  return cx * cy <= 1 << DMGS_CELL_KEY_BITS;
+}
+
+dmgs_batch view_batch(const dmgs_settings* s, int64_t P, const ViewLayout& V, void* state, int64_t K, void* lists,
+                      void* bwd_ws) {
+  dmgs_batch b{};
+  b.views = at<dmgs_view>(state, V.record);
+  b.num_views = 1;
+  b.num_gaussians = P;
+  b.total_tiles = V.grid_x * V.grid_y;
+  b.total_cells = b.max_view_cells = V.cells;
+  b.total_pixels = (int64_t)s->image_width * s->image_height;
+  b.capacity = K;
+  b.state = state;
+  b.lists = lists;
+  b.bwd_ws = bwd_ws;
+  b.cell_mode = V.cells <= 4096 ? 1 : 0;
+  return b;
+}
+
+dmgs::ViewArgs view_args(const dmgs_settings* s, const dmgs_gaussians* g, const ViewLayout& V) {
+  dmgs::ViewArgs a{};
+  a.P = (int)g->count;
+  a.W = s->image_width;
+  a.H = s->image_height;
+  a.grid_x = V.grid_x;
+  a.grid_y = V.grid_y;
+  a.tanfovx = s->tanfovx;
+  a.tanfovy = s->tanfovy;
+  a.focal_x = (float)a.W / (2.0f * s->tanfovx);
+  a.focal_y = (float)a.H / (2.0f * s->tanfovy);
+  a.scale_modifier = s->scale_modifier;
+  a.sh_degree = s->sh_degree;
+  a.sh_coeffs = g->shs ? s->sh_coeffs : 0;
+  a.raw = g->raw;
+  a.means3D = g->means3D;
+  a.scales = g->scales;
+  a.rotations = g->rotations;
+  a.opacities = g->opacities;
+  a.shs = g->shs;
+  a.shs_rest = g->shs_rest;
+  a.colors_precomp = g->colors_precomp;
+  a.cov3D_precomp = g->cov3D_precomp;
+  a.viewmatrix = s->viewmatrix;
+  a.projmatrix = s->projmatrix;
+  a.campos = s->campos;
+  a.bg = s->bg;
+  return a;
+}
+
+int check_gaussians(const dmgs_settings* s, const dmgs_gaussians* g, const void* state) {
+  if (!g) return bfail(DMGS_EINVAL, "gaussians is null");
+  const int rc = dmgs::check_view(s, g->count, g->means3D, g->opacities, g->shs, g->colors_precomp, g->scales,
+                                  g->rotations, g->cov3D_precomp);
+  if (rc) return rc;
+  if (g->count <= 0) return bfail(DMGS_EINVAL, "no Gaussians");
+  if (!view_has_cells(s->image_width, s->image_height)) return bfail(DMGS_EINVAL, "more than 65536 cells");
+  if (g->raw & ~7) return bfail(DMGS_EINVAL, "invalid raw mask %d", g->raw);
+  if (g->shs_rest && (!g->shs || (s->sh_coeffs != 4 && s->sh_coeffs != 9 && s->sh_coeffs != 16)))
+    return bfail(DMGS_EINVAL, "shs_rest needs shs and 4, 9 or 16 coefficients");
+  for (const float* p : {g->shs, g->shs_rest, g->rotations})
+    if (reinterpret_cast<uintptr_t>(p) & 15u) return bfail(DMGS_EINVAL, "tensors must be 16-byte aligned");
+  if (!state || (reinterpret_cast<uintptr_t>(state) & 255u))
+    return bfail(DMGS_EINVAL, "state is required, 256-byte aligned");
+  return DMGS_OK;
 }
 
 }  // namespace
@@ -318,92 +508,21 @@ int dmgs_batched_forward(const dmgs_batch* b, const float* params, float* images
   if ((stages & DMGS_STAGE_BLEND) && !images) return bfail(DMGS_EINVAL, "images is required for the blend");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const Ctx c(b);
-  const size_t N = c.N;
-  const dmgs::MVArgs a = mv_args(b, c, params);
-  uint32_t* offs = at<uint32_t>(b->state, c.S.offsets);
-  uint32_t* status = at<uint32_t>(b->state, c.S.status);
   bool chunks_ready = false;  // the duplicate's chunk table was filled by this call's scan
   if (stages & DMGS_STAGE_GEOMETRY) {
-    dmgs::MVArgs ap = a;
-    ap.status = status;  // zeroed by the preprocess, set by the depth sort
-    dmgs::launch_mv_preprocess(ap, st);
-    uint32_t* gs = at<uint32_t>(b->state, c.S.gscratch);
-    // the visible entries, in entry order, sorted by their keys; culled entries drop out in the first pass
-    uint32_t* V_dev = at<uint32_t>(b->state, c.S.visible);
-    dmgs::radix_sort_entry_keys(a.depth_keys, a.order, at<uint32_t>(b->state, c.S.keys_b),
-                                at<uint32_t>(b->state, c.S.order_b), N, gs, st, V_dev,
-                                b->cell_mode == 1 ? status : nullptr);
-    dmgs::launch_gather_rects(a.rects, a.order, at<uint2>(b->state, c.S.rects_sorted), offs, N, st, V_dev);
-    if ((stages & DMGS_STAGE_BINNING) && b->capacity > 0 && b->lists) {
-      // the binning follows in this call: the scan also fills the duplicate's chunk table
-      dmgs::launch_inclusive_scan_chunks(offs, offs, N, gs, at<uint32_t>(b->lists, c.L.chunk),
-                                         (uint32_t)b->capacity, st);
-      chunks_ready = true;
-    } else {
-      dmgs::launch_inclusive_scan(offs, offs, N, gs, st);
-    }
+    dmgs::MVArgs a = mv_args(b, c, params);
+    a.status = at<uint32_t>(b->state, c.S.status);  // zeroed by the preprocess, set by the depth sort
+    dmgs::launch_mv_preprocess(a, st);
+    // the binning may follow in this call: the scan then also fills the duplicate's chunk table
+    chunks_ready = (stages & DMGS_STAGE_BINNING) && b->capacity > 0 && b->lists;
+    order_entries(b, c, chunks_ready, st);
     if ((rc = bcheck("batch preprocess / depth sort / scan", st))) return rc;
   }
   if (stages & DMGS_STAGE_BINNING) {
-    const uint32_t K = (uint32_t)b->capacity;
-    dmgs::DupArgs d{};
-    d.P = (int)N;
-    d.order = a.order;
-    d.offsets = offs;
-    d.splats = a.splats;
-    d.rects = at<uint2>(b->state, c.S.rects_sorted);
-    d.views = a.views;
-    d.per_view = (uint32_t)b->num_gaussians;
-    d.tile_keys = at<uint32_t>(b->lists, c.L.tkeys_a);
-    d.values = at<uint32_t>(b->lists, c.L.vals_a);
-    d.K = K;
-    d.K_dev = c.count(b);
-    d.chunk_first = at<uint32_t>(b->lists, c.L.chunk);
-    d.chunk_ready = chunks_ready;
-    d.view_major = b->cell_mode == 1;
-    // the duplicate also zeroes the tile-order histogram and the cell ranges (adjacent)
-    d.zero = at<uint32_t>(b->state, c.S.bucket_hist);
-    d.zero_n = 512 + 2 * (size_t)b->total_cells;
-    // view-major lists: the duplicate also counts the first sort pass's digits
-    const int w0 = d.view_major ? dmgs::radix_min_passes_first_width(K, c.local_bits) : -1;
-    if (w0 > 0) {
-      d.hist = at<uint32_t>(b->lists, c.L.scratch);
-      d.hist_bits = w0;
-    }
-    dmgs::launch_duplicate(d, st);
-    uint32_t* kb = at<uint32_t>(b->lists, c.L.tkeys_b);
-    uint32_t* vb = at<uint32_t>(b->lists, c.L.vals_b);
-    if (d.view_major) {  // sort the cell-within-view bits only; the view order is already there
-      const bool in_b = dmgs::radix_sort_pairs_min_passes(d.tile_keys, d.values, kb, vb, K,
-                                                          c.local_bits,
-                                                          at<uint32_t>(b->lists, c.L.scratch), st, d.K_dev,
-                                                          w0 > 0);
-      if (in_b != c.lists_in_b()) return bfail(DMGS_EHIP, "internal: sorted list buffer mismatch");
-      dmgs::launch_view_cell_ranges(in_b ? kb : d.tile_keys, K, at<uint2>(b->state, c.S.ranges), b->total_cells,
-                                    a.views, st, d.K_dev, true);
-    } else {
-      dmgs::radix_sort_pairs(d.tile_keys, d.values, kb, vb, K, c.global_bits,
-                             at<uint32_t>(b->lists, c.L.scratch), st, d.K_dev);
-      dmgs::launch_tile_ranges(d.tile_keys, K, at<uint2>(b->state, c.S.ranges), b->total_cells, st, d.K_dev,
-                               DMGS_CELL_KEY_MASK);
-    }
-    // blend dispatch order: tiles with the longest lists first
-    dmgs::launch_tile_order(render_args(b, c), at<uint32_t>(b->state, c.S.tile_order),
-                            at<uint8_t>(b->state, c.S.tile_bucket), at<uint32_t>(b->state, c.S.bucket_hist), st,
-                            true);
-    if ((rc = bcheck("batch binning", st))) return rc;
+    if ((rc = bin_entries(b, c, chunks_ready, st))) return rc;
   }
   if (stages & DMGS_STAGE_BLEND) {
-    dmgs::RenderArgs r = render_args(b, c);
-    r.out_color = images;
-    if (b->bwd_ws) {  // the blend work-groups also clear the backward accumulator
-      r.clear = static_cast<float4*>(b->bwd_ws);
-      r.clear_n = (c.N * DMGS_GACC_STRIDE + 3) / 4;  // inside the 256-byte-aligned workspace
-    }
-    r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);  // for the backward's tile order
-    r.clear_words_n = 512;
-    dmgs::launch_render_fwd(r, st);
-    if ((rc = bcheck("batch render forward", st))) return rc;
+    if ((rc = blend_views(b, c, images, st))) return rc;
   }
   return DMGS_OK;
 }
@@ -421,17 +540,8 @@ int dmgs_batched_backward(const dmgs_batch* b, const float* params, const float*
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const Ctx c(b);
   dmgs::MVArgs a = mv_args(b, c, params);
-  if (stages & DMGS_STAGE_BLEND) {  // accumulates into bwd_ws, which holds zeros on entry
-    dmgs::RenderArgs r = render_args(b, c);
-    r.dL_dpix = dL_dimages;
-    // re-order the tiles by the list lengths the forward measured (the
-    // forward blend, and then each backward blend, zero the histogram)
-    r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);
-    r.clear_words_n = 512;
-    if (r.seg.len == 0) dmgs::launch_tile_order_bwd(r, at<uint32_t>(b->state, c.S.tile_order), at<uint8_t>(b->state, c.S.tile_bucket),
-                                at<uint32_t>(b->state, c.S.bucket_hist), st, true);
-    dmgs::launch_render_bwd(r, st);
-    if ((rc = bcheck("batch render backward", st))) return rc;
+  if (stages & DMGS_STAGE_BLEND) {
+    if ((rc = blend_views_backward(b, c, dL_dimages, st))) return rc;
   }
   if (stages & DMGS_STAGE_GEOMETRY) {
     a.grads = grads;
@@ -439,6 +549,98 @@ int dmgs_batched_backward(const dmgs_batch* b, const float* params, const float*
     if ((rc = bcheck("batch geometry backward", st))) return rc;
   }
   return DMGS_OK;
+}
+
+int dmgs_view_supported(int32_t width, int32_t height) { return view_has_cells(width, height) ? 1 : 0; }
+
+size_t dmgs_view_state_size(int64_t P, int32_t width, int32_t height, int32_t keep) {
+  if (P <= 0 || P > (int64_t)0x7fffffff || !view_has_cells(width, height)) return 0;
+  return ViewLayout(P, width, height, keep != 0).total;
+}
+
+int dmgs_view_geometry(const dmgs_settings* s, const dmgs_gaussians* g, int32_t keep, int32_t* radii, void* state,
+                       uint32_t counts[2], dmgs_stream_t stream) {
+  int rc = check_gaussians(s, g, state);
+  if (rc) return rc;
+  if (!radii || !counts) return bfail(DMGS_EINVAL, "radii and counts are required");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const ViewLayout V(g->count, s->image_width, s->image_height, keep != 0);
+  const dmgs_batch b = view_batch(s, g->count, V, state, 0, nullptr, nullptr);
+  const Ctx c(&b, keep != 0);
+  dmgs::ViewArgs a = view_args(s, g, V);
+  a.view = at<dmgs::ViewDesc>(state, V.record);
+  a.tile_sums = at<uint32_t>(state, V.tile_sums);
+  a.radii = radii;
+  a.splats = at<float4>(state, c.S.splats);
+  a.rects = at<uint2>(state, c.S.rects);
+  a.depth_keys = at<uint32_t>(state, c.S.keys_a);
+  dmgs::launch_view_preprocess(a, st);
+  order_entries(&b, c, false, st);
+  uint32_t* dev = at<uint32_t>(state, V.counts);
+  dmgs::launch_view_counts(c.count(&b), a.tile_sums, dev, st);
+  if ((rc = bcheck("view preprocess / depth sort / scan", st))) return rc;
+  if (hipMemcpyAsync(counts, dev, 8, hipMemcpyDeviceToHost, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
+    return bcheck("view counts", st) ? DMGS_EHIP : bfail(DMGS_EHIP, "reading the instance counts failed");
+  return DMGS_OK;
+}
+
+int dmgs_view_binning(const dmgs_settings* s, int64_t P, int32_t keep, int64_t K, void* state, void* lists,
+                      dmgs_stream_t stream) {
+  if (!s || P <= 0 || K <= 0 || !state || !lists || !view_has_cells(s->image_width, s->image_height))
+    return bfail(DMGS_EINVAL, "invalid view");
+  const ViewLayout V(P, s->image_width, s->image_height, keep != 0);
+  const dmgs_batch b = view_batch(s, P, V, state, K, lists, nullptr);
+  const int rc = check_batch(&b);
+  return rc ? rc : bin_entries(&b, Ctx(&b, keep != 0), false, reinterpret_cast<hipStream_t>(stream));
+}
+
+int dmgs_view_blend(const dmgs_settings* s, int64_t P, int32_t keep, int64_t K, void* state, void* lists, void* bwd_ws,
+                    float* out_color, dmgs_stream_t stream) {
+  if (!s || P <= 0 || K <= 0 || !state || !lists || !out_color || (keep != 0) != (bwd_ws != nullptr) ||
+      !view_has_cells(s->image_width, s->image_height))
+    return bfail(DMGS_EINVAL, "invalid view");
+  const ViewLayout V(P, s->image_width, s->image_height, keep != 0);
+  const dmgs_batch b = view_batch(s, P, V, state, K, lists, bwd_ws);
+  const int rc = check_batch(&b);
+  return rc ? rc : blend_views(&b, Ctx(&b, keep != 0), out_color, reinterpret_cast<hipStream_t>(stream));
+}
+
+int dmgs_view_blend_backward(const dmgs_settings* s, int64_t P, int64_t K, void* state, void* lists, void* bwd_ws,
+                             const float* dL_dout, dmgs_stream_t stream) {
+  if (!s || P <= 0 || K <= 0 || !state || !lists || !bwd_ws || !dL_dout ||
+      !view_has_cells(s->image_width, s->image_height))
+    return bfail(DMGS_EINVAL, "invalid view");
+  const ViewLayout V(P, s->image_width, s->image_height, true);
+  const dmgs_batch b = view_batch(s, P, V, state, K, lists, bwd_ws);
+  const int rc = check_batch(&b);
+  return rc ? rc : blend_views_backward(&b, Ctx(&b), dL_dout, reinterpret_cast<hipStream_t>(stream));
+}
+
+int dmgs_view_geometry_backward(const dmgs_settings* s, const dmgs_gaussians* g, const int32_t* radii,
+                                const void* bwd_ws, const dmgs_gaussian_grads* d, dmgs_stream_t stream) {
+  int rc = check_gaussians(s, g, bwd_ws);
+  if (rc) return rc;
+  if (!radii || !d || !d->means2D || !d->means3D || !d->opacities || (g->shs && !d->shs) ||
+      (g->shs_rest && !d->shs_rest) || (g->scales && (!d->scales || !d->rotations)))
+    return bfail(DMGS_EINVAL, "missing gradients");
+  for (const float* p : {d->shs, d->shs_rest, d->rotations})
+    if (reinterpret_cast<uintptr_t>(p) & 15u) return bfail(DMGS_EINVAL, "gradients must be 16-byte aligned");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const ViewLayout V(g->count, s->image_width, s->image_height, true);
+  dmgs::ViewArgs a = view_args(s, g, V);
+  a.radii = const_cast<int32_t*>(radii);
+  a.gacc = static_cast<const float*>(bwd_ws);
+  a.dL_dmeans2D = d->means2D;
+  a.dL_dmeans3D = d->means3D;
+  a.dL_dopacity = d->opacities;
+  a.dL_dsh = d->shs;
+  a.dL_dsh_rest = d->shs_rest;
+  a.dL_dcolors = d->colors;
+  a.dL_dcov3D = d->cov3D;
+  a.dL_dscales = d->scales;
+  a.dL_drotations = d->rotations;
+  dmgs::launch_view_geometry_bwd(a, st);
+  return bcheck("view geometry backward", st);
 }
 
 }  // extern "C"

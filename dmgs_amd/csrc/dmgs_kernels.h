@@ -153,6 +153,51 @@ void launch_gather_rects(const uint2* rects, const uint32_t* order, uint2* rects
 // the accumulator; the blend backward filled it).
 void launch_mv_geometry_bwd(const MVArgs& a, hipStream_t s);
 
+// ---- one view over a model's own tensors (view.hip) ----
+#define DMGS_RAW_SCALES 1     // scales are log-scales
+#define DMGS_RAW_ROTATIONS 2  // rotations are not normalised
+#define DMGS_RAW_OPACITIES 4  // opacities are logits
+constexpr int kTileSums = 64;
+struct ViewArgs {
+  int P, W, H, grid_x, grid_y;
+  float tanfovx, tanfovy, focal_x, focal_y, scale_modifier;
+  int sh_degree, sh_coeffs, raw;
+  const float* means3D;
+  const float* scales;
+  const float* rotations;
+  const float* opacities;
+  const float* shs;             // (P, M, 3), or (P, 1, 3) beside shs_rest
+  const float* shs_rest;        // (P, M - 1, 3) with M 4, 9 or 16, or null
+  const float* colors_precomp;
+  const float* cov3D_precomp;
+  const float* viewmatrix;
+  const float* projmatrix;
+  const float* campos;
+  const float* bg;
+  // forward outputs
+  ViewDesc* view;               // the view's record for the list and blend kernels
+  uint32_t* tile_sums;          // kTileSums partial sums of tiles touched
+  int32_t* radii;
+  float4* splats;
+  uint2* rects;
+  uint32_t* depth_keys;         // kSortSkip for culled Gaussians
+  // backward
+  const float* gacc;
+  float* dL_dmeans2D;
+  float* dL_dmeans3D;
+  float* dL_dopacity;
+  float* dL_dsh;                // like shs
+  float* dL_dsh_rest;
+  float* dL_dcolors;            // these may be null
+  float* dL_dcov3D;
+  float* dL_dscales;
+  float* dL_drotations;
+};
+void launch_view_preprocess(const ViewArgs& a, hipStream_t s);
+// counts[0] = *cells, counts[1] = the sum of tile_sums
+void launch_view_counts(const uint32_t* cells, const uint32_t* tile_sums, uint32_t* counts, hipStream_t s);
+void launch_view_geometry_bwd(const ViewArgs& a, hipStream_t s);
+
 // ---- blend ----
 // List segments that a forward keeps for its backward (render.hip).  At most kSegmentTiles tiles: with 8160
 // tiles (1920x1080) keeping them costs as much as it gives (forward + backward of 1M Gaussians 335 us with,

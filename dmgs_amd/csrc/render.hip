@@ -30,9 +30,9 @@
 // running totals would lose it).  That is the whole state of the backward recursion at the boundary, so
 // every 64-member segment is a work-group of its own.  Slots (4 KB) come from a counter; a tile that gets
 // none has a longer last segment.  Launches of more than kSegmentTiles tiles fill the GPU without it.
-// Blend backward of one view, us, before and after (MI355X): 10k Gaussians at 200x200 375 -> 77, 1M at
-// 800x800 225 -> 107, 491k face-bound at 800x800 1385 -> 216, 500k at 333x251 1731 -> 177 (their forwards
-// get 7-45 us longer: the states are written, summed and cleared).
+// Blend backward of one view, us, before and after (MI355X): 10k Gaussians at 200x200 375 -> 80, 1M at
+// 800x800 225 -> 105, 491k face-bound at 800x800 1385 -> 234, 500k at 333x251 1731 -> 173 (their forwards
+// get 12-43 us longer: the states are written, summed and cleared).
 #include "dmgs_common.h"
 #include "dmgs_kernels.h"
 
@@ -306,7 +306,7 @@ __device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile) {
   int list = c.tile;
   c.bit = 0;
   if (a.views) {
-    const ViewDesc& v = a.views[a.tile_view[c.tile]];
+    const ViewDesc& v = a.views[a.tile_view ? a.tile_view[c.tile] : 0];
     lt = c.tile - v.tile_base;
     gx = v.grid_x;
     const int ltx = lt % gx, lty = lt / gx;
@@ -415,11 +415,11 @@ struct FwdGroup {
   float4 xyq[kN], qorg[kN];
 };
 
-// One list position per lane of a 256-lane work-group: the members of the tile (every position of a
-// single view's list; the instances of a cell list whose mask holds the tile's bit) are packed, in list
-// order, into id[] / pos[].
+// The members of a tile in one chunk of its list (every position of a single view's tile list; the instances
+// of a cell list whose mask holds the tile's bit), packed in list order.
+template <int N>
 struct MemberList {
-  uint32_t id[256], pos[256];
+  uint32_t id[N], pos[N];
 };
 
 // Forward: four waves per 16x16 tile, one pixel per lane, wave k covering the 8x8 quadrant k.  VALU issue
@@ -428,8 +428,8 @@ struct MemberList {
 // instructions of any kind as possible: each wave first packs the LDS offsets of the staged splats that reach
 // its quadrant, then takes four at a time, reading the next four while it evaluates the four alphas (whose
 // latencies overlap) and applies them in order with selects instead of branches.  Against one wave per tile
-// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 310 us, 16 uneven views of 3M
-// 5.33 -> 4.21 ms, one 800x800 view 154 -> 53 us, 333x251 of 500k 1377 -> 364 us.  Quadrants because a splat
+// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 325 us, 16 uneven views of 3M
+// 5.33 -> 3.51 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
 // reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on KEEP,
 // CELLS or the launch.
 template <bool CELLS, bool KEEP>
@@ -438,8 +438,9 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
   constexpr int G = KEEP ? 64 : NT;  // staged splats blended per round
   constexpr int kPad = NT * 16;      // offset of the filling splat
   __shared__ FwdSplats<NT + 1> L;    // slot NT: a splat of zero opacity, which fills up groups
-  __shared__ MemberList M;
-  __shared__ uint32_t s_wc[2][NT / DMGS_WAVE];
+  constexpr int C = CELLS ? 4 : 1;   // list positions per lane and chunk
+  __shared__ MemberList<C * NT> M;
+  __shared__ uint32_t s_wc[2][C][NT / DMGS_WAVE];
   __shared__ uint32_t s_slot[KEEP ? kTileSegments : 1];
   __shared__ __align__(16) uint32_t s_reach[NT / DMGS_WAVE][G + 12];
   const TileCtx c = tile_ctx<true>(a, ordered_tile(a, blockIdx.x));
@@ -457,63 +458,95 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
   float D0 = 0.f, D1 = 0.f, D2 = 0.f;
   int seg_begin = 0, seg_members = 0, segs = 0;
 
-  // The list is taken 256 positions at a time, in three overlapping steps: the keys and ids of one chunk
-  // are on their way while the records of the chunk before it are, and while the one before that is blended.
-  uint32_t key = 0, id = 0;
-  auto request = [&](int at) {  // positions past the list read its first entry and are no members
-    const uint32_t p = c.range.x + (at + (int)threadIdx.x < len ? (uint32_t)(at + (int)threadIdx.x) : 0u);
-    if constexpr (CELLS) key = a.list_keys[p];
-    id = a.point_list[p];
-  };
-  // packs the chunk at `at`; returns the number of members (the barrier that follows is the caller's)
-  int flip = 0;
-  auto pack = [&](int at) {
-    const int q = at + (int)threadIdx.x;
-    const bool member = q < len && (!CELLS || ((key >> DMGS_CELL_KEY_BITS) & c.bit));
-    const uint64_t bal = __ballot(member);
-    if (lane == 0) s_wc[flip][wave] = (uint32_t)__popcll(bal);
-    __syncthreads();
-    int before = (int)__popcll(bal & lanemask_lt()), total = 0;
+  // Three overlapping steps: the keys and ids of a chunk of the list are on their way while the records of
+  // the next 256 members are, and while the 256 before those are blended.  A chunk of a cell list is four
+  // positions per lane: about a third of them are members, and a round of fewer than 256 costs as much to
+  // stage.  One position per lane: one view of 333x251 of 500k Gaussians 364 us (195 with four), 16 uneven views
+  // 4.21 ms (3.51); two: 255 us and 3.69 ms; on shallow lists (8 views of 800x800) the three are within 4 %.
+  uint32_t key[C], id[C];
+  int next_chunk = 0;  // the first position not asked for
+  auto request = [&]() {  // positions past the list read its first entry and are no members
 #pragma unroll
-    for (int w = 0; w < NT / DMGS_WAVE; ++w) {
-      const int cnt = (int)s_wc[flip][w];
-      before += w < wave ? cnt : 0;
-      total += cnt;
+    for (int k = 0; k < C; ++k) {
+      const int q = next_chunk + k * NT + (int)threadIdx.x;
+      const uint32_t p = c.range.x + (q < len ? (uint32_t)q : 0u);
+      if constexpr (CELLS) key[k] = a.list_keys[p];
+      id[k] = a.point_list[p];
+    }
+    next_chunk += C * NT;
+  };
+  // packs the requested chunk; returns the number of members (the barrier that follows is the caller's)
+  int flip = 0;
+  auto pack = [&]() {
+    const int at = next_chunk - C * NT;
+    uint64_t bal[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const bool member = at + k * NT + (int)threadIdx.x < len && (!CELLS || ((key[k] >> DMGS_CELL_KEY_BITS) & c.bit));
+      bal[k] = __ballot(member);
+      if (lane == 0) s_wc[flip][k][wave] = (uint32_t)__popcll(bal[k]);
+    }
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      int before = total + (int)__popcll(bal[k] & lanemask_lt());
+#pragma unroll
+      for (int w = 0; w < NT / DMGS_WAVE; ++w) {
+        const int cnt = (int)s_wc[flip][k][w];
+        before += w < wave ? cnt : 0;
+        total += cnt;
+      }
+      if ((bal[k] >> lane) & 1u) {
+        M.id[before] = id[k];
+        M.pos[before] = (uint32_t)(at + k * NT + (int)threadIdx.x);
+      }
     }
     flip ^= 1;
-    if (member) {
-      M.id[before] = id;
-      M.pos[before] = (uint32_t)q;
-    }
     return total;
   };
-  float4 r0, r1, r2;  // this lane's record of the packed chunk
+  float4 r0, r1, r2;  // this lane's record of the next round
   uint32_t my_id = 0, my_pos = 0;
-  auto gather = [&](int n) {
-    const int s = min((int)threadIdx.x, max(n - 1, 0));  // no lane's loads are conditional
-    my_id = M.id[s];
-    my_pos = M.pos[s];
+  int members = 0, used = 0;  // of the packed chunk: all, and those whose records were asked for
+  auto gather = [&]() {
+    const int n = min(NT, members - used);
+    const int s = used + min((int)threadIdx.x, max(n - 1, 0));  // no lane's loads are conditional
+    my_id = M.id[min(s, C * NT - 1)];
+    my_pos = M.pos[min(s, C * NT - 1)];
     const float4* sp = a.splats + (size_t)DMGS_SPLAT_F4 * min(my_id, a.P - 1);
     r0 = sp[0];
     r1 = sp[1];
     r2 = sp[2];
+    used += n;
+    return n;
   };
-  int n_next = 0;  // members of the chunk whose records are on their way
+  int n_next = 0;  // members whose records are on their way
+  bool asked = false;  // a chunk is on its way
+  auto ask = [&]() {  // only once the packed one runs out: a tile may be finished before
+    if (used == members && next_chunk < len) {
+      request();
+      asked = true;
+    }
+  };
   if (len > 0) {
-    request(0);
-    n_next = pack(0);
+    request();
+    members = pack();
     __syncthreads();
-    gather(n_next);
-    request(NT);
+    n_next = gather();
+    ask();
   }
-  for (int at = 0; at < len; at += NT) {
+  while (n_next > 0 || asked) {
     if (__syncthreads_count(T < 0.f) == NT) break;
     const int n = n_next;
     if ((int)threadIdx.x < n) put_splat(L, threadIdx.x, r0, r1, r2, my_id, a.P, c.rows, my_pos + 1);
-    n_next = pack(at + NT);  // its barrier also orders the records; no members past the list
+    if (asked) {
+      members = pack();  // its barrier also orders the records
+      used = 0;
+      asked = false;
+    }
     __syncthreads();
-    gather(n_next);
-    request(at + 2 * NT);
+    n_next = gather();
+    ask();
     if constexpr (KEEP) {
       // segment boundaries inside this chunk: before a round, once enough members have passed
       int want = 0, m = seg_members;
@@ -680,12 +713,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       const uint4 r = a.seg.rec[blockIdx.x];
       if (r.x >= (uint32_t)a.num_tiles) return;  // never used
       tile = (int)r.x;
-      lo = (int)r.y;
+      lo = max((int)r.y, 0);
       hi = (int)r.z;
       seg_end = blockIdx.x;
     } else {
       tile = (int)blockIdx.x - a.seg.cap;
-      if (kept) lo = (int)a.seg.tile_last[tile];
+      if (kept) lo = max((int)a.seg.tile_last[tile], 0);
     }
   } else {
     tile = ordered_tile(a, blockIdx.x);
@@ -854,7 +887,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 // (8 buckets per octave, 256 in all) and emitted heaviest bucket first.  Only
 // the dispatch order changes; every tile's result is the same in any order.
 __device__ __forceinline__ uint32_t tile_cost_bucket(const RenderArgs& a, int t, uint32_t K, bool use_work) {
-  const ViewDesc& v = a.views[a.tile_view[t]];
+  const ViewDesc& v = a.views[a.tile_view ? a.tile_view[t] : 0];
   const int lt = t - v.tile_base, gx = v.grid_x;
   const int ltx = lt % gx, lty = lt / gx;
   const int cell = v.cell_base + (lty >> DMGS_CELL_SHIFT) * cells_x(gx) + (ltx >> DMGS_CELL_SHIFT);

@@ -1,0 +1,471 @@
+// Per-Gaussian stages of one view over a model's own tensors, for gfx950.
+//
+// The drop-in renderer takes one camera and the tensors a model holds, (P, k) rows; the lists, the blend and
+// the sorts are the batched engine's with one view.  Two things are done here so that no pass over HBM exists
+// only to prepare an input:
+//   * activations: scales may be log-scales, rotations raw quaternions and opacities logits (DMGS_RAW_*); the
+//     exp, normalisation and sigmoid then run in these kernels, rounded exactly as torch rounds them, and the
+//     backward returns raw gradients;
+//   * SH coefficients may come as two tensors, (P, 1, 3) and (P, M - 1, 3).  A row of the second is 180 bytes
+//     at degree 3, which no aligned vector load fits, so a work-group copies its 256 rows through LDS with
+//     16-byte accesses and its lanes read them there (odd row strides: no bank conflicts).
+// The math is the single-view kernels' (gs_math.h).  The forward's is written out with every fused
+// multiply-add named and contraction off, in the order the compiler gives preprocess_fwd_kernel: which of two
+// products it fuses depends on the surrounding code, and a last-bit difference in a covariance changes a few
+// radii in a million Gaussians and the pixels that sit on a blend threshold.  So this route's radii and images
+// equal the per-tile-list route's bit for bit, whatever surrounds the arithmetic.
+#include "dmgs_common.h"
+#include "dmgs_kernels.h"
+#include "gs_math.h"
+
+namespace dmgs {
+
+constexpr int kRows = 256;  // Gaussians per work-group
+
+// kRows rows of R floats in LDS at an odd row stride.
+template <int R>
+struct LdsRows {
+  static constexpr int S = R % 2 ? R : R + 1;
+  __align__(16) float v[kRows * S];
+  __device__ __forceinline__ float* row(int t) { return v + t * S; }
+  // rows [0, n) from / to consecutive global rows (16-byte aligned: the first row is a multiple of kRows)
+  __device__ __forceinline__ void load(const float* __restrict__ src, int n) {
+    const int f4 = n * R / 4, rest = n * R - 4 * f4;
+    const float4* s4 = reinterpret_cast<const float4*>(src);
+    if (f4 > 0) {
+      constexpr int kIter = (kRows * R / 4 + kRows - 1) / kRows;
+      float4 x[kIter];  // every load before the first LDS store; positions past the end read the last vector
+#pragma unroll
+      for (int i = 0; i < kIter; ++i) x[i] = s4[min(i * kRows + (int)threadIdx.x, f4 - 1)];
+#pragma unroll
+      for (int i = 0; i < kIter; ++i) {
+        const int f = i * kRows + (int)threadIdx.x;
+        if (f < f4) put4(f, x[i]);
+      }
+    }
+    if ((int)threadIdx.x < rest) at(4 * f4 + (int)threadIdx.x) = src[4 * f4 + threadIdx.x];
+  }
+  __device__ __forceinline__ void store(float* __restrict__ dst, int n) {
+    const int f4 = n * R / 4, rest = n * R - 4 * f4;
+    float4* d4 = reinterpret_cast<float4*>(dst);
+    for (int f = threadIdx.x; f < f4; f += kRows) d4[f] = get4(f);
+    if ((int)threadIdx.x < rest) dst[4 * f4 + threadIdx.x] = at(4 * f4 + (int)threadIdx.x);
+  }
+
+ private:
+  __device__ __forceinline__ float& at(int e) {
+    if constexpr (S == R) return v[e];
+    return v[e / R * S + e % R];
+  }
+  __device__ __forceinline__ void put4(int f, float4 x) {
+    if constexpr (S == R) {
+      reinterpret_cast<float4*>(v)[f] = x;
+    } else {
+      at(4 * f) = x.x;
+      at(4 * f + 1) = x.y;
+      at(4 * f + 2) = x.z;
+      at(4 * f + 3) = x.w;
+    }
+  }
+  __device__ __forceinline__ float4 get4(int f) {
+    if constexpr (S == R) return reinterpret_cast<float4*>(v)[f];
+    return make_float4(at(4 * f), at(4 * f + 1), at(4 * f + 2), at(4 * f + 3));
+  }
+};
+
+__device__ __forceinline__ float view_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
+
+// torch.nn.functional.normalize of a row of four: the norm's pairwise sum without contraction, clamped
+__device__ __forceinline__ float quat_norm(float4 q) {
+#pragma clang fp contract(off)
+  return fmaxf(sqrtf((q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w)), 1e-12f);
+}
+
+// One Gaussian's SH coefficients: the first three from registers, the others from its LDS row.
+struct ShSplit {
+  const float* dc;
+  const float* rest;
+  int n;
+  __device__ __forceinline__ float operator[](int k) const { return k < 3 ? dc[k] : (k - 3 < n ? rest[k - 3] : 0.f); }
+};
+struct ShRow {
+  const float* row;
+  int n;
+  __device__ __forceinline__ float operator[](int k) const { return k < n ? row[k] : 0.f; }
+};
+
+struct ViewGaussian {
+  float3 e, s;   // scale, modifier x scale
+  float4 q;      // rotation as the covariance uses it
+  float qn;      // norm of the raw quaternion
+  float R[9], c3[6];
+};
+
+// Rotation matrix and Sigma = R diag(s)^2 R^T (quat_to_R, cov3d_from_sR).
+__device__ __forceinline__ void view_cov3d(ViewGaussian& G) {
+#pragma clang fp contract(off)
+  const float r = G.q.x, x = G.q.y, y = G.q.z, z = G.q.w;
+  const float zz = z * z, rz = r * z, ry = r * y, yz = y * z, yy = y * y;
+  float* R = G.R;
+  R[0] = fmaf(fmaf(y, y, zz), -2.0f, 1.0f);
+  R[1] = 2.0f * fmaf(x, y, -rz);
+  R[2] = 2.0f * fmaf(x, z, ry);
+  R[3] = 2.0f * fmaf(x, y, rz);
+  R[4] = fmaf(fmaf(x, x, zz), -2.0f, 1.0f);
+  R[5] = 2.0f * fmaf(-r, x, yz);
+  R[6] = 2.0f * fmaf(x, z, -ry);
+  R[7] = 2.0f * fmaf(r, x, yz);
+  R[8] = fmaf(fmaf(x, x, yy), -2.0f, 1.0f);
+  const float M00 = G.s.x * R[0], M01 = G.s.y * R[1], M02 = G.s.z * R[2];
+  const float M10 = G.s.x * R[3], M11 = G.s.y * R[4], M12 = G.s.z * R[5];
+  const float M20 = G.s.x * R[6], M21 = G.s.y * R[7], M22 = G.s.z * R[8];
+  G.c3[0] = fmaf(M02, M02, fmaf(M01, M01, M00 * M00));
+  G.c3[1] = fmaf(M02, M12, fmaf(M10, M00, M01 * M11));
+  G.c3[2] = fmaf(M02, M22, fmaf(M01, M21, M20 * M00));
+  G.c3[3] = fmaf(M12, M12, fmaf(M10, M10, M11 * M11));
+  G.c3[4] = fmaf(M12, M22, fmaf(M10, M20, M21 * M11));
+  G.c3[5] = fmaf(M22, M22, fmaf(M20, M20, M21 * M21));
+}
+
+// project_splat of gs_math.h.
+__device__ __forceinline__ bool view_project(float3 p, const float (&c)[6], const ViewParams& v, SplatGeom& o) {
+#pragma clang fp contract(off)
+  const float* vm = v.vm;
+  const float* pm = v.pm;
+  const float tz = fmaf(vm[10], p.z, fmaf(vm[2], p.x, vm[6] * p.y)) + vm[14];
+  if (tz <= 0.2f) return false;
+  const float tx0 = fmaf(vm[8], p.z, fmaf(vm[4], p.y, vm[0] * p.x)) + vm[12];
+  const float ty0 = fmaf(vm[9], p.z, fmaf(vm[5], p.y, vm[1] * p.x)) + vm[13];
+  const float limx = 1.3f * v.tanx, limy = 1.3f * v.tany;
+  const float tx = fminf(limx, fmaxf(-limx, tx0 / tz)) * tz;
+  const float ty = fminf(limy, fmaxf(-limy, ty0 / tz)) * tz;
+  const float iz = 1.0f / tz, iz2 = iz * iz;
+  const float j00 = v.fx * iz, j02 = -(v.fx * tx) * iz2;
+  const float j11 = v.fy * iz, j12 = -(v.fy * ty) * iz2;
+  const float m00 = fmaf(j00, vm[0], j02 * vm[2]), m01 = fmaf(j00, vm[4], j02 * vm[6]);
+  const float m02 = fmaf(j00, vm[8], j02 * vm[10]);
+  const float m10 = fmaf(j11, vm[1], j12 * vm[2]), m11 = fmaf(j11, vm[5], j12 * vm[6]);
+  const float m12 = fmaf(j11, vm[9], j12 * vm[10]);
+  const float s0x = fmaf(c[2], m02, fmaf(c[0], m00, c[1] * m01));
+  const float s0y = fmaf(c[4], m02, fmaf(c[1], m00, c[3] * m01));
+  const float s0z = fmaf(c[5], m02, fmaf(c[2], m00, c[4] * m01));
+  const float s1x = fmaf(c[2], m12, fmaf(c[0], m10, c[1] * m11));
+  const float s1y = fmaf(c[4], m12, fmaf(c[1], m10, c[3] * m11));
+  const float s1z = fmaf(c[5], m12, fmaf(c[2], m10, c[4] * m11));
+  const float ca = fmaf(m02, s0z, fmaf(m00, s0x, m01 * s0y)) + 0.3f;
+  const float cb = fmaf(m12, s0z, fmaf(m10, s0x, m11 * s0y));
+  const float cc = fmaf(m12, s1z, fmaf(m10, s1x, m11 * s1y)) + 0.3f;
+  const float det = fmaf(cc, ca, -(cb * cb));
+  if (det == 0.0f) return false;
+  const float phw = (fmaf(pm[11], p.z, fmaf(pm[3], p.x, pm[7] * p.y)) + pm[15]) + 0.0000001f;
+  const float phx = fmaf(pm[8], p.z, fmaf(pm[0], p.x, pm[4] * p.y)) + pm[12];
+  const float phy = fmaf(pm[9], p.z, fmaf(pm[1], p.x, pm[5] * p.y)) + pm[13];
+  const float pw = 1.0f / phw, det_inv = 1.0f / det;
+  const float sum = ca + cc, mid = 0.5f * sum;
+  const float disc = sqrtf(fmaxf(0.1f, fmaf(mid, mid, -det)));
+  const float radius = ceilf(3.f * sqrtf(fmaxf(fmaf(0.5f, sum, disc), fmaf(0.5f, sum, -disc))));
+  o.pix = make_float2(0.5f * fmaf(fmaf(phx, pw, 1.0f), (float)v.W, -1.0f),
+                      0.5f * fmaf(fmaf(phy, pw, 1.0f), (float)v.H, -1.0f));
+  tile_rect(o.pix, (int)radius, v.gx, v.gy, o.rmin, o.rmax);
+  o.tiles = (o.rmax.x - o.rmin.x) * (o.rmax.y - o.rmin.y);
+  if (o.tiles == 0) return false;
+  o.conic = make_float3(cc * det_inv, -cb * det_inv, ca * det_inv);
+  o.radius = (int)radius;
+  o.depth = tz;
+  return true;
+}
+
+// sh_to_rgb of gs_math.h with the view direction, clamped at zero.
+template <typename SH>
+__device__ __forceinline__ float3 view_rgb(int deg, const SH& sh, float3 p, const float (&campos)[3]) {
+#pragma clang fp contract(off)
+  float3 r = make_float3(kSH_C0 * sh[0], kSH_C0 * sh[1], kSH_C0 * sh[2]);
+  auto add = [&](int k, float b) {
+    r = make_float3(fmaf(b, sh[3 * k], r.x), fmaf(b, sh[3 * k + 1], r.y), fmaf(b, sh[3 * k + 2], r.z));
+  };
+  if (deg > 0) {
+    const float dx = p.x - campos[0], dy = p.y - campos[1], dz = p.z - campos[2];
+    const float inv = 1.0f / sqrtf(fmaf(dz, dz, fmaf(dx, dx, dy * dy)));
+    const float x = dx * inv, y = dy * inv, z = dz * inv;
+    const float b1 = -kSH_C1 * y, b2 = kSH_C1 * z, b3 = -kSH_C1 * x;
+    r = make_float3(fmaf(b3, sh[9], fmaf(b2, sh[6], b1 * sh[3])) + r.x, fmaf(b3, sh[10], fmaf(b2, sh[7], b1 * sh[4])) + r.y,
+                    fmaf(b3, sh[11], fmaf(b2, sh[8], b1 * sh[5])) + r.z);
+    if (deg > 1) {
+      const float xx = x * x, yy = y * y, zz = z * z, xy = x * y, yz = y * z, xz = x * z;
+      const float d = fmaf(x, x, -yy);
+      add(4, kSH_C2[0] * xy);
+      add(5, kSH_C2[1] * yz);
+      add(6, kSH_C2[2] * fmaf(-y, y, fmaf(zz, 2.0f, -xx)));
+      add(7, kSH_C2[3] * xz);
+      add(8, kSH_C2[4] * d);
+      if (deg > 2) {
+        const float q = fmaf(zz, 4.0f, -xx) - yy;
+        add(9, (kSH_C3[0] * y) * fmaf(xx, 3.0f, -yy));
+        add(10, z * (kSH_C3[1] * xy));
+        add(11, (kSH_C3[2] * y) * q);
+        add(12, (kSH_C3[3] * z) * fmaf(-3.0f, yy, fmaf(-3.0f, xx, zz + zz)));
+        add(13, (kSH_C3[4] * x) * q);
+        add(14, (kSH_C3[5] * z) * d);
+        add(15, (kSH_C3[6] * x) * fmaf(-3.0f, yy, xx));
+      }
+    }
+  }
+  return make_float3(fmaxf(r.x + 0.5f, 0.0f), fmaxf(r.y + 0.5f, 0.0f), fmaxf(r.z + 0.5f, 0.0f));
+}
+
+__device__ __forceinline__ void load_shape(const ViewArgs& a, int g, ViewGaussian& G) {
+  if (a.cov3D_precomp) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) G.c3[k] = a.cov3D_precomp[6 * (size_t)g + k];
+    return;
+  }
+  G.e = make_float3(a.scales[3 * (size_t)g], a.scales[3 * (size_t)g + 1], a.scales[3 * (size_t)g + 2]);
+  if (a.raw & DMGS_RAW_SCALES) G.e = make_float3(expf(G.e.x), expf(G.e.y), expf(G.e.z));
+  const float m = a.scale_modifier;
+  G.s = make_float3(m * G.e.x, m * G.e.y, m * G.e.z);
+  G.q = reinterpret_cast<const float4*>(a.rotations)[g];
+  G.qn = 1.0f;
+  if (a.raw & DMGS_RAW_ROTATIONS) {
+    G.qn = quat_norm(G.q);
+    G.q = make_float4(G.q.x / G.qn, G.q.y / G.qn, G.q.z / G.qn, G.q.w / G.qn);
+  }
+  view_cov3d(G);
+}
+
+__global__ __launch_bounds__(64) void view_setup_kernel(ViewArgs a) {
+  const int t = threadIdx.x;
+  ViewDesc& v = *a.view;
+  a.tile_sums[t] = 0u;
+  if (t < 16) {
+    v.view[t] = a.viewmatrix[t];
+    v.proj[t] = a.projmatrix[t];
+  }
+  if (t < 4) {
+    v.campos[t] = t < 3 ? a.campos[t] : 0.f;
+    v.bg[t] = t < 3 ? a.bg[t] : 0.f;
+  }
+  if (t == 0) {
+    v.tanfovx = a.tanfovx;
+    v.tanfovy = a.tanfovy;
+    v.focal_x = a.focal_x;
+    v.focal_y = a.focal_y;
+    v.W = a.W;
+    v.H = a.H;
+    v.grid_x = a.grid_x;
+    v.grid_y = a.grid_y;
+    v.tile_base = v.cell_base = 0;
+    v.pixel_base = 0;
+  }
+}
+
+// REST: floats in a row of the second SH tensor (3 (M - 1)), or -1: one SH tensor of any M, or given colours.
+template <int REST>
+__global__ __launch_bounds__(kRows) void view_preprocess_kernel(ViewArgs a) {
+  __shared__ LdsRows<(REST > 0 ? REST : 1)> rows;
+  __shared__ uint32_t s_tiles;
+  const int g0 = blockIdx.x * kRows, g = g0 + (int)threadIdx.x;
+  if (threadIdx.x == 0) s_tiles = 0u;
+  if constexpr (REST > 0) rows.load(a.shs_rest + (size_t)g0 * REST, min(kRows, a.P - g0));
+  __syncthreads();
+  uint32_t tiles = 0;
+  if (g < a.P) {
+    const float3 p = make_float3(a.means3D[3 * (size_t)g], a.means3D[3 * (size_t)g + 1], a.means3D[3 * (size_t)g + 2]);
+    ViewGaussian G;
+    load_shape(a, g, G);
+    const ViewParams v = view_params(a.viewmatrix, a.projmatrix, a.campos, a.W, a.H, a.grid_x, a.grid_y, a.focal_x,
+                                     a.focal_y, a.tanfovx, a.tanfovy);
+    SplatGeom o;
+    if (!view_project(p, G.c3, v, o)) {
+      a.radii[g] = 0;
+      a.depth_keys[g] = kSortSkip;
+    } else {
+      float3 rgb;
+      if (a.colors_precomp) {
+        rgb = make_float3(a.colors_precomp[3 * (size_t)g], a.colors_precomp[3 * (size_t)g + 1],
+                          a.colors_precomp[3 * (size_t)g + 2]);
+      } else {
+        if constexpr (REST >= 0) {
+          const float dc[3] = {a.shs[3 * (size_t)g], a.shs[3 * (size_t)g + 1], a.shs[3 * (size_t)g + 2]};
+          rgb = view_rgb(a.sh_degree, ShSplit{dc, rows.row(threadIdx.x), REST}, p, v.campos);
+        } else {
+          float sh[48];
+          load_sh16(a.shs + (size_t)g * a.sh_coeffs * 3, a.sh_coeffs, sh);
+          rgb = view_rgb(a.sh_degree, sh, p, v.campos);
+        }
+      }
+      const float op = a.opacities[g];
+      float4* sp = a.splats + (size_t)DMGS_SPLAT_F4 * g;
+      sp[0] = make_float4(o.pix.x, o.pix.y, o.conic.x, o.conic.y);
+      sp[1] = make_float4(o.conic.z, a.raw & DMGS_RAW_OPACITIES ? view_sigmoid(op) : op, rgb.x, rgb.y);
+      sp[2] = make_float4(rgb.z, o.depth, __int_as_float(o.radius), 0.0f);
+      a.radii[g] = o.radius;
+      a.rects[g] = pack_rect(o.rmin, o.rmax);
+      a.depth_keys[g] = __float_as_uint(o.depth);
+      tiles = (uint32_t)o.tiles;
+    }
+  }
+  if (tiles) atomicAdd(&s_tiles, tiles);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_tiles) atomicAdd(&a.tile_sums[blockIdx.x % kTileSums], s_tiles);
+}
+
+__global__ __launch_bounds__(64) void view_counts_kernel(const uint32_t* __restrict__ cells,
+                                                         const uint32_t* __restrict__ tile_sums,
+                                                         uint32_t* __restrict__ counts) {
+  uint32_t x = tile_sums[threadIdx.x];
+  for (int off = 32; off > 0; off >>= 1) x += (uint32_t)__shfl_xor((int)x, off, 64);
+  if (threadIdx.x == 0) {
+    counts[0] = *cells;
+    counts[1] = x;
+  }
+}
+
+// The blend backward's accumulator to the gradients of the model's tensors.
+// SPLIT: two SH tensors of 1 and M - 1 coefficients; M = 0: given colours; M < 0: one SH tensor of any M.
+template <int M, bool SPLIT>
+__global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
+  constexpr int R = M > 0 ? (SPLIT ? 3 * (M - 1) : 3 * M) : 0;
+  __shared__ LdsRows<(R > 0 ? R : 1)> rows;
+  const int g0 = blockIdx.x * kRows, g = g0 + (int)threadIdx.x;
+  const int n = min(kRows, a.P - g0);
+  if constexpr (R > 0) rows.load((SPLIT ? a.shs_rest : a.shs) + (size_t)g0 * R, n);
+  const bool live = g < a.P;
+  const size_t i = live ? (size_t)g : 0;
+  const float2* gg = reinterpret_cast<const float2*>(a.gacc + gacc_index(a.P, i, 0));
+  const float2 r0 = gg[0], r1 = gg[1], r2 = gg[2];
+  const float* gc = a.gacc + gacc_index(a.P, i, DMGS_GACC_GEO);
+  const float3 dcol = make_float3(gc[0], gc[1], gc[2]);
+  const bool vis = live && a.radii[i] > 0;
+  const float3 p = make_float3(a.means3D[3 * i], a.means3D[3 * i + 1], a.means3D[3 * i + 2]);
+  float3 dmean = make_float3(0.f, 0.f, 0.f), ds = dmean;
+  float4 dq = make_float4(0.f, 0.f, 0.f, 0.f);
+  float dc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const ViewParams v = view_params(a.viewmatrix, a.projmatrix, a.campos, a.W, a.H, 0, 0, a.focal_x, a.focal_y,
+                                   a.tanfovx, a.tanfovy);
+  if (vis) {
+    ViewGaussian G;
+    load_shape(a, g, G);
+    dmean = ewa_backward(p, G.c3, v, r0.x, r0.y, r1.x, r1.y, r2.x, dc);
+    if (!a.cov3D_precomp) {
+      cov3d_backward(dc, G.s, G.R, G.q, ds, dq);
+      if (a.raw & DMGS_RAW_SCALES)  // scale = exp(log-scale)
+        ds = make_float3(ds.x * G.e.x, ds.y * G.e.y, ds.z * G.e.z);
+      if (a.raw & DMGS_RAW_ROTATIONS) {  // q = raw / max(|raw|, 1e-12)
+        const float qd = G.qn > 1e-12f ? G.q.x * dq.x + G.q.y * dq.y + G.q.z * dq.z + G.q.w * dq.w : 0.f;
+        dq = make_float4((dq.x - G.q.x * qd) / G.qn, (dq.y - G.q.y * qd) / G.qn, (dq.z - G.q.z * qd) / G.qn,
+                         (dq.w - G.q.w * qd) / G.qn);
+      }
+    }
+  }
+  if constexpr (M != 0) {
+    float b[16];
+    float3 gm = make_float3(0.f, 0.f, 0.f), dd = gm;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) b[k] = 0.f;
+    if constexpr (M > 0) {
+      __syncthreads();  // the rows are in LDS
+      float* row = rows.row(threadIdx.x);
+      if (vis) {
+        if constexpr (SPLIT) {
+          const float c0[3] = {a.shs[3 * i], a.shs[3 * i + 1], a.shs[3 * i + 2]};
+          dd = sh_backward(a.sh_degree, ShSplit{c0, row, R}, p, v.campos, dcol, b, gm);
+        } else {
+          dd = sh_backward(a.sh_degree, ShRow{row, R}, p, v.campos, dcol, b, gm);
+        }
+      }
+      // the lane's row becomes its gradient
+#pragma unroll
+      for (int k = SPLIT ? 1 : 0; k < M; ++k) {
+        const int o = 3 * (SPLIT ? k - 1 : k);
+        row[o] = b[k] * gm.x;
+        row[o + 1] = b[k] * gm.y;
+        row[o + 2] = b[k] * gm.z;
+      }
+      if (SPLIT && live) {
+        a.dL_dsh[3 * i] = b[0] * gm.x;
+        a.dL_dsh[3 * i + 1] = b[0] * gm.y;
+        a.dL_dsh[3 * i + 2] = b[0] * gm.z;
+      }
+      __syncthreads();
+      if constexpr (R > 0) rows.store((SPLIT ? a.dL_dsh_rest : a.dL_dsh) + (size_t)g0 * R, n);
+    } else if (live) {
+      if (vis) {
+        float sh[48];
+        load_sh16(a.shs + i * 3 * a.sh_coeffs, a.sh_coeffs, sh);
+        dd = sh_backward(a.sh_degree, sh, p, v.campos, dcol, b, gm);
+      }
+      float* d = a.dL_dsh + i * 3 * a.sh_coeffs;
+      for (int k = 0; k < a.sh_coeffs; ++k) {
+        float bk = 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) bk = j == k ? b[j] : bk;
+        d[3 * k] = bk * gm.x;
+        d[3 * k + 1] = bk * gm.y;
+        d[3 * k + 2] = bk * gm.z;
+      }
+    }
+    dmean = make_float3(dmean.x + dd.x, dmean.y + dd.y, dmean.z + dd.z);
+  }
+  if (!live) return;
+  auto put3 = [&](float* o, float x, float y, float z) {
+    o[3 * i] = x;
+    o[3 * i + 1] = y;
+    o[3 * i + 2] = z;
+  };
+  put3(a.dL_dmeans2D, r0.x, r0.y, 0.f);
+  put3(a.dL_dmeans3D, dmean.x, dmean.y, dmean.z);
+  float dop = r2.y;
+  if (a.raw & DMGS_RAW_OPACITIES) {
+    const float o = view_sigmoid(a.opacities[i]);
+    dop *= o * (1.0f - o);
+  }
+  a.dL_dopacity[i] = dop;
+  if (a.dL_dcolors) put3(a.dL_dcolors, dcol.x, dcol.y, dcol.z);
+  if (a.dL_dcov3D) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a.dL_dcov3D[6 * i + k] = dc[k];
+  }
+  if (a.dL_dscales) put3(a.dL_dscales, ds.x, ds.y, ds.z);
+  if (a.dL_drotations) reinterpret_cast<float4*>(a.dL_drotations)[i] = dq;
+}
+
+void launch_view_preprocess(const ViewArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(view_setup_kernel, dim3(1), dim3(64), 0, s, a);
+  const dim3 grid((a.P + kRows - 1) / kRows), block(kRows);
+  if (!a.shs_rest) {
+    hipLaunchKernelGGL(view_preprocess_kernel<-1>, grid, block, 0, s, a);
+    return;
+  }
+  switch (a.sh_coeffs) {
+    case 4: hipLaunchKernelGGL(view_preprocess_kernel<9>, grid, block, 0, s, a); break;
+    case 9: hipLaunchKernelGGL(view_preprocess_kernel<24>, grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL(view_preprocess_kernel<45>, grid, block, 0, s, a); break;
+  }
+}
+
+void launch_view_counts(const uint32_t* cells, const uint32_t* tile_sums, uint32_t* counts, hipStream_t s) {
+  hipLaunchKernelGGL(view_counts_kernel, dim3(1), dim3(64), 0, s, cells, tile_sums, counts);
+}
+
+void launch_view_geometry_bwd(const ViewArgs& a, hipStream_t s) {
+  const dim3 grid((a.P + kRows - 1) / kRows), block(kRows);
+  if (!a.shs) {
+    hipLaunchKernelGGL((view_geometry_bwd_kernel<0, false>), grid, block, 0, s, a);
+  } else if (a.shs_rest) {
+    switch (a.sh_coeffs) {
+      case 4: hipLaunchKernelGGL((view_geometry_bwd_kernel<4, true>), grid, block, 0, s, a); break;
+      case 9: hipLaunchKernelGGL((view_geometry_bwd_kernel<9, true>), grid, block, 0, s, a); break;
+      default: hipLaunchKernelGGL((view_geometry_bwd_kernel<16, true>), grid, block, 0, s, a); break;
+    }
+  } else {
+    switch (a.sh_coeffs) {
+      case 1: hipLaunchKernelGGL((view_geometry_bwd_kernel<1, false>), grid, block, 0, s, a); break;
+      case 4: hipLaunchKernelGGL((view_geometry_bwd_kernel<4, false>), grid, block, 0, s, a); break;
+      case 9: hipLaunchKernelGGL((view_geometry_bwd_kernel<9, false>), grid, block, 0, s, a); break;
+      case 16: hipLaunchKernelGGL((view_geometry_bwd_kernel<16, false>), grid, block, 0, s, a); break;
+      default: hipLaunchKernelGGL((view_geometry_bwd_kernel<-1, false>), grid, block, 0, s, a); break;
+    }
+  }
+}
+
+}  // namespace dmgs

@@ -13,7 +13,10 @@ import math
 
 import torch
 
-from .rasterizer import GaussianRasterizationSettings, GaussianRasterizer
+from .binding import FaceBoundGaussians
+from .rasterizer import (RAW_OPACITIES, RAW_ROTATIONS, RAW_SCALES, GaussianRasterizationSettings, GaussianRasterizer,
+                         _cells_route, model_inputs_fit, rasterize_model)
+from .scenes import FreeGaussians
 from .sh_utils import eval_sh
 
 
@@ -51,10 +54,31 @@ def _python_colors(features_view, xyz, cam, active_sh_degree):
     return torch.sigmoid(eval_sh(active_sh_degree, features_view, dirs))
 
 
+def _model_tensors(pc):
+    """(xyz, dc, rest, opacity, scales, rotations, raw mask) of this package's
+    own models, whose getters the rasterizer's kernels evaluate themselves, or
+    None (any other model, a subclass included, is read through its getters)."""
+    if type(pc) is FreeGaussians:
+        return (pc._xyz, pc._features_dc, pc._features_rest, pc._opacity, pc._scaling, pc._rotation,
+                RAW_SCALES | RAW_ROTATIONS | RAW_OPACITIES)
+    if type(pc) is FaceBoundGaussians:
+        return (pc._xyz, pc._masked(pc._features_dc), pc._masked(pc._features_rest), pc._masked(pc._opacity),
+                pc._scale, pc._rot, RAW_OPACITIES)
+    return None
+
+
 def render(viewpoint_camera, pc, pipe, bg_color: torch.Tensor, scaling_modifier=1.0, override_color=None):
     """Render the scene (gaussian_renderer/__init__.py:18-101)."""
     screenspace_points = _screenspace(pc.get_xyz)
     rs = _settings(viewpoint_camera, bg_color, pc.active_sh_degree, scaling_modifier, pipe.debug)
+    if not pipe.compute_cov3D_python and not pipe.convert_SHs_python and override_color is None and _cells_route(rs):
+        m = _model_tensors(pc)
+        if m is not None and model_inputs_fit(*m[:-1]):
+            xyz, dc, rest, opacity, scales, rotations, raw = m
+            rendered_image, radii = rasterize_model(xyz, screenspace_points, dc, rest, opacity, scales, rotations,
+                                                    raw, rs)
+            return {"render": rendered_image, "viewspace_points": screenspace_points,
+                    "visibility_filter": radii > 0, "radii": radii}
     rasterizer = GaussianRasterizer(raster_settings=rs)
     means3D = pc.get_xyz
     opacity = pc.get_opacity

@@ -18,7 +18,12 @@ given; P == 0 returns an all-zero image.  With ``debug`` every kernel is
 synchronised and checked, and a failing call saves its CPU-copied arguments to
 ``snapshot_fw.dump`` / ``snapshot_bw.dump`` before re-raising.
 
-All compute runs in the gfx950 HIP library through ``dmgs_amd._native``.
+All compute runs in the gfx950 HIP library through ``dmgs_amd._native``.  An
+image takes the cell-list route (``view_forward``: the batched engine's lists
+and blend with one view); ``forward_raw`` / ``backward_raw`` are the route of
+the reference's per-tile lists, taken with ``debug`` (every kernel
+synchronised), for images of more than 65536 cells of 64x64 pixels, and by
+callers that want those lists.  Both give the same image bit for bit.
 """
 import ctypes
 from typing import NamedTuple
@@ -112,8 +117,17 @@ def _cpu_copy(args):
 
 def rasterize_gaussians(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
                         raster_settings):
-    return _RasterizeGaussians.apply(means3D, means2D, sh, colors_precomp, opacities, scales, rotations,
-                                     cov3Ds_precomp, raster_settings)
+    fn = _RasterizeGaussians if torch.is_grad_enabled() else _RasterizeGaussiansNoGrad
+    return fn.apply(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
+                    raster_settings)
+
+
+def _check_color_and_shape(sh, colors_precomp, scales, rotations, cov3Ds_precomp):
+    if _present(sh) == _present(colors_precomp):
+        raise Exception("Please provide excatly one of either SHs or precomputed colors!")
+    if (_present(scales) or _present(rotations)) == _present(cov3Ds_precomp) or \
+            (_present(scales) != _present(rotations)):
+        raise Exception("Please provide exactly one of either scale/rotation pair or precomputed 3D covariance!")
 
 
 def forward_raw(means3D, opacities, sh, colors_precomp, scales, rotations, cov3Ds_precomp, rs):
@@ -131,11 +145,7 @@ def forward_raw(means3D, opacities, sh, colors_precomp, scales, rotations, cov3D
     radii = torch.zeros(P, dtype=torch.int32, device=dev)
     if P == 0:
         return torch.zeros(3, H, W, dtype=torch.float32, device=dev), radii, None
-    if _present(sh) == _present(colors_precomp):
-        raise Exception("Please provide excatly one of either SHs or precomputed colors!")
-    if (_present(scales) or _present(rotations)) == _present(cov3Ds_precomp) or \
-            (_present(scales) != _present(rotations)):
-        raise Exception("Please provide exactly one of either scale/rotation pair or precomputed 3D covariance!")
+    _check_color_and_shape(sh, colors_precomp, scales, rotations, cov3Ds_precomp)
     fr = _Frame(rs, dev, M)
     t = dict(
         means3D=_f32(means3D, dev), opacities=_f32(opacities, dev),
@@ -200,27 +210,127 @@ def ctypes_ref(struct):
     return ctypes.byref(struct)
 
 
+# ---- the cell-list route -------------------------------------------------
+RAW_SCALES, RAW_ROTATIONS, RAW_OPACITIES = 1, 2, 4
+_INPUTS = ("means3D", "opacities", "shs", "shs_rest", "colors_precomp", "scales", "rotations", "cov3D_precomp")
+
+
+def _gaussians(P, t, raw):
+    g = N.DmgsGaussians()
+    g.count, g.raw = P, raw
+    for name in _INPUTS:
+        x = t.get(name)
+        if x is not None:
+            setattr(g, name, x.data_ptr())
+    return g
+
+
+def view_forward(t, sh_coeffs, raw, rs, keep):
+    """One image from a model's tensors: ``t`` maps the names of ``_INPUTS``
+    to contiguous float32, 16-byte aligned device tensors, ``raw`` marks what
+    the kernels activate, ``keep`` says that a backward will follow.  Returns
+    (color, radii, state); state holds what ``view_backward`` needs beside
+    the inputs."""
+    means = t["means3D"]
+    dev, P = means.device, means.shape[0]
+    H, W = int(rs.image_height), int(rs.image_width)
+    fr = _Frame(rs, dev, sh_coeffs)
+    lib = N.load()
+    stream = N.stream_handle(dev)
+    byte = dict(dtype=torch.uint8, device=dev)
+    nbytes = lib.dmgs_view_state_size(P, W, H, int(keep))
+    ws = torch.empty(nbytes, **byte)
+    radii = torch.empty(P, dtype=torch.int32, device=dev)
+    counts = torch.empty(2, dtype=torch.int32, pin_memory=True)
+    s = ctypes_ref(fr.c)
+    g = _gaussians(P, t, raw)
+    with _stage("geometry"):  # ends with the one host synchronisation of the path (as in the reference)
+        N.check(lib.dmgs_view_geometry(s, ctypes_ref(g), int(keep), N.ptr(radii), N.ptr(ws), N.ptr(counts), stream),
+                "dmgs_view_geometry")
+    cells, tiles = (int(c) & 0xFFFFFFFF for c in counts.tolist())
+    K = max(1, cells)
+    lists = torch.empty(lib.dmgs_batched_lists_size(K), **byte)
+    bws = torch.empty(lib.dmgs_batched_backward_size(1, P), **byte) if keep else None
+    color = torch.empty(3, H, W, dtype=torch.float32, device=dev)
+    with _stage("binning"):
+        N.check(lib.dmgs_view_binning(s, P, int(keep), K, N.ptr(ws), N.ptr(lists), stream), "dmgs_view_binning")
+    with _stage("render_forward"):
+        N.check(lib.dmgs_view_blend(s, P, int(keep), K, N.ptr(ws), N.ptr(lists), N.ptr(bws), N.ptr(color), stream),
+                "dmgs_view_blend")
+    return color, radii, dict(frame=fr, ws=ws, lists=lists, bws=bws, cells=K, K=tiles, P=P, M=sh_coeffs, raw=raw)
+
+
+def view_backward(t, state, radii, grad_color, colors=False, cov3D=False):
+    """Gradients of ``view_forward`` (dict by input name, and ``means2D``);
+    colour and covariance gradients where asked for."""
+    fr, P = state["frame"], state["P"]
+    dev = radii.device
+    lib = N.load()
+    f = lambda *shape: torch.empty(*shape, dtype=torch.float32, device=dev)
+    like = lambda name: None if t.get(name) is None else torch.empty_like(t[name])
+    out = dict(means2D=f(P, 3), means3D=f(P, 3), opacities=f(P, 1), shs=like("shs"), shs_rest=like("shs_rest"),
+               scales=like("scales"), rotations=like("rotations"), colors_precomp=f(P, 3) if colors else None,
+               cov3D_precomp=f(P, 6) if cov3D else None)
+    d = N.DmgsGaussianGrads()
+    for field, name in (("means2D", "means2D"), ("means3D", "means3D"), ("opacities", "opacities"), ("shs", "shs"),
+                        ("shs_rest", "shs_rest"), ("colors", "colors_precomp"), ("cov3D", "cov3D_precomp"),
+                        ("scales", "scales"), ("rotations", "rotations")):
+        if out[name] is not None:
+            setattr(d, field, out[name].data_ptr())
+    gc = grad_color.to(dtype=torch.float32).contiguous()
+    stream = N.stream_handle(dev)
+    s = ctypes_ref(fr.c)
+    with _stage("render_backward"):
+        N.check(lib.dmgs_view_blend_backward(s, P, state["cells"], N.ptr(state["ws"]), N.ptr(state["lists"]),
+                                             N.ptr(state["bws"]), N.ptr(gc), stream), "dmgs_view_blend_backward")
+    with _stage("geometry_backward"):
+        N.check(lib.dmgs_view_geometry_backward(s, ctypes_ref(_gaussians(P, t, state["raw"])), N.ptr(radii),
+                                                N.ptr(state["bws"]), ctypes_ref(d), stream),
+                "dmgs_view_geometry_backward")
+    return out
+
+
+def _cells_route(rs):
+    return not rs.debug and N.load().dmgs_view_supported(int(rs.image_width), int(rs.image_height)) == 1
+
+
+def _rasterize(ctx, args, keep):
+    """Shared forward of the two autograd functions below."""
+    means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp, rs = args
+    raw_args = (means3D, opacities, sh, colors_precomp, scales, rotations, cov3Ds_precomp, rs)
+    if rs.debug:
+        try:
+            color, radii, state = forward_raw(*raw_args)
+        except Exception:
+            torch.save(_cpu_copy(raw_args[:-1]), "snapshot_fw.dump")
+            print("\nAn error occured in forward. Please forward snapshot_fw.dump for debugging.")
+            raise
+    elif means3D.device.type != "cuda" or means3D.dim() != 2 or means3D.shape[1] != 3 or means3D.shape[0] == 0 or \
+            not _cells_route(rs):
+        color, radii, state = forward_raw(*raw_args)
+    else:
+        _check_color_and_shape(sh, colors_precomp, scales, rotations, cov3Ds_precomp)
+        dev = means3D.device
+        opt = lambda x: _f32(x, dev) if _present(x) else None
+        t = dict(means3D=_f32(means3D, dev), opacities=_f32(opacities, dev), shs=opt(sh), colors_precomp=opt(colors_precomp),
+                 scales=opt(scales), rotations=opt(rotations), cov3D_precomp=opt(cov3Ds_precomp))
+        color, radii, state = view_forward(t, sh.shape[1] if _present(sh) else 0, 0, rs, keep)
+        state["tensors"] = t
+    ctx.state = state if keep else None
+    ctx.raster_settings = rs
+    ctx.num_rendered = 0 if state is None else state["K"]
+    ctx.shapes = [None if x is None else x.shape for x in args[:-1]]
+    ctx.mark_non_differentiable(radii)
+    return color, radii
+
+
 class _RasterizeGaussians(torch.autograd.Function):
     @staticmethod
     def forward(ctx, means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
                 raster_settings):
-        args = (means3D, opacities, sh, colors_precomp, scales, rotations, cov3Ds_precomp, raster_settings)
-        if raster_settings.debug:
-            try:
-                color, radii, state = forward_raw(*args)
-            except Exception:
-                torch.save(_cpu_copy(args[:-1]), "snapshot_fw.dump")
-                print("\nAn error occured in forward. Please forward snapshot_fw.dump for debugging.")
-                raise
-        else:
-            color, radii, state = forward_raw(*args)
-        ctx.state = state
-        ctx.raster_settings = raster_settings
-        ctx.num_rendered = 0 if state is None else state["K"]
-        ctx.shapes = [None if x is None else x.shape for x in
-                      (means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp)]
+        color, radii = _rasterize(ctx, (means3D, means2D, sh, colors_precomp, opacities, scales, rotations,
+                                        cov3Ds_precomp, raster_settings), True)
         ctx.save_for_backward(radii)
-        ctx.mark_non_differentiable(radii)
         return color, radii
 
     @staticmethod
@@ -233,17 +343,22 @@ class _RasterizeGaussians(torch.autograd.Function):
             z = [None if (s is None or not needs[i]) else torch.zeros(s, device=grad_out_color.device)
                  for i, s in enumerate(shapes)]
             return tuple(z) + (None,)
-        if ctx.raster_settings.debug:
-            try:
-                g = backward_raw(state, radii, grad_out_color)
-            except Exception:
-                torch.save(_cpu_copy((grad_out_color,) + tuple(state["tensors"].values())), "snapshot_bw.dump")
-                print("\nAn error occured in backward. Writing snapshot_bw.dump for debugging.\n")
-                raise
+        if "ws" in state:
+            g = view_backward(state["tensors"], state, radii, grad_out_color, colors=needs[3], cov3D=needs[7])
+            ordered = [g["means3D"], g["means2D"], g["shs"], g["colors_precomp"], g["opacities"], g["scales"],
+                       g["rotations"], g["cov3D_precomp"]]
         else:
-            g = backward_raw(state, radii, grad_out_color)
-        ordered = [g["means3D"], g["means2D"], g["sh"], g["colors"], g["opacity"], g["scales"], g["rotations"],
-                   g["cov3D"]]
+            if ctx.raster_settings.debug:
+                try:
+                    g = backward_raw(state, radii, grad_out_color)
+                except Exception:
+                    torch.save(_cpu_copy((grad_out_color,) + tuple(state["tensors"].values())), "snapshot_bw.dump")
+                    print("\nAn error occured in backward. Writing snapshot_bw.dump for debugging.\n")
+                    raise
+            else:
+                g = backward_raw(state, radii, grad_out_color)
+            ordered = [g["means3D"], g["means2D"], g["sh"], g["colors"], g["opacity"], g["scales"], g["rotations"],
+                       g["cov3D"]]
         grads = []
         for i, (gr, s) in enumerate(zip(ordered, shapes)):
             if not needs[i] or s is None or gr is None or s.numel() == 0:
@@ -252,6 +367,72 @@ class _RasterizeGaussians(torch.autograd.Function):
                 grads.append(gr.reshape(s))
         ctx.state = None
         return tuple(grads) + (None,)
+
+
+class _RasterizeGaussiansNoGrad(torch.autograd.Function):
+    """The forward with autograd off: nothing is kept for a backward."""
+
+    @staticmethod
+    def forward(ctx, *args):
+        return _rasterize(ctx, args, False)
+
+
+class _RasterizeModel(torch.autograd.Function):
+    """A model's own tensors (``raw`` as in ``view_forward``), SH in two
+    tensors; gradients reach those tensors directly."""
+
+    @staticmethod
+    def forward(ctx, xyz, means2D, dc, rest, opacity, scales, rotations, raw, rs, keep):
+        t = dict(means3D=xyz, opacities=opacity, shs=dc, scales=scales, rotations=rotations)
+        if rest.numel():
+            t["shs_rest"] = rest
+        color, radii, state = view_forward(t, 1 + rest.shape[1], raw, rs, keep)
+        if keep:
+            ctx.save_for_backward(radii, xyz, dc, rest, opacity, scales, rotations)
+            ctx.state = state
+        ctx.num_rendered = state["K"]
+        ctx.mark_non_differentiable(radii)
+        return color, radii
+
+    @staticmethod
+    def backward(ctx, grad_out_color, _grad_radii):
+        radii, xyz, dc, rest, opacity, scales, rotations = ctx.saved_tensors
+        inputs = (xyz, radii, dc, rest, opacity, scales, rotations)
+        needs = ctx.needs_input_grad
+        state, ctx.state = ctx.state, None
+        if state is None:  # a second backward through one image, as in _RasterizeGaussians
+            z = [torch.zeros(xyz.shape if i == 1 else x.shape, device=xyz.device) if needs[i] else None
+                 for i, x in enumerate(inputs)]
+            return tuple(z) + (None, None, None)
+        t = dict(means3D=xyz, opacities=opacity, shs=dc, scales=scales, rotations=rotations)
+        if rest.numel():
+            t["shs_rest"] = rest
+        g = view_backward(t, state, radii, grad_out_color)
+        out = (g["means3D"], g["means2D"], g["shs"], rest.new_zeros(rest.shape) if g["shs_rest"] is None else g["shs_rest"],
+               g["opacities"], g["scales"], g["rotations"])
+        return tuple(x if n else None for x, n in zip(out, needs)) + (None, None, None)
+
+
+def model_inputs_fit(xyz, dc, rest, opacity, scales, rotations):
+    """Whether a model's tensors have the form ``rasterize_model`` reads in
+    place: contiguous float32 on one GPU, 16-byte aligned, at least one row,
+    and 1, 4, 9 or 16 SH coefficients."""
+    P = xyz.shape[0]
+    if xyz.dim() != 2 or P == 0 or dc.dim() != 3 or rest.dim() != 3:
+        return False
+    M = 1 + rest.shape[1]
+    want = ((xyz, (P, 3)), (dc, (P, 1, 3)), (rest, (P, M - 1, 3)), (opacity, (P, 1)), (scales, (P, 3)),
+            (rotations, (P, 4)))
+    dev = xyz.device
+    return dev.type == "cuda" and M in (1, 4, 9, 16) and all(
+        tuple(x.shape) == s and x.dtype == torch.float32 and x.device == dev and x.is_contiguous() and
+        x.data_ptr() % 16 == 0 for x, s in want)
+
+
+def rasterize_model(xyz, means2D, dc, rest, opacity, scales, rotations, raw, raster_settings):
+    """``rasterize_gaussians`` on a model's own tensors (see ``model_inputs_fit``)."""
+    return _RasterizeModel.apply(xyz, means2D, dc, rest, opacity, scales, rotations, raw, raster_settings,
+                                 torch.is_grad_enabled())
 
 
 class GaussianRasterizer(nn.Module):

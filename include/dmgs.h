@@ -372,6 +372,64 @@ int dmgs_batched_forward(const dmgs_batch* batch, const float* params, float* im
 int dmgs_batched_backward(const dmgs_batch* batch, const float* params, const float* dL_dimages, float* grads,
                           int32_t stages, dmgs_stream_t stream);
 
+/* ---- One view over a model's own tensors ----
+ * The drop-in renderer's route: the batched engine's cell lists and blend
+ * with one view, whose per-Gaussian stages read (P, k) tensors as a model
+ * holds them.  `raw` marks what the kernels activate themselves (rounded as
+ * torch.exp, torch.nn.functional.normalize and torch.sigmoid round), and the
+ * gradients are then those of the raw tensors; shs_rest, when given, holds
+ * the coefficients past the first in a (P, M - 1, 3) tensor of its own
+ * (M = 4, 9 or 16), shs then being (P, 1, 3).  Tensors are 16-byte aligned.
+ * Images equal those of dmgs_forward_* bit for bit. */
+#define DMGS_GAUSSIANS_LOG_SCALES 1
+#define DMGS_GAUSSIANS_RAW_ROTATIONS 2
+#define DMGS_GAUSSIANS_OPACITY_LOGITS 4
+typedef struct dmgs_gaussians {
+  int64_t count;
+  const float* means3D;
+  const float* opacities;
+  const float* shs;
+  const float* shs_rest;
+  const float* colors_precomp;
+  const float* scales;
+  const float* rotations;
+  const float* cov3D_precomp;
+  int32_t raw;
+  int32_t reserved;
+} dmgs_gaussians;
+typedef struct dmgs_gaussian_grads { /* shaped like the inputs; colors, cov3D, scales, rotations may be NULL */
+  float* means2D; /* (P, 3), NDC */
+  float* means3D;
+  float* opacities;
+  float* shs;
+  float* shs_rest;
+  float* colors;
+  float* cov3D;
+  float* scales;
+  float* rotations;
+} dmgs_gaussian_grads;
+/* Whether an image size has lists here (at most 65536 cells of 64x64 pixels). */
+int dmgs_view_supported(int32_t width, int32_t height);
+/* keep: a backward will follow (the same value in every call of one image). */
+size_t dmgs_view_state_size(int64_t P, int32_t width, int32_t height, int32_t keep);
+/* Preprocess, depth sort and scan; waits for the stream and returns in
+ * counts (host memory, pinned for speed) the cell instances (size the lists
+ * with dmgs_batched_lists_size(max(1, counts[0]))) and the reference's
+ * num_rendered. */
+int dmgs_view_geometry(const dmgs_settings* settings, const dmgs_gaussians* g, int32_t keep, int32_t* radii,
+                       void* state, uint32_t counts[2], dmgs_stream_t stream);
+/* K: the capacity the lists were sized for. */
+int dmgs_view_binning(const dmgs_settings* settings, int64_t P, int32_t keep, int64_t K, void* state, void* lists,
+                      dmgs_stream_t stream);
+/* bwd_ws (dmgs_batched_backward_size(1, P)) exactly when keep is set. */
+int dmgs_view_blend(const dmgs_settings* settings, int64_t P, int32_t keep, int64_t K, void* state, void* lists,
+                    void* bwd_ws, float* out_color, dmgs_stream_t stream);
+/* Accumulates into bwd_ws, which the forward blend cleared. */
+int dmgs_view_blend_backward(const dmgs_settings* settings, int64_t P, int64_t K, void* state, void* lists,
+                             void* bwd_ws, const float* dL_dout, dmgs_stream_t stream);
+int dmgs_view_geometry_backward(const dmgs_settings* settings, const dmgs_gaussians* g, const int32_t* radii,
+                                const void* bwd_ws, const dmgs_gaussian_grads* grads, dmgs_stream_t stream);
+
 /* ---- Scene and frame conversions ---- */
 /* PLY vertex rows (P x row_floats float32, row-major, as the 3DGS writer of
  * scene/gaussian_model.py:191-210 lays them out) -> the 59-channel

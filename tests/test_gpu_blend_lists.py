@@ -1,9 +1,9 @@
 """The blend kernels at the edges of their list handling, against the FP64 oracle.
 
-The forward takes a tile's list 256 positions at a time and keeps a segment
-for the backward every 64 members: lists of one entry, around 64 and 256, and
-longer than several chunks; a list cut off by saturation; more segments than
-the workspace has slots for.  Tolerances are those of the other parity tests
+The forward takes a cell's list in chunks of 1024 positions, stages 256
+members at a time and keeps a segment for the backward every 64 members:
+lists of no entry, one entry, around 64 and 256, and longer than a chunk; a
+list cut off by saturation; more segments than the workspace has slots for.  Tolerances are those of the other parity tests
 (images 1e-4, gradients 1e-3 norm-relative; 1e-5 between two groupings of the
 same sums)."""
 import math
@@ -20,24 +20,26 @@ from oracle import raster as OR
 pytestmark = pytest.mark.gpu
 
 
-def _covering(n, logit, seed=0):
-    """n splats that each cover the whole view."""
+def _covering(n, logit, scale, seed=0):
+    """n splats; of log-scale 0.5 each covers the whole view."""
     g = torch.Generator().manual_seed(seed)
     xyz = torch.rand(n, 3, generator=g) - 0.5
     dc = torch.randn(n, 1, 3, generator=g) * 0.5
-    scale = torch.randn(n, 3, generator=g) * 0.1 + 0.5
+    scale = torch.randn(n, 3, generator=g) * 0.1 + scale
     return S.FreeGaussians(xyz, dc, torch.randn(n, 3, 3, generator=g) * 0.1, scale, torch.randn(n, 4, generator=g),
                            logit + 0.3 * torch.randn(n, 1, generator=g), 1)
 
 
-@pytest.mark.parametrize("n,logit,size", [
-    (1, -2.0, (16, 16)), (63, -4.0, (17, 16)), (64, -4.0, (16, 33)), (65, -4.0, (33, 17)), (128, -4.0, (16, 16)),
-    (255, -4.5, (20, 20)), (256, -4.5, (20, 20)), (257, -4.5, (20, 20)), (700, -4.5, (48, 40)),
-    (300, 1.0, (40, 40)),       # saturates within the first chunk
-    (600, -4.5, (320, 320))])   # 400 tiles of nine segments, 1024 slots
-def test_list_edges(n, logit, size):
-    print(f"case: list edges n={n} logit={logit} size={size}", flush=True)
-    m = _covering(n, logit)
+@pytest.mark.parametrize("n,logit,size,scale", [
+    (1, -2.0, (16, 16), 0.5), (63, -4.0, (17, 16), 0.5), (64, -4.0, (16, 33), 0.5), (65, -4.0, (33, 17), 0.5), (128, -4.0, (16, 16), 0.5),
+    (255, -4.5, (20, 20), 0.5), (256, -4.5, (20, 20), 0.5), (257, -4.5, (20, 20), 0.5), (700, -4.5, (48, 40), 0.5),
+    (300, 1.0, (40, 40), 0.5),       # saturates within the first chunk
+    (600, -4.5, (320, 320), 0.5),  # 400 tiles of nine segments, 1024 slots
+    (1100, -4.5, (16, 16), 0.5),   # more than one chunk of a cell list
+    (40, 0.0, (300, 180), -3.0)])  # most tiles, and whole cells, are empty
+def test_list_edges(n, logit, size, scale):
+    print(f"case: list edges n={n} logit={logit} size={size} scale={scale}", flush=True)
+    m = _covering(n, logit, scale)
     cam = C.camera_at((0.3, -0.2, -4.0), *size, device="cpu")
     bg = torch.tensor([0.2, 0.5, 0.8])
     st = OR.settings_for(cam, bg.double(), 1)
