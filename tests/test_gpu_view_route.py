@@ -1,0 +1,81 @@
+"""The cell-list route of the drop-in renderer (rasterizer.view_forward) against
+the per-tile-list route (forward_raw / backward_raw) on the same inputs.
+
+Radii and images equal bit for bit, with activations in the kernels (exp,
+normalisation, sigmoid, as torch rounds them) or before them, SH in one tensor
+or two, every SH size that has its own kernel and one that has none, given
+colours and covariances, and row counts around a work-group's 256.  Gradients
+agree within 1e-5 (two orders of the same sums)."""
+import pytest
+import torch
+
+from dmgs_amd import cameras as C
+from dmgs_amd import rasterizer as RZ
+from dmgs_amd import scenes as S
+from dmgs_amd.gaussian_renderer import PipelineParams, render
+from helpers import grad_rel_err, settings_from_cam
+
+pytestmark = pytest.mark.gpu
+
+
+class _Plain(S.FreeGaussians):
+    """A subclass: read through its getters."""
+
+
+@pytest.mark.parametrize("P,deg,active,mod", [(1, 3, 3, 1.0), (255, 0, 0, 1.0), (256, 1, 1, 0.7), (257, 2, 2, 1.0),
+                                              (1000, 3, 1, 1.0), (5001, 3, 3, 0.8)])
+def test_model_tensors_equal_getters(P, deg, active, mod):
+    print(f"case: view route P={P} degree={deg} active={active} modifier={mod}", flush=True)
+    m = S.free_scene(P, seed=P, sh_degree=deg).to("cuda")
+    m._rotation[0] = 0.0  # a quaternion whose norm is clamped
+    parts = [p.clone() for p in m.parameters()]
+    cam = C.camera_at((0.4, 0.3, -3.5), 173, 119)
+    bg = torch.tensor([0.1, 0.6, 0.3], device="cuda")
+    g = torch.randn(3, 119, 173, generator=torch.Generator().manual_seed(1)).cuda()
+    got = {}
+    for name, cls, pipe in (("model", S.FreeGaussians, PipelineParams()), ("getters", _Plain, PipelineParams()),
+                            ("tiles", _Plain, PipelineParams(debug=True))):  # debug: the per-tile lists
+        mm = cls(*[p.clone() for p in parts], sh_degree=deg).requires_grad_(True)
+        mm.active_sh_degree = active
+        out = render(cam, mm, pipe, bg, mod)
+        (out["render"] * g).sum().backward()
+        with torch.no_grad():
+            eager = render(cam, mm, pipe, bg, mod)
+        assert torch.equal(eager["render"], out["render"]) and torch.equal(eager["radii"], out["radii"])
+        got[name] = (out["render"].detach(), out["radii"], out["viewspace_points"].grad,
+                     [p.grad for p in mm.parameters()])
+    for name in ("model", "getters"):
+        assert torch.equal(got[name][1], got["tiles"][1]), name
+        assert torch.equal(got[name][0], got["tiles"][0]), name
+        assert grad_rel_err(got[name][2], got["tiles"][2]) < 1e-5, name
+        for a, b in zip(got[name][3], got["tiles"][3]):
+            assert (a is None) == (b is None)
+            if a is not None and a.numel():
+                assert grad_rel_err(a, b) < 1e-5, name
+
+
+@pytest.mark.parametrize("P,M,colors,cov", [(300, 5, False, False), (257, 0, True, False), (300, 16, False, True),
+                                            (513, 0, True, True)])
+def test_rasterizer_inputs(P, M, colors, cov):
+    """An SH size without a kernel of its own, given colours and covariances, through GaussianRasterizer."""
+    print(f"case: view route inputs P={P} M={M} colors={colors} cov={cov}", flush=True)
+    gen = torch.Generator().manual_seed(P)
+    base = S.free_scene(P, seed=P).to("cuda")
+    cam = C.camera_at((0.4, 0.3, -3.5), 90, 70)
+    col = torch.rand(P, 3, generator=gen).cuda() if colors else None
+    sh = None if colors else (torch.randn(P, M, 3, generator=gen) * 0.3).cuda()
+    g = torch.randn(3, 70, 90, generator=gen).cuda()
+    got = []
+    for debug in (False, True):
+        rs = settings_from_cam(cam, torch.ones(3), 1 if M == 5 else 3, debug=debug)
+        leaf = lambda t: None if t is None else t.detach().clone().requires_grad_(True)
+        x = dict(means3D=leaf(base._xyz), means2D=leaf(torch.zeros_like(base._xyz)), opacities=leaf(base.get_opacity),
+                 shs=leaf(sh), colors_precomp=leaf(col), scales=None if cov else leaf(base.get_scaling),
+                 rotations=None if cov else leaf(base.get_rotation),
+                 cov3D_precomp=leaf(base.get_covariance()) if cov else None)
+        color, radii = RZ.GaussianRasterizer(rs)(**x)
+        (color * g).sum().backward()
+        got.append((color.detach(), radii, {k: v.grad for k, v in x.items() if v is not None}))
+    assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][0], got[1][0])
+    for k, v in got[1][2].items():
+        assert grad_rel_err(got[0][2][k], v) < 1e-5, k
