@@ -117,6 +117,7 @@ _SIGNATURES = {
     "dmgs_batched_lists_size": (c_size_t, [c_int64]),
     "dmgs_batched_backward_size": (c_size_t, [c_int32, c_int64]),
     "dmgs_batched_offsets": (c_int32, [c_int32, c_int64, c_int32, c_int64, c_int64, ctypes.POINTER(c_size_t)]),
+    "dmgs_sh_sigmoid": (c_int32, [c_int64, c_int32, c_int32, c_int32] + [c_void_p] * 8),
     "dmgs_view_supported": (c_int32, [c_int32, c_int32]),
     "dmgs_view_state_size": (c_size_t, [c_int64, c_int32, c_int32, c_int32]),
     "dmgs_view_geometry": (c_int32, [ctypes.POINTER(DmgsSettings), ctypes.POINTER(DmgsGaussians), c_int32, c_void_p,

@@ -616,6 +616,24 @@ int dmgs_view_blend_backward(const dmgs_settings* s, int64_t P, int64_t K, void*
   return rc ? rc : blend_views_backward(&b, Ctx(&b), dL_dout, reinterpret_cast<hipStream_t>(stream));
 }
 
+int dmgs_sh_sigmoid(int64_t n, int32_t coeffs, int32_t degree, int32_t color_major, const float* feats,
+                    const float* xyz, const float* campos, float* colors, const float* dL_dcolors, float* dL_dfeats,
+                    float* dL_dxyz, dmgs_stream_t stream) {
+  if (n < 0 || n > (int64_t)0x7fffffff - 256) return bfail(DMGS_EINVAL, "invalid n");
+  if ((coeffs != 1 && coeffs != 4 && coeffs != 9 && coeffs != 16) || degree < 0 || degree > 3 ||
+      (degree + 1) * (degree + 1) > coeffs)
+    return bfail(DMGS_EINVAL, "degree %d needs 1, 4, 9 or 16 coefficients, at least (degree + 1)^2", degree);
+  if (n == 0) return DMGS_OK;
+  if (!feats || !xyz || !campos || !colors || (dL_dcolors && (!dL_dfeats || !dL_dxyz)))
+    return bfail(DMGS_EINVAL, "null pointer");
+  if ((reinterpret_cast<uintptr_t>(feats) | reinterpret_cast<uintptr_t>(dL_dfeats)) & 15u)
+    return bfail(DMGS_EINVAL, "features must be 16-byte aligned");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const dmgs::ShSigmoidArgs a{(int)n, degree, feats, xyz, campos, colors, dL_dcolors, dL_dfeats, dL_dxyz};
+  dmgs::launch_sh_sigmoid(a, coeffs, color_major != 0, dL_dcolors != nullptr, st);
+  return bcheck("sh sigmoid", st);
+}
+
 int dmgs_view_geometry_backward(const dmgs_settings* s, const dmgs_gaussians* g, const int32_t* radii,
                                 const void* bwd_ws, const dmgs_gaussian_grads* d, dmgs_stream_t stream) {
   int rc = check_gaussians(s, g, bwd_ws);

@@ -197,6 +197,18 @@ void launch_view_preprocess(const ViewArgs& a, hipStream_t s);
 // counts[0] = *cells, counts[1] = the sum of tile_sums
 void launch_view_counts(const uint32_t* cells, const uint32_t* tile_sums, uint32_t* counts, hipStream_t s);
 void launch_view_geometry_bwd(const ViewArgs& a, hipStream_t s);
+// sigmoid of the SH sum in the view direction (coeffs 1, 4, 9 or 16 per colour)
+struct ShSigmoidArgs {
+  int n, degree;
+  const float* feats;   // (n, 3 M), colour-major or coefficient-major
+  const float* xyz;     // (n, 3)
+  const float* campos;  // 3
+  float* colors;        // (n, 3); read by the backward
+  const float* dL_dcolors;
+  float* dL_dfeats;
+  float* dL_dxyz;
+};
+void launch_sh_sigmoid(const ShSigmoidArgs& a, int coeffs, bool color_major, bool backward, hipStream_t s);
 
 // ---- blend ----
 // List segments that a forward keeps for its backward (render.hip).  At most kSegmentTiles tiles: with 8160

@@ -281,7 +281,8 @@ __device__ __forceinline__ float3 ewa_backward(float3 p, const float c[6], const
 // the 16 basis values b (zero past the active degree) and the masked colour
 // gradient g, and returns dL/dmean through the normalised view direction.
 // The basis partials are those of the polynomials in sh_to_rgb.
-template <typename SH>
+// CLAMP false: the colour has no clamp at zero, so g is dL_dRGB.
+template <bool CLAMP = true, typename SH>
 __device__ __forceinline__ float3 sh_backward(int deg, const SH& sh, float3 pos, const float* campos,
                                               float3 dL_dRGB, float (&b)[16], float3& g) {
   const float3 v = make_float3(pos.x - campos[0], pos.y - campos[1], pos.z - campos[2]);
@@ -356,7 +357,9 @@ __device__ __forceinline__ float3 sh_backward(int deg, const SH& sh, float3 pos,
       }
     }
   }
-  g = make_float3(rgb.x < 0.f ? 0.f : dL_dRGB.x, rgb.y < 0.f ? 0.f : dL_dRGB.y, rgb.z < 0.f ? 0.f : dL_dRGB.z);
+  g = dL_dRGB;
+  if constexpr (CLAMP)
+    g = make_float3(rgb.x < 0.f ? 0.f : dL_dRGB.x, rgb.y < 0.f ? 0.f : dL_dRGB.y, rgb.z < 0.f ? 0.f : dL_dRGB.z);
   const float3 ddir = make_float3(dRx.x * g.x + dRx.y * g.y + dRx.z * g.z, dRy.x * g.x + dRy.y * g.y + dRy.z * g.z,
                                   dRz.x * g.x + dRz.y * g.y + dRz.z * g.z);
   // d normalize(v) / dv applied to ddir (|v|^-3 only scales the gradient:

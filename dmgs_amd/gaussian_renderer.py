@@ -13,6 +13,7 @@ import math
 
 import torch
 
+from . import _native as N
 from .binding import FaceBoundGaussians
 from .rasterizer import (RAW_OPACITIES, RAW_ROTATIONS, RAW_SCALES, GaussianRasterizationSettings, GaussianRasterizer,
                          _cells_route, model_inputs_fit, rasterize_model)
@@ -48,10 +49,60 @@ def _screenspace(xyz):
     return pts
 
 
-def _python_colors(features_view, xyz, cam, active_sh_degree):
-    dirs = xyz - cam.camera_center.to(xyz.device).repeat(features_view.shape[0], 1)
+def _torch_colors(features_view, xyz, campos, active_sh_degree):
+    dirs = xyz - campos.repeat(features_view.shape[0], 1)
     dirs = dirs / dirs.norm(dim=1, keepdim=True)
     return torch.sigmoid(eval_sh(active_sh_degree, features_view, dirs))
+
+
+# The Python SH path as one kernel each way (352 launches per training iteration of 122 880 Gaussians before).
+class _ShSigmoid(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, feats, xyz, campos, degree):
+        n, _, M = feats.shape
+        color_major = int(feats.stride(2) == 1)
+        colors = torch.empty(n, 3, dtype=torch.float32, device=xyz.device)
+        N.check(N.load().dmgs_sh_sigmoid(n, M, degree, color_major, N.ptr(feats), N.ptr(xyz), N.ptr(campos),
+                                         N.ptr(colors), None, None, None, N.stream_handle(xyz.device)),
+                "dmgs_sh_sigmoid")
+        ctx.save_for_backward(feats, xyz, campos, colors)
+        ctx.degree, ctx.color_major = degree, color_major
+        return colors
+
+    @staticmethod
+    def backward(ctx, grad):
+        feats, xyz, campos, colors = ctx.saved_tensors
+        n, _, M = feats.shape
+        if torch.is_grad_enabled():  # create_graph: the derivative of the torch ops, itself differentiable
+            out = _torch_colors(feats, xyz, campos, ctx.degree)
+            grads = torch.autograd.grad(out, (feats, xyz), grad, create_graph=True, allow_unused=True)
+            return grads[0], grads[1], None, None
+        g = grad.to(torch.float32).contiguous()
+        dfeats = torch.empty_strided(feats.shape, feats.stride(), dtype=torch.float32, device=feats.device)
+        dxyz = torch.empty_like(xyz)
+        N.check(N.load().dmgs_sh_sigmoid(n, M, ctx.degree, ctx.color_major, N.ptr(feats), N.ptr(xyz), N.ptr(campos),
+                                         N.ptr(colors), N.ptr(g), N.ptr(dfeats), N.ptr(dxyz),
+                                         N.stream_handle(xyz.device)), "dmgs_sh_sigmoid")
+        return dfeats, dxyz, None, None
+
+
+def _sh_kernel_fits(feats, xyz, degree):
+    """Whether (n, 3, M) features are rows the SH kernel reads in place."""
+    if feats.dim() != 3 or feats.shape[1] != 3 or xyz.dim() != 2 or tuple(xyz.shape) != (feats.shape[0], 3):
+        return False
+    n, _, M = feats.shape
+    return (n > 0 and M in (1, 4, 9, 16) and 0 <= degree <= 3 and (degree + 1) ** 2 <= M and
+            feats.device.type == "cuda" and feats.device == xyz.device and
+            feats.dtype == torch.float32 and xyz.dtype == torch.float32 and xyz.is_contiguous() and
+            feats.stride() in ((3 * M, M, 1), (3 * M, 1, 3)) and feats.data_ptr() % 16 == 0)
+
+
+def _python_colors(features_view, xyz, cam, active_sh_degree):
+    if _sh_kernel_fits(features_view, xyz, active_sh_degree):
+        campos = cam.camera_center.to(device=xyz.device, dtype=torch.float32).contiguous()
+        if campos.numel() == 3 and not campos.requires_grad:
+            return _ShSigmoid.apply(features_view, xyz, campos, active_sh_degree)
+    return _torch_colors(features_view, xyz, cam.camera_center.to(xyz.device), active_sh_degree)
 
 
 def _model_tensors(pc):

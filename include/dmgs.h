@@ -430,6 +430,15 @@ int dmgs_view_blend_backward(const dmgs_settings* settings, int64_t P, int64_t K
 int dmgs_view_geometry_backward(const dmgs_settings* settings, const dmgs_gaussians* g, const int32_t* radii,
                                 const void* bwd_ws, const dmgs_gaussian_grads* grads, dmgs_stream_t stream);
 
+/* Colours of the reference adapter's Python SH path: sigmoid of the SH sum
+ * in the direction from campos (gaussian_renderer/__init__.py:74-78), rows of
+ * 3 x coeffs features, color_major (3, coeffs) or (coeffs, 3).  Without
+ * dL_dcolors: writes colors (n, 3).  With it: reads the colors of the
+ * forward and writes dL_dfeats (like feats) and dL_dxyz (n, 3). */
+int dmgs_sh_sigmoid(int64_t n, int32_t coeffs, int32_t degree, int32_t color_major, const float* feats,
+                    const float* xyz, const float* campos, float* colors, const float* dL_dcolors, float* dL_dfeats,
+                    float* dL_dxyz, dmgs_stream_t stream);
+
 /* ---- Scene and frame conversions ---- */
 /* PLY vertex rows (P x row_floats float32, row-major, as the 3DGS writer of
  * scene/gaussian_model.py:191-210 lays them out) -> the 59-channel

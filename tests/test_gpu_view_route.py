@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from dmgs_amd import cameras as C
+from dmgs_amd import gaussian_renderer as GR
 from dmgs_amd import rasterizer as RZ
 from dmgs_amd import scenes as S
 from dmgs_amd.gaussian_renderer import PipelineParams, render
@@ -79,3 +80,47 @@ def test_rasterizer_inputs(P, M, colors, cov):
     assert torch.equal(got[0][1], got[1][1]) and torch.equal(got[0][0], got[1][0])
     for k, v in got[1][2].items():
         assert grad_rel_err(got[0][2][k], v) < 1e-5, k
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 1000])
+@pytest.mark.parametrize("M,deg", [(1, 0), (4, 1), (9, 1), (9, 2), (16, 0), (16, 3)])
+def test_sh_sigmoid_kernel_equals_torch(n, M, deg):
+    """sigmoid(SH) of both feature layouts against float64 torch ops.
+
+    The sum has up to 16 products of factors below 3 in magnitude (|sh| < 5): its float32 error stays below
+    16 * 15 * 2^-23 = 3e-5, and a quarter of that after the sigmoid."""
+    print(f"case: sh sigmoid n={n} M={M} degree={deg}", flush=True)
+    gen = torch.Generator().manual_seed(n * 31 + M + deg)
+    cam = C.camera_at((0.4, 0.3, -3.5), 64, 64)
+    xyz = (torch.rand(n, 3, generator=gen) * 2 - 1).cuda()
+    g = torch.randn(n, 3, generator=gen).cuda()
+    base = torch.randn(n, 3 * M, generator=gen).cuda()
+    for color_major in (True, False):
+        view = (lambda t: t.view(-1, 3, M)) if color_major else (lambda t: t.view(-1, M, 3).transpose(1, 2))
+        f32, x32 = base.clone().requires_grad_(True), xyz.clone().requires_grad_(True)
+        f64, x64 = base.double().requires_grad_(True), xyz.double().requires_grad_(True)
+        assert GR._sh_kernel_fits(view(f32), x32, deg)
+        assert not GR._sh_kernel_fits(view(f64), x64, deg)
+        out, ref = GR._python_colors(view(f32), x32, cam, deg), GR._python_colors(view(f64), x64, cam, deg)
+        assert (out.double() - ref).abs().max() < 8e-6
+        (out * g).sum().backward()
+        (ref * g.double()).sum().backward()
+        assert grad_rel_err(f32.grad.double(), f64.grad) < 1e-5
+        if deg:
+            assert grad_rel_err(x32.grad.double(), x64.grad) < 1e-5
+        else:
+            assert not x32.grad.any()
+
+
+def test_sh_sigmoid_second_order():
+    """A graph of the backward (create_graph) goes through the torch ops."""
+    gen = torch.Generator().manual_seed(3)
+    cam = C.camera_at((0.4, 0.3, -3.5), 64, 64)
+    xyz = (torch.rand(7, 3, generator=gen) * 2 - 1).cuda().requires_grad_(True)
+    f = torch.randn(7, 3, 16, generator=gen).cuda().requires_grad_(True)
+    second = []
+    for ff, xx in ((f, xyz), (f.detach().double().requires_grad_(True), xyz.detach().double().requires_grad_(True))):
+        a, b = torch.autograd.grad(GR._python_colors(ff, xx, cam, 3).sum(), (ff, xx), create_graph=True)
+        second.append(torch.autograd.grad((a ** 2).sum() + (b ** 2).sum(), (ff, xx)))
+    for s, r in zip(*second):
+        assert grad_rel_err(s.double(), r) < 1e-4
