@@ -12,10 +12,9 @@
 // with L the affine triangle matrix built without gradient and
 // k = tanh(scale_factor) * max_scale, shared by the face's Gaussians.
 //
-// Backward: one thread per face walks its G Gaussians, sums their
-// contributions to the face frame and the three vertices, back-propagates
-// through the frame construction once, and adds into the vertex gradient
-// with 9 atomics per face.  The quaternion gradient is mapped to the rotation
+// Backward: the contributions of a face's G Gaussians to its frame and its
+// three vertices are summed, go back through the frame construction once, and
+// are added into the vertex gradient with 9 atomics per face.  The quaternion gradient is mapped to the rotation
 // through the body-frame angular gradient g_w = 1/2 Im(conj(q) * dL/dq): any
 // variation of R here is a rotation, so a matrix gradient that agrees with the
 // true one on rotation tangents gives exact vertex gradients.
@@ -141,98 +140,174 @@ __global__ __launch_bounds__(256) void bind_fwd_kernel(BindArgs a) {
   }
 }
 
-__global__ __launch_bounds__(256) void bind_bwd_kernel(BindArgs a) {
-  const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= a.F) return;
-  const int i0 = face_vertex(a.faces, f, 0), i1 = face_vertex(a.faces, f, 1), i2 = face_vertex(a.faces, f, 2);
-  const V3 v0 = load3(a.verts, i0), v1 = load3(a.verts, i1), v2 = load3(a.verts, i2);
-  const Frame fr = make_frame(v0, v1, v2);
-  V3 dv0 = v3(0.f, 0.f, 0.f), dv1 = dv0, dv2 = dv0;
-  V3 gx = dv0, gy = dv0, gn = dv0;  // gradient of the frame columns
-  for (int j = 0; j < a.G; ++j) {
-    const int gi = f * a.G + j;
-    const float* bc = a.bc + 3 * (a.bc_per_gaussian ? gi : j);
-    const V3 dp = load3(a.dxyz, gi);
-    dv0 = dv0 + bc[0] * dp;
-    dv1 = dv1 + bc[1] * dp;
-    dv2 = dv2 + bc[2] * dp;
-    if (a.rot2d && a.drot) {
-      const float ra = a.rot2d[2 * gi], rb = a.rot2d[2 * gi + 1];
-      const float rr = ra * ra + rb * rb;
-      const float ic = 1.0f / fmaxf(sqrtf(rr), 1e-12f);
-      const float ca = ra * ic, cb = rb * ic;
-      float R[3][3];
-      rotation_of(fr, ca, cb, R);
-      float4 q = mat_to_quat(R);
-      const float iq = 1.0f / fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);
-      q = make_float4(q.x * iq, q.y * iq, q.z * iq, q.w * iq);
-      const float4 g = reinterpret_cast<const float4*>(a.drot)[gi];
-      // g_w = 1/2 Im(conj(q) * g), quaternions (w, x, y, z)
-      const V3 qv = v3(q.y, q.z, q.w), gv = v3(g.y, g.z, g.w);
-      const V3 gw = 0.5f * (q.x * gv - g.x * qv - cross(qv, gv));
-      // rotation about z by theta = atan2(rb, ra): dL/dtheta = gw.z
-      if (a.drot2d) {
-        const float s = rr > 0.f ? gw.z / rr : 0.f;
-        a.drot2d[2 * gi] = -rb * s;
-        a.drot2d[2 * gi + 1] = ra * s;
+// A lane per Gaussian: whole faces per block (as many as fit 256 lanes, or one face whose Gaussians the lanes walk
+// with stride 256).  The frames of the block's faces are made once, by one lane each; every Gaussian's
+// contributions to its face (up to 24 sums) go through LDS and are added there in the Gaussians' order.
+// Bound by the atomics on the vertices: neighbouring lanes add the three components of one vertex, so that they
+// leave as one request.  A lane per face with nine adds of its own took 57 us for 81 920 faces x 6 with rotations
+// (24 now; 44 with this split but the adds left with the face's lane) and 61 us for 98 528 x 6 covariances (26).
+constexpr int kBindLanes = 256;
+// Blocks whose faces add to the one dk: same-address adds take 8.5 ns each, so a block walks several groups of
+// faces (98 528 x 6: 41 us with 2346 blocks, 34 with 1536, 32 with 1024, 26 with 512).
+constexpr int kBindCovBlocks = 512;
+
+template <bool ROT, bool COV>
+__global__ __launch_bounds__(kBindLanes) void bind_bwd_kernel(BindArgs a, int block_faces) {
+  // sums per face: dv0, dv1, dv2; ROT: frame columns x, y, n; COV: the covariance's 6
+  constexpr int kCov = ROT ? 18 : 9, kBindSums = kCov + (COV ? 6 : 0);
+  __shared__ float s_part[kBindSums * kBindLanes];       // [sum][lane]
+  __shared__ float s_frame[9 * kBindLanes];              // [component][face]: frame, later the vertex gradients
+  __shared__ int s_vertex[3 * kBindLanes];               // [corner][face]
+  __shared__ float s_dk[kBindLanes / 64];
+  const int tid = threadIdx.x;
+  float dk = 0.f;
+  for (uint32_t f0 = blockIdx.x * block_faces; f0 < (uint32_t)a.F; f0 += gridDim.x * block_faces) {
+    const int nf = min(block_faces, a.F - (int)f0);
+    const uint32_t ng = (uint32_t)nf * a.G;  // Gaussians of this block
+    const size_t g0 = (size_t)f0 * a.G;
+    Frame fr;
+    if (tid < nf) {
+      int iv[3];
+      for (int t = 0; t < 3; ++t) s_vertex[t * kBindLanes + tid] = iv[t] = face_vertex(a.faces, f0 + tid, t);
+      fr = make_frame(load3(a.verts, iv[0]), load3(a.verts, iv[1]), load3(a.verts, iv[2]));
+      if constexpr (ROT) {
+        const float c[9] = {fr.x.x, fr.x.y, fr.x.z, fr.y.x, fr.y.y, fr.y.z, fr.n.x, fr.n.y, fr.n.z};
+        for (int t = 0; t < 9; ++t) s_frame[t * kBindLanes + tid] = c[t];
       }
-      // frame angular gradient g1 = R_t gw; column gradients 1/2 R_t2w (g1 x e_j)
-      const V3 g1 = v3(ca * gw.x - cb * gw.y, cb * gw.x + ca * gw.y, gw.z);
-      // R_t2w (g1 x e_x) = R_t2w (0, g1.z, -g1.y) = g1.z y - g1.y n, etc.
-      gx = gx + 0.5f * (g1.z * fr.y - g1.y * fr.n);
-      gy = gy + 0.5f * (g1.x * fr.n - g1.z * fr.x);
-      gn = gn + 0.5f * (g1.y * fr.x - g1.x * fr.y);
     }
-    if (a.scale2d && a.dscale && a.dscale2d) {
-      a.dscale2d[2 * gi] = a.dscale[3 * gi] * __expf(a.scale2d[2 * gi]);
-      a.dscale2d[2 * gi + 1] = a.dscale[3 * gi + 1] * __expf(a.scale2d[2 * gi + 1]);
+    __syncthreads();
+    float sum[kBindSums];
+#pragma unroll
+    for (int t = 0; t < kBindSums; ++t) sum[t] = 0.f;
+    for (uint32_t i = tid; i < ng; i += kBindLanes) {  // one pass, or several over one face
+      const uint32_t fl = i / (uint32_t)a.G, j = i - fl * a.G;
+      const size_t gi = g0 + i;
+      const float* bc = a.bc + 3 * (a.bc_per_gaussian ? gi : j);
+      const V3 dp = v3(a.dxyz[3 * gi], a.dxyz[3 * gi + 1], a.dxyz[3 * gi + 2]);
+      for (int t = 0; t < 3; ++t) {
+        sum[3 * t] += bc[t] * dp.x;
+        sum[3 * t + 1] += bc[t] * dp.y;
+        sum[3 * t + 2] += bc[t] * dp.z;
+      }
+      if constexpr (ROT) {
+        Frame fq;
+        const float* c = s_frame + fl;
+        fq.x = v3(c[0], c[kBindLanes], c[2 * kBindLanes]);
+        fq.y = v3(c[3 * kBindLanes], c[4 * kBindLanes], c[5 * kBindLanes]);
+        fq.n = v3(c[6 * kBindLanes], c[7 * kBindLanes], c[8 * kBindLanes]);
+        const float ra = a.rot2d[2 * gi], rb = a.rot2d[2 * gi + 1];
+        const float rr = ra * ra + rb * rb;
+        const float ic = 1.0f / fmaxf(sqrtf(rr), 1e-12f);
+        const float ca = ra * ic, cb = rb * ic;
+        float R[3][3];
+        rotation_of(fq, ca, cb, R);
+        float4 q = mat_to_quat(R);
+        const float iq = 1.0f / fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);
+        q = make_float4(q.x * iq, q.y * iq, q.z * iq, q.w * iq);
+        const float4 g = reinterpret_cast<const float4*>(a.drot)[gi];
+        // g_w = 1/2 Im(conj(q) * g), quaternions (w, x, y, z)
+        const V3 qv = v3(q.y, q.z, q.w), gv = v3(g.y, g.z, g.w);
+        const V3 gw = 0.5f * (q.x * gv - g.x * qv - cross(qv, gv));
+        // rotation about z by theta = atan2(rb, ra): dL/dtheta = gw.z
+        if (a.drot2d) {
+          const float s = rr > 0.f ? gw.z / rr : 0.f;
+          a.drot2d[2 * gi] = -rb * s;
+          a.drot2d[2 * gi + 1] = ra * s;
+        }
+        // frame angular gradient g1 = R_t gw; column gradients 1/2 R_t2w (g1 x e_j)
+        const V3 g1 = v3(ca * gw.x - cb * gw.y, cb * gw.x + ca * gw.y, gw.z);
+        // R_t2w (g1 x e_x) = R_t2w (0, g1.z, -g1.y) = g1.z y - g1.y n, etc.
+        const V3 d[3] = {0.5f * (g1.z * fq.y - g1.y * fq.n), 0.5f * (g1.x * fq.n - g1.z * fq.x),
+                         0.5f * (g1.y * fq.x - g1.x * fq.y)};
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+          sum[9 + 3 * t] += d[t].x;
+          sum[9 + 3 * t + 1] += d[t].y;
+          sum[9 + 3 * t + 2] += d[t].z;
+        }
+      }
+      if constexpr (COV)
+#pragma unroll
+        for (int t = 0; t < 6; ++t) sum[kCov + t] += a.dcov[6 * gi + t];
+      if (a.scale2d && a.dscale && a.dscale2d) {
+        a.dscale2d[2 * gi] = a.dscale[3 * gi] * __expf(a.scale2d[2 * gi]);
+        a.dscale2d[2 * gi + 1] = a.dscale[3 * gi + 1] * __expf(a.scale2d[2 * gi + 1]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < kBindSums; ++t) s_part[t * kBindLanes + tid] = sum[t];
+    __syncthreads();
+    if (tid < nf) {
+      const int gl = min(a.G, kBindLanes), first = tid * gl;  // one face alone: every lane holds a part of it
+#pragma unroll
+      for (int t = 0; t < kBindSums; ++t) sum[t] = 0.f;
+      for (int j = first; j < first + gl; ++j) {
+#pragma unroll
+        for (int t = 0; t < kBindSums; ++t) sum[t] += s_part[t * kBindLanes + j];
+      }
+      V3 gx = v3(0.f, 0.f, 0.f), gy = gx, gn = gx;  // gradient of the frame columns
+      if constexpr (ROT) {
+        gx = v3(sum[9], sum[10], sum[11]);
+        gy = v3(sum[12], sum[13], sum[14]);
+        gn = v3(sum[15], sum[16], sum[17]);
+      }
+      if constexpr (COV) {
+        // stage 2: Sigma = A A^T, A = R_t2w L k, shared by the face's Gaussians
+        const float* Gs = sum + kCov;
+        const float Gm[3][3] = {{Gs[0], 0.5f * Gs[1], 0.5f * Gs[2]},
+                                {0.5f * Gs[1], Gs[3], 0.5f * Gs[4]},
+                                {0.5f * Gs[2], 0.5f * Gs[4], Gs[5]}};
+        const float* L = a.Lmat + 9 * (size_t)(f0 + tid);
+        const float k = a.k[0];
+        const float Rw[3][3] = {{fr.x.x, fr.y.x, fr.n.x}, {fr.x.y, fr.y.y, fr.n.y}, {fr.x.z, fr.y.z, fr.n.z}};
+        float B[3][3];  // B = L L^T k^2
+        for (int r = 0; r < 3; ++r)
+          for (int c = 0; c < 3; ++c)
+            B[r][c] = k * k * (L[3 * r] * L[3 * c] + L[3 * r + 1] * L[3 * c + 1] + L[3 * r + 2] * L[3 * c + 2]);
+        // dL/dR = 2 G R B ; dL/dk = 2/k <G, R L L^T R^T k^2>
+        float RB[3][3], dR[3][3], gk = 0.f;
+        for (int r = 0; r < 3; ++r)
+          for (int c = 0; c < 3; ++c) RB[r][c] = Rw[r][0] * B[0][c] + Rw[r][1] * B[1][c] + Rw[r][2] * B[2][c];
+        for (int r = 0; r < 3; ++r)
+          for (int c = 0; c < 3; ++c) {
+            dR[r][c] = 2.f * (Gm[r][0] * RB[0][c] + Gm[r][1] * RB[1][c] + Gm[r][2] * RB[2][c]);
+            const float S = RB[r][0] * Rw[c][0] + RB[r][1] * Rw[c][1] + RB[r][2] * Rw[c][2];
+            gk += Gm[r][c] * S;
+          }
+        gx = gx + v3(dR[0][0], dR[1][0], dR[2][0]);
+        gy = gy + v3(dR[0][1], dR[1][1], dR[2][1]);
+        gn = gn + v3(dR[0][2], dR[1][2], dR[2][2]);
+        if (k != 0.f) dk += 2.f * gk / k;
+      }
+      V3 de1, de2;
+      frame_bwd(fr, gx, gy, gn, de1, de2);
+      const V3 dv[3] = {v3(sum[0], sum[1], sum[2]) - de1 - de2, v3(sum[3], sum[4], sum[5]) + de1,
+                        v3(sum[6], sum[7], sum[8]) + de2};
+      for (int t = 0; t < 3; ++t) {
+        s_frame[3 * t * kBindLanes + tid] = dv[t].x;
+        s_frame[(3 * t + 1) * kBindLanes + tid] = dv[t].y;
+        s_frame[(3 * t + 2) * kBindLanes + tid] = dv[t].z;
+      }
+    }
+    __syncthreads();
+    for (int e = tid; e < 9 * nf; e += kBindLanes) {  // neighbouring lanes add to neighbouring addresses
+      const int fl = e / 9, c = e - 9 * fl;
+      unsafeAtomicAdd(a.dverts + 3 * (size_t)s_vertex[c / 3 * kBindLanes + fl] + c % 3, s_frame[c * kBindLanes + fl]);
+    }
+    __syncthreads();
+  }
+  if constexpr (COV) {
+    if (a.dk) {  // one atomic per block
+      for (int off = 32; off > 0; off >>= 1) dk += __shfl_xor(dk, off, 64);
+      if ((tid & 63) == 0) s_dk[tid >> 6] = dk;
+      __syncthreads();
+      if (tid == 0) {
+        float t = 0.f;
+        for (int w = 0; w < kBindLanes / 64; ++w) t += s_dk[w];
+        if (t != 0.f) unsafeAtomicAdd(a.dk, t);
+      }
     }
   }
-  if (a.dcov) {
-    // stage 2: Sigma = A A^T, A = R_t2w L k, shared by the face's Gaussians
-    float Gs[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < a.G; ++j)
-      for (int k = 0; k < 6; ++k) Gs[k] += a.dcov[6 * (f * a.G + j) + k];
-    const float Gm[3][3] = {{Gs[0], 0.5f * Gs[1], 0.5f * Gs[2]},
-                            {0.5f * Gs[1], Gs[3], 0.5f * Gs[4]},
-                            {0.5f * Gs[2], 0.5f * Gs[4], Gs[5]}};
-    const float* L = a.Lmat + 9 * f;
-    const float k = a.k[0];
-    const float Rw[3][3] = {{fr.x.x, fr.y.x, fr.n.x}, {fr.x.y, fr.y.y, fr.n.y}, {fr.x.z, fr.y.z, fr.n.z}};
-    float B[3][3];  // B = L L^T k^2
-    for (int r = 0; r < 3; ++r)
-      for (int c = 0; c < 3; ++c)
-        B[r][c] = k * k * (L[3 * r] * L[3 * c] + L[3 * r + 1] * L[3 * c + 1] + L[3 * r + 2] * L[3 * c + 2]);
-    // dL/dR = 2 G R B ; dL/dk = 2/k <G, R L L^T R^T k^2>
-    float RB[3][3], dR[3][3];
-    for (int r = 0; r < 3; ++r)
-      for (int c = 0; c < 3; ++c) RB[r][c] = Rw[r][0] * B[0][c] + Rw[r][1] * B[1][c] + Rw[r][2] * B[2][c];
-    float gk = 0.f;
-    for (int r = 0; r < 3; ++r)
-      for (int c = 0; c < 3; ++c) {
-        dR[r][c] = 2.f * (Gm[r][0] * RB[0][c] + Gm[r][1] * RB[1][c] + Gm[r][2] * RB[2][c]);
-        const float S = RB[r][0] * Rw[c][0] + RB[r][1] * Rw[c][1] + RB[r][2] * Rw[c][2];
-        gk += Gm[r][c] * S;
-      }
-    gx = gx + v3(dR[0][0], dR[1][0], dR[2][0]);
-    gy = gy + v3(dR[0][1], dR[1][1], dR[2][1]);
-    gn = gn + v3(dR[0][2], dR[1][2], dR[2][2]);
-    if (a.dk && k != 0.f) unsafeAtomicAdd(a.dk, 2.f * gk / k);
-  }
-  V3 de1, de2;
-  frame_bwd(fr, gx, gy, gn, de1, de2);
-  dv0 = dv0 - de1 - de2;
-  dv1 = dv1 + de1;
-  dv2 = dv2 + de2;
-  unsafeAtomicAdd(a.dverts + 3 * i0, dv0.x);
-  unsafeAtomicAdd(a.dverts + 3 * i0 + 1, dv0.y);
-  unsafeAtomicAdd(a.dverts + 3 * i0 + 2, dv0.z);
-  unsafeAtomicAdd(a.dverts + 3 * i1, dv1.x);
-  unsafeAtomicAdd(a.dverts + 3 * i1 + 1, dv1.y);
-  unsafeAtomicAdd(a.dverts + 3 * i1 + 2, dv1.z);
-  unsafeAtomicAdd(a.dverts + 3 * i2, dv2.x);
-  unsafeAtomicAdd(a.dverts + 3 * i2 + 1, dv2.y);
-  unsafeAtomicAdd(a.dverts + 3 * i2 + 2, dv2.z);
 }
 
 // --------------------------------------------------------------- stage 2 --
@@ -311,7 +386,18 @@ void launch_bind_cov_fwd(const BindArgs& a, hipStream_t s) {
 
 void launch_bind_bwd(const BindArgs& a, hipStream_t s) {
   if (a.F <= 0) return;
-  hipLaunchKernelGGL(bind_bwd_kernel, dim3((a.F + 255) / 256), dim3(256), 0, s, a);
+  const int block_faces = a.G < kBindLanes ? kBindLanes / a.G : 1;
+  const bool rot = a.rot2d && a.drot, cov = a.dcov != nullptr;
+  const int groups = (a.F + block_faces - 1) / block_faces;
+  const dim3 grid(cov && groups > kBindCovBlocks ? kBindCovBlocks : groups), block(kBindLanes);
+  if (rot && cov)
+    hipLaunchKernelGGL((bind_bwd_kernel<true, true>), grid, block, 0, s, a, block_faces);
+  else if (rot)
+    hipLaunchKernelGGL((bind_bwd_kernel<true, false>), grid, block, 0, s, a, block_faces);
+  else if (cov)
+    hipLaunchKernelGGL((bind_bwd_kernel<false, true>), grid, block, 0, s, a, block_faces);
+  else
+    hipLaunchKernelGGL((bind_bwd_kernel<false, false>), grid, block, 0, s, a, block_faces);
 }
 
 void launch_faces_in_frustum(int F, const float* verts, const int32_t* faces, const float* proj, uint8_t* mask,

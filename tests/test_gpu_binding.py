@@ -270,3 +270,33 @@ def test_stage2_render_dyn():
         e = grad_rel_err(got, ref)
         print(f"  {name}: rel err {e:.2e}", flush=True)
         assert ref.abs().max() > 0 and e < 1e-3
+
+
+@pytest.mark.parametrize("F,G", [(1, 1), (257, 1), (20, 255), (20, 256), (3, 257), (1, 700), (129, 2), (86, 3), (43, 6)])
+def test_binding_backward_block_edges(F, G):
+    """Faces that fill a block's 256 lanes, leave lanes over, or span several passes of one block.
+
+    A vertex gradient sums up to G terms per face in float32: G * 2^-24 of the terms' magnitude, and the chain through
+    the frame about 100 roundings: 1e-4 of the largest gradient."""
+    print(f"case: bind backward F={F} G={G}", flush=True)
+    g = torch.Generator().manual_seed(F * 1000 + G)
+    v, f = S.icosphere(2)
+    v, f, n = v + torch.randn(v.shape, generator=g) * 0.02, f[torch.arange(F) % f.shape[0]], F * G
+    e = -torch.log(torch.rand(n, 3, generator=g))
+    bc, rot2d, scale2d = e / e.sum(1, keepdim=True), torch.randn(n, 2, generator=g), torch.randn(n, 2, generator=g) * 0.3
+    ov, orot, osc, osf = [t.double().requires_grad_(True) for t in (v, rot2d, scale2d, torch.tensor([0.4]))]
+    gv, grot, gsc, gsf = [t.detach().float().cuda().requires_grad_(True) for t in (ov, orot, osc, osf)]
+    wx, wq, ws, wc = [torch.randn(n, k, generator=g) for k in (3, 4, 3, 6)]
+    xyz_o, q_o, s_o, _ = OB.stage3(ov, f, bc.double(), orot, osc, 1e-4)
+    xyz, q, s = PB.bind_stage3(gv, f.cuda(), bc.cuda(), grot, gsc, 1e-4)
+    sign = torch.sign((q.detach().cpu().double() * q_o.detach()).sum(1, keepdim=True))
+    ref = torch.autograd.grad((xyz_o * wx).sum() + (q_o * (sign * wq)).sum() + (s_o * ws).sum(), [ov, orot, osc])
+    got = torch.autograd.grad((xyz * wx.cuda()).sum() + (q * wq.cuda()).sum() + (s * ws.cuda()).sum(), [gv, grot, gsc])
+    xyz_o, cov_o, _ = OB.stage2(ov, f, bc.double(), G, torch.tanh(osf.reshape(())) * 2.0, 0.2, 2.5e-6)
+    xyz, cov, _ = PB.bind_stage2(gv, f.cuda(), bc.cuda(), gsf, 0.2, 2.0, 2.5, gaussians_per_face=G)
+    ref += torch.autograd.grad((xyz_o * wx).sum() + (cov_o * wc).sum() * 1e2, [ov, osf])
+    got += torch.autograd.grad((xyz * wx.cuda()).sum() + (cov * wc.cuda()).sum() * 1e2, [gv, gsf])
+    for name, a, b in zip(("verts 3", "rotation", "scaling", "verts 2", "scale_factor"), got, ref):
+        e = grad_rel_err(a, b)
+        print(f"  {name}: rel err {e:.2e}")
+        assert e < 1e-4
