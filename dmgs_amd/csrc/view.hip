@@ -26,22 +26,30 @@ constexpr int kRows = 256;  // Gaussians per work-group
 template <int R>
 struct LdsRows {
   static constexpr int S = R % 2 ? R : R + 1;
+  static constexpr int kIter = (kRows * R / 4 + kRows - 1) / kRows;
   __align__(16) float v[kRows * S];
   __device__ __forceinline__ float* row(int t) { return v + t * S; }
   // rows [0, n) from / to consecutive global rows (16-byte aligned: the first row is a multiple of kRows)
   __device__ __forceinline__ void load(const float* __restrict__ src, int n) {
-    const int f4 = n * R / 4, rest = n * R - 4 * f4;
+    float4 x[kIter];  // every load before the first LDS store
+    request(src, n, x);
+    put(src, n, x);
+  }
+  // load in two halves; positions past the end read the last vector
+  __device__ __forceinline__ void request(const float* __restrict__ src, int n, float4 (&x)[kIter]) {
+    const int f4 = n * R / 4;
     const float4* s4 = reinterpret_cast<const float4*>(src);
     if (f4 > 0) {
-      constexpr int kIter = (kRows * R / 4 + kRows - 1) / kRows;
-      float4 x[kIter];  // every load before the first LDS store; positions past the end read the last vector
 #pragma unroll
       for (int i = 0; i < kIter; ++i) x[i] = s4[min(i * kRows + (int)threadIdx.x, f4 - 1)];
+    }
+  }
+  __device__ __forceinline__ void put(const float* __restrict__ src, int n, const float4 (&x)[kIter]) {
+    const int f4 = n * R / 4, rest = n * R - 4 * f4;
 #pragma unroll
-      for (int i = 0; i < kIter; ++i) {
-        const int f = i * kRows + (int)threadIdx.x;
-        if (f < f4) put4(f, x[i]);
-      }
+    for (int i = 0; i < kIter; ++i) {
+      const int f = i * kRows + (int)threadIdx.x;
+      if (f < f4) put4(f, x[i]);
     }
     if ((int)threadIdx.x < rest) at(4 * f4 + (int)threadIdx.x) = src[4 * f4 + threadIdx.x];
   }
@@ -225,10 +233,13 @@ __device__ __forceinline__ void load_shape(const ViewArgs& a, int g, ViewGaussia
     return;
   }
   G.e = make_float3(a.scales[3 * (size_t)g], a.scales[3 * (size_t)g + 1], a.scales[3 * (size_t)g + 2]);
+  G.q = reinterpret_cast<const float4*>(a.rotations)[g];
+}
+__device__ __forceinline__ void make_shape(const ViewArgs& a, ViewGaussian& G) {
+  if (a.cov3D_precomp) return;
   if (a.raw & DMGS_RAW_SCALES) G.e = make_float3(expf(G.e.x), expf(G.e.y), expf(G.e.z));
   const float m = a.scale_modifier;
   G.s = make_float3(m * G.e.x, m * G.e.y, m * G.e.z);
-  G.q = reinterpret_cast<const float4*>(a.rotations)[g];
   G.qn = 1.0f;
   if (a.raw & DMGS_RAW_ROTATIONS) {
     G.qn = quat_norm(G.q);
@@ -269,18 +280,31 @@ __global__ __launch_bounds__(kRows) void view_preprocess_kernel(ViewArgs a) {
   __shared__ LdsRows<(REST > 0 ? REST : 1)> rows;
   __shared__ uint32_t s_tiles;
   const int g0 = blockIdx.x * kRows, g = g0 + (int)threadIdx.x;
+  const bool live = g < a.P;
+  const size_t i = live ? (size_t)g : 0;
   if (threadIdx.x == 0) s_tiles = 0u;
-  if constexpr (REST > 0) rows.load(a.shs_rest + (size_t)g0 * REST, min(kRows, a.P - g0));
+  // the Gaussian's own loads, then the rows', all in flight together; the projection runs while the rows arrive
+  const float3 p = make_float3(a.means3D[3 * i], a.means3D[3 * i + 1], a.means3D[3 * i + 2]);
+  ViewGaussian G;
+  load_shape(a, i, G);
+  const float op = a.opacities[i];
+  float dc[3] = {0.f, 0.f, 0.f};
+  if constexpr (REST >= 0)
+    if (!a.colors_precomp)
+      for (int k = 0; k < 3; ++k) dc[k] = a.shs[3 * i + k];
+  float4 x[LdsRows<(REST > 0 ? REST : 1)>::kIter];
+  const int n = min(kRows, a.P - g0);
+  if constexpr (REST > 0) rows.request(a.shs_rest + (size_t)g0 * REST, n, x);
+  const ViewParams v = view_params(a.viewmatrix, a.projmatrix, a.campos, a.W, a.H, a.grid_x, a.grid_y, a.focal_x,
+                                   a.focal_y, a.tanfovx, a.tanfovy);
+  make_shape(a, G);
+  SplatGeom o;
+  const bool seen = view_project(p, G.c3, v, o) && live;
+  if constexpr (REST > 0) rows.put(a.shs_rest + (size_t)g0 * REST, n, x);
   __syncthreads();
   uint32_t tiles = 0;
-  if (g < a.P) {
-    const float3 p = make_float3(a.means3D[3 * (size_t)g], a.means3D[3 * (size_t)g + 1], a.means3D[3 * (size_t)g + 2]);
-    ViewGaussian G;
-    load_shape(a, g, G);
-    const ViewParams v = view_params(a.viewmatrix, a.projmatrix, a.campos, a.W, a.H, a.grid_x, a.grid_y, a.focal_x,
-                                     a.focal_y, a.tanfovx, a.tanfovy);
-    SplatGeom o;
-    if (!view_project(p, G.c3, v, o)) {
+  if (live) {
+    if (!seen) {
       a.radii[g] = 0;
       a.depth_keys[g] = kSortSkip;
     } else {
@@ -290,7 +314,6 @@ __global__ __launch_bounds__(kRows) void view_preprocess_kernel(ViewArgs a) {
                           a.colors_precomp[3 * (size_t)g + 2]);
       } else {
         if constexpr (REST >= 0) {
-          const float dc[3] = {a.shs[3 * (size_t)g], a.shs[3 * (size_t)g + 1], a.shs[3 * (size_t)g + 2]};
           rgb = view_rgb(a.sh_degree, ShSplit{dc, rows.row(threadIdx.x), REST}, p, v.campos);
         } else {
           float sh[48];
@@ -298,7 +321,6 @@ __global__ __launch_bounds__(kRows) void view_preprocess_kernel(ViewArgs a) {
           rgb = view_rgb(a.sh_degree, sh, p, v.campos);
         }
       }
-      const float op = a.opacities[g];
       float4* sp = a.splats + (size_t)DMGS_SPLAT_F4 * g;
       sp[0] = make_float4(o.pix.x, o.pix.y, o.conic.x, o.conic.y);
       sp[1] = make_float4(o.conic.z, a.raw & DMGS_RAW_OPACITIES ? view_sigmoid(op) : op, rgb.x, rgb.y);
@@ -350,6 +372,7 @@ __global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
   if (vis) {
     ViewGaussian G;
     load_shape(a, g, G);
+    make_shape(a, G);
     dmean = ewa_backward(p, G.c3, v, r0.x, r0.y, r1.x, r1.y, r2.x, dc);
     if (!a.cov3D_precomp) {
       cov3d_backward(dc, G.s, G.R, G.q, ds, dq);
