@@ -116,7 +116,7 @@ struct ListLayout {
     tkeys_b = o; o += align_up(K * 4);
     vals_a = o; o += align_up(K * 4);
     vals_b = o; o += align_up(K * 4);
-    scratch = o; o += align_up(dmgs::radix_scratch_words(K) * 4);   // sort histograms
+    scratch = o; o += align_up(dmgs::radix_list_scratch_words(K) * 4);  // sort histograms
     chunk = o; o += align_up(dmgs::duplicate_scratch_words(K) * 4);  // duplicate chunk starts
     total = o;
   }
@@ -152,12 +152,13 @@ struct Ctx {
   explicit Ctx(const dmgs_batch* b, bool segments = true)
       : N((size_t)b->num_views * b->num_gaussians),
         S(N, (size_t)b->total_tiles, (size_t)b->total_pixels, segments),
-        L((size_t)b->capacity), mode(b->cell_mode),
+        L((size_t)b->capacity), capacity((size_t)b->capacity), mode(b->cell_mode),
         local_bits(b->cell_mode == 1 ? std::max(1, bits_for((uint32_t)(b->max_view_cells - 1))) : 0),
         global_bits(std::max(1, bits_for((uint32_t)(b->total_cells - 1)))) {}
   // the depth keys also order by view (with one view plain depth bits do, at any depth)
   bool view_keys(const dmgs_batch* b) const { return mode == 1 && b->num_views > 1; }
   uint32_t* count(const dmgs_batch* b) const { return at<uint32_t>(b->state, S.offsets) + (N - 1); }
+  size_t capacity;
   int mode;
   // key bits of the cell sort: the cell within the view (mode 1) or the
   // global cell id (mode 0; cell ids 0 .. total_cells - 1, so 65536 cells
@@ -165,8 +166,8 @@ struct Ctx {
   int local_bits;
   int global_bits;
   int cell_sort_bits() const { return mode == 1 ? local_bits : global_bits; }
-  // a one-pass sort (view-major lists, at most 256 cells per view) leaves the lists in the b buffers
-  bool lists_in_b() const { return mode == 1 && local_bits <= 8; }
+  // a one-pass sort (view-major lists of at most 256 cells per view, or 512 on large ones) leaves the lists in the b buffers
+  bool lists_in_b() const { return mode == 1 && dmgs::radix_one_pass(capacity, local_bits); }
 };
 
 dmgs::MVArgs mv_args(const dmgs_batch* b, const Ctx& c, const float* params) {
@@ -257,7 +258,8 @@ int bin_entries(const dmgs_batch* b, const Ctx& c, bool chunks_ready, hipStream_
   d.zero = at<uint32_t>(b->state, c.S.bucket_hist);
   d.zero_n = 512 + 2 * (size_t)b->total_cells;
   // view-major lists: the duplicate also counts the first sort pass's digits
-  const int w0 = d.view_major ? dmgs::radix_min_passes_first_width(K, c.local_bits) : -1;
+  const bool wide = d.view_major && c.local_bits == 9 && c.lists_in_b();
+  const int w0 = wide ? 9 : d.view_major ? dmgs::radix_min_passes_first_width(K, c.local_bits) : -1;
   if (w0 > 0) {
     d.hist = at<uint32_t>(b->lists, c.L.scratch);
     d.hist_bits = w0;
@@ -266,8 +268,10 @@ int bin_entries(const dmgs_batch* b, const Ctx& c, bool chunks_ready, hipStream_
   uint32_t* kb = at<uint32_t>(b->lists, c.L.tkeys_b);
   uint32_t* vb = at<uint32_t>(b->lists, c.L.vals_b);
   if (d.view_major) {  // sort the cell-within-view bits only; the view order is already there
-    const bool in_b = dmgs::radix_sort_pairs_min_passes(d.tile_keys, d.values, kb, vb, K, c.local_bits,
-                                                        at<uint32_t>(b->lists, c.L.scratch), st, d.K_dev, w0 > 0);
+    uint32_t* scratch = at<uint32_t>(b->lists, c.L.scratch);
+    if (wide) dmgs::radix_sort_pairs_wide_digit(d.tile_keys, d.values, kb, vb, K, scratch, st, d.K_dev);
+    const bool in_b = wide || dmgs::radix_sort_pairs_min_passes(d.tile_keys, d.values, kb, vb, K, c.local_bits, scratch,
+                                                                st, d.K_dev, w0 > 0);
     if (in_b != c.lists_in_b()) return bfail(DMGS_EHIP, "internal: sorted list buffer mismatch");
     dmgs::launch_view_cell_ranges(in_b ? kb : d.tile_keys, K, at<uint2>(b->state, c.S.ranges), b->total_cells,
                                   d.views, st, d.K_dev, true);

@@ -72,6 +72,12 @@ bool radix_sort_pairs_min_passes(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint3
 // counted with plain LDS atomics.
 void radix_sort_entry_keys(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1, size_t n, uint32_t* scratch,
                            hipStream_t s, uint32_t* n_out, uint32_t* flags);
+// Whether the cell lists are sorted in one pass (of 8 bits, or of 9 on lists of at least 4 M).
+bool radix_one_pass(size_t n, int bits);
+// One pass of 9 bits over pairs whose digits the duplicate has counted; the sorted pairs are in k1, v1.
+void radix_sort_pairs_wide_digit(const uint32_t* k0, const uint32_t* v0, uint32_t* k1, uint32_t* v1, size_t n,
+                                 uint32_t* scratch, hipStream_t s, const uint32_t* n_dev);
+size_t radix_list_scratch_words(size_t n);  // of either cell-list sort
 // Digit width of the first pass of radix_sort_pairs_min_passes, or -1 when
 // its blocks are not 4096 keys (the duplicate's chunks) for this n.
 int radix_min_passes_first_width(size_t n, int bits);

@@ -225,6 +225,23 @@ __device__ __forceinline__ uint64_t digit_peers(uint32_t d, int nbits, bool vali
   return peers;
 }
 
+// Work-groups go to the XCDs in turn.  The tile of this one, such that each XCD works on runs of up to 32 consecutive
+// ones: the counts (32 to a cache line) and the short pieces of a digit which neighbouring tiles write lie side by
+// side and meet in one L2.  Longer runs gain nothing and leave the XCDs unequal work; few tiles take shorter runs, so
+// that every XCD has some.  Grids of xcd_grid(tiles).
+constexpr uint32_t kXcds = 8;
+__host__ __device__ __forceinline__ uint32_t xcd_run_shift(uint32_t tiles) {
+  return tiles < 128u ? 0u : tiles >= 2048u ? 5u : 25u - (uint32_t)__builtin_clz(tiles);
+}
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t tiles) {
+  const uint32_t sh = xcd_run_shift(tiles), run = (1u << sh) - 1u, i = blockIdx.x;
+  return (i & ~((kXcds << sh) - 1u)) | (i % kXcds) << sh | (i / kXcds & run);
+}
+static uint32_t xcd_grid(uint32_t tiles) {
+  const uint32_t span = kXcds << xcd_run_shift(tiles);
+  return (tiles + span - 1u) / span * span;
+}
+
 // SPREAD: the digits are close to uniform (the low bytes of depth keys), so
 // per-wave counters with one plain LDS atomic per key rarely collide;
 // otherwise lanes with equal digits are grouped by ballots first.
@@ -240,14 +257,16 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
   __shared__ uint32_t cnt[256];
   __shared__ uint32_t wcnt[SPREAD ? kSortWaves : 1][256];
   if (n_dev) n = min(n, (size_t)*n_dev);  // device-side length (blocks past it count nothing)
+  const uint32_t tile = xcd_tile(nb);
   const uint32_t mask = (1u << nbits) - 1u;
+  if (tile >= nb) return;  // uniform per block
   cnt[threadIdx.x] = 0;
   if constexpr (SPREAD) {
 #pragma unroll
     for (int w = 0; w < kSortWaves; ++w) wcnt[w][threadIdx.x] = 0;
   }
   __syncthreads();
-  const size_t base = (size_t)blockIdx.x * (kSortThreads * ITEMS);
+  const size_t base = (size_t)tile * (kSortThreads * ITEMS);
   const int lane = threadIdx.x & 63;
   if (base < n) {  // uniform per block; then n >= 1
     // every key of the thread is requested before the first is used
@@ -290,7 +309,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_hist_kernel(const uint32_t
 #pragma unroll
       for (int w = 0; w < kSortWaves; ++w) c += wcnt[w][threadIdx.x];
     }
-    hist[(size_t)threadIdx.x * nb + blockIdx.x] = c;
+    hist[(size_t)threadIdx.x * nb + tile] = c;
   }
 }
 
@@ -349,42 +368,39 @@ __global__ __launch_bounds__(NT) void radix_rowscan_kernel(uint32_t* __restrict_
 
 // Ranking (5 instructions a key and digit bit) and the random access of the write-out bound a pass over a few million
 // keys, memory one over more.  The values are requested with the keys, a key leaves with its value in one write-out
-// of one LDS read per digit, and work-groups, which go to the XCDs in turn, take a run of consecutive tiles per XCD,
-// so that the short pieces which neighbouring tiles append to a digit meet in one L2.  Per pass, before and now:
+// of one LDS read per digit.  Per pass, before and now:
 // the passes of eight 800 x 800 views of 1 M Gaussians (5 M keys, 18 M pairs) 48 and 36 us, of 0.7 M keys 11.8 and
 // 9.1 us; 164 M pairs with 5-bit digits 521 us (2.6 GB at 5.0 TB/s).
-constexpr uint32_t kXcds = 8;
 // FIRST: keys equal to kSortSkip are dropped, each value is its key's input
 // position (vin unused), and work-group 0 stores the number of keys kept in
 // *n_out.
-// BITS: ballots per key, at least the digit's width.
-template <int ITEMS, int BITS, bool FIRST = false>
-__global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
+// BITS: ballots per key, at least the digit's width.  NT: lanes, at least one per digit.
+template <int ITEMS, int BITS, bool FIRST = false, int NT = kSortThreads>
+__global__ __launch_bounds__(NT) void radix_scatter_kernel(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, uint32_t* __restrict__ kout,
     uint32_t* __restrict__ vout, size_t n, int shift, int nbits, const uint32_t* __restrict__ hist_excl,
     const uint32_t* __restrict__ totals, uint32_t nb, const uint32_t* __restrict__ n_dev,
     uint32_t* __restrict__ n_out) {
-  constexpr int kTile = kSortThreads * ITEMS;
+  constexpr int kTile = NT * ITEMS, kWaves = NT / 64;
   constexpr int kSlice = 64 * ITEMS;
   if (n_dev) n = min(n, (size_t)*n_dev);
-  const uint32_t per_xcd = ((uint32_t)((n + kTile - 1) / kTile) + kXcds - 1) / kXcds;
-  const uint32_t tile = blockIdx.x % kXcds * per_xcd + blockIdx.x / kXcds;
-  if (blockIdx.x / kXcds >= per_xcd || (size_t)tile * kTile >= n) return;  // uniform per block
-  __shared__ uint32_t wcnt[kSortWaves][256];  // counts, then the block-local position of each wave's first key of a digit
-  __shared__ uint32_t goff[256];              // global minus block-local position of each digit
+  const uint32_t tile = xcd_tile(nb);
+  if ((size_t)tile * kTile >= n) return;  // uniform per block
+  __shared__ uint32_t wcnt[kWaves][NT];  // counts, then the block-local position of each wave's first key of a digit
+  __shared__ uint32_t goff[NT];              // global minus block-local position of each digit
   __shared__ uint2 sbuf[kTile];               // (key, value) in block-sorted order
-  __shared__ uint32_t s_wave[kSortWaves];
+  __shared__ uint32_t s_wave[kWaves];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar addressing
   const uint32_t mask = (1u << nbits) - 1u;
-  for (int w = 0; w < kSortWaves; ++w) wcnt[w][threadIdx.x] = 0;
+  for (int w = 0; w < kWaves; ++w) wcnt[w][threadIdx.x] = 0;
   // global position of the block's first element of each digit (one thread
   // per digit), before any key is held in registers
   const uint32_t dg = threadIdx.x;
   uint32_t gbase = 0;
   {
     uint32_t all_total;
-    const uint32_t digit_base = block_exclusive_scan<kSortWaves>(dg <= mask ? totals[dg] : 0u, s_wave, all_total);
+    const uint32_t digit_base = block_exclusive_scan<kWaves>(dg <= mask ? totals[dg] : 0u, s_wave, all_total);
     if (dg <= mask) gbase = digit_base + hist_excl[(size_t)dg * nb + tile];
     if constexpr (FIRST) {
       if (n_out && tile == 0 && threadIdx.x == 0) *n_out = all_total;
@@ -423,15 +439,15 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
   __syncthreads();
   // per digit (one thread each): exclusive prefix over waves and block-local
   // digit start
-  uint32_t c[kSortWaves], tot = 0;
-  for (int w = 0; w < kSortWaves; ++w) {
+  uint32_t c[kWaves], tot = 0;
+  for (int w = 0; w < kWaves; ++w) {
     c[w] = wcnt[w][dg];
     tot += c[w];
   }
   uint32_t count;  // the keys this block sorts (all of its slice unless skipped ones)
-  uint32_t start = block_exclusive_scan<kSortWaves>(tot, s_wave, count);
+  uint32_t start = block_exclusive_scan<kWaves>(tot, s_wave, count);
   goff[dg] = gbase - start;
-  for (int w = 0; w < kSortWaves; ++w) {
+  for (int w = 0; w < kWaves; ++w) {
     wcnt[w][dg] = start;
     start += c[w];
   }
@@ -448,7 +464,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_scatter_kernel(
   __syncthreads();
   // coalesced write-out: each digit's run is contiguous in LDS and in memory
 #pragma unroll 4
-  for (uint32_t i = threadIdx.x; i < count; i += kSortThreads) {
+  for (uint32_t i = threadIdx.x; i < count; i += NT) {
     const uint2 e = sbuf[i];
     const uint32_t pos = goff[digit(e.x)] + i;
     if (pos < n) {  // always true for a consistent histogram; guards the write
@@ -466,6 +482,26 @@ static void launch_rowscan(uint32_t* hist, uint32_t nb, uint32_t* totals, uint32
 }
 
 static int sort_items(size_t n) { return n >= ((size_t)4 << 20) ? 16 : 4; }
+
+// 512 digits in one pass instead of two passes of 5 and 4 bits: the lists of a view of 257 to 512 cells (1600 x 900,
+// 1920 x 1080) in one trip through memory.  From the size on whose blocks are the duplicate's chunks.  164 M pairs:
+// 2 x 521 us and 172 us of counting become 726 us, and the duplicate's count of 512 digits 80 us more; 6 M pairs
+// (1920 x 1080, 1 M Gaussians) 58 us become 25.
+bool radix_one_pass(size_t n, int bits) { return bits <= 8 || (bits == 9 && sort_items(n) == 16); }
+
+void radix_sort_pairs_wide_digit(const uint32_t* k0, const uint32_t* v0, uint32_t* k1, uint32_t* v1, size_t n,
+                                 uint32_t* scratch, hipStream_t s, const uint32_t* n_dev) {
+  if (n == 0) return;
+  const uint32_t nb = (uint32_t)((n + 4095) / 4096), grid = xcd_grid(nb);
+  uint32_t* totals = scratch + 512 * (size_t)nb;
+  launch_rowscan(scratch, nb, totals, 512, s);
+  hipLaunchKernelGGL((radix_scatter_kernel<8, 9, false, 512>), dim3(grid), dim3(512), 0, s, k0, v0, k1, v1, n, 0, 9,
+                     (const uint32_t*)scratch, (const uint32_t*)totals, nb, n_dev, (uint32_t*)nullptr);
+}
+
+size_t radix_list_scratch_words(size_t n) {
+  return sort_items(n) == 16 ? 512 * ((n + 4095) / 4096) + 512 + 64 : radix_scratch_words(n);
+}
 
 size_t radix_scratch_words(size_t n) {
   const size_t tile = (size_t)kSortThreads * sort_items(n);
@@ -486,7 +522,7 @@ static void radix_passes(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1,
                          uint32_t* scratch, hipStream_t s, const uint32_t* n_dev, int passes,
                          bool first_hist_ready = false, int spread_below = 0, const EntryPass* entry = nullptr) {
   constexpr size_t kTile = (size_t)kSortThreads * ITEMS;
-  const uint32_t nb = (uint32_t)((n + kTile - 1) / kTile), grid = (nb + kXcds - 1) / kXcds * kXcds;
+  const uint32_t nb = (uint32_t)((n + kTile - 1) / kTile), grid = xcd_grid(nb);
   int widths[4];
   int left = bits;
   for (int p = 0; p < passes; ++p) {
@@ -501,7 +537,7 @@ static void radix_passes(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1,
   for (int p = 0; p < passes; ++p) {
     const int w = widths[p];
     if (p == 0 && entry) {
-      hipLaunchKernelGGL((radix_hist_kernel<ITEMS, true, true>), dim3(nb), dim3(kSortThreads), 0, s,
+      hipLaunchKernelGGL((radix_hist_kernel<ITEMS, true, true>), dim3(grid), dim3(kSortThreads), 0, s,
                          (const uint32_t*)ka, n, shift, w, hist, nb, (const uint32_t*)nullptr, entry->flags);
       launch_rowscan(hist, nb, totals, 1u << w, s);
       hipLaunchKernelGGL((radix_scatter_kernel<ITEMS, 8, true>), dim3(grid), dim3(kSortThreads), 0, s,
@@ -515,10 +551,10 @@ static void radix_passes(uint32_t* k0, uint32_t* v0, uint32_t* k1, uint32_t* v1,
     }
     if (p == 0 && first_hist_ready) {
     } else if (shift + w <= spread_below) {
-      hipLaunchKernelGGL((radix_hist_kernel<ITEMS, true>), dim3(nb), dim3(kSortThreads), 0, s, (const uint32_t*)ka, n,
+      hipLaunchKernelGGL((radix_hist_kernel<ITEMS, true>), dim3(grid), dim3(kSortThreads), 0, s, (const uint32_t*)ka, n,
                          shift, w, hist, nb, n_dev);
     } else {
-      hipLaunchKernelGGL((radix_hist_kernel<ITEMS, false>), dim3(nb), dim3(kSortThreads), 0, s, (const uint32_t*)ka,
+      hipLaunchKernelGGL((radix_hist_kernel<ITEMS, false>), dim3(grid), dim3(kSortThreads), 0, s, (const uint32_t*)ka,
                          n, shift, w, hist, nb, n_dev);
     }
     launch_rowscan(hist, nb, totals, 1u << w, s);
@@ -627,20 +663,24 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
   __shared__ uint32_t s_rx[256], s_ry[256];  // multi-view: tile rectangle, [lo, hi) packed 16:16
   __shared__ int s_vcx[kDupViews];           // multi-view: cells per row of view v
   __shared__ uint32_t s_vtb[kDupViews];      // multi-view: key base of view v
-  __shared__ uint32_t s_hist[256];           // digit counts of this chunk (first sort pass)
+  __shared__ uint32_t s_hist[512];           // digit counts of this chunk (first sort pass)
   const uint32_t K = device_count(a.K, a.K_dev);
-  const uint32_t lo_slot = blockIdx.x * kDupChunk;
+  const uint32_t chunks = (uint32_t)(((size_t)a.K + kDupChunk - 1) / kDupChunk);
+  const uint32_t chunk = xcd_tile(chunks);
   const uint32_t hmask = (1u << a.hist_bits) - 1u;
   if (a.zero) {  // this work-group's share of the words a later step needs zeroed
     const size_t per = (a.zero_n + gridDim.x - 1) / gridDim.x;
     const size_t zlo = (size_t)blockIdx.x * per, zhi = min(a.zero_n, zlo + per);
     for (size_t i = zlo + threadIdx.x; i < zhi; i += 256) a.zero[i] = 0u;
   }
+  if (chunk >= chunks) return;  // uniform per block
+  const uint32_t lo_slot = chunk * kDupChunk;
   if (lo_slot >= K) {  // uniform per block: an empty chunk counts nothing
-    if (a.hist && threadIdx.x <= hmask) a.hist[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = 0u;
+    if (a.hist)
+      for (uint32_t d = threadIdx.x; d <= hmask; d += 256) a.hist[(size_t)d * chunks + chunk] = 0u;
     return;
   }
-  if (a.hist) s_hist[threadIdx.x] = 0u;
+  if (a.hist) s_hist[threadIdx.x] = s_hist[threadIdx.x + 256] = 0u;
   const uint32_t hi_slot = min(K, lo_slot + kDupChunk);
   const uint32_t P = (uint32_t)a.P;
   const uint32_t nviews = a.views ? (P + a.per_view - 1) / a.per_view : 0u;
@@ -652,7 +692,7 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
     s_vtb[v] = view_tb(v);
   }
   __syncthreads();
-  uint32_t first = a.chunk_first[blockIdx.x];
+  uint32_t first = a.chunk_first[chunk];
   uint32_t win_begin = (first == 0) ? 0u : min(a.offsets[first - 1], K);
   // A window's per-entry loads (entry, its slot range, its rectangle), issued
   // together; the next window's are in flight while this one is emitted.
@@ -789,7 +829,8 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
   }
   // the chunk is the first sort pass's block: its digit histogram, in the
   // radix histogram's layout (digit-major over blocks)
-  if (a.hist && threadIdx.x <= hmask) a.hist[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = s_hist[threadIdx.x];
+  if (a.hist)
+    for (uint32_t d = threadIdx.x; d <= hmask; d += 256) a.hist[(size_t)d * chunks + chunk] = s_hist[d];
 }
 
 size_t duplicate_scratch_words(size_t K) { return (K + kDupChunk - 1) / kDupChunk + 64; }
@@ -797,8 +838,8 @@ size_t duplicate_scratch_words(size_t K) { return (K + kDupChunk - 1) / kDupChun
 void launch_duplicate(const DupArgs& a, hipStream_t s) {
   if (a.P <= 0 || a.K == 0) return;
   if (!a.chunk_ready) hipLaunchKernelGGL(chunk_first_kernel, dim3((a.P + 255) / 256), dim3(256), 0, s, a);
-  const uint32_t chunks = (a.K + kDupChunk - 1) / kDupChunk;
-  hipLaunchKernelGGL(duplicate_kernel, dim3(chunks), dim3(256), 0, s, a);
+  const uint32_t chunks = (uint32_t)(((size_t)a.K + kDupChunk - 1) / kDupChunk);
+  hipLaunchKernelGGL(duplicate_kernel, dim3(xcd_grid(chunks)), dim3(256), 0, s, a);
 }
 
 __global__ void fill_u32_kernel(uint32_t* __restrict__ p, size_t n, uint32_t v) {

@@ -1,9 +1,12 @@
 """The radix sort's scatter at the edges of its tiles (1024 and 4096 keys), of the runs of tiles that the XCDs take
-(8 per round) and of its digit widths (6 and 8 ballots a key): keys and values equal torch's stable sort."""
+(8 per round) and of its digit widths (6, 8 and 9 ballots a key): keys and values equal torch's stable sort."""
 import pytest
 import torch
 
 from dmgs_amd import _native as N
+from dmgs_amd import batched as BT
+from dmgs_amd import cameras as C
+from dmgs_amd import scenes as S
 
 pytestmark = pytest.mark.gpu
 LARGE = 4 << 20  # from here on a tile holds 4096 keys
@@ -28,3 +31,34 @@ def test_sort_pairs_tile_edges(n, bits):
                                 N.stream_handle(k0.device)), "dmgs_sort_pairs")
     order = torch.sort(k, stable=True).indices
     assert torch.equal(k0.cpu(), to32(k[order])) and torch.equal(v0.cpu(), v[order])
+
+
+@pytest.mark.parametrize("P,sizes", [(3000, [(1100, 1000), (64, 64)]), (20000, [(1920, 1080)]),
+                                     (20000, [(1088, 960), (2048, 1024), (33, 17)]), (700_000, [(1600, 900)] * 3)])
+def test_wide_digit_lists_equal_two_passes(P, sizes):
+    """Cell lists of views of 257 to 512 cells: one pass of 512 digits (capacities from 4 Mi) equals two passes."""
+    print(f"case: wide digit P={P} sizes={sizes}", flush=True)
+    model = S.free_scene(P, seed=6, layout="mixture")
+    cams = [C.camera_at((0.3 * k, 0.2, -4.0), w, h) for k, (w, h) in enumerate(sizes)]
+    r = BT.BatchedRenderer(cams, [torch.zeros(3, device="cuda")] * len(cams), P, sh_degree=3, cell_mode=1)
+    params = BT.pack_model(model.to("cuda"))
+    K = r.count_instances(params)
+    got = []
+    for cap in (max(K, LARGE), min(K, LARGE - 1)):
+        r.plan(params, K_cap=cap)
+        images = r.forward(params)
+        got.append([t.cpu() for t in r.cell_lists()] + [images.cpu()])
+    if K >= LARGE:  # a truncated list cannot be compared; the order can
+        assert P == 700_000
+        ranges, keys, ids = got[0][:3]
+        k = keys.long() & 0xFFFF
+        cell, view = k & 0xFFF, k >> 12
+        pos = torch.arange(k.numel())
+        assert torch.all(cell[1:] >= cell[:-1]) and torch.all((cell[1:] > cell[:-1]) | (view[1:] >= view[:-1]))
+        base = torch.tensor([r.views[v].cell_base for v in range(r.B)])
+        same = (cell[1:] == cell[:-1]) & (view[1:] == view[:-1])
+        first = torch.cat([torch.zeros(1, dtype=torch.long), pos[1:][~same]])
+        assert torch.equal(ranges[base[view[first]] + cell[first], 0].long(), first)
+    else:
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
