@@ -15,8 +15,8 @@
 // n_contrib of the tile (entries behind every pixel's last contributor
 // cannot contribute), transmittance is recomputed (times 1 / (1 - alpha), one
 // reciprocal) instead of being stored, and the wave sums its 9 per-splat
-// partial gradients into a per-batch LDS accumulator; the work-group flushes
-// that accumulator with one global atomic per (splat, value) per batch.
+// partial gradients into a set of LDS accumulators, flushed with one global
+// atomic per (splat, value) and tile.
 //
 // Several views in one launch: a global tile id indexes the ranges; the view
 // table gives each tile's image size, background and packed output offset.
@@ -30,9 +30,9 @@
 // running totals would lose it).  That is the whole state of the backward recursion at the boundary, so
 // every 64-member segment is a work-group of its own.  Slots (4 KB) come from a counter; a tile that gets
 // none has a longer last segment.  Launches of more than kSegmentTiles tiles fill the GPU without it.
-// Blend backward of one view, us, before and after (MI355X): 10k Gaussians at 200x200 375 -> 80, 1M at
-// 800x800 225 -> 105, 491k face-bound at 800x800 1385 -> 234, 500k at 333x251 1731 -> 173 (their forwards
-// get 12-43 us longer: the states are written, summed and cleared).
+// Blend backward of one view, us, one wave per tile and with segments (MI355X): 10k Gaussians at 200x200 375
+// and 58, 1M at 800x800 225 and 89, 491k face-bound at 800x800 1385 and 172 (their forwards get 12-43 us longer:
+// the states are written, summed and cleared).
 #include "dmgs_common.h"
 #include "dmgs_kernels.h"
 
@@ -159,81 +159,79 @@ __device__ __forceinline__ float splat_exp2(float p) { return __builtin_amdgcn_e
 
 #define DMGS_DPP_ADD(v, ctrl) ((v) + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), (ctrl), 0xF, 0xF, true)))
 
-// Sums over a one-wave work-group of nine per-lane values, through LDS: each
-// lane stores its values 0-7 (red[q][lane]); lane (row r, row position p)
-// then adds value 2r + (p >> 3) of the eight lanes 8 (p & 7) .. 8 (p & 7) + 7
-// (two 16-byte reads, seven adds), and two quad butterflies plus a shift by
-// four lanes leave the sum over all 64 lanes in row positions 7 and 15.
-// Value 8 takes DPP row sums and two row broadcasts (lane 63 ends with its
-// total).  About 17 VALU instead of row_sums9's 28 plus its selects.
-struct WaveSum9 {
+// Sums over a one-wave work-group of eight per-lane values, through LDS: each
+// lane stores its values (red[q][lane]); lane (row r, row position p) then adds
+// value 2r + (p >> 3) of the eight lanes 8 (p & 7) .. 8 (p & 7) + 7 (two 16-byte
+// reads, seven adds), and two quad butterflies plus a shift by four lanes leave
+// the sum over all 64 lanes in row positions 7 and 15: 11 VALU instructions.
+// A ninth value would take ten more by itself; it waits in a row of LDS until
+// four splats' fill the wave (row_sums4, 7 for the four).  The same tree in
+// registers (half-wave and row exchanges) takes 24 and 8.
+struct WaveSum8 {
   int q;       // the value this lane sums in the LDS step (0..7)
   int src;     // the first of its eight source lanes
   bool owner;  // row position 7 or 15: ends with the total of value q
-  bool last;   // lane 63: ends with the total of value 8
 };
-__device__ __forceinline__ WaveSum9 wave_sum9_lane(unsigned lane) {
+__device__ __forceinline__ WaveSum8 wave_sum8_lane(unsigned lane) {
   const unsigned p = lane & 15u, r = lane >> 4;
-  return {(int)(2u * r + (p >> 3)), (int)(8u * (p & 7u)), (p & 7u) == 7u, lane == 63u};
+  return {(int)(2u * r + (p >> 3)), (int)(8u * (p & 7u)), (p & 7u) == 7u};
 }
-// Rows named in row_mask add lane 15 (ctrl 0x142) or lane 31 (0x143) of the
-// wave; the other rows add zero.
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float add_row_bcast(float v) {
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xF, false));
+// Orders the LDS accesses of a one-wave work-group.  The LDS serves a wave's accesses in their order, so no wait for
+// the stores is needed before a load of what they wrote; only the compiler has to keep the order.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
-// acc[0..8] receive the totals by plain stores.  Called by the whole wave.
-__device__ __forceinline__ void wave_sums9(const float (&v)[DMGS_GACC_USED], float (*red)[DMGS_WAVE],
-                                           const WaveSum9& w, unsigned lane, float* acc) {
-  __syncthreads();  // the previous call's reads of red are done
+// acc[0..7] receive the totals by plain stores.  Called by the whole wave.
+__device__ __forceinline__ void wave_sums8(const float (&v)[8], float (*red)[DMGS_WAVE], const WaveSum8& w,
+                                           float* acc) {
+  const unsigned lane = threadIdx.x & 63;
+  wave_lds_order();  // the previous call's reads of red
 #pragma unroll
   for (int q = 0; q < 8; ++q) red[q][lane] = v[q];
-  __syncthreads();
+  wave_lds_order();
   const float4 a = *reinterpret_cast<const float4*>(&red[w.q][w.src]);
   const float4 b = *reinterpret_cast<const float4*>(&red[w.q][w.src + 4]);
   float s = ((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w));
   s = DMGS_DPP_ADD(s, 0xB1);   // quad_perm [1,0,3,2]
   s = DMGS_DPP_ADD(s, 0x4E);   // quad_perm [2,3,0,1]: each quad holds its four sources' sum
   s = DMGS_DPP_ADD(s, 0x114);  // row_shr 4: position 7 (15) adds position 3 (11)
-  float e = DMGS_DPP_ADD(v[8], 0xB1);
-  e = DMGS_DPP_ADD(e, 0x4E);
-  e = DMGS_DPP_ADD(DMGS_DPP_ADD(e, 0x124), 0x128);  // row_ror 4, row_ror 8: every lane holds its row's sum
-  e = add_row_bcast<0x142, 0xA>(e);                  // rows 1, 3 add rows 0, 2
-  e = add_row_bcast<0x143, 0xC>(e);                  // rows 2, 3 add rows 0 + 1
   if (w.owner) acc[w.q] = s;
-  if (w.last) acc[8] = e;
+}
+// The sums of four rows of 64 values: row r of the wave leaves with that of rows[r] in each of its lanes.
+__device__ __forceinline__ float row_sums4(const float (*rows)[DMGS_WAVE]) {
+  const unsigned lane = threadIdx.x & 63;
+  wave_lds_order();  // the rows are written
+  const float4 a = *reinterpret_cast<const float4*>(&rows[0][4u * lane]);
+  float s = (a.x + a.y) + (a.z + a.w);
+  s = DMGS_DPP_ADD(s, 0xB1);
+  s = DMGS_DPP_ADD(s, 0x4E);
+  return DMGS_DPP_ADD(DMGS_DPP_ADD(s, 0x124), 0x128);  // row_ror 4, row_ror 8
 }
 
 // Backward state of one pixel, walking its list back to front.  The reference
 // keeps per channel ch an accumulator acc_ch (colour behind the current splat)
 // and needs only  sum_ch (col_ch - acc_ch) g_ch  (g = dL/dpixel), so one
 // recursion on S = sum_ch acc_ch g_ch replaces three:
-// S <- alpha' <col', g> + (1 - alpha') S, with alpha', col' the splat behind.
+// S <- S + alpha (<col, g> - S).  The background is the colour behind the
+// last splat: S starts from <bg, g>, and the reference's separate term
+// -T_final <bg, g> / (1 - alpha) is part of S.
 struct BwdPixel {
-  float T;    // transmittance in front of the splat last processed
-  float S;    // sum_ch acc_ch g_ch
-  float pcg;  // alpha' <col', g>: the recursion's next term
-  float om;   // 1 - alpha': its factor
+  float T;  // transmittance in front of the splat last processed
+  float S;  // sum_ch acc_ch g_ch behind the next one, the background included
 };
-__device__ __forceinline__ BwdPixel bwd_pixel(float T_final) { return {T_final, 0.f, 0.f, 1.f}; }
 
 // One contributing splat (alpha, colour col) at a pixel with dL/dpixel =
-// (g0, g1, g2) and bg_term = -T_final <bg, g>: updates the state and returns
-// dL/dalpha; w = alpha T is dL/dcolour_ch / g_ch.
+// (g0, g1, g2): updates the state and returns dL/dalpha; w = alpha T is
+// dL/dcolour_ch / g_ch.
 __device__ __forceinline__ float bwd_step(BwdPixel& st, float alpha, const float4& col, float g0, float g1,
-                                          float g2, float bg_term, float& w) {
-  // each state value is read before it is replaced, so it can be updated in
-  // place; the FMA names its destination (S's own register) because the
-  // compiler's two-address form would land it in pcg's register and cost two
-  // moves per pixel to restore the loop's registers
-  asm("v_fma_f32 %0, %1, %0, %2" : "+v"(st.S) : "v"(st.om), "v"(st.pcg));
-  st.om = 1.f - alpha;
-  const float inv = __builtin_amdgcn_rcpf(st.om);  // T before this splat = T / (1 - alpha)
+                                          float g2, float& w) {
+  const float inv = __builtin_amdgcn_rcpf(1.f - alpha);  // T before this splat = T / (1 - alpha)
   st.T *= inv;
   w = alpha * st.T;
-  const float cg = fmaf(col.z, g2, fmaf(col.y, g1, col.x * g0));
-  st.pcg = alpha * cg;
-  return fmaf(bg_term, inv, (cg - st.S) * st.T);
+  const float d = fmaf(col.z, g2, fmaf(col.y, g1, col.x * g0)) - st.S;
+  st.S = fmaf(alpha, d, st.S);
+  return d * st.T;
 }
 
 // Gradients through G = exp(power), with t = dL/dG G = o G dL/dalpha (the
@@ -241,9 +239,9 @@ __device__ __forceinline__ float bwd_step(BwdPixel& st, float alpha, const float
 // -t (b dx + c dy), dL/d(a, b, c) = -t (dx^2, dx dy, dy^2) / 2, dL/do =
 // t / o.  From the scaled conic q = log2(e) (-a/2, -b, -c/2):
 // -(a X + b Y) = ln 2 (2 q.x X + q.y Y) and -(b X + c Y) = ln 2 (q.y X + 2 q.z Y).
-// The kernels accumulate, per splat, (2 q.x X + q.y Y, q.y X + 2 q.z Y,
-// sum t dx^2, sum t dx dy, sum t dy^2, sum G dL/dalpha, sum w g_ch) with
-// X = sum t dx, Y = sum t dy; the flush applies the constant factors.
+// The kernel sums, per splat, X = t dx, Y = t dy, t dx^2, t dx dy, t dy^2, t
+// and w g_ch over the pixels; the linear forms of X, Y and t are applied once
+// per splat and tile, the constant factors in the flush.
 __device__ __forceinline__ float grad_scale(int k, float ddelx_dx, float ddely_dy) {
   constexpr float kLn2 = 0.693147180559945309f;
   return k == 0 ? kLn2 * ddelx_dx : (k == 1 ? kLn2 * ddely_dy : (k < 5 ? -0.5f : 1.0f));
@@ -369,36 +367,49 @@ __device__ __forceinline__ void clear_share(const RenderArgs& a) {
 }
 
 // Stage the next instances of this tile from its cell list, back to front (one wave): visit the list
-// positions cursor-1, cursor-2, ... down to lo, 64 at a time, and keep those whose key holds this tile's
-// bit, in visit order, while another chunk surely fits in the BATCH slots; then stage the kept records in
-// one pass, one lane per record (the footprint test then runs once per 64 records instead of once per
-// chunk visited).  Moves cursor down; returns the number staged; ends with a barrier.
+// positions cursor-1, cursor-2, ... down to lo, four times 64 a round, and keep those whose key holds this tile's
+// bit, in visit order, until BATCH are found; then stage the kept records in one pass, one lane per record.  Full
+// batches share the loads, the footprint test (250 instructions) and the waits among 64 members; about a third of a
+// cell's positions are a tile's members, so a batch of one round of 64 held 20.  Moves cursor down to the last
+// position taken; returns the number staged; ends with a barrier.
 template <int BATCH>
 __device__ __forceinline__ int stage_cell_batch(BwdSplats<BATCH>& L, const RenderArgs& a, const TileCtx& c, int& cursor,
                                                 int lo) {
-  constexpr int CH = DMGS_WAVE < BATCH ? DMGS_WAVE : BATCH;  // positions per chunk
+  constexpr int U = 4;  // positions per lane and round
+  const int s = (int)threadIdx.x;
   const uint64_t lt = lanemask_lt();
   int run = 0;
   do {
-    const int s = (int)threadIdx.x;
-    const int q = cursor - 1 - s;
-    const bool valid = s < CH && q >= lo;
-    // The entry id is requested with the key, both without a branch (lanes
+    const int base = cursor;
+    // The entry ids are requested with the keys, all without a branch (lanes
     // past the list read its first entry and ignore it): one memory round
-    // trip, not two.
-    const uint32_t at = c.range.x + (valid ? (uint32_t)q : 0u);
-    const uint32_t key = a.list_keys[at];
-    const uint32_t id = a.point_list[at];
-    const bool member = valid && ((key >> DMGS_CELL_KEY_BITS) & c.bit);
-    const uint64_t bal = __ballot(member);
-    if (member) {
-      const int slot = run + (int)__popcll(bal & lt);
-      // id and position wait in the record for the staging pass
-      L.xym[slot] = make_float4(0.f, 0.f, __uint_as_float(id), __uint_as_float((uint32_t)q));
+    // trip per round.
+    uint32_t key[U], id[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = base - 1 - s - u * DMGS_WAVE;
+      const uint32_t at = c.range.x + (q >= lo ? (uint32_t)q : 0u);
+      key[u] = a.list_keys[at];
+      id[u] = a.point_list[at];
     }
-    run += (int)__popcll(bal);
-    cursor -= CH;
-  } while (run + CH <= BATCH && cursor > lo);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (run == BATCH) break;  // the rest of the round is read again
+      const int q = base - 1 - s - u * DMGS_WAVE;
+      const bool member = q >= lo && ((key[u] >> DMGS_CELL_KEY_BITS) & c.bit);
+      const uint64_t bal = __ballot(member);
+      const int slot = run + (int)__popcll(bal & lt);
+      if (member && slot < BATCH)  // id and position wait in the record for the staging pass
+        L.xym[slot] = make_float4(0.f, 0.f, __uint_as_float(id[u]), __uint_as_float((uint32_t)q));
+      run += (int)__popcll(bal);
+      cursor = base - (u + 1) * DMGS_WAVE;
+      if (run > BATCH) {  // the batch ends before its first member without a slot
+        const uint64_t first = __ballot(member && slot == BATCH);
+        cursor = base - u * DMGS_WAVE - (int)__builtin_ctzll(first);
+        run = BATCH;
+      }
+    }
+  } while (run < BATCH && cursor > lo);
   __syncthreads();
   for (int s = (int)threadIdx.x; s < run; s += DMGS_WAVE) {
     const float4 t = L.xym[s];
@@ -694,10 +705,18 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
 
 // Backward with one wave per 16x16 tile: lane (lx, ly) owns the pixels
 // (lx, ly + 4k), k = 0..3, i.e. one pixel in each of four 16x4 strips.  The
-// footprint test runs per strip, each pixel is evaluated exactly as in
-// render_bwd_kernel, and a lane first sums its four pixels' partial
-// gradients, so each (tile, splat) pays for one wave reduction instead of
-// four.
+// footprint test runs per strip, each pixel is evaluated exactly as in the
+// forward, and a lane first sums its four pixels' partial gradients, so each
+// (tile, splat) pays for one wave reduction instead of four.
+//
+// Bound by the instructions of its waves, vector and scalar, at five waves per
+// SIMD (91 registers; six spill, and four take 24 % longer): so a batch is
+// filled before it is walked, what can be decided for 64 staged splats at once
+// (which strips are live) is, one lane per splat, and so are the linear forms
+// of the sums; the ninth sum waits for three others'.  The background is the
+// colour behind the last splat rather than a term of its own.  Before and now:
+// sixteen uneven views of 3 M Gaussians 6.96 and 4.87 ms, eight 800x800 views
+// of 1 M 462 and 375 us.
 //
 // SEGS: the work-groups below a.seg.cap each take one kept segment of a tile's
 // list (see Segments), the others the rest of a tile's list.
@@ -724,23 +743,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     tile = ordered_tile(a, blockIdx.x);
   }
   __shared__ BwdSplats<BATCH> L;
-  // Two accumulator sets: a batch's global atomics are issued after the next
-  // batch has been staged, so no staging load waits behind them (the memory
-  // counter is in order) and they complete while that batch is computed.
-  __shared__ __align__(16) float s_acc[2][BATCH][DMGS_GACC_USED];
-  __shared__ uint32_t s_gid[2][BATCH];
-  static_assert(BATCH * DMGS_GACC_USED >= 8 * DMGS_WAVE && (BATCH * DMGS_GACC_USED) % 4 == 0,
-                "one accumulator set holds a splat's 8 x 64 per-lane values");
+  // Two accumulator sets of a quarter of a batch: a set's global atomics are
+  // issued after the next batch has been staged (or before the batch's next
+  // quarter), so no staging load waits behind them (the memory counter is in
+  // order) and they complete while that one is computed.
+  constexpr int SET = BATCH / 4;
+  __shared__ float s_acc[2][SET][DMGS_GACC_USED];
+  uint32_t set_id = 0;  // lane i: the Gaussian of slot i of the set to be flushed
+  __shared__ __align__(16) float s_red[8][DMGS_WAVE];    // a splat's per-lane values 0..7
+  __shared__ __align__(16) float s_ninth[4][DMGS_WAVE];  // value 8 of the last splats, until there are four
   const TileCtx c = tile_ctx<false>(a, tile);  // pixel k = 0 of this lane: (lx, ly), ly in 0..3
   const unsigned lane = threadIdx.x & 63;
-  const WaveSum9 wsum = wave_sum9_lane(lane);
+  const WaveSum8 wsum = wave_sum8_lane(lane);
   const float pxf = (float)c.px;
   const float ddelx_dx = 0.5f * (float)c.W, ddely_dy = 0.5f * (float)c.H;  // d pixel / d NDC
   float pyf[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) pyf[k] = (float)(c.py + 4 * k);
 
-  float g0[4], g1[4], g2[4], bg_term[4];
+  float g0[4], g1[4], g2[4];
   BwdPixel st[4];
   uint32_t last_contributor[4];
   uint32_t m = 0;
@@ -761,13 +782,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       g1[k] = dp[c.plane + pid];
       g2[k] = dp[2 * c.plane + pid];
     }
-    bg_term[k] = -T_final * (c.bg0 * g0[k] + c.bg1 * g1[k] + c.bg2 * g2[k]);
-    st[k] = bwd_pixel(T_final);
+    st[k] = {T_final, c.bg0 * g0[k] + c.bg1 * g1[k] + c.bg2 * g2[k]};
     if constexpr (SEGS) {
       if (seg_end != kNoSegment) {  // start from the state at hi: T, and the colour behind it
         const float4 e = a.seg.state[(size_t)seg_end * 256 + threadIdx.x + 64 * k];
         st[k].T = e.x;
-        st[k].S = (e.y * g0[k] + e.z * g1[k] + e.w * g2[k]) / e.x;
+        st[k].S = (e.y * g0[k] + e.z * g1[k] + e.w * g2[k] + T_final * st[k].S) / e.x;
       }
     }
   }
@@ -783,24 +803,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
   }
   const int todo_total = min(min((int)(c.range.y - c.range.x), (int)m), hi);
 
-  // one batch's accumulated sums -> one global atomic per (splat, value)
-  auto flush = [&](int buf, int cnt) {
-    for (int i = threadIdx.x; i < cnt * DMGS_GACC_USED; i += NT) {
+  // one set's sums -> one global atomic per (splat, value)
+  auto flush = [&](int buf, uint32_t slots) {
+    static_assert(SET * DMGS_GACC_USED <= 3 * NT, "slot positions of three rounds");
+#pragma unroll 1
+    for (int r = 0; r < 3; ++r) {  // whole rounds: every lane hands out its slot's id
+      const int i = r * NT + (int)threadIdx.x;
       const int slot = i / DMGS_GACC_USED, q = i - slot * DMGS_GACC_USED;
+      const uint32_t gid = (uint32_t)__shfl((int)set_id, slot);
+      if (!((slots >> slot) & 1u)) continue;
       const float val = s_acc[buf][slot][q] * grad_scale(q, ddelx_dx, ddely_dy);
-      if (val != 0.f) unsafeAtomicAdd(a.gacc + gacc_index(a.P, s_gid[buf][slot], q), val);
+      if (val != 0.f) unsafeAtomicAdd(a.gacc + gacc_index(a.P, gid, q), val);
     }
   };
-  int buf = 0, prev_n = 0;
+  int buf = 0;
+  uint32_t summed = 0;      // slots of set buf that hold sums
   int cursor = todo_total;  // list positions in [lo, cursor) are still to do
   while (cursor > lo) {
     __syncthreads();
     const int top = cursor;
     int n;
-    for (int s = threadIdx.x; s < BATCH; s += NT) {
-#pragma unroll
-      for (int k = 0; k < DMGS_GACC_USED; ++k) s_acc[buf][s][k] = 0.f;
-    }
     if constexpr (CELLS) {
       n = stage_cell_batch(L, a, c, cursor, lo);
     } else {
@@ -812,72 +834,90 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       n = min(BATCH, top - lo);
       cursor -= n;
     }
-    for (int s = threadIdx.x; s < n; s += NT) s_gid[buf][s] = L.id(s);
     // Every staging load has landed here; saying so keeps the compiler from
     // waiting later (behind the atomics below) for a load it cannot rule out.
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    flush(buf ^ 1, prev_n);  // the previous batch's atomics overlap this batch
-    __syncthreads();
-    // the flushed set is free until the next batch zeroes it: it holds the
-    // per-lane values of the wave sums (wave_sums9) meanwhile
-    float(*const s_red)[DMGS_WAVE] = reinterpret_cast<float(*)[DMGS_WAVE]>(&s_acc[buf ^ 1][0][0]);
-    uint32_t mask_next = n > 0 ? L.mask(0) : 0u;  // read one splat ahead
-    for (int j = 0; j < n; ++j) {
-      const uint32_t reach = __builtin_amdgcn_readfirstlane(mask_next);
-      if (j + 1 < n) mask_next = L.mask(j + 1);
-      if (reach == 0u) continue;
-      uint32_t contributor;
-      if constexpr (CELLS) {
-        contributor = __builtin_amdgcn_readfirstlane(L.pos(j));
-      } else {
-        contributor = (uint32_t)(top - 1 - j);
-      }
-      uint32_t live = reach;  // strips the splat reaches and that still have pixels behind it
+    // lane s: the strips that slot s reaches and that still have pixels behind it
+    const uint32_t pos = L.pos(lane);
+    uint32_t live_of = (int)lane < n ? L.mask(lane) : 0u;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (contributor >= strip_max[k]) live &= ~(1u << k);
-      if (live == 0u) continue;
-      const float2 xy = make_float2(L.xym[j].x, L.xym[j].y);
-      const float4 q = L.qo[j];
-      const float4 col = L.rgb_id[j];
-      const float dx = xy.x - pxf;
-      const PowerDx pd = power_dx(q.x, q.y, dx);  // shared by the lane's four pixels (one column)
-      // per-lane sums over its pixels: sum t, sum t dy, sum t dy^2 (dx is the
-      // same for the four pixels, so its powers multiply in once per splat)
-      float s_t = 0.f, s_tdy = 0.f, s_tdy2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f;
-      bool any = false;
+    for (int k = 0; k < 4; ++k)
+      if (pos >= strip_max[k]) live_of &= ~(1u << k);
+    const uint64_t todo = __ballot(live_of != 0u);
+    for (int j0 = 0; j0 < n; j0 += SET) {
+      uint32_t left = (uint32_t)(todo >> j0) & ((1u << SET) - 1u);
+      if (left == 0u) continue;
+      flush(buf, summed);  // overlaps this quarter
+      buf ^= 1;
+      summed = 0;
+      set_id = L.id(j0 + (int)(lane & (SET - 1u)));
+      uint32_t ninth = 0, ninths = 0;  // slots of s_ninth's rows, a byte each, the last one lowest
+      auto sum_ninths = [&]() {
+        const float e = row_sums4(s_ninth);
+        const uint32_t r = lane >> 4;
+        if (r < ninths && (lane & 15u) == 0u) s_acc[buf][(ninth >> (8u * (ninths - 1u - r))) & (SET - 1u)][8] = e;
+        ninths = 0;
+      };
+      while (left) {
+        const int slot = __builtin_ctz(left), j = j0 + slot;
+        left &= left - 1u;
+        const uint32_t live = __builtin_amdgcn_readlane(live_of, j), contributor = __builtin_amdgcn_readlane(pos, j);
+        const float2 xy = make_float2(L.xym[j].x, L.xym[j].y);
+        const float4 q = L.qo[j];
+        const float4 col = L.rgb_id[j];
+        const float dx = xy.x - pxf;
+        const PowerDx pd = power_dx(q.x, q.y, dx);  // shared by the lane's four pixels (one column)
+        // per-lane sums over its pixels: sum t, sum t dy, sum t dy^2 (dx is the
+        // same for the four pixels, so its powers multiply in once per splat)
+        float s_t = 0.f, s_tdy = 0.f, s_tdy2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f;
+        bool any = false;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        if (!((live >> k) & 1u)) continue;  // wave-uniform
-        const float dy = xy.y - pyf[k];
-        const float p = power_at(pd, q.z, dy);
-        const float G = splat_exp2(p);
-        const float ga = q.w * G;  // o G: alpha before the 0.99 clamp
-        const float alpha = fminf(0.99f, ga);
-        if (contributor < last_contributor[k] && p <= 0.0f && alpha >= 1.0f / 255.0f) {
-          any = true;
-          float w;
-          const float t = ga * bwd_step(st[k], alpha, col, g0[k], g1[k], g2[k], bg_term[k], w);
-          c0 = fmaf(w, g0[k], c0);
-          c1 = fmaf(w, g1[k], c1);
-          c2 = fmaf(w, g2[k], c2);
-          s_t += t;
-          const float tdy = t * dy;
-          s_tdy += tdy;
-          s_tdy2 = fmaf(tdy, dy, s_tdy2);
+        for (int k = 0; k < 4; ++k) {
+          if (!((live >> k) & 1u)) continue;  // wave-uniform
+          const float dy = xy.y - pyf[k];
+          const float p = power_at(pd, q.z, dy);
+          const float G = splat_exp2(p);
+          const float ga = q.w * G;  // o G: alpha before the 0.99 clamp
+          const float alpha = fminf(0.99f, ga);
+          if (contributor < last_contributor[k] && p <= 0.0f && alpha >= 1.0f / 255.0f) {
+            any = true;
+            float w;
+            const float t = ga * bwd_step(st[k], alpha, col, g0[k], g1[k], g2[k], w);
+            c0 = fmaf(w, g0[k], c0);
+            c1 = fmaf(w, g1[k], c1);
+            c2 = fmaf(w, g2[k], c2);
+            s_t += t;
+            const float tdy = t * dy;
+            s_tdy += tdy;
+            s_tdy2 = fmaf(tdy, dy, s_tdy2);
+          }
         }
+        if (__ballot(any) == 0) continue;
+        const float s_tdx = s_t * dx;
+        const float v[8] = {s_tdx, s_tdy, s_tdx * dx, s_tdy * dx, s_tdy2, s_t, c0, c1};
+        int at = (buf * SET + slot) * DMGS_GACC_USED;
+        asm("" : "+s"(at));  // a scalar product, not a 64-bit one per lane
+        wave_sums8(v, s_red, wsum, &s_acc[0][0][0] + at);
+        s_ninth[ninths][lane] = c2;
+        ninth = ninth << 8 | (uint32_t)slot;
+        summed |= 1u << slot;
+        if (++ninths == 4u) sum_ninths();
       }
-      if (__ballot(any) == 0) continue;
-      const float s_tdx = s_t * dx;
-      const float v[DMGS_GACC_USED] = {dmean_x(q, s_tdx, s_tdy), dmean_y(q, s_tdx, s_tdy), s_tdx * dx, s_tdy * dx,
-                                       s_tdy2, s_t * __builtin_amdgcn_rcpf(q.w), c0, c1, c2};
-      wave_sums9(v, s_red, wsum, lane, s_acc[buf][j]);
+      if (ninths) sum_ninths();
+      __syncthreads();
+      // what is linear in the sums is left to one lane per splat
+      if (lane < SET && ((summed >> lane) & 1u)) {
+        const float4 q = L.qo[j0 + (int)lane];
+        float* const acc = s_acc[buf][lane];
+        const float X = acc[0], Y = acc[1];
+        acc[0] = dmean_x(q, X, Y);
+        acc[1] = dmean_y(q, X, Y);
+        acc[5] *= __builtin_amdgcn_rcpf(q.w);
+      }
+      __syncthreads();
     }
-    prev_n = n;
-    buf ^= 1;
   }
-  __syncthreads();
-  flush(buf ^ 1, prev_n);
+  flush(buf, summed);
   if (a.clear_words && blockIdx.x == 0)  // the tile-order histogram, ready for another backward's
     for (int i = threadIdx.x; i < a.clear_words_n; i += NT) a.clear_words[i] = 0u;
 }
