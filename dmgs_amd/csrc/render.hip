@@ -295,8 +295,10 @@ __device__ __forceinline__ int ordered_tile(const RenderArgs& a, int slot) {
 
 // QUADS (256 lanes): wave k covers the 8x8 quadrant k (k & 1: right, k >> 1: lower); otherwise (64 lanes) a
 // lane's first pixel is in the tile's top 16x4 strip.
+// half: a work-group of the whole tile (-1), or of its upper (0) or lower (1) 16x8 pixels, of which each wave then
+// owns 8x4 with two lanes each (see render_fwd_quads_kernel).
 template <bool QUADS>
-__device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile) {
+__device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile, int half = -1) {
   TileCtx c;
   c.tile = tile;
   int lt = c.tile, gx = a.grid_x;
@@ -329,16 +331,16 @@ __device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile) {
   if constexpr (QUADS) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     lx = (wave & 1) * 8 + (lane & 7);
-    ly = (wave >> 1) * 8 + (lane >> 3);
+    ly = half < 0 ? (wave >> 1) * 8 + (lane >> 3) : half * 8 + (wave >> 1) * 4 + (lane >> 3 & 3);
   }
   const int ox = tx * DMGS_BLOCK_X, oy = ty * DMGS_BLOCK_Y;
   c.px = ox + lx;
   c.py = oy + ly;
-  // rectangle k: quadrant k, or 16x4 strip k
+  // rectangle k: quadrant k of the tile or of its half, or 16x4 strip k
   c.rows.x0 = (float)ox;
-  c.rows.y0 = (float)oy;
+  c.rows.y0 = (float)(half > 0 ? oy + 8 : oy);
   c.rows.w = QUADS ? 8.0f : 16.0f;
-  c.rows.h = QUADS ? 8.0f : 4.0f;
+  c.rows.h = QUADS && half < 0 ? 8.0f : 4.0f;
   c.rows.cols = QUADS ? 2 : 1;
   c.rows.n = 4;
   c.inside = c.px < c.W && c.py < c.H;
@@ -426,6 +428,15 @@ struct FwdGroup {
   float4 xyq[kN], qorg[kN];
 };
 
+// Two pairs of staged splats as one of a pixel's two lanes reads them: of each pair its own splat's shape, and both
+// splats' colours in its channels (red and green, or blue); and the LDS byte offsets of the next four splats.
+struct FwdPairs {
+  uint4 at;
+  float4 xyq[2];
+  float2 qo[2], col[2][2];
+  uint32_t pos[2];
+};
+
 // The members of a tile in one chunk of its list (every position of a single view's tile list; the instances
 // of a cell list whose mask holds the tile's bit), packed in list order.
 template <int N>
@@ -443,7 +454,13 @@ struct MemberList {
 // 5.33 -> 3.51 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
 // reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on KEEP,
 // CELLS or the launch.
-template <bool CELLS, bool KEEP>
+// SPLIT: a tile's list is a chain (each pixel's transmittance goes from splat to splat), so a launch of few tiles
+// takes as long as its longest list, however empty the GPU is: 24 instructions a splat in each of four waves.  Two
+// work-groups blend a tile then, 16x8 pixels each with two lanes a pixel: the lanes evaluate the alphas of two
+// consecutive splats side by side, exchange them, and both carry the transmittance over the two in order; one adds
+// red and green, the other blue.  16 instructions a splat, in twice as many waves, with the same operations in the
+// same order on every value.  (Eight waves of one work-group share a CU's SIMDs and gain nothing.)
+template <bool CELLS, bool KEEP, bool SPLIT>
 __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
   constexpr int NT = 256, U = FwdGroup::kN;
   constexpr int G = KEEP ? 64 : NT;  // staged splats blended per round
@@ -454,7 +471,8 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
   __shared__ uint32_t s_wc[2][C][NT / DMGS_WAVE];
   __shared__ uint32_t s_slot[KEEP ? kTileSegments : 1];
   __shared__ __align__(16) uint32_t s_reach[NT / DMGS_WAVE][G + 12];
-  const TileCtx c = tile_ctx<true>(a, ordered_tile(a, blockIdx.x));
+  const int half = SPLIT ? (int)(blockIdx.x & 1u) : -1;
+  const TileCtx c = tile_ctx<true>(a, ordered_tile(a, SPLIT ? (int)(blockIdx.x >> 1) : (int)blockIdx.x), half);
   const float pxf = (float)c.px, pyf = (float)c.py;
   const int len = (int)(c.range.y - c.range.x);
   const int lane = threadIdx.x & 63;
@@ -607,6 +625,63 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
       }
       if (count == 0) continue;
       if (lane < 12) reach[count + lane] = kPad;
+      if constexpr (SPLIT) {
+        const bool second = lane >= 32;  // of the pixel's two lanes
+        const char* const channels =
+            second ? reinterpret_cast<const char*>(L.bpmi) : reinterpret_cast<const char*>(L.qorg) + 8;
+        auto fetch = [&](FwdPairs& g, const uint4& at, int next) {
+          const uint32_t own[2] = {second ? at.y : at.x, second ? at.w : at.z};
+          const uint32_t both[2][2] = {{at.x, at.y}, {at.z, at.w}};
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            g.xyq[p] = lds_at(L.xyq, own[p]);
+            g.qo[p] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(L.qorg) + own[p]);
+            g.pos[p] = __float_as_uint(lds_at(L.bpmi, own[p]).y);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) g.col[p][e] = *reinterpret_cast<const float2*>(channels + both[p][e]);
+          }
+          g.at = *reinterpret_cast<const uint4*>(reach + next);
+        };
+        // blends `cur` while `next` is on its way; false when nothing is left to do
+        int done = 0;
+        auto step = [&](FwdPairs& cur, FwdPairs& next) {
+          fetch(next, cur.at, done + 8);
+          float alpha[2];
+          bool ok[2];
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const float4 g = cur.xyq[p];
+            const float power = power_at(power_dx(g.z, g.w, g.x - pxf), cur.qo[p].x, g.y - pyf);
+            const float al = fminf(0.99f, cur.qo[p].y * splat_exp2(power));
+            ok[p] = (power <= 0.0f) & (al >= 1.0f / 255.0f);
+            alpha[p] = ok[p] ? al : 0.0f;
+          }
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(alpha[p]), __float_as_uint(alpha[p]), false, false);
+            bool take[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {  // both lanes: the first lane's splat, then the second's
+              const float al = __uint_as_float(x[e]);
+              const float test_T = T * (1.0f - al);
+              take[e] = test_T >= 0.0001f;
+              const float w = take[e] ? al * T : 0.0f;
+              C0 = fmaf(cur.col[p][e].x, w, C0);
+              C1 = fmaf(cur.col[p][e].y, w, C1);  // the blue lane's is not used
+              T = take[e] ? test_T : -fabsf(T);
+            }
+            const bool mine = (second & take[1]) | (!second & take[0]);
+            last_contributor = (mine & ok[p]) ? cur.pos[p] : last_contributor;
+          }
+          done += 4;
+          return done < count && __ballot(T > 0.f) != 0;
+        };
+        FwdPairs g0, g1;
+        fetch(g0, *reinterpret_cast<const uint4*>(reach), 4);
+        while (step(g0, g1) && step(g1, g0)) {
+        }
+        continue;
+      }
       auto fetch = [&](FwdGroup& g, const uint4& at, int next) {
         const uint32_t o[U] = {at.x, at.y, at.z, at.w};
 #pragma unroll
@@ -688,17 +763,29 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
     for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
     if (lane == 0) s_max[wave] = m;
     __syncthreads();
-    if (threadIdx.x == 0) a.tile_work[c.tile] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+    if (threadIdx.x == 0) {
+      m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+      if constexpr (SPLIT)
+        atomicMax(&a.tile_work[c.tile], m);  // zero since the tiles were ordered
+      else
+        a.tile_work[c.tile] = m;
+    }
+  }
+  if constexpr (SPLIT) {
+    last_contributor = max(last_contributor, (uint32_t)__shfl_xor((int)last_contributor, 32, 64));
+    if (lane >= 32) C2 = C0;
   }
   if (c.inside) {
     const size_t pid = c.pix - c.img / 3;  // pixel index within the view
     T = fabsf(T);
-    a.final_T[c.pix] = T;
-    a.n_contrib[c.pix] = last_contributor;
     float* out = a.out_color + c.img;
-    out[pid] = C0 + T * c.bg0;
-    out[c.plane + pid] = C1 + T * c.bg1;
-    out[2 * c.plane + pid] = C2 + T * c.bg2;
+    if (!SPLIT || lane < 32) {
+      a.final_T[c.pix] = T;
+      a.n_contrib[c.pix] = last_contributor;
+      out[pid] = C0 + T * c.bg0;
+      out[c.plane + pid] = C1 + T * c.bg1;
+    }
+    if (!SPLIT || lane >= 32) out[2 * c.plane + pid] = C2 + T * c.bg2;
   }
   clear_share(a);
 }
@@ -951,6 +1038,7 @@ __global__ __launch_bounds__(256) void tile_bucket_kernel(RenderArgs a, uint8_t*
   if (t < a.num_tiles) {
     const uint32_t b = tile_cost_bucket(a, t, K, use_work != 0);
     bucket[t] = (uint8_t)b;
+    if (!use_work && a.tile_work) a.tile_work[t] = 0u;  // the forward's halves of a tile take the larger of theirs
     atomicAdd(&cnt[b], 1u);
   }
   __syncthreads();
@@ -1006,16 +1094,22 @@ __global__ void seg_reset_kernel(uint32_t* head) {
   if (threadIdx.x < 2) head[threadIdx.x] = threadIdx.x == 0 ? 0u : kSegMagic;
 }
 
+// Two work-groups per tile while they find idle SIMDs, us before and after: 336 tiles of long lists (500k Gaussians,
+// 333x251, near) 196 and 150, 169 tiles (10k, 200x200) 48 and 39, 475 tiles 220 and 171; 512 tiles of 2 views 72 and
+// 59, or 23 and 26 where the lists end after a few splats.  625 tiles of such lists 20 and 28, 1024 24 and 33.
+constexpr int kSplitTiles = 512;
 void launch_render_fwd(const RenderArgs& a, hipStream_t s) {
   if (a.num_tiles <= 0) return;
   const dim3 grid(a.num_tiles), block(256);
   if (a.seg.len > 0) {
     hipLaunchKernelGGL(seg_reset_kernel, dim3(1), dim3(64), 0, s, a.seg.head);
-    hipLaunchKernelGGL((render_fwd_quads_kernel<true, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, true, false>), grid, block, 0, s, a);
+  } else if (a.views && a.num_tiles <= kSplitTiles) {
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false, true>), dim3(2 * a.num_tiles), block, 0, s, a);
   } else if (a.views) {
-    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false, false>), grid, block, 0, s, a);
   } else {
-    hipLaunchKernelGGL((render_fwd_quads_kernel<false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((render_fwd_quads_kernel<false, false, false>), grid, block, 0, s, a);
   }
 }
 

@@ -70,3 +70,31 @@ def test_list_edges(n, logit, size, scale):
     whole = r.backward(params, dL.cuda().reshape(-1).contiguous())
     assert grad_rel_err(whole, grads) < 1e-5
     assert grad_rel_err(twice, grads) < 1e-5
+
+
+@pytest.mark.parametrize("n,logit,size,scale", [(1, 0.0, (17, 9), 0.5), (2, 0.0, (16, 24), 0.5), (3, 0.0, (31, 8), 0.5),
+                                                (257, -4.5, (40, 40), 0.5), (300, 1.0, (33, 41), 0.5),
+                                                (3000, 0.0, (352, 368), -2.5), (40, 0.0, (300, 180), -3.0)])
+def test_two_work_groups_per_tile(n, logit, size, scale):
+    """A forward without a backward to follow blends up to 512 tiles with two work-groups each: the same operations
+    on every value as the one that keeps segments, so images, transmittances and counts are equal bit for bit."""
+    print(f"case: split tiles n={n} logit={logit} size={size} scale={scale}", flush=True)
+    model = _covering(n, logit, scale)
+    cams = [C.camera_at((0.2, 0.1, -3.0), *size)]
+    r = BT.BatchedRenderer(cams, [torch.tensor([0.1, 0.5, 0.9], device="cuda")], n, sh_degree=1)
+    params = BT.pack_model(model.to("cuda"))
+    r.plan(params)
+    assert r.total_tiles <= 512
+    got = []
+    for keep in (True, False):
+        if not keep:
+            r.bwd_ws = None
+        img = r.forward(params).clone()
+        X = r.total_pixels
+        T = r.state[r._offsets[3]:r._offsets[3] + 4 * X].view(torch.float32).clone()
+        cnt = r.state[r._offsets[4]:r._offsets[4] + 4 * X].view(torch.int32).clone()
+        got.append((img, T, cnt))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    # and twice: the halves' largest counts do not depend on an earlier forward
+    assert torch.equal(r.forward(params), got[0][0])
