@@ -117,6 +117,7 @@ _SIGNATURES = {
     "dmgs_batched_lists_size": (c_size_t, [c_int64]),
     "dmgs_batched_backward_size": (c_size_t, [c_int32, c_int64]),
     "dmgs_batched_offsets": (c_int32, [c_int32, c_int64, c_int32, c_int64, c_int64, ctypes.POINTER(c_size_t)]),
+    "dmgs_view_counts": (c_int32, [c_void_p]),
     "dmgs_sh_sigmoid": (c_int32, [c_int64, c_int32, c_int32, c_int32] + [c_void_p] * 8),
     "dmgs_view_supported": (c_int32, [c_int32, c_int32]),
     "dmgs_view_state_size": (c_size_t, [c_int64, c_int32, c_int32, c_int32]),
@@ -179,11 +180,16 @@ def check(rc, what):
 
 
 def ptr(t):
-    """Device pointer of a tensor (None -> NULL)."""
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (None -> NULL), as ctypes takes it for a void pointer."""
+    return None if t is None else t.data_ptr()
+
+
+# the stream's handle without a Stream object around it (6 us a call) where torch offers it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def stream_handle(device=None):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    index = getattr(device, "index", None)
+    if _raw_stream is None or index is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(index)

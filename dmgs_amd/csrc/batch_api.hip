@@ -583,7 +583,14 @@ int dmgs_view_geometry(const dmgs_settings* s, const dmgs_gaussians* g, int32_t 
   uint32_t* dev = at<uint32_t>(state, V.counts);
   dmgs::launch_view_counts(c.count(&b), a.tile_sums, dev, st);
   if ((rc = bcheck("view preprocess / depth sort / scan", st))) return rc;
-  if (hipMemcpyAsync(counts, dev, 8, hipMemcpyDeviceToHost, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
+  if (hipMemcpyAsync(counts, dev, 8, hipMemcpyDeviceToHost, st) != hipSuccess)
+    return bcheck("view counts", st) ? DMGS_EHIP : bfail(DMGS_EHIP, "requesting the instance counts failed");
+  return DMGS_OK;
+}
+
+int dmgs_view_counts(dmgs_stream_t stream) {
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (hipStreamSynchronize(st) != hipSuccess)
     return bcheck("view counts", st) ? DMGS_EHIP : bfail(DMGS_EHIP, "reading the instance counts failed");
   return DMGS_OK;
 }

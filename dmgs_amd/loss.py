@@ -8,11 +8,12 @@ instead of five depthwise convolutions plus autograd.
 """
 import torch
 
+from . import _native as N
+
 
 class _FusedDssimL1(torch.autograd.Function):
     @staticmethod
     def forward(ctx, image, gt, lambda_dssim):
-        from . import _native as N
         img = image.detach().to(torch.float32).contiguous()
         ref = gt.detach().to(device=img.device, dtype=torch.float32).contiguous()
         if img.dim() == 4 and img.shape[0] == 1:
@@ -32,7 +33,6 @@ class _FusedDssimL1(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_loss):
-        from . import _native as N
         img, ref, ws = ctx.saved_tensors
         C, H, W = img.shape
         g = grad_loss.detach().to(torch.float32).reshape(1).contiguous()

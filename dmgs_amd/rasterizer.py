@@ -247,11 +247,15 @@ def view_forward(t, sh_coeffs, raw, rs, keep):
     with _stage("geometry"):  # ends with the one host synchronisation of the path (as in the reference)
         N.check(lib.dmgs_view_geometry(s, ctypes_ref(g), int(keep), N.ptr(radii), N.ptr(ws), N.ptr(counts), stream),
                 "dmgs_view_geometry")
+        try:  # what does not depend on the counts is allocated while they are on their way
+            bws = torch.empty(lib.dmgs_batched_backward_size(1, P), **byte) if keep else None
+            color = torch.empty(3, H, W, dtype=torch.float32, device=dev)
+        finally:  # also on an error: the copy writes into counts
+            rc = lib.dmgs_view_counts(stream)
+        N.check(rc, "dmgs_view_counts")
     cells, tiles = (int(c) & 0xFFFFFFFF for c in counts.tolist())
     K = max(1, cells)
     lists = torch.empty(lib.dmgs_batched_lists_size(K), **byte)
-    bws = torch.empty(lib.dmgs_batched_backward_size(1, P), **byte) if keep else None
-    color = torch.empty(3, H, W, dtype=torch.float32, device=dev)
     with _stage("binning"):
         N.check(lib.dmgs_view_binning(s, P, int(keep), K, N.ptr(ws), N.ptr(lists), stream), "dmgs_view_binning")
     with _stage("render_forward"):

@@ -412,12 +412,14 @@ typedef struct dmgs_gaussian_grads { /* shaped like the inputs; colors, cov3D, s
 int dmgs_view_supported(int32_t width, int32_t height);
 /* keep: a backward will follow (the same value in every call of one image). */
 size_t dmgs_view_state_size(int64_t P, int32_t width, int32_t height, int32_t keep);
-/* Preprocess, depth sort and scan; waits for the stream and returns in
- * counts (host memory, pinned for speed) the cell instances (size the lists
- * with dmgs_batched_lists_size(max(1, counts[0]))) and the reference's
+/* Preprocess, depth sort and scan.  counts (host memory, pinned, valid after
+ * dmgs_view_counts) receives the cell instances (size the lists with
+ * dmgs_batched_lists_size(max(1, counts[0]))) and the reference's
  * num_rendered. */
 int dmgs_view_geometry(const dmgs_settings* settings, const dmgs_gaussians* g, int32_t keep, int32_t* radii,
                        void* state, uint32_t counts[2], dmgs_stream_t stream);
+/* Waits for the stream: the counts of the geometry call before it are there. */
+int dmgs_view_counts(dmgs_stream_t stream);
 /* K: the capacity the lists were sized for. */
 int dmgs_view_binning(const dmgs_settings* settings, int64_t P, int32_t keep, int64_t K, void* state, void* lists,
                       dmgs_stream_t stream);
