@@ -11,8 +11,8 @@ import torch  # noqa: F401  (loads the HIP runtime the library binds to)
 
 from . import build as _build
 
-c_int32, c_int64, c_size_t, c_void_p, c_float = (ctypes.c_int32, ctypes.c_int64, ctypes.c_size_t,
-                                                  ctypes.c_void_p, ctypes.c_float)
+c_int32, c_uint32, c_int64, c_size_t, c_void_p, c_float = (ctypes.c_int32, ctypes.c_uint32, ctypes.c_int64, ctypes.c_size_t,
+                                                            ctypes.c_void_p, ctypes.c_float)
 
 
 class DmgsSettings(ctypes.Structure):
@@ -44,6 +44,11 @@ class DmgsBatch(ctypes.Structure):
         ("state", c_void_p), ("lists", c_void_p), ("bwd_ws", c_void_p),
         ("cell_mode", c_int32), ("max_view_cells", c_int32), ("dens", c_void_p),
     ]
+
+
+class DmgsDssimView(ctypes.Structure):
+    _fields_ = [("height", c_int32), ("width", c_int32), ("first_tile", c_uint32), ("first_pixel", c_uint32),
+                ("index", c_uint32), ("reserved", c_uint32 * 3)]
 
 
 class DmgsGaussians(ctypes.Structure):
@@ -100,6 +105,9 @@ _SIGNATURES = {
                                                c_void_p, c_void_p, c_void_p]),
     "dmgs_dssim_l1_backward_groups": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_float,
                                                 c_void_p, c_void_p, c_void_p, c_void_p]),
+    "dmgs_dssim_views": (c_int32, [c_int32, c_void_p, c_void_p, c_void_p]),
+    "dmgs_dssim_l1_forward_views": (c_int32, [c_void_p] * 4 + [c_int32, c_uint32, c_float] + [c_void_p] * 3),
+    "dmgs_dssim_l1_backward_views": (c_int32, [c_void_p] * 3 + [c_int32, c_uint32, c_float] + [c_void_p] * 4),
     "dmgs_dssim_target_stats": (c_int32, [c_void_p, c_int32, c_int32, c_int32, c_void_p, c_void_p]),
     "dmgs_dssim_l1_forward_groups_stats": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32,
                                                      c_int32, c_float, c_void_p, c_void_p, c_void_p]),

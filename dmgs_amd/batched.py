@@ -376,43 +376,62 @@ class BatchedLoss:
         self.targets = renderer.new_images()
         for v, t in enumerate(targets):
             renderer.image(self.targets, v).copy_(t.to(device=dev, dtype=torch.float32))
-        # consecutive views of one size are back to back in the packed buffers:
-        # each such run is one grouped launch pair (one loss per view)
-        self.runs = []
-        for v, hw in enumerate(renderer.sizes):
-            if self.runs and self.runs[-1][2] == hw:
-                self.runs[-1][1] = v + 1
-            else:
-                self.runs.append([v, v + 1, hw])
-        self.ws = [torch.empty(self.lib.dmgs_dssim_l1_workspace_size(3 * (v1 - v0), h, w), dtype=torch.uint8,
-                               device=dev) for v0, v1, (h, w) in self.runs]
-        # the targets' blurred maps (G*y, G*y^2) are fixed: computed once here
-        self.stats = []
+        # Every view in one launch each way.  Views of one size are groups of planes; others go through a table of
+        # their sizes and places in the packed buffers, which a work-group looks its tile up in (eight 800 x 800
+        # views 103 and 109 us forward; sixteen uneven views 888 us as one launch per run of equal sizes, 653 so).
+        # The targets' blurred maps (G*y, G*y^2) are fixed: computed once here.
         s = N.stream_handle(dev)
-        for v0, v1, (h, w) in self.runs:
-            st = torch.empty(2 * 3 * (v1 - v0) * h * w, dtype=torch.float32, device=dev)
-            N.check(self.lib.dmgs_dssim_target_stats(N.ptr(renderer.image(self.targets, v0)), 3 * (v1 - v0), h, w,
-                                                     N.ptr(st), s), "dmgs_dssim_target_stats")
-            self.stats.append(st)
+        self.stats = torch.empty(6 * renderer.total_pixels, dtype=torch.float32, device=dev)
+        self.shape = renderer.sizes[0] if len(set(renderer.sizes)) == 1 else None
+        if self.shape is not None:
+            C, (h, w) = 3 * renderer.B, self.shape
+            nbytes = self.lib.dmgs_dssim_l1_workspace_size(C, h, w)
+            N.check(self.lib.dmgs_dssim_target_stats(N.ptr(self.targets), C, h, w, N.ptr(self.stats), s),
+                    "dmgs_dssim_target_stats")
+        else:
+            table = (N.DmgsDssimView * renderer.B)()
+            for v, (h, w) in enumerate(renderer.sizes):
+                table[v].height, table[v].width, table[v].first_pixel = h, w, renderer.pixel_base[v]
+                N.check(self.lib.dmgs_dssim_target_stats(N.ptr(renderer.image(self.targets, v)), 3, h, w,
+                                                         N.ptr(self.stats[6 * renderer.pixel_base[v]:]), s),
+                        "dmgs_dssim_target_stats")
+            tiles, size = N.c_uint32(0), N.c_size_t(0)
+            N.check(self.lib.dmgs_dssim_views(renderer.B, table, ctypes.byref(tiles), ctypes.byref(size)),
+                    "dmgs_dssim_views")
+            self.tiles, nbytes = tiles.value, size.value
+            self.views = torch.frombuffer(bytearray(table), dtype=torch.uint8).to(dev)
+        self.ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         self.losses = torch.zeros(renderer.B, 3, dtype=torch.float32, device=dev)
         self.ones = torch.ones(renderer.B, dtype=torch.float32, device=dev)
 
+    def _packed(self, t):
+        if t.numel() != 3 * self.r.total_pixels or t.dtype != torch.float32 or not t.is_contiguous() or \
+                t.device.type != "cuda":
+            raise ValueError("images must be a contiguous float32 buffer packed like the renderer's")
+        return N.ptr(t)
+
     def forward(self, images):
         """(B, 3) device tensor: (loss, l1, ssim) per view."""
-        r, s = self.r, N.stream_handle(self.r.device)
-        for ws, st, (v0, v1, (h, w)) in zip(self.ws, self.stats, self.runs):
-            N.check(self.lib.dmgs_dssim_l1_forward_groups_stats(
-                N.ptr(r.image(images, v0)), N.ptr(r.image(self.targets, v0)), N.ptr(st), v1 - v0, 3, h, w, self.lam,
-                N.ptr(ws), N.ptr(self.losses[v0]), s), "dmgs_dssim_l1_forward_groups_stats")
+        x, s = self._packed(images), N.stream_handle(self.r.device)
+        y, st, ws, out = N.ptr(self.targets), N.ptr(self.stats), N.ptr(self.ws), N.ptr(self.losses)
+        if self.shape is not None:
+            N.check(self.lib.dmgs_dssim_l1_forward_groups_stats(x, y, st, self.r.B, 3, *self.shape, self.lam, ws, out, s),
+                    "dmgs_dssim_l1_forward_groups_stats")
+        else:
+            N.check(self.lib.dmgs_dssim_l1_forward_views(x, y, st, N.ptr(self.views), self.r.B, self.tiles, self.lam,
+                                                         ws, out, s), "dmgs_dssim_l1_forward_views")
         return self.losses
 
     def backward(self, images, dimages):
         """dL/dimages of the summed per-view loss (every view's dloss = 1)."""
-        r, s = self.r, N.stream_handle(self.r.device)
-        for ws, (v0, v1, (h, w)) in zip(self.ws, self.runs):
-            N.check(self.lib.dmgs_dssim_l1_backward_groups(
-                N.ptr(r.image(images, v0)), N.ptr(r.image(self.targets, v0)), v1 - v0, 3, h, w, self.lam, N.ptr(ws),
-                N.ptr(self.ones[v0:v1]), N.ptr(r.image(dimages, v0)), s), "dmgs_dssim_l1_backward_groups")
+        x, dx, s = self._packed(images), self._packed(dimages), N.stream_handle(self.r.device)
+        y, ws, ones = N.ptr(self.targets), N.ptr(self.ws), N.ptr(self.ones)
+        if self.shape is not None:
+            N.check(self.lib.dmgs_dssim_l1_backward_groups(x, y, self.r.B, 3, *self.shape, self.lam, ws, ones, dx, s),
+                    "dmgs_dssim_l1_backward_groups")
+        else:
+            N.check(self.lib.dmgs_dssim_l1_backward_views(x, y, N.ptr(self.views), self.r.B, self.tiles, self.lam, ws,
+                                                          ones, dx, s), "dmgs_dssim_l1_backward_views")
         return dimages
 
 

@@ -582,6 +582,64 @@ int dmgs_dssim_l1_backward_groups(const float* img, const float* gt, int32_t G, 
   return check_launch("dssim backward", st, false);
 }
 
+static_assert(sizeof(dmgs_dssim_view) == sizeof(dmgs::DssimView) &&
+                  offsetof(dmgs_dssim_view, index) == offsetof(dmgs::DssimView, index),
+              "dmgs_dssim_view layout");
+
+int dmgs_dssim_views(int32_t n, dmgs_dssim_view* views, uint32_t* tiles, size_t* ws_bytes) {
+  if (n <= 0 || !views || !tiles || !ws_bytes) return fail(DMGS_EINVAL, "invalid views");
+  uint64_t t = 0, pixels = 0;
+  for (int32_t v = 0; v < n; ++v) {
+    const int32_t H = views[v].height, W = views[v].width;
+    if (H <= 0 || W <= 0 || H >= (1 << 24) || W >= (1 << 24) || (int64_t)3 * H * W > ((int64_t)1 << 31))
+      return fail(DMGS_EINVAL, "invalid image shape 3 x %d x %d", H, W);
+    views[v].first_tile = (uint32_t)t;
+    views[v].index = (uint32_t)v;
+    t += dmgs::dssim_tiles(3, H, W);
+    pixels = std::max(pixels, (uint64_t)views[v].first_pixel + (uint64_t)H * W);
+    if (t > 0x7fffffffull || pixels > 0xffffffffull) return fail(DMGS_EINVAL, "the views are too large together");
+  }
+  *tiles = (uint32_t)t;
+  *ws_bytes = align_up(pixels * 9 * 4) + align_up(t * 2 * 4);
+  return DMGS_OK;
+}
+
+static int check_views(const void* img, const void* gt, const void* views, int32_t n, uint32_t tiles, const void* ws) {
+  if (!img || !gt || !views || !ws) return fail(DMGS_EINVAL, "null pointer");
+  if (n <= 0 || tiles == 0 || tiles > 0x7fffffffu) return fail(DMGS_EINVAL, "invalid views");
+  if (misaligned(ws)) return fail(DMGS_EINVAL, "ws must be 256-byte aligned");
+  return DMGS_OK;
+}
+
+int dmgs_dssim_l1_forward_views(const float* img, const float* gt, const float* gt_stats, const dmgs_dssim_view* views,
+                                int32_t n, uint32_t tiles, float lambda_dssim, void* ws, float* loss_out,
+                                dmgs_stream_t stream) {
+  if (const int rc = check_views(img, gt, views, n, tiles, ws)) return rc;
+  if (!gt_stats || !loss_out) return fail(DMGS_EINVAL, "null pointer");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  float w[11];
+  ssim_window(w);
+  const dmgs::DssimViews vs{reinterpret_cast<const dmgs::DssimView*>(views), n, tiles};
+  float* partials = static_cast<float*>(ws);  // before the maps: their size is the launch's alone
+  dmgs::launch_dssim_forward_views(img, gt, gt_stats, vs, w, lambda_dssim, at<float>(ws, align_up((size_t)tiles * 2 * 4)),
+                                   partials, loss_out, st);
+  return check_launch("dssim forward of views", st, false);
+}
+
+int dmgs_dssim_l1_backward_views(const float* img, const float* gt, const dmgs_dssim_view* views, int32_t n,
+                                 uint32_t tiles, float lambda_dssim, const void* ws, const float* dloss, float* dimg,
+                                 dmgs_stream_t stream) {
+  if (const int rc = check_views(img, gt, views, n, tiles, ws)) return rc;
+  if (!dloss || !dimg) return fail(DMGS_EINVAL, "null pointer");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  float w[11];
+  ssim_window(w);
+  const dmgs::DssimViews vs{reinterpret_cast<const dmgs::DssimView*>(views), n, tiles};
+  dmgs::launch_dssim_backward_views(img, gt, at<float>(ws, align_up((size_t)tiles * 2 * 4)), vs, w, lambda_dssim, dloss,
+                                    dimg, st);
+  return check_launch("dssim backward of views", st, false);
+}
+
 int dmgs_dssim_l1_forward(const float* img, const float* gt, int32_t C, int32_t H, int32_t W, float lambda_dssim,
                           void* ws, float* loss_out, dmgs_stream_t stream) {
   return dmgs_dssim_l1_forward_groups(img, gt, 1, C, H, W, lambda_dssim, ws, loss_out, stream);

@@ -349,6 +349,23 @@ void launch_faces_in_frustum(int F, const float* verts, const int32_t* faces, co
 
 // ---- fused L1 + SSIM loss ----
 size_t dssim_partials(int C, int H, int W);
+uint32_t dssim_tiles(int C, int H, int W);
+// RGB views of any sizes in one launch (views: a device table; tile0 and index ascend).
+struct DssimView {
+  int32_t H, W;
+  uint32_t tile0, pix0;  // its first tile of the launch, its first pixel of the packed images
+  uint32_t index;        // its place among the losses
+  uint32_t pad[3];
+};
+struct DssimViews {
+  const DssimView* views;
+  int n;
+  uint32_t tiles;
+};
+void launch_dssim_forward_views(const float* x, const float* y, const float* ystats, const DssimViews& vs,
+                                const float* w11, float lam, float* coef, float* partials, float* out, hipStream_t s);
+void launch_dssim_backward_views(const float* x, const float* y, const float* coef, const DssimViews& vs,
+                                 const float* w11, float lam, const float* dloss, float* dx, hipStream_t s);
 // C planes in C / group loss groups of `group` consecutive planes each.
 // ystats: the target's blurred maps from launch_dssim_target, or null.
 void launch_dssim_forward(const float* x, const float* y, const float* ystats, int C, int group, int H, int W,

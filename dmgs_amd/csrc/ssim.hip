@@ -97,18 +97,33 @@ __device__ __forceinline__ uint32_t pix(int px, int py, int W) {
 struct Tile {
   int bx, by, bz;
 };
-__device__ __forceinline__ Tile xcd_tile() {
+__device__ __forceinline__ uint32_t xcd_linear() {
   constexpr uint32_t kXcds = 8;
   const uint32_t gx = gridDim.x, gy = gridDim.y;
   const uint32_t n = gx * gy * gridDim.z;
   const uint32_t L = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
   const uint32_t k = L % kXcds, j = L / kXcds;
-  const uint32_t T = k * (n / kXcds) + min(k, n % kXcds) + j;
+  return k * (n / kXcds) + min(k, n % kXcds) + j;
+}
+__device__ __forceinline__ Tile tile_at(uint32_t T, uint32_t gx, uint32_t gy) {
   Tile t;
   t.bx = (int)(T % gx);
   t.by = (int)((T / gx) % gy);
   t.bz = (int)(T / (gx * gy));
   return t;
+}
+__device__ __forceinline__ Tile xcd_tile() { return tile_at(xcd_linear(), gridDim.x, gridDim.y); }
+
+// The view of tile T in a launch over views of any sizes (three planes each): the last whose first tile is not past
+// T.  Launches of their own, one per run of equal sizes, each ended in a tail of half-empty waves: sixteen uneven
+// views (18 M pixels) 436 + 72 and 380 us, in one launch 350 + 5 and 299.
+__device__ __forceinline__ DssimView view_at(const DssimViews& vs, uint32_t T) {
+  int v = -1;
+  for (int b = 0; b < vs.n; b += 64) {
+    const int l = b + (int)(threadIdx.x & 63);
+    v += (int)__popcll(__ballot((l < vs.n) & (vs.views[min(l, vs.n - 1)].tile0 <= T)));
+  }
+  return vs.views[__builtin_amdgcn_readfirstlane(v)];
 }
 
 // The 14 staged values of row r starting at column 4j (16-byte aligned).
@@ -125,11 +140,11 @@ __device__ __forceinline__ void load14(const float (*src)[kPS], int r, int j, fl
 // One loss per group of `group` consecutive planes (group = C: one loss over
 // the whole image; group = 3: one per RGB view of a batch).
 // STATS: ystats holds G*y (planes 0..C-1) and G*y^2 (planes C..2C-1).
-template <bool STATS>
+template <bool STATS, bool VIEWS>
 __global__ __launch_bounds__(256) void dssim_fwd_kernel(const float* __restrict__ x, const float* __restrict__ y,
                                                         const float* __restrict__ ystats, int H, int W, int group,
                                                         Window11 g, float lam, float* __restrict__ coef,
-                                                        float* __restrict__ partials) {
+                                                        float* __restrict__ partials, DssimViews vs) {
   constexpr int NQ = STATS ? 3 : 5;  // blurred maps: x, x^2, xy (, y, y^2)
   // the x and y patches until every row blur has read them, then the
   // row-blurred maps (one buffer: more work-groups per CU)
@@ -138,7 +153,25 @@ __global__ __launch_bounds__(256) void dssim_fwd_kernel(const float* __restrict_
     float hq[NQ][kPH][kHS];
   } u;
   __shared__ float red[2][4];
-  const Tile tl = xcd_tile();
+  Tile tl;
+  int planes = (int)gridDim.z;
+  size_t part;  // this tile's partial sums
+  if constexpr (VIEWS) {
+    const uint32_t T = xcd_linear();
+    const DssimView v = view_at(vs, T);
+    H = v.H;
+    W = v.W;
+    planes = 3;
+    tl = tile_at(T - v.tile0, (uint32_t)((W + kTW - 1) / kTW), (uint32_t)((H + kTH - 1) / kTH));
+    part = T;
+    x += 3 * (size_t)v.pix0;
+    y += 3 * (size_t)v.pix0;
+    coef += 9 * (size_t)v.pix0;
+    if constexpr (STATS) ystats += 6 * (size_t)v.pix0;
+  } else {
+    tl = xcd_tile();
+    part = ((size_t)tl.bz * gridDim.y + tl.by) * gridDim.x + tl.bx;
+  }
   const int c = tl.bz;
   const int ox = tl.bx * kTW, oy = tl.by * kTH;
   const size_t plane = (size_t)H * W;
@@ -148,7 +181,7 @@ __global__ __launch_bounds__(256) void dssim_fwd_kernel(const float* __restrict_
   if constexpr (STATS) {
     const int lx = threadIdx.x & 31, r0 = (threadIdx.x >> 5) * 4;
     const float* y0 = ystats + c * plane;
-    const float* y1 = y0 + (size_t)gridDim.z * plane;
+    const float* y1 = y0 + (size_t)planes * plane;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint32_t o = pix(min(ox + lx, W - 1), min(oy + r0 + i, H - 1), W);
@@ -243,7 +276,7 @@ __global__ __launch_bounds__(256) void dssim_fwd_kernel(const float* __restrict_
   }
   const float C1 = 0.01f * 0.01f, C2 = 0.03f * 0.03f;
   const float dS = -lam / (float)((size_t)group * plane);  // dL/dS for the mean over the group's pixels
-  const size_t all = (size_t)gridDim.z * plane;
+  const size_t all = (size_t)planes * plane;
   float* const c0 = coef + c * plane;
   float* const c1 = c0 + all;
   float* const c2 = c1 + all;
@@ -278,9 +311,8 @@ __global__ __launch_bounds__(256) void dssim_fwd_kernel(const float* __restrict_
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    const size_t b = ((size_t)tl.bz * gridDim.y + tl.by) * gridDim.x + tl.bx;
-    partials[2 * b] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-    partials[2 * b + 1] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+    partials[2 * part] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
+    partials[2 * part + 1] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
   }
 }
 
@@ -355,10 +387,19 @@ __global__ __launch_bounds__(256) void dssim_target_kernel(const float* __restri
 // One workgroup per loss group (its partials are contiguous: `nblocks`
 // blocks per group): loss = (1-lam) * L1 + lam * (1 - SSIM);
 // out[3 g ..] = (loss, l1, ssim).
+template <bool VIEWS>
 __global__ __launch_bounds__(256) void dssim_reduce_kernel(const float* __restrict__ partials, int nblocks,
-                                                           float inv_n, float lam, float* __restrict__ out) {
+                                                           float inv_n, float lam, float* __restrict__ out,
+                                                           DssimViews vs) {
   __shared__ float red[2][4];
-  partials += (size_t)2 * nblocks * blockIdx.x;
+  if constexpr (VIEWS) {
+    const DssimView v = vs.views[blockIdx.x];
+    nblocks = 3 * ((v.W + kTW - 1) / kTW) * ((v.H + kTH - 1) / kTH);
+    inv_n = 1.0f / (float)((size_t)3 * v.H * v.W);
+    partials += (size_t)2 * v.tile0;
+  } else {
+    partials += (size_t)2 * nblocks * blockIdx.x;
+  }
   out += 3 * blockIdx.x;
   float s = 0.f, l = 0.f;
   // eight pairs per thread requested at once (indices past the end read the
@@ -393,17 +434,33 @@ __global__ __launch_bounds__(256) void dssim_reduce_kernel(const float* __restri
   }
 }
 
+template <bool VIEWS>
 __global__ __launch_bounds__(256) void dssim_bwd_kernel(const float* __restrict__ x, const float* __restrict__ y,
                                                         const float* __restrict__ coef, int H, int W, int C,
                                                         int group, Window11 g, float lam,
-                                                        const float* __restrict__ dloss, float* __restrict__ dx) {
+                                                        const float* __restrict__ dloss, float* __restrict__ dx,
+                                                        DssimViews vs) {
   // the coefficient patches until every row blur has read them, then the
   // row-blurred coefficients (one buffer: more work-groups per CU)
   __shared__ __align__(16) union {
     float sa[3][kPH][kPS];
     float hq[3][kPH][kHS];
   } u;
-  const Tile tl = xcd_tile();
+  Tile tl;
+  if constexpr (VIEWS) {
+    const uint32_t T = xcd_linear();
+    const DssimView v = view_at(vs, T);
+    H = v.H;
+    W = v.W;
+    tl = tile_at(T - v.tile0, (uint32_t)((W + kTW - 1) / kTW), (uint32_t)((H + kTH - 1) / kTH));
+    x += 3 * (size_t)v.pix0;
+    y += 3 * (size_t)v.pix0;
+    dx += 3 * (size_t)v.pix0;
+    coef += 9 * (size_t)v.pix0;
+    dloss += v.index;
+  } else {
+    tl = xcd_tile();
+  }
   const int c = tl.bz;
   const int ox = tl.bx * kTW, oy = tl.by * kTH;
   const size_t plane = (size_t)H * W;
@@ -508,14 +565,30 @@ void launch_dssim_forward(const float* x, const float* y, const float* ystats, i
   for (int k = 0; k < 11; ++k) g.w[k] = w11[k];
   const dim3 grid((W + kTW - 1) / kTW, (H + kTH - 1) / kTH, C);
   if (ystats)
-    hipLaunchKernelGGL(dssim_fwd_kernel<true>, grid, dim3(256), 0, s, x, y, ystats, H, W, group, g, lam, coef,
-                       partials);
+    hipLaunchKernelGGL((dssim_fwd_kernel<true, false>), grid, dim3(256), 0, s, x, y, ystats, H, W, group, g, lam, coef,
+                       partials, DssimViews{});
   else
-    hipLaunchKernelGGL(dssim_fwd_kernel<false>, grid, dim3(256), 0, s, x, y, ystats, H, W, group, g, lam, coef,
-                       partials);
+    hipLaunchKernelGGL((dssim_fwd_kernel<false, false>), grid, dim3(256), 0, s, x, y, ystats, H, W, group, g, lam, coef,
+                       partials, DssimViews{});
   const int per_group = (int)(grid.x * grid.y) * group;
-  hipLaunchKernelGGL(dssim_reduce_kernel, dim3(C / group), dim3(256), 0, s, (const float*)partials, per_group,
-                     1.0f / (float)((size_t)group * H * W), lam, out);
+  hipLaunchKernelGGL(dssim_reduce_kernel<false>, dim3(C / group), dim3(256), 0, s, (const float*)partials, per_group,
+                     1.0f / (float)((size_t)group * H * W), lam, out, DssimViews{});
+}
+
+void launch_dssim_forward_views(const float* x, const float* y, const float* ystats, const DssimViews& vs,
+                                const float* w11, float lam, float* coef, float* partials, float* out, hipStream_t s) {
+  Window11 g;
+  for (int k = 0; k < 11; ++k) g.w[k] = w11[k];
+  hipLaunchKernelGGL((dssim_fwd_kernel<true, true>), dim3(vs.tiles), dim3(256), 0, s, x, y, ystats, 0, 0, 3, g, lam, coef,
+                     partials, vs);
+  hipLaunchKernelGGL(dssim_reduce_kernel<true>, dim3(vs.n), dim3(256), 0, s, (const float*)partials, 0, 0.f, lam, out, vs);
+}
+
+void launch_dssim_backward_views(const float* x, const float* y, const float* coef, const DssimViews& vs,
+                                 const float* w11, float lam, const float* dloss, float* dx, hipStream_t s) {
+  Window11 g;
+  for (int k = 0; k < 11; ++k) g.w[k] = w11[k];
+  hipLaunchKernelGGL(dssim_bwd_kernel<true>, dim3(vs.tiles), dim3(256), 0, s, x, y, coef, 0, 0, 3, 3, g, lam, dloss, dx, vs);
 }
 
 void launch_dssim_backward(const float* x, const float* y, const float* coef, int C, int group, int H, int W,
@@ -523,7 +596,12 @@ void launch_dssim_backward(const float* x, const float* y, const float* coef, in
   Window11 g;
   for (int k = 0; k < 11; ++k) g.w[k] = w11[k];
   const dim3 grid((W + kTW - 1) / kTW, (H + kTH - 1) / kTH, C);
-  hipLaunchKernelGGL(dssim_bwd_kernel, grid, dim3(256), 0, s, x, y, coef, H, W, C, group, g, lam, dloss, dx);
+  hipLaunchKernelGGL(dssim_bwd_kernel<false>, grid, dim3(256), 0, s, x, y, coef, H, W, C, group, g, lam, dloss, dx,
+                     DssimViews{});
+}
+
+uint32_t dssim_tiles(int C, int H, int W) {
+  return (uint32_t)((W + kTW - 1) / kTW) * (uint32_t)((H + kTH - 1) / kTH) * (uint32_t)C;
 }
 
 size_t dssim_partials(int C, int H, int W) {

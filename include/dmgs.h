@@ -234,6 +234,25 @@ int dmgs_dssim_target_stats(const float* gt, int32_t C, int32_t H, int32_t W, fl
 int dmgs_dssim_l1_forward_groups_stats(const float* img, const float* gt, const float* gt_stats, int32_t G,
                                        int32_t Cg, int32_t H, int32_t W, float lambda_dssim, void* ws,
                                        float* loss_out, dmgs_stream_t stream);
+/* RGB views of any sizes, packed one after the other, as one launch each way.
+ * dmgs_dssim_views (host): height, width and first_pixel (of the packed
+ * images, in pixels) are given; fills the rest, the tile count and the
+ * workspace size.  The calls take the table in device memory, the targets'
+ * maps at 6 * first_pixel (dmgs_dssim_target_stats per view) and one loss
+ * triple and one dloss per view; values equal the grouped calls'. */
+typedef struct dmgs_dssim_view {
+  int32_t height, width;
+  uint32_t first_tile, first_pixel;
+  uint32_t index;
+  uint32_t reserved[3];
+} dmgs_dssim_view;
+int dmgs_dssim_views(int32_t n, dmgs_dssim_view* views, uint32_t* tiles, size_t* ws_bytes);
+int dmgs_dssim_l1_forward_views(const float* img, const float* gt, const float* gt_stats, const dmgs_dssim_view* views,
+                                int32_t n, uint32_t tiles, float lambda_dssim, void* ws, float* loss_out,
+                                dmgs_stream_t stream);
+int dmgs_dssim_l1_backward_views(const float* img, const float* gt, const dmgs_dssim_view* views, int32_t n,
+                                 uint32_t tiles, float lambda_dssim, const void* ws, const float* dloss, float* dimg,
+                                 dmgs_stream_t stream);
 
 /* ---- batched views --------------------------------------------------------
  * Replaces the per-view loop of the training / evaluation scripts

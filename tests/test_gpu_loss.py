@@ -110,3 +110,31 @@ def test_fixed_target_statistics_give_identical_loss(G, H, W):
     ref_sq = torch.nn.functional.conv2d(y64 * y64, win, padding=5, groups=G * 3)[0]
     assert torch.allclose(stats[0].double().cpu(), ref_mu, atol=2e-6)
     assert torch.allclose(stats[1].double().cpu(), ref_sq, atol=2e-6)
+
+
+@pytest.mark.parametrize("sizes", [[(33, 17)], [(40, 24)] * 3, [(64, 32), (200, 150), (31, 1), (1, 40), (64, 32)],
+                                   [(16 + 7 * (k % 9), 10 + 5 * (k % 11)) for k in range(67)]])
+def test_views_in_one_launch(sizes):
+    """BatchedLoss of views of any sizes (tables past one wave's 64 entries too) equals the loss of each view alone:
+    the same operations in the same order, so bit for bit."""
+    print(f"case: loss of {len(sizes)} views, first {sizes[:5]}", flush=True)
+    from dmgs_amd import batched as BT
+    from dmgs_amd import cameras as C
+    from dmgs_amd.loss import fused_dssim_l1
+    g = torch.Generator().manual_seed(len(sizes))
+    cams = [C.camera_at((0.0, 0.0, -4.0), w, h) for w, h in sizes]
+    r = BT.BatchedRenderer(cams, torch.zeros(3, device="cuda"), 10, sh_degree=0)
+    targets = [torch.rand(3, h, w, generator=g).cuda() for w, h in sizes]
+    loss = BT.BatchedLoss(r, targets, 0.2)
+    images, grads = r.new_images(), r.new_images()
+    images.copy_(torch.rand(images.shape, generator=g))
+    got = loss.forward(images).clone()
+    loss.backward(images, grads)
+    for v, t in enumerate(targets):
+        x = r.image(images, v).clone().requires_grad_(True)
+        ref = fused_dssim_l1(x, t, 0.2)
+        ref.backward()
+        assert torch.equal(got[v, 0], ref.detach()), v
+        assert torch.equal(r.image(grads, v), x.grad), v
+    with pytest.raises(ValueError):
+        loss.forward(images[:-1])
