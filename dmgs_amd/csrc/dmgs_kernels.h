@@ -104,10 +104,11 @@ struct DupArgs {
   uint32_t K;                   // capacity of tile_keys / values
   const uint32_t* K_dev;        // optional device count (clamped to K)
   uint32_t* chunk_first;        // duplicate_scratch_words(K) words
+  uint32_t slots;               // per chunk (set by the launcher)
   bool chunk_ready;             // chunk_first already filled (launch_inclusive_scan_chunks)
   bool view_major;
   // optional: the first radix pass's histogram (digits = the low hist_bits of
-  // a key), written per 4096-slot chunk into the sort scratch
+  // a key), written per chunk into the sort scratch (from the K on whose chunks are the sort's blocks)
   uint32_t* hist;
   int hist_bits;
   // optional: words a later step needs zeroed (cleared in shares by the work-groups)
@@ -340,10 +341,12 @@ struct BindArgs {
   float* drot2d;
   float* dscale2d;
   float* dk;                // device scalar, accumulated
+  double* dk_ws;            // optional, zeroed: the blocks' parts of dk (bind_cov_workspace_bytes)
 };
 void launch_bind_fwd(const BindArgs& a, hipStream_t s);
 void launch_bind_cov_fwd(const BindArgs& a, hipStream_t s);
 void launch_bind_bwd(const BindArgs& a, hipStream_t s);
+size_t bind_cov_workspace_bytes();
 void launch_faces_in_frustum(int F, const float* verts, const int32_t* faces, const float* proj, uint8_t* mask,
                              hipStream_t s);
 

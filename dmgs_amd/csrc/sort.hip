@@ -14,6 +14,7 @@
 // Ranking inside a block is wavefront-level: each wave64 owns a contiguous
 // 1024-key slice, finds lanes with equal digits with per-bit ballots and
 // keeps running per-digit counters in LDS, so ties keep input order.
+#include <algorithm>
 #include <utility>
 
 #include "dmgs_common.h"
@@ -88,9 +89,9 @@ __device__ __forceinline__ int scan_pad(int p) { return p + (p >> 5); }
 // stores stay fully coalesced (consecutive lanes, consecutive words) while
 // each thread scans 16 consecutive elements.
 // chunk_first (inclusive scans of instance counts): also record, for every
-// 4096-slot output chunk below K, the element whose [start, end) holds the
-// chunk's first slot (what chunk_first_kernel computes from the offsets).
-constexpr uint32_t kChunkSlots = 4096;
+// output chunk below K (chunk_slots(K) slots), the element whose [start, end)
+// holds the chunk's first slot (what chunk_first_kernel computes from the
+// offsets).
 // sums_raw: `spine` holds the raw block sums (at most kPrefixBlocks of them)
 // and each work-group adds up those before it, so no spine launch is needed;
 // otherwise `spine` holds their exclusive scan.
@@ -100,7 +101,8 @@ template <bool kExclusive>
 __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t* __restrict__ in,
                                                                  uint32_t* __restrict__ out, size_t n,
                                                                  const uint32_t* __restrict__ spine, int sums_raw,
-                                                                 uint32_t* __restrict__ chunk_first, uint32_t K) {
+                                                                 uint32_t* __restrict__ chunk_first, uint32_t K,
+                                                                 uint32_t slots) {
   __shared__ uint32_t s_wave[kScanThreads / 64];
   __shared__ uint32_t tile[kScanTile + kScanTile / 32];
   const size_t base = (size_t)blockIdx.x * kScanTile;
@@ -147,8 +149,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t
     if (!kExclusive && chunk_first && x > 0u) {
       const uint32_t beg = min(run, K), end = min(run + x, K);
       const size_t idx = base + (size_t)threadIdx.x * kScanItems + i;
-      for (uint32_t c = (beg + kChunkSlots - 1) / kChunkSlots; c * kChunkSlots < end; ++c)
-        chunk_first[c] = (uint32_t)idx;
+      for (uint32_t c = (beg + slots - 1) / slots; c * slots < end; ++c) chunk_first[c] = (uint32_t)idx;
     }
     if (!kExclusive) run += x;
     tile[scan_pad((int)threadIdx.x * kScanItems + i)] = run;
@@ -165,6 +166,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_apply_kernel(const uint32_t
 
 size_t scan_scratch_words(size_t n) { return (n + kScanTile - 1) / kScanTile + 64; }
 
+static uint32_t chunk_slots(uint32_t K);
 static void scan_impl(const uint32_t* in, uint32_t* out, size_t n, uint32_t* scratch, bool exclusive,
                       hipStream_t s, uint32_t* chunk_first = nullptr, uint32_t K = 0) {
   if (n == 0) return;
@@ -174,10 +176,10 @@ static void scan_impl(const uint32_t* in, uint32_t* out, size_t n, uint32_t* scr
   if (!sums_raw) hipLaunchKernelGGL(scan_spine_kernel, dim3(1), dim3(kScanThreads), 0, s, scratch, nb);
   if (exclusive)
     hipLaunchKernelGGL(scan_apply_kernel<true>, dim3((unsigned)nb), dim3(kScanThreads), 0, s, in, out, n,
-                       (const uint32_t*)scratch, sums_raw, (uint32_t*)nullptr, 0u);
+                       (const uint32_t*)scratch, sums_raw, (uint32_t*)nullptr, 0u, 1u);
   else
     hipLaunchKernelGGL(scan_apply_kernel<false>, dim3((unsigned)nb), dim3(kScanThreads), 0, s, in, out, n,
-                       (const uint32_t*)scratch, sums_raw, chunk_first, K);
+                       (const uint32_t*)scratch, sums_raw, chunk_first, K, chunk_slots(K));
 }
 
 void launch_inclusive_scan_chunks(const uint32_t* in, uint32_t* out, size_t n, uint32_t* scratch,
@@ -632,15 +634,17 @@ void launch_gather_u32(const uint32_t* src, const uint32_t* idx, uint32_t* dst, 
   hipLaunchKernelGGL(gather_u32_kernel, dim3((n + 255) / 256), dim3(256), 0, s, src, idx, dst, n);
 }
 
-// Load-balanced emission.  The K output slots are cut into chunks of
-// kDupChunk; a first pass records, for every chunk, the depth-ordered
+// Load-balanced emission.  The K output slots are cut into chunks; a first pass records, for every chunk, the depth-ordered
 // Gaussian whose output range contains the chunk's first slot.  Each
 // workgroup then fills exactly one chunk: it stages windows of up to 256
 // consecutive Gaussians (end offset, rectangle) in LDS and maps each of its
 // slots back to its Gaussian by binary search, so stores are coalesced and a
 // few huge splats cannot serialise a workgroup.
-constexpr uint32_t kDupChunk = 4096;
-static_assert(kDupChunk == kChunkSlots, "the scan fills the duplicate's chunk table");
+// 4096 slots where the duplicate also counts the first sort pass's digits (its blocks are the sort's); fewer below,
+// because a work-group walks its chunk's entries in windows of 256, one memory latency each, and there are few
+// chunks.  With 4096, 1024 and 512 slots, us: 10 k Gaussians at 200 x 200 31, 14 and 9; 491 k face-bound ones at
+// 800 x 800 38, 15 and 11; 1 M at 800 x 800 (2.3 M slots) 25, 18 and 19.
+static uint32_t chunk_slots(uint32_t K) { return sort_items(K) == 16 ? 4096u : K >= (1u << 20) ? 1024u : 512u; }
 
 __device__ __forceinline__ uint32_t device_count(uint32_t cap, const uint32_t* dev) {
   return dev ? min(cap, *dev) : cap;
@@ -652,7 +656,7 @@ __global__ __launch_bounds__(256) void chunk_first_kernel(DupArgs a) {
   const uint32_t K = device_count(a.K, a.K_dev);
   const uint32_t beg = (s == 0) ? 0u : min(a.offsets[s - 1], K);
   const uint32_t end = min(a.offsets[s], K);
-  for (uint32_t c = (beg + kDupChunk - 1) / kDupChunk; c * kDupChunk < end; ++c) a.chunk_first[c] = (uint32_t)s;
+  for (uint32_t c = (beg + a.slots - 1) / a.slots; c * a.slots < end; ++c) a.chunk_first[c] = (uint32_t)s;
 }
 
 constexpr int kDupViews = 256;  // views whose cell-grid width and base are cached in LDS
@@ -665,7 +669,7 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
   __shared__ uint32_t s_vtb[kDupViews];      // multi-view: key base of view v
   __shared__ uint32_t s_hist[512];           // digit counts of this chunk (first sort pass)
   const uint32_t K = device_count(a.K, a.K_dev);
-  const uint32_t chunks = (uint32_t)(((size_t)a.K + kDupChunk - 1) / kDupChunk);
+  const uint32_t chunks = (uint32_t)(((size_t)a.K + a.slots - 1) / a.slots);
   const uint32_t chunk = xcd_tile(chunks);
   const uint32_t hmask = (1u << a.hist_bits) - 1u;
   if (a.zero) {  // this work-group's share of the words a later step needs zeroed
@@ -674,14 +678,14 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
     for (size_t i = zlo + threadIdx.x; i < zhi; i += 256) a.zero[i] = 0u;
   }
   if (chunk >= chunks) return;  // uniform per block
-  const uint32_t lo_slot = chunk * kDupChunk;
+  const uint32_t lo_slot = chunk * a.slots;
   if (lo_slot >= K) {  // uniform per block: an empty chunk counts nothing
     if (a.hist)
       for (uint32_t d = threadIdx.x; d <= hmask; d += 256) a.hist[(size_t)d * chunks + chunk] = 0u;
     return;
   }
   if (a.hist) s_hist[threadIdx.x] = s_hist[threadIdx.x + 256] = 0u;
-  const uint32_t hi_slot = min(K, lo_slot + kDupChunk);
+  const uint32_t hi_slot = min(K, lo_slot + a.slots);
   const uint32_t P = (uint32_t)a.P;
   const uint32_t nviews = a.views ? (P + a.per_view - 1) / a.per_view : 0u;
   auto view_tb = [&](uint32_t v) -> uint32_t {
@@ -833,12 +837,17 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
     for (uint32_t d = threadIdx.x; d <= hmask; d += 256) a.hist[(size_t)d * chunks + chunk] = s_hist[d];
 }
 
-size_t duplicate_scratch_words(size_t K) { return (K + kDupChunk - 1) / kDupChunk + 64; }
+size_t duplicate_scratch_words(size_t K) {
+  const size_t slots = chunk_slots((uint32_t)std::min<size_t>(K, 0xffffffffu));
+  return (K + slots - 1) / slots + 64;
+}
 
-void launch_duplicate(const DupArgs& a, hipStream_t s) {
-  if (a.P <= 0 || a.K == 0) return;
+void launch_duplicate(const DupArgs& args, hipStream_t s) {
+  if (args.P <= 0 || args.K == 0) return;
+  DupArgs a = args;
+  a.slots = chunk_slots(a.K);
   if (!a.chunk_ready) hipLaunchKernelGGL(chunk_first_kernel, dim3((a.P + 255) / 256), dim3(256), 0, s, a);
-  const uint32_t chunks = (uint32_t)(((size_t)a.K + kDupChunk - 1) / kDupChunk);
+  const uint32_t chunks = (uint32_t)(((size_t)a.K + a.slots - 1) / a.slots);
   hipLaunchKernelGGL(duplicate_kernel, dim3(xcd_grid(chunks)), dim3(256), 0, s, a);
 }
 

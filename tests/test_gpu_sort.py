@@ -62,3 +62,35 @@ def test_wide_digit_lists_equal_two_passes(P, sizes):
     else:
         for a, b in zip(*got):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("P,scale,cap", [(1, -2.0, None), (300, -1.0, None), (5000, -3.5, 511), (5000, -3.5, 512),
+                                         (5000, -3.5, 513), (5000, -3.5, (1 << 20) - 1), (5000, -3.5, 1 << 20),
+                                         (5000, -3.5, LARGE - 1), (5000, -3.5, LARGE), (40, 1.5, None)])
+def test_duplicate_chunk_sizes(P, scale, cap):
+    """The instances of each output chunk size (512, 1024 and 4096 slots), full, cut off and mostly empty: for every
+    capacity the lists are the first `capacity` instances in depth order, sorted by cell."""
+    print(f"case: duplicate P={P} scale={scale} capacity={cap}", flush=True)
+    model = S.free_scene(P, seed=P)
+    model._scaling = model._scaling + 3.5 + scale
+    r = BT.BatchedRenderer([C.camera_at((0.3, 0.2, -4.0), 640, 400)], [torch.zeros(3, device="cuda")], P, sh_degree=3,
+                           cell_mode=1)
+    params = BT.pack_model(model.to("cuda"))
+    K = r.count_instances(params)
+    assert K > 0
+    r.plan(params, K_cap=8 * LARGE // 4)  # 4096-slot chunks, all instances
+    r.forward(params)
+    _, keys, ids = r.cell_lists()
+    assert keys.numel() == K
+    cap = cap or K
+    r.plan(params, K_cap=cap)
+    r.forward(params)
+    ranges, k2, i2 = r.cell_lists()
+    if cap >= K:
+        assert torch.equal(keys, k2) and torch.equal(ids, i2)
+    else:  # a prefix in depth order: a subset of every cell's list, in its order
+        assert k2.numel() == cap
+        full = list(zip((keys & 0xFFFF).tolist(), ids.tolist()))
+        place = {e: n for n, e in enumerate(full)}
+        at = [place[e] for e in zip((k2 & 0xFFFF).tolist(), i2.tolist())]
+        assert at == sorted(at) and len(set(at)) == cap
