@@ -95,6 +95,9 @@ _SIGNATURES = {
                                         c_float, c_float, c_int32, c_void_p, c_void_p, c_void_p, c_void_p]),
     "dmgs_bind_cov_backward": (c_int32, [c_int64, c_void_p, c_int64, c_void_p, c_int32, c_void_p, c_int32,
                                          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "dmgs_bind_cov_workspace_size": (c_size_t, []),
+    "dmgs_bind_cov_backward_ws": (c_int32, [c_int64, c_void_p, c_int64, c_void_p, c_int32, c_void_p, c_int32,
+                                         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p] + [c_void_p]),
     "dmgs_faces_in_frustum": (c_int32, [c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_void_p]),
     "dmgs_dssim_l1_workspace_size": (c_size_t, [c_int32, c_int32, c_int32]),
     "dmgs_dssim_l1_forward": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_float, c_void_p, c_void_p,

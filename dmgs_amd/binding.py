@@ -108,11 +108,13 @@ class _Stage2(torch.autograd.Function):
         dxyz = torch.zeros(n, 3, device=dev) if dxyz is None else _f32(dxyz)
         dcov = torch.zeros(n, 6, device=dev) if dcov is None else _f32(dcov)
         dverts = torch.zeros_like(v)
-        dk = torch.zeros(1, device=dev)
-        N.check(N.load().dmgs_bind_cov_backward(v.shape[0], N.ptr(v), f.shape[0], N.ptr(f), ctx.G, N.ptr(b),
-                                                ctx.per_g, N.ptr(kk), N.ptr(L), N.ptr(dxyz), N.ptr(dcov),
-                                                N.ptr(dverts), N.ptr(dk), N.stream_handle(dev)),
-                "dmgs_bind_cov_backward")
+        lib = N.load()
+        words = lib.dmgs_bind_cov_workspace_size() // 4
+        ws = torch.zeros(words + 1, device=dev)  # the workspace, then dk
+        dk = ws[words:]
+        N.check(lib.dmgs_bind_cov_backward_ws(v.shape[0], N.ptr(v), f.shape[0], N.ptr(f), ctx.G, N.ptr(b), ctx.per_g,
+                                              N.ptr(kk), N.ptr(L), N.ptr(dxyz), N.ptr(dcov), N.ptr(dverts), N.ptr(dk),
+                                              N.ptr(ws), N.stream_handle(dev)), "dmgs_bind_cov_backward_ws")
         return dverts, dk.reshape(()), None, None, None, None, None, None
 
 

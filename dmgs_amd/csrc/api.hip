@@ -747,12 +747,14 @@ int dmgs_bind_cov_forward(int64_t V, const float* verts, int64_t F, const int32_
   return check_launch("bind cov forward", st, false);
 }
 
-int dmgs_bind_cov_backward(int64_t V, const float* verts, int64_t F, const int32_t* faces, int32_t G,
+int dmgs_bind_cov_backward_ws(int64_t V, const float* verts, int64_t F, const int32_t* faces, int32_t G,
                            const float* bc, int32_t bc_per_gaussian, const float* k, const float* Lmat,
-                           const float* dxyz, const float* dcov, float* dverts, float* dk, dmgs_stream_t stream) {
+                           const float* dxyz, const float* dcov, float* dverts, float* dk, void* ws,
+                              dmgs_stream_t stream) {
   int rc = check_mesh(V, verts, F, faces, G, bc);
   if (rc) return rc;
   if (!k || !Lmat || !dxyz || !dcov || !dverts) return fail(DMGS_EINVAL, "missing buffers");
+  if (reinterpret_cast<uintptr_t>(ws) & 7u) return fail(DMGS_EINVAL, "ws must be 8-byte aligned");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   dmgs::BindArgs a{};
   a.F = (int)F;
@@ -767,8 +769,18 @@ int dmgs_bind_cov_backward(int64_t V, const float* verts, int64_t F, const int32
   a.dcov = dcov;
   a.dverts = dverts;
   a.dk = dk;
+  a.dk_ws = static_cast<double*>(ws);
   dmgs::launch_bind_bwd(a, st);
   return check_launch("bind cov backward", st, false);
+}
+
+size_t dmgs_bind_cov_workspace_size(void) { return dmgs::bind_cov_workspace_bytes(); }
+
+int dmgs_bind_cov_backward(int64_t V, const float* verts, int64_t F, const int32_t* faces, int32_t G,
+                           const float* bc, int32_t bc_per_gaussian, const float* k, const float* Lmat,
+                           const float* dxyz, const float* dcov, float* dverts, float* dk, dmgs_stream_t stream) {
+  return dmgs_bind_cov_backward_ws(V, verts, F, faces, G, bc, bc_per_gaussian, k, Lmat, dxyz, dcov, dverts, dk, nullptr,
+                                   stream);
 }
 
 int dmgs_faces_in_frustum(int64_t V, const float* verts, int64_t F, const int32_t* faces, const float* projmatrix,

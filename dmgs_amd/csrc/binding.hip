@@ -145,11 +145,14 @@ __global__ __launch_bounds__(256) void bind_fwd_kernel(BindArgs a) {
 // contributions to its face (up to 24 sums) go through LDS and are added there in the Gaussians' order.
 // Bound by the atomics on the vertices: neighbouring lanes add the three components of one vertex, so that they
 // leave as one request.  A lane per face with nine adds of its own took 57 us for 81 920 faces x 6 with rotations
-// (24 now; 44 with this split but the adds left with the face's lane) and 61 us for 98 528 x 6 covariances (26).
+// (24 now; 44 with this split but the adds left with the face's lane) and 61 us for 98 528 x 6 covariances (28).
 constexpr int kBindLanes = 256;
 // Blocks whose faces add to the one dk: same-address adds take 8.5 ns each, so a block walks several groups of
-// faces (98 528 x 6: 41 us with 2346 blocks, 34 with 1536, 32 with 1024, 26 with 512).
+// faces (98 528 x 6: 41 us with 2346 blocks, 34 with 1536, 32 with 1024, 26 with 512).  The scalar is a sum of terms
+// of random sign: with a workspace the blocks' parts are kept in 64 bits and added in order (the atomics' rounding
+// alone was 5e-7 of a typical sum).
 constexpr int kBindCovBlocks = 512;
+size_t bind_cov_workspace_bytes() { return 8 * (1 + (size_t)kBindCovBlocks); }
 
 template <bool ROT, bool COV>
 __global__ __launch_bounds__(kBindLanes) void bind_bwd_kernel(BindArgs a, int block_faces) {
@@ -158,9 +161,9 @@ __global__ __launch_bounds__(kBindLanes) void bind_bwd_kernel(BindArgs a, int bl
   __shared__ float s_part[kBindSums * kBindLanes];       // [sum][lane]
   __shared__ float s_frame[9 * kBindLanes];              // [component][face]: frame, later the vertex gradients
   __shared__ int s_vertex[3 * kBindLanes];               // [corner][face]
-  __shared__ float s_dk[kBindLanes / 64];
+  __shared__ double s_dk[kBindLanes / 64];
   const int tid = threadIdx.x;
-  float dk = 0.f;
+  double dk = 0.0;  // of random signs: in 64 bits
   for (uint32_t f0 = blockIdx.x * block_faces; f0 < (uint32_t)a.F; f0 += gridDim.x * block_faces) {
     const int nf = min(block_faces, a.F - (int)f0);
     const uint32_t ng = (uint32_t)nf * a.G;  // Gaussians of this block
@@ -277,7 +280,7 @@ __global__ __launch_bounds__(kBindLanes) void bind_bwd_kernel(BindArgs a, int bl
         gx = gx + v3(dR[0][0], dR[1][0], dR[2][0]);
         gy = gy + v3(dR[0][1], dR[1][1], dR[2][1]);
         gn = gn + v3(dR[0][2], dR[1][2], dR[2][2]);
-        if (k != 0.f) dk += 2.f * gk / k;
+        if (k != 0.f) dk += (double)(2.f * gk / k);
       }
       V3 de1, de2;
       frame_bwd(fr, gx, gy, gn, de1, de2);
@@ -297,16 +300,38 @@ __global__ __launch_bounds__(kBindLanes) void bind_bwd_kernel(BindArgs a, int bl
     __syncthreads();
   }
   if constexpr (COV) {
-    if (a.dk) {  // one atomic per block
-      for (int off = 32; off > 0; off >>= 1) dk += __shfl_xor(dk, off, 64);
-      if ((tid & 63) == 0) s_dk[tid >> 6] = dk;
+    if (!a.dk) return;
+    auto block_sum = [&](double x) {  // thread 0 has it
+      for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+      if ((tid & 63) == 0) s_dk[tid >> 6] = x;
       __syncthreads();
-      if (tid == 0) {
-        float t = 0.f;
-        for (int w = 0; w < kBindLanes / 64; ++w) t += s_dk[w];
-        if (t != 0.f) unsafeAtomicAdd(a.dk, t);
-      }
+      double t = 0.0;
+      for (int w = 0; w < kBindLanes / 64; ++w) t += s_dk[w];
+      return t;
+    };
+    const double part = block_sum(dk);
+    if (!a.dk_ws) {
+      if (tid == 0 && part != 0.0) unsafeAtomicAdd(a.dk, (float)part);
+      return;
     }
+    // The block that arrives last adds the blocks' parts in a fixed order.  A part is exchanged, not stored: the old
+    // value's return says that it is where every XCD's atomics see it, and only then does the block count as arrived.
+    // (A releasing counter writes back an L2 per block: 52 us instead of 28.)
+    unsigned long long* parts = reinterpret_cast<unsigned long long*>(a.dk_ws) + 1;
+    __shared__ uint32_t s_arrived;
+    if (tid == 0) {
+      const unsigned long long old = __hip_atomic_exchange(parts + blockIdx.x, (unsigned long long)__double_as_longlong(part),
+                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      uint32_t one = old == ~0ull ? 2u : 1u;  // zeroed by the caller: always 1, and never before the exchange is done
+      s_arrived = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(a.dk_ws), one, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (s_arrived != gridDim.x - 1) return;
+    double t = 0.0;
+    for (uint32_t i = tid; i < gridDim.x; i += kBindLanes)
+      t += __longlong_as_double((long long)__hip_atomic_fetch_or(parts + i, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    t = block_sum(t);
+    if (tid == 0) *a.dk += (float)t;
   }
 }
 

@@ -195,6 +195,12 @@ int dmgs_bind_cov_forward(int64_t V, const float* verts, int64_t F, const int32_
 int dmgs_bind_cov_backward(int64_t V, const float* verts, int64_t F, const int32_t* faces, int32_t G,
                            const float* bc, int32_t bc_per_gaussian, const float* k, const float* Lmat,
                            const float* dxyz, const float* dcov, float* dverts, float* dk, dmgs_stream_t stream);
+/* The same with a workspace (dmgs_bind_cov_workspace_size bytes, zeroed, 8-byte
+ * aligned; may be null) in which the parts of dk are added in 64 bits. */
+size_t dmgs_bind_cov_workspace_size(void);
+int dmgs_bind_cov_backward_ws(int64_t V, const float* verts, int64_t F, const int32_t* faces, int32_t G,
+                           const float* bc, int32_t bc_per_gaussian, const float* k, const float* Lmat,
+                           const float* dxyz, const float* dcov, float* dverts, float* dk, void* ws, dmgs_stream_t stream);
 /* mask[f] = 1 if face f's centroid projects inside |ndc| < 1.05 with w > 0
  * (in_frustum, scene/gaussian_geo_model_finetune.py:33-48). */
 int dmgs_faces_in_frustum(int64_t V, const float* verts, int64_t F, const int32_t* faces, const float* projmatrix,
