@@ -94,3 +94,32 @@ def test_duplicate_chunk_sizes(P, scale, cap):
         place = {e: n for n, e in enumerate(full)}
         at = [place[e] for e in zip((k2 & 0xFFFF).tolist(), i2.tolist())]
         assert at == sorted(at) and len(set(at)) == cap
+
+
+@pytest.mark.parametrize("size", [(16, 16), (512, 512), (1024, 1024), (1040, 1008), (1025, 1024)])
+def test_tile_order_is_a_permutation_by_length(size):
+    """1, 1024, 4096 and 4095 tiles in one launch, 4160 in two: every tile once, longest lists first."""
+    print(f"case: tile order {size}", flush=True)
+    P = 4000
+    r = BT.BatchedRenderer([C.camera_at((0.3, 0.2, -4.0), *size)], [torch.zeros(3, device="cuda")], P, sh_degree=0)
+    params = BT.pack_model(S.free_scene(P, seed=2, sh_degree=0).to("cuda"))
+    r.plan(params)
+    images = r.forward(params).clone()
+    T = r.total_tiles
+    gx, cx = (size[0] + 15) // 16, ((size[0] + 15) // 16 + 3) // 4
+    ranges = r.cell_lists()[0].long()
+    length = ranges[:, 1] - ranges[:, 0]
+    t = torch.arange(T)
+    cost = length[(t // gx // 4) * cx + t % gx // 4].clamp(min=0).double()
+    bucket = torch.where(cost > 0, 254 - (8 * torch.log2(cost.clamp(min=1))).floor().clamp(max=254), 255.0)
+    # the order lies before the range table in the state: the one run of T words that is a permutation
+    words = r.state[:r._offsets[2]].view(torch.int32).cpu()
+    found = 0
+    for at in range(0, words.numel() - T + 1, 64):  # sub-buffers are 256-byte aligned
+        o = words[at:at + T].long()
+        if int(o[0]) < T and torch.equal(torch.sort(o).values, t):
+            b = bucket[o]
+            if bool((b[1:] >= b[:-1] - 1).all()):  # log2 rounds either way at a bucket's edge
+                found += 1
+    assert found >= 1
+    assert torch.isfinite(images).all()

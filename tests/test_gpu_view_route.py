@@ -124,3 +124,27 @@ def test_sh_sigmoid_second_order():
         second.append(torch.autograd.grad((a ** 2).sum() + (b ** 2).sum(), (ff, xx)))
     for s, r in zip(*second):
         assert grad_rel_err(s.double(), r) < 1e-4
+
+
+def test_counts_in_plain_and_pinned_memory():
+    """The geometry call writes pinned counts from its kernel and copies to plain host memory: the same numbers."""
+    import ctypes
+    from dmgs_amd import _native as N
+    from dmgs_amd.gaussian_renderer import _settings
+    lib, P = N.load(), 3000
+    m = S.free_scene(P, seed=4).to("cuda")
+    rs = _settings(C.camera_at((0.4, 0.3, -3.5), 173, 119), torch.zeros(3, device="cuda"), 3, 1.0, False)
+    fr = RZ._Frame(rs, m._xyz.device, 16)
+    g = RZ._gaussians(P, dict(means3D=m._xyz, opacities=m._opacity, shs=m._features_dc, shs_rest=m._features_rest,
+                              scales=m._scaling, rotations=m._rotation),
+                      RZ.RAW_SCALES | RZ.RAW_ROTATIONS | RZ.RAW_OPACITIES)
+    state = torch.empty(lib.dmgs_view_state_size(P, 173, 119, 0), dtype=torch.uint8, device="cuda")
+    radii = torch.empty(P, dtype=torch.int32, device="cuda")
+    stream = N.stream_handle(m._xyz.device)
+    got = []
+    for counts in (torch.zeros(4, dtype=torch.int32, pin_memory=True)[1:3], torch.zeros(4, dtype=torch.int32)[1:3]):
+        N.check(lib.dmgs_view_geometry(ctypes.byref(fr.c), ctypes.byref(g), 0, N.ptr(radii), N.ptr(state),
+                                       N.ptr(counts), stream), "dmgs_view_geometry")
+        N.check(lib.dmgs_view_counts(stream), "dmgs_view_counts")
+        got.append(counts.tolist())
+    assert got[0] == got[1] and min(got[0]) > 0
