@@ -257,7 +257,7 @@ struct RenderArgs {
   float* gacc;           // P x DMGS_GACC_STRIDE floats, two planes (gacc_index)
   // optional (multi-view): work-group slot -> tile, heaviest tiles first
   const uint32_t* tile_order;
-  // optional (multi-view, strip forward): per tile, the largest last
+  // optional (multi-view): per tile, the largest last
   // contributor of its pixels (the backward's list length)
   uint32_t* tile_work;
   // optional (forward): the backward accumulator, zeroed by the forward's
@@ -276,7 +276,7 @@ void launch_render_fwd(const RenderArgs& a, hipStream_t s);
 // byte per tile, hist: 512 words of scratch.
 void launch_tile_order(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, hipStream_t s,
                        bool hist_zeroed = false);
-// The same with a.tile_work (written by the strip forward) as each tile's
+// The same with a.tile_work (written by the forward) as each tile's
 // cost: the backward's exact list length.
 void launch_tile_order_bwd(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, hipStream_t s,
                            bool hist_zeroed = false);

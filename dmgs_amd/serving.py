@@ -119,10 +119,9 @@ class _Batch:
         self.phase = "render"
 
 
-# Blend shapes the server chooses between when no variant is fixed: quarter
-# tiles of 8x8 pixels (fastest for small views and short lists) and one wave
-# per 16x16 tile (fastest for large views and long lists).  All shapes give
-# bit-identical images, so the choice changes only the time.
+# The variants the server times when none is fixed.  They name the same blend
+# kernels (the launch picks their form from its own sizes), so the choice
+# changes nothing; the numbers are kept for callers that read them.
 AUTO_VARIANTS = (3, 4)
 
 
@@ -131,10 +130,9 @@ class RenderServer:
 
     scenes: {name: params (59, P) float32 on ``device``} or {name: (params,
     sh_degree)}.  hbm_budget: bytes the server may hold for in-flight work
-    (default 80 % of the free HBM at start-up).  variant: the blend shape of
-    every batch, or None to time each of AUTO_VARIANTS on the first batches
-    of a (scene, size class) and keep the faster (size class: the bit length
-    of the batch's tile count)."""
+    (default 80 % of the free HBM at start-up).  variant: passed on to every
+    batch, or None to time AUTO_VARIANTS on the first batches of a (scene,
+    size class) (size class: the bit length of the batch's tile count)."""
 
     def __init__(self, scenes, device="cuda", hbm_budget=None, max_views=8, num_streams=4, variant=None,
                  initial_instances_per_pixel=32.0):
