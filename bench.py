@@ -518,18 +518,19 @@ def list_counts(r):
     return K, int(bits.sum().item())
 
 
-def _reach_strips(cx, cy, a, b, c, o, x0, y0):
-    """Which of the four 16x4 pixel strips of the tile at (x0, y0) each
-    splat's alpha >= 1/255 ellipse reaches, by the blend kernels' staging
-    test (same margins); (4, L) bool."""
+def _reach(cx, cy, a, b, c, o, x0, y0, quads):
+    """Which of the four 8x8 quadrants (``quads``) or 16x4 pixel strips of
+    the tile at (x0, y0) each splat's alpha >= 1/255 ellipse reaches, by the
+    blend kernels' staging test (same margins); (4, L) bool."""
     with np.errstate(divide="ignore", invalid="ignore", over="ignore"):
         tau = 2.0 * np.log(255.0 * o)
     t = tau * 1.001 + 0.001
     out = np.zeros((4, cx.size), dtype=bool)
     m = 0.01
     for k in range(4):
-        rx0, rx1 = x0 - m, x0 + 15.0 + m
-        ry0, ry1 = y0 + 4.0 * k - m, y0 + 4.0 * k + 3.0 + m
+        bx, by, bw, bh = (8 * (k & 1), 8 * (k >> 1), 8, 8) if quads else (0, 4 * k, 16, 4)
+        rx0, rx1 = x0 + bx - m, x0 + bx + bw - 1.0 + m
+        ry0, ry1 = y0 + by - m, y0 + by + bh - 1.0 + m
         inside = (cx >= rx0) & (cx <= rx1) & (cy >= ry0) & (cy <= ry1)
         best = np.full(cx.size, np.inf)
         with np.errstate(divide="ignore", invalid="ignore"):
@@ -551,9 +552,9 @@ def pair_counts(r, view, n_tiles, seed=0):
     (float64 restatement of the per-pixel rules):
       reference:        a per-pixel loop, every list entry up to and including
                         the pixel's stopping entry (the reference kernel's work);
-      strips_forward:   the one-wave-per-tile forward, 64 lanes per (splat,
-                        16x4 strip) the splat's footprint reaches while a pixel
-                        of the strip still blends;
+      quads_forward:    the forward, 64 lanes per (splat, 8x8 quadrant) the
+                        splat's footprint reaches while a pixel of the
+                        quadrant still blends;
       strips_backward:  the strip backward, 64 lanes per (splat, reached strip)
                         in front of the strip's last contributor;
       contributing:     pairs that pass the alpha test before the pixel stops.
@@ -571,7 +572,7 @@ def pair_counts(r, view, n_tiles, seed=0):
     N.check(r.lib.dmgs_batched_list_offsets(ctypes.byref(r._desc()), ctypes.byref(ko), ctypes.byref(vo)), "offsets")
     o2 = r._offsets[2]
     rng = np.random.default_rng(seed)
-    counts = dict(reference=0, strips_forward=0, strips_backward=0, contributing=0, tile_instances=0, tiles=0)
+    counts = dict(reference=0, quads_forward=0, strips_backward=0, contributing=0, tile_instances=0, tiles=0)
     for t in rng.permutation(gx * gy)[:n_tiles]:
         tx, ty = int(t) % gx, int(t) // gx
         cell = d.cell_base + (ty // 4) * cgx + tx // 4
@@ -587,7 +588,7 @@ def pair_counts(r, view, n_tiles, seed=0):
             continue
         cx, cy, a, b, c, o = (rec[g, i] for i in (0, 1, 2, 3, 4, 5))
         x0, y0 = 16.0 * tx, 16.0 * ty
-        reach = _reach_strips(cx, cy, a, b, c, o, x0, y0)
+        reach = {q: _reach(cx, cy, a, b, c, o, x0, y0, q) for q in (True, False)}
         py, px = np.mgrid[0:16, 0:16]
         px, py = (px + x0).reshape(-1), (py + y0).reshape(-1)
         dx = cx[None, :] - px[:, None]
@@ -605,14 +606,16 @@ def pair_counts(r, view, n_tiles, seed=0):
         counts["reference"] += int(np.minimum(sidx + 1, L)[inside].sum())
         counts["contributing"] += int(include[inside].sum())
         strip = (py - int(y0)) // 4
+        quad = (py - int(y0)) // 8 * 2 + (px - int(x0)) // 8
         for k in range(4):
+            sel = inside & (quad == k)
+            if sel.any():
+                alive_to = sidx[sel].max()     # the quadrant blends up to its last stopping entry
+                counts["quads_forward"] += 64 * int((reach[True][k] & (np.arange(L) <= alive_to)).sum())
             sel = inside & (strip == k)
-            if not sel.any():
-                continue
-            alive_to = sidx[sel].max()          # the strip blends up to its last stopping entry
-            counts["strips_forward"] += 64 * int((reach[k] & (np.arange(L) <= alive_to)).sum())
-            behind = ncontrib[sel].max()       # entries in front of the strip's last contributor
-            counts["strips_backward"] += 64 * int((reach[k] & (np.arange(L) < behind)).sum())
+            if sel.any():
+                behind = ncontrib[sel].max()   # entries in front of the strip's last contributor
+                counts["strips_backward"] += 64 * int((reach[False][k] & (np.arange(L) < behind)).sum())
     return counts
 
 
@@ -647,11 +650,11 @@ def main():
     # pair evaluations on sampled tiles of the first view, scaled to the step by tile instances
     pc = pair_counts(r, 0, args.pair_tiles, seed=1)
     scale = m["K_tile"] / max(pc["tile_instances"], 1)
-    pairs = {k: int(round(pc[k] * scale)) for k in ("reference", "strips_forward", "strips_backward", "contributing")}
+    pairs = {k: int(round(pc[k] * scale)) for k in ("reference", "quads_forward", "strips_backward", "contributing")}
     valu = _valu_issue(f"batched_{kern}", stage_ms[kern], args)
     pairs_note = {"sample": f"{pc['tiles']} random tiles of view 0 ({pc['tile_instances']} tile instances), "
                             f"scaled by the step's {m['K_tile']} tile instances",
-                  "forward_evaluated_per_contributing": round(pc["strips_forward"] / max(pc["contributing"], 1), 3),
+                  "forward_evaluated_per_contributing": round(pc["quads_forward"] / max(pc["contributing"], 1), 3),
                   "backward_evaluated_per_contributing": round(pc["strips_backward"] / max(pc["contributing"], 1), 3),
                   "reference_evaluated_per_contributing": round(pc["reference"] / max(pc["contributing"], 1), 3)}
     if valu:

@@ -91,52 +91,72 @@ __device__ __forceinline__ T lds_at(const T (&a)[N], uint32_t byte_offset) {
 // against each rectangle of pixel centres a wave (or a strip of the tile)
 // covers and keeps one bit per rectangle; a wave skips the splat when its
 // bit is clear: no pixel there could pass the alpha test, so results are
-// unchanged.  Margins (rectangle +0.01 px, tau x 1.001 + 0.001) keep the test
-// conservative against rounding.
-struct PixelRects {  // n rectangles of w x h pixels, `cols` (1 or 2) to a row, the first at (x0, y0)
+// unchanged.  Margins (rectangle +0.01 px, tau x 1.001 + 0.001, and 1e-6 of the
+// form's terms at the work-group's far edges, which bounds what rounding adds to
+// it here and in a pixel) keep the test conservative.
+struct PixelRects {  // four rectangles of w x h pixels, `cols` (1 or 2) to a row, the first at (x0, y0)
   float x0, y0, w, h;
-  int cols, n;
+  int cols;
 };
 
-// min over the rectangle of q(p - centre) <= tau, q(d) = a dx^2 + 2 b dx dy + c dy^2
-// (convex: the minimum is the centre if it is inside, else on an edge, where
-// the one-dimensional minimiser is clamped to the edge).
-__device__ __forceinline__ bool ellipse_meets_rect(float cx, float cy, float a, float b, float c, float tau,
-                                                   float x0, float x1, float y0, float y1) {
-  if (cx >= x0 && cx <= x1 && cy >= y0 && cy <= y1) return true;
-  // (an approximate reciprocal only moves the edge point off the exact
-  // minimiser, which raises the value found by far less than the margins)
+// Per rectangle: the minimum over it of q(d) = a dx^2 + 2 b dx dy + c dy^2, d = p - centre, against t.  q grows along
+// every ray from the centre (or is negative on all of it), so what counts are the edges that face the centre: at most
+// one vertical and one horizontal, each with its one-dimensional minimiser clamped to the edge.  Where the centre
+// lies between two edges the line through it stands in for them, whose point is in the rectangle too; for a
+// rectangle that holds the centre that is the centre.  (An approximate reciprocal only moves the edge point off the
+// minimiser, which raises the value found by far less than the margins.)  Rectangles side by side share a row's or
+// column's terms: 150 instructions for four rectangles, where four edges of each, a rectangle at a time behind a
+// branch, took REACH_BEFORE.
+template <int NX, int NY>
+__device__ __forceinline__ uint32_t reach_rects(float cx, float cy, float a, float b, float c, float t,
+                                                const PixelRects& rr) {
+  constexpr float m = 0.01f;
   const float ia = __builtin_amdgcn_rcpf(a), ic = __builtin_amdgcn_rcpf(c);
-  float best = INFINITY;
+  const float b2 = b + b, to_y = -b * ic, to_x = -b * ia;
+  const float ox = rr.x0 - cx, oy = rr.y0 - cy;
+  float xl[NX], xh[NX], ey_at[NX], xb[NX], xx[NX];  // of a column: its edges, and the terms of the edge that counts
+  float yl[NY], yh[NY], ex_at[NY], yb[NY], yy[NY];
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const float dx = (e ? x1 : x0) - cx;
-    const float dy = fminf(fmaxf(-b * dx * ic, y0 - cy), y1 - cy);
-    best = fminf(best, a * dx * dx + 2.0f * b * dx * dy + c * dy * dy);
+  for (int i = 0; i < NX; ++i) {
+    xl[i] = ox + (i ? rr.w * (float)i - m : -m);
+    xh[i] = ox + (rr.w * (float)(i + 1) - 1.0f + m);
+    const float e = __builtin_amdgcn_fmed3f(xl[i], 0.f, xh[i]);
+    ey_at[i] = to_y * e;
+    xb[i] = b2 * e;
+    xx[i] = a * e * e;
   }
 #pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const float dy = (e ? y1 : y0) - cy;
-    const float dx = fminf(fmaxf(-b * dy * ia, x0 - cx), x1 - cx);
-    best = fminf(best, a * dx * dx + 2.0f * b * dx * dy + c * dy * dy);
+  for (int j = 0; j < NY; ++j) {
+    yl[j] = oy + (j ? rr.h * (float)j - m : -m);
+    yh[j] = oy + (rr.h * (float)(j + 1) - 1.0f + m);
+    const float e = __builtin_amdgcn_fmed3f(yl[j], 0.f, yh[j]);
+    ex_at[j] = to_x * e;
+    yb[j] = b2 * e;
+    yy[j] = c * e * e;
   }
-  return best <= tau;
+  const float fx = fmaxf(fabsf(xl[0]), fabsf(xh[NX - 1])), fy = fmaxf(fabsf(yl[0]), fabsf(yh[NY - 1]));
+  t = fmaf(1e-6f, fmaf(a * fx, fx, c * fy * fy), t);
+  uint32_t mask = 0;
+#pragma unroll
+  for (int j = 0; j < NY; ++j) {
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const float dy = __builtin_amdgcn_fmed3f(yl[j], ey_at[i], yh[j]);
+      const float dx = __builtin_amdgcn_fmed3f(xl[i], ex_at[j], xh[i]);
+      const float q = fminf(fmaf(dy, fmaf(c, dy, xb[i]), xx[i]), fmaf(dx, fmaf(a, dx, yb[j]), yy[j]));
+      mask |= q > t ? 0u : 1u << (j * NX + i);
+    }
+  }
+  return mask;
 }
 
 __device__ __forceinline__ uint32_t reach_mask(float cx, float cy, float a, float b, float c, float o,
                                                const PixelRects& rr) {
-  const float tau = 2.0f * logf(255.0f * o);
-  if (!(tau > 0.0f)) return 0u;  // o < 1/255: alpha never reaches the threshold
-  if (!(a > 0.0f && c > 0.0f)) return 0xFu;
-  const float t = tau * 1.001f + 0.001f, m = 0.01f;
-  uint32_t mask = 0;
-  for (int k = 0; k < rr.n; ++k) {
-    const int row = rr.cols == 2 ? k >> 1 : k, col = rr.cols == 2 ? k & 1 : 0;
-    const float x0 = rr.x0 + (float)col * rr.w, y0 = rr.y0 + (float)row * rr.h;
-    if (ellipse_meets_rect(cx, cy, a, b, c, t, x0 - m, x0 + rr.w - 1.0f + m, y0 - m, y0 + rr.h - 1.0f + m))
-      mask |= 1u << k;
-  }
-  return mask;
+  const float t = fmaf(1.001f * 1.3862943611f, __builtin_amdgcn_logf(255.0f * o), 0.001f);  // tau from a log2
+  const uint32_t mask =
+      rr.cols == 2 ? reach_rects<2, 2>(cx, cy, a, b, c, t, rr) : reach_rects<1, 4>(cx, cy, a, b, c, t, rr);
+  if (!(255.0f * o > 1.0f)) return 0u;  // alpha never reaches the threshold
+  return (a > 0.0f) & (c > 0.0f) ? mask : 0xFu;
 }
 
 // p = log2(e) power = (q.x dx) dx + dy (q.y dx + q.z dy) for power = -1/2 (a dx^2
@@ -342,7 +362,6 @@ __device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile, int h
   c.rows.w = QUADS ? 8.0f : 16.0f;
   c.rows.h = QUADS && half < 0 ? 8.0f : 4.0f;
   c.rows.cols = QUADS ? 2 : 1;
-  c.rows.n = 4;
   c.inside = c.px < c.W && c.py < c.H;
   c.plane = (size_t)c.W * c.H;
   c.pix = (size_t)pbase + (size_t)c.py * c.W + c.px;

@@ -98,3 +98,39 @@ def test_two_work_groups_per_tile(n, logit, size, scale):
         assert torch.equal(a, b)
     # and twice: the halves' largest counts do not depend on an earlier forward
     assert torch.equal(r.forward(params), got[0][0])
+
+
+@pytest.mark.parametrize("n,logit,size,long", [(60, 1.0, (16, 16), -1.0), (200, 0.0, (33, 41), -1.0),
+                                               (400, -1.0, (120, 70), -0.5), (300, -5.4, (48, 48), -1.0),
+                                               (2000, 0.0, (300, 200), -2.5)])
+def test_needles_across_quadrants_and_strips(n, logit, size, long):
+    """Thin splats in any direction, centres inside and outside the image: which quadrants and strips they reach
+    decides what is evaluated, so a rectangle wrongly left out is missing from the image or the gradients.  Opacities
+    around 1/255 included.  Tolerances of the other parity tests."""
+    print(f"case: needles n={n} logit={logit} size={size} long={long}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    xyz = (torch.rand(n, 3, generator=g) - 0.5) * 4.0
+    scale = torch.tensor([long, -4.5, -4.5]) + 0.2 * torch.randn(n, 3, generator=g)
+    m = S.FreeGaussians(xyz, torch.randn(n, 1, 3, generator=g) * 0.5, torch.randn(n, 3, 3, generator=g) * 0.1, scale,
+                        torch.randn(n, 4, generator=g), logit + 0.3 * torch.randn(n, 1, generator=g), 1)
+    cam = C.camera_at((0.3, -0.2, -4.0), *size, device="cpu")
+    bg = torch.tensor([0.2, 0.5, 0.8])
+    st = OR.settings_for(cam, bg.double(), 1)
+    kw = dict(shs=m.get_features, scales=m.get_scaling, rotations=m.get_rotation)
+    col, _, state = OR.rasterize(m.get_xyz, m.get_opacity, st, **kw)
+    dL = torch.randn(col.shape, generator=torch.Generator().manual_seed(1))
+    dL[:, state["ambiguous"]] = 0.0
+    want = OR.rasterize_backward(state, st, m.get_xyz, dL.double(), **kw)
+    params = BT.pack_model(m.to("cuda"))
+    r = BT.BatchedRenderer([cam], bg, n, sh_degree=1)
+    r.plan(params)
+    images = r.forward(params).clone()
+    grads = r.backward(params, dL.cuda().reshape(-1).contiguous())
+    ok = ~state["ambiguous"]
+    assert (r.image(images, 0).cpu().double() - col).abs()[:, ok].max().item() < 1e-4
+    got = BT.unpack_grads(grads, 4)
+    o = torch.sigmoid(m._opacity.double())
+    for name, ref in (("_xyz", want[0]), ("_opacity", want[4] * o * (1 - o)), ("_features_dc", want[2][:, :1])):
+        assert grad_rel_err(got[name], ref) < 1e-3, name
+    r.bwd_ws = None  # without a backward to follow: two work-groups a tile
+    assert torch.equal(r.forward(params), images)
