@@ -105,8 +105,9 @@ struct PixelRects {  // four rectangles of w x h pixels, `cols` (1 or 2) to a ro
 // lies between two edges the line through it stands in for them, whose point is in the rectangle too; for a
 // rectangle that holds the centre that is the centre.  (An approximate reciprocal only moves the edge point off the
 // minimiser, which raises the value found by far less than the margins.)  Rectangles side by side share a row's or
-// column's terms: 150 instructions for four rectangles, where four edges of each, a rectangle at a time behind a
-// branch, took REACH_BEFORE.
+// column's terms, and the logarithm is the hardware's: against four edges of each rectangle behind a branch, 158 vector
+// instructions less per staged splat in the forward's code and 129 in the backward's.  Issued on 8 views of 800x800 of
+// 1M Gaussians 202.5M -> 189.8M and 265.9M -> 259.5M; one 333x251 view of 500k, near, 319 -> 303 us.
 template <int NX, int NY>
 __device__ __forceinline__ uint32_t reach_rects(float cx, float cy, float a, float b, float c, float t,
                                                 const PixelRects& rr) {
@@ -469,8 +470,8 @@ struct MemberList {
 // instructions of any kind as possible: each wave first packs the LDS offsets of the staged splats that reach
 // its quadrant, then takes four at a time, reading the next four while it evaluates the four alphas (whose
 // latencies overlap) and applies them in order with selects instead of branches.  Against one wave per tile
-// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 325 us, 16 uneven views of 3M
-// 5.33 -> 3.51 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
+// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 312 us, 16 uneven views of 3M
+// 5.33 -> 3.36 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
 // reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on KEEP,
 // CELLS or the launch.
 // SPLIT: a tile's list is a chain (each pixel's transmittance goes from splat to splat), so a launch of few tiles
