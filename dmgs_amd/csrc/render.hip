@@ -470,8 +470,8 @@ struct MemberList {
 // instructions of any kind as possible: each wave first packs the LDS offsets of the staged splats that reach
 // its quadrant, then takes four at a time, reading the next four while it evaluates the four alphas (whose
 // latencies overlap) and applies them in order with selects instead of branches.  Against one wave per tile
-// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 312 us, 16 uneven views of 3M
-// 5.33 -> 3.36 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
+// with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 294 us, 16 uneven views of 3M
+// 5.33 -> 2.99 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
 // reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on KEEP,
 // CELLS or the launch.
 // SPLIT: a tile's list is a chain (each pixel's transmittance goes from splat to splat), so a launch of few tiles
@@ -480,8 +480,13 @@ struct MemberList {
 // consecutive splats side by side, exchange them, and both carry the transmittance over the two in order; one adds
 // red and green, the other blue.  16 instructions a splat, in twice as many waves, with the same operations in the
 // same order on every value.  (Eight waves of one work-group share a CU's SIMDs and gain nothing.)
+// Five waves per SIMD where one work-group blends a tile and keeps nothing: the compiler takes 106 registers (four
+// waves) if left alone and 96 without a spill if asked; 16 uneven views 3.34 -> 2.99 ms, 8 views of 800x800 312 -> 294 us,
+// 1920x1080 134 -> 125 us.  Six waves spill 48 bytes (8 views of 800x800 330 us); with kept segments five spill 24
+// (a 10k view 57 -> 59 us, 82k faces 249 -> 255); two work-groups a tile have few waves in flight at any register count.
 template <bool CELLS, bool KEEP, bool SPLIT>
-__global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPLIT ? 1 : 5, 8))) void render_fwd_quads_kernel(
+    RenderArgs a) {
   constexpr int NT = 256, U = FwdGroup::kN;
   constexpr int G = KEEP ? 64 : NT;  // staged splats blended per round
   constexpr int kPad = NT * 16;      // offset of the filling splat
@@ -822,8 +827,8 @@ __global__ __launch_bounds__(256) void render_fwd_quads_kernel(RenderArgs a) {
 // (which strips are live) is, one lane per splat, and so are the linear forms
 // of the sums; the ninth sum waits for three others'.  The background is the
 // colour behind the last splat rather than a term of its own.  Before and now:
-// sixteen uneven views of 3 M Gaussians 6.96 and 4.87 ms, eight 800x800 views
-// of 1 M 462 and 375 us.
+// sixteen uneven views of 3 M Gaussians 6.96 and 4.82 ms, eight 800x800 views
+// of 1 M 462 and 370 us.
 //
 // SEGS: the work-groups below a.seg.cap each take one kept segment of a tile's
 // list (see Segments), the others the rest of a tile's list.
