@@ -234,25 +234,32 @@ __device__ __forceinline__ float row_sums4(const float (*rows)[DMGS_WAVE]) {
 // keeps per channel ch an accumulator acc_ch (colour behind the current splat)
 // and needs only  sum_ch (col_ch - acc_ch) g_ch  (g = dL/dpixel), so one
 // recursion on S = sum_ch acc_ch g_ch replaces three:
-// S <- S + alpha (<col, g> - S).  The background is the colour behind the
-// last splat: S starts from <bg, g>, and the reference's separate term
-// -T_final <bg, g> / (1 - alpha) is part of S.
+// S <- (1 - alpha) S + alpha <col, g>.  The background stays out of S: its
+// share of dL/dalpha is -T_final <bg, g> / (1 - alpha), one multiply-add from
+// a per-pixel constant, whose rounding does not grow along the list (as the
+// start of S, <bg, g> is rounded once per splat in front).
 struct BwdPixel {
   float T;  // transmittance in front of the splat last processed
-  float S;  // sum_ch acc_ch g_ch behind the next one, the background included
+  float S;  // sum_ch acc_ch g_ch behind the next one
 };
 
 // One contributing splat (alpha, colour col) at a pixel with dL/dpixel =
 // (g0, g1, g2): updates the state and returns dL/dalpha; w = alpha T is
-// dL/dcolour_ch / g_ch.
+// dL/dcolour_ch / g_ch.  The rounding sequence is fixed: gradients of scales
+// and rotations are small differences of these values' sums, so another
+// sequence of equal accuracy moves single elements by up to 1e-3 of their rms
+// (S + alpha (<col, g> - S), one instruction less, and the background in S:
+// 4e-7 of the gradients' norm, a repeated run 1e-7).
 __device__ __forceinline__ float bwd_step(BwdPixel& st, float alpha, const float4& col, float g0, float g1,
-                                          float g2, float& w) {
-  const float inv = __builtin_amdgcn_rcpf(1.f - alpha);  // T before this splat = T / (1 - alpha)
+                                          float g2, float bg_term, float& w) {
+  const float om = 1.f - alpha;
+  const float inv = __builtin_amdgcn_rcpf(om);  // T before this splat = T / (1 - alpha)
   st.T *= inv;
   w = alpha * st.T;
-  const float d = fmaf(col.z, g2, fmaf(col.y, g1, col.x * g0)) - st.S;
-  st.S = fmaf(alpha, d, st.S);
-  return d * st.T;
+  const float cg = fmaf(col.z, g2, fmaf(col.y, g1, col.x * g0));
+  const float d = cg - st.S;
+  st.S = fmaf(om, st.S, __fmul_rn(alpha, cg));
+  return fmaf(bg_term, inv, __fmul_rn(d, st.T));
 }
 
 // Gradients through G = exp(power), with t = dL/dG G = o G dL/dalpha (the
@@ -260,9 +267,9 @@ __device__ __forceinline__ float bwd_step(BwdPixel& st, float alpha, const float
 // -t (b dx + c dy), dL/d(a, b, c) = -t (dx^2, dx dy, dy^2) / 2, dL/do =
 // t / o.  From the scaled conic q = log2(e) (-a/2, -b, -c/2):
 // -(a X + b Y) = ln 2 (2 q.x X + q.y Y) and -(b X + c Y) = ln 2 (q.y X + 2 q.z Y).
-// The kernel sums, per splat, X = t dx, Y = t dy, t dx^2, t dx dy, t dy^2, t
-// and w g_ch over the pixels; the linear forms of X, Y and t are applied once
-// per splat and tile, the constant factors in the flush.
+// The kernel sums, per splat, (2 q.x X + q.y Y, q.y X + 2 q.z Y, t dx^2,
+// t dx dy, t dy^2, t / o, w g_ch) with X = t dx, Y = t dy over the pixels; the
+// flush applies the constant factors.
 __device__ __forceinline__ float grad_scale(int k, float ddelx_dx, float ddely_dy) {
   constexpr float kLn2 = 0.693147180559945309f;
   return k == 0 ? kLn2 * ddelx_dx : (k == 1 ? kLn2 * ddely_dy : (k < 5 ? -0.5f : 1.0f));
@@ -822,13 +829,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
 // (tile, splat) pays for one wave reduction instead of four.
 //
 // Bound by the instructions of its waves, vector and scalar, at five waves per
-// SIMD (91 registers; six spill, and four take 24 % longer): so a batch is
+// SIMD (95 registers; six spill, and four take 24 % longer): so a batch is
 // filled before it is walked, what can be decided for 64 staged splats at once
-// (which strips are live) is, one lane per splat, and so are the linear forms
-// of the sums; the ninth sum waits for three others'.  The background is the
-// colour behind the last splat rather than a term of its own.  Before and now:
-// sixteen uneven views of 3 M Gaussians 6.96 and 4.82 ms, eight 800x800 views
-// of 1 M 462 and 370 us.
+// (which strips are live) is, one lane per splat, and the ninth sum waits for
+// three others'.  Before and now: sixteen uneven views of 3 M Gaussians 6.96
+// and 5.29 ms, eight 800x800 views of 1 M 462 and 434 us (5.06 ms and 407 us
+// with the background in the recursion and the linear forms after the sums,
+// whose gradients differ, see bwd_step).
 //
 // SEGS: the work-groups below a.seg.cap each take one kept segment of a tile's
 // list (see Segments), the others the rest of a tile's list.
@@ -873,7 +880,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
 #pragma unroll
   for (int k = 0; k < 4; ++k) pyf[k] = (float)(c.py + 4 * k);
 
-  float g0[4], g1[4], g2[4];
+  float g0[4], g1[4], g2[4], bg_term[4];
   BwdPixel st[4];
   uint32_t last_contributor[4];
   uint32_t m = 0;
@@ -894,12 +901,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
       g1[k] = dp[c.plane + pid];
       g2[k] = dp[2 * c.plane + pid];
     }
-    st[k] = {T_final, c.bg0 * g0[k] + c.bg1 * g1[k] + c.bg2 * g2[k]};
+    bg_term[k] = -T_final * (c.bg0 * g0[k] + c.bg1 * g1[k] + c.bg2 * g2[k]);
+    st[k] = {T_final, 0.f};
     if constexpr (SEGS) {
       if (seg_end != kNoSegment) {  // start from the state at hi: T, and the colour behind it
         const float4 e = a.seg.state[(size_t)seg_end * 256 + threadIdx.x + 64 * k];
         st[k].T = e.x;
-        st[k].S = (e.y * g0[k] + e.z * g1[k] + e.w * g2[k] + T_final * st[k].S) / e.x;
+        st[k].S = (e.y * g0[k] + e.z * g1[k] + e.w * g2[k]) / e.x;
       }
     }
   }
@@ -994,7 +1002,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
           if (contributor < last_contributor[k] && p <= 0.0f && alpha >= 1.0f / 255.0f) {
             any = true;
             float w;
-            const float t = ga * bwd_step(st[k], alpha, col, g0[k], g1[k], g2[k], w);
+            const float t = ga * bwd_step(st[k], alpha, col, g0[k], g1[k], g2[k], bg_term[k], w);
             c0 = fmaf(w, g0[k], c0);
             c1 = fmaf(w, g1[k], c1);
             c2 = fmaf(w, g2[k], c2);
@@ -1006,7 +1014,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         }
         if (__ballot(any) == 0) continue;
         const float s_tdx = s_t * dx;
-        const float v[8] = {s_tdx, s_tdy, s_tdx * dx, s_tdy * dx, s_tdy2, s_t, c0, c1};
+        // the linear forms before the sums over the lanes: X and Y of a long splat cancel in them
+        const float v[8] = {dmean_x(q, s_tdx, s_tdy), dmean_y(q, s_tdx, s_tdy), s_tdx * dx, s_tdy * dx, s_tdy2,
+                            s_t * __builtin_amdgcn_rcpf(q.w), c0, c1};
         int at = (buf * SET + slot) * DMGS_GACC_USED;
         asm("" : "+s"(at));  // a scalar product, not a 64-bit one per lane
         wave_sums8(v, s_red, wsum, &s_acc[0][0][0] + at);
@@ -1016,16 +1026,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
         if (++ninths == 4u) sum_ninths();
       }
       if (ninths) sum_ninths();
-      __syncthreads();
-      // what is linear in the sums is left to one lane per splat
-      if (lane < SET && ((summed >> lane) & 1u)) {
-        const float4 q = L.qo[j0 + (int)lane];
-        float* const acc = s_acc[buf][lane];
-        const float X = acc[0], Y = acc[1];
-        acc[0] = dmean_x(q, X, Y);
-        acc[1] = dmean_y(q, X, Y);
-        acc[5] *= __builtin_amdgcn_rcpf(q.w);
-      }
       __syncthreads();
     }
   }
