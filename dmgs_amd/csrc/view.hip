@@ -9,11 +9,14 @@
 //   * SH coefficients may come as two tensors, (P, 1, 3) and (P, M - 1, 3).  A row of the second is 180 bytes
 //     at degree 3, which no aligned vector load fits, so a work-group copies its 256 rows through LDS with
 //     16-byte accesses and its lanes read them there (odd row strides: no bank conflicts).
-// The math is the single-view kernels' (gs_math.h).  The forward's is written out with every fused
-// multiply-add named and contraction off, in the order the compiler gives preprocess_fwd_kernel: which of two
-// products it fuses depends on the surrounding code, and a last-bit difference in a covariance changes a few
-// radii in a million Gaussians and the pixels that sit on a blend threshold.  So this route's radii and images
-// equal the per-tile-list route's bit for bit, whatever surrounds the arithmetic.
+// The math is the single-view kernels' (gs_math.h), written out with every fused multiply-add named and
+// contraction off, in the order the compiler gives preprocess_fwd_kernel and geometry_bwd_kernel: which of two
+// products it fuses depends on the surrounding code.  A last-bit difference in a covariance changes a few radii in a
+// million Gaussians and the pixels that sit on a blend threshold, and the gradients of long splats are differences
+// that magnify one (4e-6 to 1e-3 of the scale and rotation gradients' norm between two choices).  So this route's
+// radii and images equal the per-tile-list route's bit for bit, and its gradients those of the same blend sums,
+// through torch's activations where the kernels activate.  (The SH gradient is gs_math.h's in both; the tests
+// compare it too.)
 #include "dmgs_common.h"
 #include "dmgs_kernels.h"
 #include "gs_math.h"
@@ -83,10 +86,19 @@ struct LdsRows {
 
 __device__ __forceinline__ float view_sigmoid(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-// torch.nn.functional.normalize of a row of four: the norm's pairwise sum without contraction, clamped
+// torch.nn.functional.normalize of a row of four, x / max(norm, 1e-12): the norm's pairwise sum without contraction
+constexpr float kNormEps = 1e-12f;
 __device__ __forceinline__ float quat_norm(float4 q) {
 #pragma clang fp contract(off)
-  return fmaxf(sqrtf((q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w)), 1e-12f);
+  return sqrtf((q.x * q.x + q.y * q.y) + (q.z * q.z + q.w * q.w));
+}
+// Its gradient, rounded as torch's operations round it: dq / n, and through the norm, whose own gradient is the
+// pairwise sum of -dq (q / n) (q the normalised row).
+__device__ __forceinline__ float4 quat_norm_backward(float4 q, float norm, float4 dq) {
+#pragma clang fp contract(off)
+  const float n = fmaxf(norm, kNormEps);
+  const float dn = norm >= kNormEps ? (-dq.x * (q.x / n) + -dq.y * (q.y / n)) + (-dq.z * (q.z / n) + -dq.w * (q.w / n)) : 0.f;
+  return make_float4(dq.x / n + dn * q.x, dq.y / n + dn * q.y, dq.z / n + dn * q.z, dq.w / n + dn * q.w);
 }
 
 // One Gaussian's SH coefficients: the first three from registers, the others from its LDS row.
@@ -183,6 +195,119 @@ __device__ __forceinline__ bool view_project(float3 p, const float (&c)[6], cons
   return true;
 }
 
+// ewa_backward of gs_math.h as geometry_bwd_kernel has it: dL/dSigma in dc, dL/dmean returned.
+__device__ __forceinline__ float3 view_ewa_backward(float3 p, const float (&c)[6], const ViewParams& v, float dmx,
+                                                    float dmy, float dqa, float dqb, float dqc, float (&dc)[6]) {
+#pragma clang fp contract(off)
+  const float* vm = v.vm;
+  const float* pm = v.pm;
+  const float tz = fmaf(vm[10], p.z, fmaf(vm[2], p.x, vm[6] * p.y)) + vm[14];
+  const float tx0 = fmaf(vm[8], p.z, fmaf(vm[0], p.x, vm[4] * p.y)) + vm[12];
+  const float ty0 = fmaf(vm[9], p.z, fmaf(vm[1], p.x, vm[5] * p.y)) + vm[13];
+  const float limx = 1.3f * v.tanx, limy = 1.3f * v.tany;
+  const float txtz = tx0 / tz, tytz = ty0 / tz;
+  const float tx = tz * fminf(limx, fmaxf(-limx, txtz)), ty = tz * fminf(limy, fmaxf(-limy, tytz));
+  const float xmul = (txtz < -limx || txtz > limx) ? 0.f : 1.f;
+  const float ymul = (tytz < -limy || tytz > limy) ? 0.f : 1.f;
+  const float iz = __builtin_amdgcn_rcpf(tz), iz2 = iz * iz, iz3 = iz * iz2;
+  const float fx = v.fx, fy = v.fy;
+  const float j00 = fx * iz, j02 = iz2 * (fx * -tx), j11 = fy * iz, j12 = iz2 * (fy * -ty);
+  const float V0[3] = {vm[0], vm[4], vm[8]}, V1[3] = {vm[1], vm[5], vm[9]}, V2[3] = {vm[2], vm[6], vm[10]};
+  float m0[3], m1[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    m0[k] = fmaf(V0[k], j00, V2[k] * j02);
+    m1[k] = fmaf(V1[k], j11, V2[k] * j12);
+  }
+  float S0[3], S1[3];  // Sigma m0, Sigma m1
+  S0[0] = fmaf(c[2], m0[2], fmaf(c[0], m0[0], c[1] * m0[1]));
+  S0[1] = fmaf(c[4], m0[2], fmaf(c[1], m0[0], c[3] * m0[1]));
+  S0[2] = fmaf(c[5], m0[2], fmaf(c[2], m0[0], c[4] * m0[1]));
+  S1[0] = fmaf(c[2], m1[2], fmaf(c[0], m1[0], c[1] * m1[1]));
+  S1[1] = fmaf(c[4], m1[2], fmaf(c[1], m1[0], c[3] * m1[1]));
+  S1[2] = fmaf(c[5], m1[2], fmaf(c[2], m1[0], c[4] * m1[1]));
+  const float ca = fmaf(m0[2], S0[2], fmaf(m0[0], S0[0], m0[1] * S0[1])) + 0.3f;
+  const float cb = fmaf(m1[2], S0[2], fmaf(m1[0], S0[0], m1[1] * S0[1]));
+  const float cc = fmaf(m1[2], S1[2], fmaf(m1[0], S1[0], m1[1] * S1[1])) + 0.3f;
+  // conic -> cov2D
+  const float ac = ca * cc, denom = fmaf(-cb, cb, ac);
+  const float d2inv = __builtin_amdgcn_rcpf(fmaf(denom, denom, 0.0000001f));
+  float dLa = 0.f, dLb = 0.f, dLc = 0.f;
+  if (d2inv != 0.f) {
+    const float cb2 = cb + cb, e = denom - ac;
+    dLa = d2inv * fmaf(dqc, e, fmaf(dqb, cb2 * cc, -(dqa * (cc * cc))));
+    dLc = d2inv * fmaf(dqa, e, fmaf(dqb, cb * (ca + ca), -(dqc * (ca * ca))));
+    dLb = (d2inv + d2inv) * fmaf(dqc, cb * ca, fmaf(dqa, cb * cc, -(dqb * fmaf(cb, cb2, denom))));
+  }
+  // cov2D -> cov3D (6-vector)
+  const float dLa2 = dLa + dLa, dLc2 = dLc + dLc;
+  auto square = [&](int k) { return fmaf(m1[k], m1[k] * dLc, fmaf(m1[k], m0[k] * dLb, m0[k] * (m0[k] * dLa))); };
+  auto mixed = [&](int i, int j) {
+    return fmaf(m1[j], m1[i] * dLc2, fmaf(fmaf(m1[j], m0[i], m1[i] * m0[j]), dLb, m0[j] * (m0[i] * dLa2)));
+  };
+  dc[0] = square(0);
+  dc[1] = mixed(0, 1);
+  dc[2] = mixed(0, 2);
+  dc[3] = square(1);
+  dc[4] = mixed(1, 2);
+  dc[5] = square(2);
+  // cov2D -> J -> t -> mean
+  float dm0[3], dm1[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    dm0[k] = fmaf(S1[k], dLb, S0[k] * dLa2);
+    dm1[k] = fmaf(S1[k], dLc2, S0[k] * dLb);
+  }
+  auto along = [](const float (&V)[3], const float (&d)[3]) { return fmaf(V[2], d[2], fmaf(V[0], d[0], V[1] * d[1])); };
+  const float dj00 = along(V0, dm0), dj02 = along(V2, dm0), dj11 = along(V1, dm1), dj12 = along(V2, dm1);
+  const float dtx = iz2 * (xmul * -fx) * dj02, dty = iz2 * (ymul * -fy) * dj12;
+  const float dtz = fmaf(iz3 * ((fy + fy) * ty), dj12,
+                         fmaf(iz3 * ((fx + fx) * tx), dj02, fmaf(iz2 * -fx, dj00, -((fy * iz2) * dj11))));
+  // projection (means2D gradient is in NDC)
+  const float phw = fmaf(pm[11], p.z, fmaf(pm[3], p.x, pm[7] * p.y)) + pm[15];
+  const float phx = fmaf(pm[8], p.z, fmaf(pm[0], p.x, pm[4] * p.y)) + pm[12];
+  const float phy = fmaf(pm[9], p.z, fmaf(pm[1], p.x, pm[5] * p.y)) + pm[13];
+  const float mw = __builtin_amdgcn_rcpf(phw + 0.0000001f);
+  const float mul1 = mw * (phx * mw), mul2 = mw * (phy * mw);
+  auto mean = [&](int k) {
+    return fmaf(dmx, fmaf(pm[4 * k], mw, -(pm[4 * k + 3] * mul1)),
+                dmy * fmaf(pm[4 * k + 1], mw, -(pm[4 * k + 3] * mul2))) +
+           fmaf(vm[4 * k + 2], dtz, fmaf(vm[4 * k + 1], dty, vm[4 * k] * dtx));
+  };
+  return make_float3(mean(0), mean(1), mean(2));
+}
+
+// cov3d_backward of gs_math.h, likewise.
+__device__ __forceinline__ void view_cov3d_backward(const float (&dc)[6], float3 s3, const float (&R)[9], float4 q,
+                                                    float3& ds, float4& dq) {
+#pragma clang fp contract(off)
+  // dL/dM = 2 G M, M = R diag(s); off the diagonal G has half of dc
+  const float G01 = 0.5f * dc[1], G02 = 0.5f * dc[2], G12 = 0.5f * dc[4];
+  const float sv[3] = {s3.x, s3.y, s3.z};
+  float d[3], g[9];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const float two_s = sv[j] + sv[j], R0 = R[j], R1 = R[3 + j], R2 = R[6 + j];
+    const float dM0 = two_s * fmaf(R2, G02, fmaf(R0, dc[0], R1 * G01));
+    const float dM1 = two_s * fmaf(R2, G12, fmaf(R1, dc[3], R0 * G01));
+    const float dM2 = two_s * fmaf(R2, dc[5], fmaf(R0, G02, R1 * G12));
+    d[j] = fmaf(R2, dM2, fmaf(R0, dM0, R1 * dM1));
+    g[j] = sv[j] * dM0;
+    g[3 + j] = sv[j] * dM1;
+    g[6 + j] = sv[j] * dM2;
+  }
+  ds = make_float3(d[0], d[1], d[2]);
+  const float r = q.x, x = q.y, y = q.z, z = q.w, x2 = x + x, y2 = y + y, z2 = z + z;
+  const float dr = fmaf(x, g[7], fmaf(-y, g[6], fmaf(-x, g[5], fmaf(z, g[3], fmaf(y, g[2], -(z * g[1]))))));
+  const float dx = fmaf(-x2, g[8], fmaf(r, g[7], fmaf(z, g[6], fmaf(-r, g[5],
+                        fmaf(-x2, g[4], fmaf(y, g[3], fmaf(y, g[1], z * g[2])))))));
+  const float dy = fmaf(-y2, g[8], fmaf(z, g[7], fmaf(-r, g[6], fmaf(z, g[5],
+                        fmaf(x, g[3], fmaf(r, g[2], fmaf(x, g[1], -(y2 * g[0]))))))));
+  const float dz = fmaf(y, g[7], fmaf(x, g[6], fmaf(y, g[5], fmaf(-z2, g[4],
+                        fmaf(r, g[3], fmaf(x, g[2], fmaf(-z2, g[0], -(r * g[1]))))))));
+  dq = make_float4(dr + dr, dx + dx, dy + dy, dz + dz);
+}
+
 // The SH sum of sh_to_rgb (gs_math.h) in the view direction.
 template <typename SH>
 __device__ __forceinline__ float3 view_sh(int deg, const SH& sh, float3 p, const float (&campos)[3]) {
@@ -243,7 +368,8 @@ __device__ __forceinline__ void make_shape(const ViewArgs& a, ViewGaussian& G) {
   G.qn = 1.0f;
   if (a.raw & DMGS_RAW_ROTATIONS) {
     G.qn = quat_norm(G.q);
-    G.q = make_float4(G.q.x / G.qn, G.q.y / G.qn, G.q.z / G.qn, G.q.w / G.qn);
+    const float n = fmaxf(G.qn, kNormEps);
+    G.q = make_float4(G.q.x / n, G.q.y / n, G.q.z / n, G.q.w / n);
   }
   view_cov3d(G);
 }
@@ -379,21 +505,18 @@ __global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
     ViewGaussian G;
     load_shape(a, g, G);
     make_shape(a, G);
-    dmean = ewa_backward(p, G.c3, v, r0.x, r0.y, r1.x, r1.y, r2.x, dc);
+    dmean = view_ewa_backward(p, G.c3, v, r0.x, r0.y, r1.x, r1.y, r2.x, dc);
     if (!a.cov3D_precomp) {
-      cov3d_backward(dc, G.s, G.R, G.q, ds, dq);
+      view_cov3d_backward(dc, G.s, G.R, G.q, ds, dq);
       if (a.raw & DMGS_RAW_SCALES)  // scale = exp(log-scale)
         ds = make_float3(ds.x * G.e.x, ds.y * G.e.y, ds.z * G.e.z);
-      if (a.raw & DMGS_RAW_ROTATIONS) {  // q = raw / max(|raw|, 1e-12)
-        const float qd = G.qn > 1e-12f ? G.q.x * dq.x + G.q.y * dq.y + G.q.z * dq.z + G.q.w * dq.w : 0.f;
-        dq = make_float4((dq.x - G.q.x * qd) / G.qn, (dq.y - G.q.y * qd) / G.qn, (dq.z - G.q.z * qd) / G.qn,
-                         (dq.w - G.q.w * qd) / G.qn);
-      }
+      if (a.raw & DMGS_RAW_ROTATIONS) dq = quat_norm_backward(G.q, G.qn, dq);
     }
   }
   if constexpr (M != 0) {
     float b[16];
-    float3 gm = make_float3(0.f, 0.f, 0.f), dd = gm;
+    float3 gm = make_float3(0.f, 0.f, 0.f);
+    auto add = [&](float3 d) { dmean = make_float3(dmean.x + d.x, dmean.y + d.y, dmean.z + d.z); };
 #pragma unroll
     for (int k = 0; k < 16; ++k) b[k] = 0.f;
     if constexpr (M > 0) {
@@ -402,9 +525,9 @@ __global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
       if (vis) {
         if constexpr (SPLIT) {
           const float c0[3] = {a.shs[3 * i], a.shs[3 * i + 1], a.shs[3 * i + 2]};
-          dd = sh_backward(a.sh_degree, ShSplit{c0, row, R}, p, v.campos, dcol, b, gm);
+          add(sh_backward(a.sh_degree, ShSplit{c0, row, R}, p, v.campos, dcol, b, gm));
         } else {
-          dd = sh_backward(a.sh_degree, ShRow{row, R}, p, v.campos, dcol, b, gm);
+          add(sh_backward(a.sh_degree, ShRow{row, R}, p, v.campos, dcol, b, gm));
         }
       }
       // the lane's row becomes its gradient
@@ -426,7 +549,7 @@ __global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
       if (vis) {
         float sh[48];
         load_sh16(a.shs + i * 3 * a.sh_coeffs, a.sh_coeffs, sh);
-        dd = sh_backward(a.sh_degree, sh, p, v.campos, dcol, b, gm);
+        add(sh_backward(a.sh_degree, sh, p, v.campos, dcol, b, gm));
       }
       float* d = a.dL_dsh + i * 3 * a.sh_coeffs;
       for (int k = 0; k < a.sh_coeffs; ++k) {
@@ -438,7 +561,6 @@ __global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
         d[3 * k + 2] = bk * gm.z;
       }
     }
-    dmean = make_float3(dmean.x + dd.x, dmean.y + dd.y, dmean.z + dd.z);
   }
   if (!live) return;
   auto put3 = [&](float* o, float x, float y, float z) {
@@ -451,7 +573,7 @@ __global__ __launch_bounds__(kRows) void view_geometry_bwd_kernel(ViewArgs a) {
   float dop = r2.y;
   if (a.raw & DMGS_RAW_OPACITIES) {
     const float o = view_sigmoid(a.opacities[i]);
-    dop *= o * (1.0f - o);
+    dop = dop * (1.0f - o) * o;
   }
   a.dL_dopacity[i] = dop;
   if (a.dL_dcolors) put3(a.dL_dcolors, dcol.x, dcol.y, dcol.z);
