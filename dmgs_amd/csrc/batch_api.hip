@@ -122,6 +122,9 @@ struct ListLayout {
   }
 };
 
+// A splat's tile rectangle holds 16 bits per edge, the exclusive upper one included (pack_rect): 65535 tiles a side.
+bool tiles_fit_rect(int32_t W, int32_t H) { return W <= 0xFFFF * DMGS_BLOCK_X && H <= 0xFFFF * DMGS_BLOCK_Y; }
+
 int check_batch(const dmgs_batch* b) {
   if (!b) return bfail(DMGS_EINVAL, "batch is null");
   if (b->num_views <= 0 || b->num_gaussians <= 0 || (int64_t)b->num_views * b->num_gaussians > (int64_t)0x7fffffff)
@@ -334,7 +337,7 @@ struct ViewLayout {
   static int cells_along(int tiles) { return (tiles + (1 << DMGS_CELL_SHIFT) - 1) >> DMGS_CELL_SHIFT; }
 };
 bool view_has_cells(int32_t W, int32_t H) {
-  if (W <= 0 || H <= 0 || (int64_t)W * H > (int64_t)1 << 30) return false;
+  if (W <= 0 || H <= 0 || (int64_t)W * H > (int64_t)1 << 30 || !tiles_fit_rect(W, H)) return false;
   const int64_t cx = ViewLayout::cells_along((W + DMGS_BLOCK_X - 1) / DMGS_BLOCK_X);
   const int64_t cy = ViewLayout::cells_along((H + DMGS_BLOCK_Y - 1) / DMGS_BLOCK_Y);
   return cx * cy <= 1 << DMGS_CELL_KEY_BITS;
@@ -393,7 +396,8 @@ int check_gaussians(const dmgs_settings* s, const dmgs_gaussians* g, const void*
                                   g->rotations, g->cov3D_precomp);
   if (rc) return rc;
   if (g->count <= 0) return bfail(DMGS_EINVAL, "no Gaussians");
-  if (!view_has_cells(s->image_width, s->image_height)) return bfail(DMGS_EINVAL, "more than 65536 cells");
+  if (!view_has_cells(s->image_width, s->image_height))
+    return bfail(DMGS_EINVAL, "more than 65536 cells, or 65535 tiles a side");
   if (g->raw & ~7) return bfail(DMGS_EINVAL, "invalid raw mask %d", g->raw);
   if (g->shs_rest && (!g->shs || (s->sh_coeffs != 4 && s->sh_coeffs != 9 && s->sh_coeffs != 16)))
     return bfail(DMGS_EINVAL, "shs_rest needs shs and 4, 9 or 16 coefficients");
@@ -417,6 +421,7 @@ int dmgs_batched_prepare_views(dmgs_view* views, int32_t B, int32_t* total_tiles
     dmgs_view& d = views[v];
     if (d.width <= 0 || d.height <= 0 || !(d.tanfovx > 0.f) || !(d.tanfovy > 0.f))
       return bfail(DMGS_EINVAL, "view %d: invalid size or field of view", v);
+    if (!tiles_fit_rect(d.width, d.height)) return bfail(DMGS_EINVAL, "view %d: more than 65535 tiles a side", v);
     d.focal_x = (float)d.width / (2.0f * d.tanfovx);
     d.focal_y = (float)d.height / (2.0f * d.tanfovy);
     d.grid_x = (d.width + DMGS_BLOCK_X - 1) / DMGS_BLOCK_X;

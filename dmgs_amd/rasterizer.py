@@ -22,8 +22,8 @@ All compute runs in the gfx950 HIP library through ``dmgs_amd._native``.  An
 image takes the cell-list route (``view_forward``: the batched engine's lists
 and blend with one view); ``forward_raw`` / ``backward_raw`` are the route of
 the reference's per-tile lists, taken with ``debug`` (every kernel
-synchronised), for images of more than 65536 cells of 64x64 pixels, and by
-callers that want those lists.  Both give the same image bit for bit.
+synchronised), for images of more than 65536 cells of 64x64 pixels or 65535
+tiles a side, and by callers that want those lists.  Both give the same image bit for bit.
 """
 import ctypes
 from typing import NamedTuple

@@ -433,7 +433,7 @@ typedef struct dmgs_gaussian_grads { /* shaped like the inputs; colors, cov3D, s
   float* scales;
   float* rotations;
 } dmgs_gaussian_grads;
-/* Whether an image size has lists here (at most 65536 cells of 64x64 pixels). */
+/* Whether an image size has lists here (at most 65536 cells of 64x64 pixels and 65535 tiles of 16x16 a side). */
 int dmgs_view_supported(int32_t width, int32_t height);
 /* keep: a backward will follow (the same value in every call of one image). */
 size_t dmgs_view_state_size(int64_t P, int32_t width, int32_t height, int32_t keep);
