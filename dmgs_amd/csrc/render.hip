@@ -51,6 +51,8 @@ struct StagedSplat {
   float r, g, b;
   uint32_t pos, mask, id;  // list position, reach mask (reach_mask), splat id
 };
+// In a forward mask: the colour is not finite (see render_fwd_quads_kernel).
+constexpr uint32_t kOddColor = 16u;
 template <int SLOTS>
 struct FwdSplats {
   float4 xyq[SLOTS];   // x, y, q.x, q.y
@@ -59,7 +61,8 @@ struct FwdSplats {
   __device__ __forceinline__ void put(int j, const StagedSplat& s) {
     xyq[j] = make_float4(s.x, s.y, s.qx, s.qy);
     qorg[j] = make_float4(s.qz, s.o, s.r, s.g);
-    bpmi[j] = make_float4(s.b, __uint_as_float(s.pos), __uint_as_float(s.mask), __uint_as_float(s.id));
+    const bool odd = s.r * 0.f + s.g * 0.f + s.b * 0.f != 0.f;  // NaN unless all three are finite
+    bpmi[j] = make_float4(s.b, __uint_as_float(s.pos), __uint_as_float(s.mask | (odd ? kOddColor : 0u)), __uint_as_float(s.id));
   }
   __device__ __forceinline__ uint32_t mask(int j) const { return __float_as_uint(bpmi[j].z); }
   __device__ __forceinline__ uint32_t pos(int j) const { return __float_as_uint(bpmi[j].y); }
@@ -488,7 +491,7 @@ struct MemberList {
 // red and green, the other blue.  16 instructions a splat, in twice as many waves, with the same operations in the
 // same order on every value.  (Eight waves of one work-group share a CU's SIMDs and gain nothing.)
 // Five waves per SIMD where one work-group blends a tile and keeps nothing: the compiler takes 106 registers (four
-// waves) if left alone and 96 without a spill if asked; 16 uneven views 3.34 -> 2.99 ms, 8 views of 800x800 312 -> 294 us,
+// waves) if left alone and 96 if asked (one spilled in the path for odd colours); 16 uneven views 3.34 -> 2.99 ms, 8 views of 800x800 312 -> 294 us,
 // 1920x1080 134 -> 125 us.  Six waves spill 48 bytes (8 views of 800x800 330 us); with kept segments five spill 24
 // (a 10k view 57 -> 59 us, 82k faces 249 -> 255); two work-groups a tile have few waves in flight at any register count.
 template <bool CELLS, bool KEEP, bool SPLIT>
@@ -648,14 +651,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
       // and for the two groups read ahead
       uint32_t* const reach = s_reach[wave];
       int count = 0;
+      uint64_t odd = 0;
 #pragma unroll
       for (int k = 0; k < G; k += 64) {
         const int s = h + k + lane;
-        const uint64_t bits = __ballot(s < n && ((L.mask(min(s, NT)) >> wave) & 1u));
+        const uint32_t mask = L.mask(min(s, NT));
+        const bool reached = s < n && ((mask >> wave) & 1u);
+        const uint64_t bits = __ballot(reached);
+        odd |= __ballot(reached && (mask & kOddColor));
         if ((bits >> lane) & 1u) reach[count + (int)__popcll(bits & lanemask_lt())] = (uint32_t)s * 16u;
         count += (int)__popcll(bits);
       }
       if (count == 0) continue;
+      if (odd != 0) {
+        // The groups below add skipped splats with weight zero, which a colour that is not finite would turn into
+        // NaN in pixels that it does not touch: such a round goes splat by splat, adding only what contributes.
+        for (int i = 0; i < count; ++i) {
+          const uint32_t o = reach[i];
+          const float4 g = lds_at(L.xyq, o), q = lds_at(L.qorg, o), b = lds_at(L.bpmi, o);
+          const float power = power_at(power_dx(g.z, g.w, g.x - pxf), q.x, g.y - pyf);
+          const float alpha = fminf(0.99f, q.y * splat_exp2(power));
+          if (!((power <= 0.0f) & (alpha >= 1.0f / 255.0f) & (T > 0.f))) continue;
+          const float test_T = T * (1.0f - alpha), w = alpha * T;
+          if (test_T >= 0.0001f) {
+            const bool blue = SPLIT && lane >= 32;  // of a pixel's two lanes the one that adds blue, in C0
+            C0 = fmaf(blue ? b.x : q.z, w, C0);
+            C1 = fmaf(q.w, w, C1);
+            C2 = fmaf(b.x, w, C2);
+            if constexpr (KEEP) {
+              D0 = fmaf(q.z, w, D0);
+              D1 = fmaf(q.w, w, D1);
+              D2 = fmaf(b.x, w, D2);
+            }
+            T = test_T;
+            last_contributor = __float_as_uint(b.y);
+          } else {
+            T = -T;
+          }
+        }
+        continue;
+      }
       if (lane < 12) reach[count + lane] = kPad;
       if constexpr (SPLIT) {
         const bool second = lane >= 32;  // of the pixel's two lanes
