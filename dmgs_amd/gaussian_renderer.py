@@ -74,9 +74,11 @@ class _ShSigmoid(torch.autograd.Function):
         feats, xyz, campos, colors = ctx.saved_tensors
         n, _, M = feats.shape
         if torch.is_grad_enabled():  # create_graph: the derivative of the torch ops, itself differentiable
+            asked = [t for t, need in zip((feats, xyz), ctx.needs_input_grad) if need]
             out = _torch_colors(feats, xyz, campos, ctx.degree)
-            grads = torch.autograd.grad(out, (feats, xyz), grad, create_graph=True, allow_unused=True)
-            return grads[0], grads[1], None, None
+            grads = iter(torch.autograd.grad(out, asked, grad, create_graph=True, allow_unused=True)
+                         if out.requires_grad else [None] * len(asked))
+            return tuple(next(grads) if need else None for need in ctx.needs_input_grad[:2]) + (None, None)
         g = grad.to(torch.float32).contiguous()
         dfeats = torch.empty_strided(feats.shape, feats.stride(), dtype=torch.float32, device=feats.device)
         dxyz = torch.empty_like(xyz)
