@@ -16,7 +16,7 @@ import torch
 from . import _native as N
 from .binding import FaceBoundGaussians
 from .rasterizer import (RAW_OPACITIES, RAW_ROTATIONS, RAW_SCALES, GaussianRasterizationSettings, GaussianRasterizer,
-                         _cells_route, model_inputs_fit, rasterize_model)
+                         _cells_route, _f32, model_inputs_fit, rasterize_model)
 from .scenes import FreeGaussians
 from .sh_utils import eval_sh
 
@@ -60,13 +60,12 @@ class _ShSigmoid(torch.autograd.Function):
     @staticmethod
     def forward(ctx, feats, xyz, campos, degree):
         n, _, M = feats.shape
-        color_major = int(feats.stride(2) == 1)
         colors = torch.empty(n, 3, dtype=torch.float32, device=xyz.device)
-        N.check(N.load().dmgs_sh_sigmoid(n, M, degree, color_major, N.ptr(feats), N.ptr(xyz), N.ptr(campos),
-                                         N.ptr(colors), None, None, None, N.stream_handle(xyz.device)),
+        N.check(N.load().dmgs_sh_sigmoid(n, M, degree, int(feats.stride(2) == 1), N.ptr(feats), N.ptr(xyz),
+                                         N.ptr(campos), N.ptr(colors), None, None, None, N.stream_handle(xyz.device)),
                 "dmgs_sh_sigmoid")
         ctx.save_for_backward(feats, xyz, campos, colors)
-        ctx.degree, ctx.color_major = degree, color_major
+        ctx.degree = degree
         return colors
 
     @staticmethod
@@ -79,11 +78,14 @@ class _ShSigmoid(torch.autograd.Function):
             grads = iter(torch.autograd.grad(out, asked, grad, create_graph=True, allow_unused=True)
                          if out.requires_grad else [None] * len(asked))
             return tuple(next(grads) if need else None for need in ctx.needs_input_grad[:2]) + (None, None)
-        g = grad.to(torch.float32).contiguous()
+        # saved-tensor hooks may give the tensors back in another layout or type
+        xyz, campos, colors, g = (_f32(t, xyz.device) for t in (xyz, campos, colors, grad))
+        if not _sh_kernel_fits(feats, xyz, ctx.degree):
+            feats = _f32(feats, xyz.device)
         dfeats = torch.empty_strided(feats.shape, feats.stride(), dtype=torch.float32, device=feats.device)
         dxyz = torch.empty_like(xyz)
-        N.check(N.load().dmgs_sh_sigmoid(n, M, ctx.degree, ctx.color_major, N.ptr(feats), N.ptr(xyz), N.ptr(campos),
-                                         N.ptr(colors), N.ptr(g), N.ptr(dfeats), N.ptr(dxyz),
+        N.check(N.load().dmgs_sh_sigmoid(n, M, ctx.degree, int(feats.stride(2) == 1), N.ptr(feats), N.ptr(xyz),
+                                         N.ptr(campos), N.ptr(colors), N.ptr(g), N.ptr(dfeats), N.ptr(dxyz),
                                          N.stream_handle(xyz.device)), "dmgs_sh_sigmoid")
         return dfeats, dxyz, None, None
 

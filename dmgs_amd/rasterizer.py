@@ -400,7 +400,8 @@ class _RasterizeModel(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_out_color, _grad_radii):
-        radii, xyz, dc, rest, opacity, scales, rotations = ctx.saved_tensors
+        radii, *saved = ctx.saved_tensors
+        xyz, dc, rest, opacity, scales, rotations = (_f32(x, radii.device) for x in saved)  # hooks may change them
         inputs = (xyz, radii, dc, rest, opacity, scales, rotations)
         needs = ctx.needs_input_grad
         state, ctx.state = ctx.state, None

@@ -15,7 +15,7 @@ def test_create_graph_with_a_frozen_input(needs, degree):
     xyz = torch.randn(5, 3, generator=g, dtype=torch.float64).requires_grad_(needs[1])
     campos = torch.tensor([0.1, 3.0, -0.4], dtype=torch.float64)
     grad = torch.randn(5, 3, generator=g, dtype=torch.float64)
-    ctx = SimpleNamespace(saved_tensors=(feats, xyz, campos, None), degree=degree, color_major=1,
+    ctx = SimpleNamespace(saved_tensors=(feats, xyz, campos, None), degree=degree,
                           needs_input_grad=needs + (False, False))
     got = GR._ShSigmoid.backward(ctx, grad)
     assert got[2:] == (None, None)
