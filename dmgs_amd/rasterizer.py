@@ -261,7 +261,8 @@ def view_forward(t, sh_coeffs, raw, rs, keep):
     with _stage("render_forward"):
         N.check(lib.dmgs_view_blend(s, P, int(keep), K, N.ptr(ws), N.ptr(lists), N.ptr(bws), N.ptr(color), stream),
                 "dmgs_view_blend")
-    return color, radii, dict(frame=fr, ws=ws, lists=lists, bws=bws, cells=K, K=tiles, P=P, M=sh_coeffs, raw=raw)
+    return color, radii, dict(frame=fr, ws=ws, lists=lists, bws=bws, cells=K, K=tiles, P=P, M=sh_coeffs, raw=raw,
+                              walked=False)
 
 
 def view_backward(t, state, radii, grad_color, colors=False, cov3D=False):
@@ -285,6 +286,9 @@ def view_backward(t, state, radii, grad_color, colors=False, cov3D=False):
     stream = N.stream_handle(dev)
     s = ctypes_ref(fr.c)
     with _stage("render_backward"):
+        if state["walked"]:  # the forward left the accumulator cleared for one backward
+            state["bws"][:lib.dmgs_backward_workspace_size(P)].zero_()
+        state["walked"] = True
         N.check(lib.dmgs_view_blend_backward(s, P, state["cells"], N.ptr(state["ws"]), N.ptr(state["lists"]),
                                              N.ptr(state["bws"]), N.ptr(gc), stream), "dmgs_view_blend_backward")
     with _stage("geometry_backward"):
@@ -296,6 +300,23 @@ def view_backward(t, state, radii, grad_color, colors=False, cov3D=False):
 
 def _cells_route(rs):
     return not rs.debug and N.load().dmgs_view_supported(int(rs.image_width), int(rs.image_height)) == 1
+
+
+def _take_state(ctx):
+    """The forward's state, for one backward: kept for another one while the graph is (``retain_graph``), released
+    with it otherwise, so that the workspaces do not live as long as the image does."""
+    if ctx.state is _RELEASED:
+        raise RuntimeError("Trying to backward through a rendered image a second time: specify retain_graph=True for "
+                           "the first")
+    state = ctx.state
+    if not _graph_is_kept():
+        ctx.state = _RELEASED
+    return state
+
+
+_RELEASED = object()
+# torch's own test, as its compiled functions use it; without it nothing is released early
+_graph_is_kept = getattr(torch._C._autograd, "_get_current_graph_task_keep_graph", lambda: True)
 
 
 def _rasterize(ctx, args, keep):
@@ -340,10 +361,10 @@ class _RasterizeGaussians(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out_color, _grad_radii):
         (radii,) = ctx.saved_tensors
-        state = ctx.state
+        state = _take_state(ctx)
         shapes = ctx.shapes
         needs = ctx.needs_input_grad
-        if state is None:
+        if state is None:  # no Gaussians
             z = [None if (s is None or not needs[i]) else torch.zeros(s, device=grad_out_color.device)
                  for i, s in enumerate(shapes)]
             return tuple(z) + (None,)
@@ -369,7 +390,6 @@ class _RasterizeGaussians(torch.autograd.Function):
                 grads.append(None)
             else:
                 grads.append(gr.reshape(s))
-        ctx.state = None
         return tuple(grads) + (None,)
 
 
@@ -402,13 +422,8 @@ class _RasterizeModel(torch.autograd.Function):
     def backward(ctx, grad_out_color, _grad_radii):
         radii, *saved = ctx.saved_tensors
         xyz, dc, rest, opacity, scales, rotations = (_f32(x, radii.device) for x in saved)  # hooks may change them
-        inputs = (xyz, radii, dc, rest, opacity, scales, rotations)
         needs = ctx.needs_input_grad
-        state, ctx.state = ctx.state, None
-        if state is None:  # a second backward through one image, as in _RasterizeGaussians
-            z = [torch.zeros(xyz.shape if i == 1 else x.shape, device=xyz.device) if needs[i] else None
-                 for i, x in enumerate(inputs)]
-            return tuple(z) + (None, None, None)
+        state = _take_state(ctx)
         t = dict(means3D=xyz, opacities=opacity, shs=dc, scales=scales, rotations=rotations)
         if rest.numel():
             t["shs_rest"] = rest
