@@ -401,6 +401,26 @@ class _RasterizeGaussiansNoGrad(torch.autograd.Function):
         return _rasterize(ctx, args, False)
 
 
+def _through_activations(t, state, radii, grad_color):
+    """``view_backward`` of a model's tensors with a graph of its own (create_graph): the rasterizer's gradients,
+    which have none, through torch's activations, which do."""
+    raw = state["raw"]
+    acts = dict(t)
+    if raw & RAW_SCALES:
+        acts["scales"] = torch.exp(t["scales"])
+    if raw & RAW_ROTATIONS:
+        acts["rotations"] = nn.functional.normalize(t["rotations"])
+    if raw & RAW_OPACITIES:
+        acts["opacities"] = torch.sigmoid(t["opacities"])
+    with torch.no_grad():
+        g = view_backward({k: x.detach() for k, x in acts.items()}, dict(state, raw=0), radii, grad_color)
+    state["walked"] = True
+    for k in ("scales", "rotations", "opacities"):
+        if acts[k] is not t[k] and acts[k].requires_grad:
+            g[k], = torch.autograd.grad(acts[k], t[k], g[k], create_graph=True)
+    return g
+
+
 class _RasterizeModel(torch.autograd.Function):
     """A model's own tensors (``raw`` as in ``view_forward``), SH in two
     tensors; gradients reach those tensors directly."""
@@ -427,7 +447,10 @@ class _RasterizeModel(torch.autograd.Function):
         t = dict(means3D=xyz, opacities=opacity, shs=dc, scales=scales, rotations=rotations)
         if rest.numel():
             t["shs_rest"] = rest
-        g = view_backward(t, state, radii, grad_out_color)
+        if torch.is_grad_enabled():
+            g = _through_activations(t, state, radii, grad_out_color)
+        else:
+            g = view_backward(t, state, radii, grad_out_color)
         out = (g["means3D"], g["means2D"], g["shs"], rest.new_zeros(rest.shape) if g["shs_rest"] is None else g["shs_rest"],
                g["opacities"], g["scales"], g["rotations"])
         return tuple(x if n else None for x, n in zip(out, needs)) + (None, None, None)
