@@ -147,16 +147,24 @@ class BatchedRenderer:
         self.state = self.lists = self.bwd_ws = None
         self.dens = None
         self._offsets = None
+        self._state_backward = False  # the state has room for what a forward keeps for its backward
 
     # ---- planning ---------------------------------------------------------
-    def _alloc_state(self):
-        n = self.lib.dmgs_batched_state_size(self.B, self.P, self.total_tiles, self.total_pixels)
+    def _alloc_state(self, backward=True):
+        """The state; without ``backward`` without the list segments that a
+        forward keeps for one.  An existing state's contents are kept."""
+        size = self.lib.dmgs_batched_state_size if backward else self.lib.dmgs_batched_forward_state_size
+        n = size(self.B, self.P, self.total_tiles, self.total_pixels)
         if n == 0:
             raise RuntimeError("dmgs_batched_state_size rejected the batch")
+        old = self.state
         offs = (N.c_size_t * 9)()
         N.check(self.lib.dmgs_batched_offsets(self.B, self.P, self.total_tiles, self.total_pixels, 0, offs),
                 "dmgs_batched_offsets")
         self.state = torch.empty(n, dtype=torch.uint8, device=self.device)
+        if old is not None:
+            self.state[:old.numel()].copy_(old)
+        self._state_backward = backward
         self._offsets = list(offs)
 
     def _after_tables(self):
@@ -168,6 +176,8 @@ class BatchedRenderer:
 
     def _desc(self, capacity=None):
         self._after_tables()
+        if self.bwd_ws is not None and not self._state_backward:  # planned for a forward only before
+            self._alloc_state()
         d = N.DmgsBatch()
         d.views, d.tile_view = self.views_dev.data_ptr(), self.tile_view.data_ptr()
         d.num_views, d.sh_degree, d.num_gaussians = self.B, self.sh_degree, self.P
@@ -185,7 +195,7 @@ class BatchedRenderer:
         """Run preprocess + depth sort + scan only and return the number of
         (Gaussian, tile) instances of the batch (one host read)."""
         if self.state is None:
-            self._alloc_state()
+            self._alloc_state(backward=False)
         self._check_params(params)
         N.check(self.lib.dmgs_batched_forward(ctypes.byref(self._desc(0)), N.ptr(params), None, STAGE_GEOMETRY,
                                               N.stream_handle(self.device)), "dmgs_batched_forward")
@@ -197,7 +207,7 @@ class BatchedRenderer:
         status word (bit 0: see ``depth_clamped``) into ``host_out[1]`` when
         it has two elements; valid once the current stream has reached it."""
         if self.state is None:
-            self._alloc_state()
+            self._alloc_state(backward=False)
         self._check_params(params)
         N.check(self.lib.dmgs_batched_forward(ctypes.byref(self._desc(0)), N.ptr(params), None, STAGE_GEOMETRY,
                                               N.stream_handle(self.device)), "dmgs_batched_forward")
@@ -210,7 +220,7 @@ class BatchedRenderer:
         """Size the instance lists for ``params`` (with headroom) and allocate
         the workspaces.  Returns the capacity."""
         if self.state is None:
-            self._alloc_state()
+            self._alloc_state(backward)
         if K_cap is None:
             K = self.count_instances(params)
             K_cap = max(1024, int(math.ceil(K * self.headroom)))
@@ -220,6 +230,8 @@ class BatchedRenderer:
             self.bwd_ws = torch.empty(self.lib.dmgs_batched_backward_size(self.B, self.P), dtype=torch.uint8,
                                       device=self.device)
             self._acc_clear = False
+        if backward and not self._state_backward:
+            self._alloc_state()
         return self.K_cap
 
     def _require_plan(self):

@@ -98,9 +98,10 @@ struct StateLayout {
     ranges = o; o += align_up(T * 8);
     final_T = o; o += align_up(X * 4);
     n_contrib = o; o += align_up(X * 4);
+    // all that a forward without a backward touches ends here, in either form
+    seg_head = o; o += align_up(8);
     seg_cap = segments && T <= (size_t)dmgs::kSegmentTiles ? (int)std::min<size_t>(16384, std::max<size_t>(1024, N / 16)) : 0;
     tile_last = o; o += align_up(seg_cap ? T * 4 : 0);
-    seg_head = o; o += align_up(8);
     seg_rec = o; o += align_up((size_t)seg_cap * 16);
     seg_state = o; o += (size_t)seg_cap * 256 * 16;
     total = o;
@@ -458,6 +459,11 @@ int dmgs_batched_tile_view(const dmgs_view* views, int32_t B, int32_t* tile_view
 size_t dmgs_batched_state_size(int32_t B, int64_t P, int32_t total_tiles, int64_t total_pixels) {
   if (B <= 0 || P <= 0 || total_tiles <= 0 || total_pixels <= 0) return 0;
   return StateLayout((size_t)B * P, (size_t)total_tiles, (size_t)total_pixels).total;
+}
+
+size_t dmgs_batched_forward_state_size(int32_t B, int64_t P, int32_t total_tiles, int64_t total_pixels) {
+  if (B <= 0 || P <= 0 || total_tiles <= 0 || total_pixels <= 0) return 0;
+  return StateLayout((size_t)B * P, (size_t)total_tiles, (size_t)total_pixels, false).total;
 }
 
 size_t dmgs_batched_lists_size(int64_t capacity) {

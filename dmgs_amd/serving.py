@@ -86,7 +86,7 @@ class _Batch:
                                         sh_degree=sh, scale_modifier=requests[0].scaling_modifier,
                                         device=server.device)
             self.r.variant, self.vkey = server._choose_variant(scene, self.r.total_tiles)
-            self.r._alloc_state()
+            self.r._alloc_state(backward=False)
             self.images = self.r.new_images()
             self.count = torch.empty(2, dtype=torch.int32, pin_memory=True)  # instances, status word
         self.reserved = 0
@@ -169,7 +169,7 @@ class RenderServer:
         lib = BT.N.load()
         tiles = sum(((c.image_width + 15) // 16) * ((c.image_height + 15) // 16) for c in cams)
         pixels = sum(c.image_width * c.image_height for c in cams)
-        return int(lib.dmgs_batched_state_size(len(cams), P, tiles, pixels)) + 12 * pixels, pixels
+        return int(lib.dmgs_batched_forward_state_size(len(cams), P, tiles, pixels)) + 12 * pixels, pixels
 
     def footprint(self, scene, cams):
         """Estimated bytes of a batch (state + images exact, lists from the

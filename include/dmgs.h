@@ -310,8 +310,10 @@ int dmgs_batched_tile_view(const dmgs_view* views, int32_t B, int32_t* tile_view
 /* Workspaces of a batch (device memory, caller-owned):
  *   state   K-independent: per (view, Gaussian) splats, keys, radii, scan;
  *           per-tile ranges; per-pixel blend state; up to 4096 tiles, also
- *           list segments a forward with bwd_ws keeps for its backward.
- *           Kept until backward.
+ *           list segments a forward with bwd_ws keeps for its backward
+ *           (4 to 64 MB; the forward size is without them, for batches whose
+ *           bwd_ws is always null; the rest is laid out alike).  Kept until
+ *           backward.
  *   lists   the (Gaussian, tile) instance lists for up to `capacity`
  *           instances and their sort scratch.  Kept until backward.
  *   bwd_ws  per (view, Gaussian) gradient accumulator (backward only).  A
@@ -321,6 +323,7 @@ int dmgs_batched_tile_view(const dmgs_view* views, int32_t B, int32_t* tile_view
  *           backward needs a forward BLEND since the previous backward, or
  *           zeros in it. */
 size_t dmgs_batched_state_size(int32_t B, int64_t P, int32_t total_tiles, int64_t total_pixels);
+size_t dmgs_batched_forward_state_size(int32_t B, int64_t P, int32_t total_tiles, int64_t total_pixels);
 size_t dmgs_batched_lists_size(int64_t capacity);
 size_t dmgs_batched_backward_size(int32_t B, int64_t P);
 /* Byte offsets inside `state`: [0] radii (B*P int32, view-major), [1] instance
