@@ -578,6 +578,13 @@ int dmgs_view_geometry(const dmgs_settings* s, const dmgs_gaussians* g, int32_t 
   int rc = check_gaussians(s, g, state);
   if (rc) return rc;
   if (!radii || !counts) return bfail(DMGS_EINVAL, "radii and counts are required");
+  // pinned memory is written by the kernel itself: the wait ends one copy earlier (about 5 us).  Asked before the first
+  // launch, so that the error which the question leaves for plain host memory is not taken for a launch's, nor clears one.
+  hipPointerAttribute_t attr{};
+  void* mapped = nullptr;
+  const bool pinned = hipPointerGetAttributes(&attr, counts) == hipSuccess && attr.type == hipMemoryTypeHost &&
+                      hipHostGetDevicePointer(&mapped, counts, 0) == hipSuccess && mapped;
+  if (!pinned) (void)hipGetLastError();
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   const ViewLayout V(g->count, s->image_width, s->image_height, keep != 0);
   const dmgs_batch b = view_batch(s, g->count, V, state, 0, nullptr, nullptr);
@@ -591,12 +598,6 @@ int dmgs_view_geometry(const dmgs_settings* s, const dmgs_gaussians* g, int32_t 
   a.depth_keys = at<uint32_t>(state, c.S.keys_a);
   dmgs::launch_view_preprocess(a, st);
   order_entries(&b, c, false, st);
-  // pinned memory is written by the kernel itself: the wait ends one copy earlier (about 5 us)
-  hipPointerAttribute_t attr{};
-  void* mapped = nullptr;
-  const bool pinned = hipPointerGetAttributes(&attr, counts) == hipSuccess && attr.type == hipMemoryTypeHost &&
-                      hipHostGetDevicePointer(&mapped, counts, 0) == hipSuccess && mapped;
-  if (!pinned) (void)hipGetLastError();  // plain host memory
   uint32_t* dev = pinned ? static_cast<uint32_t*>(mapped) : at<uint32_t>(state, V.counts);
   dmgs::launch_view_counts(c.count(&b), a.tile_sums, dev, st);
   if ((rc = bcheck("view preprocess / depth sort / scan", st))) return rc;
