@@ -417,8 +417,9 @@ class BatchedLoss:
         self.ones = torch.ones(renderer.B, dtype=torch.float32, device=dev)
 
     def _packed(self, t):
-        if t.numel() != 3 * self.r.total_pixels or t.dtype != torch.float32 or not t.is_contiguous() or \
-                t.device.type != "cuda":
+        n = 3 * self.r.total_pixels  # a buffer may be longer than the images in it
+        if not (t.numel() == n or (t.dim() == 1 and t.numel() > n)) or t.dtype != torch.float32 or \
+                not t.is_contiguous() or t.device.type != "cuda":
             raise ValueError("images must be a contiguous float32 buffer packed like the renderer's")
         return N.ptr(t)
 

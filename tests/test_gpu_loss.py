@@ -138,3 +138,22 @@ def test_views_in_one_launch(sizes):
         assert torch.equal(r.image(grads, v), x.grad), v
     with pytest.raises(ValueError):
         loss.forward(images[:-1])
+
+
+@pytest.mark.parametrize("sizes", [[(40, 24)] * 2, [(33, 17), (20, 40)]])
+def test_images_in_a_longer_buffer(sizes):
+    """The images may be the front of a longer buffer, at any offset: what lies behind stays as it is."""
+    print(f"case: loss in a longer buffer {sizes}", flush=True)
+    from dmgs_amd import batched as BT
+    from dmgs_amd import cameras as C
+    g = torch.Generator().manual_seed(1)
+    cams = [C.camera_at((0.0, 0.0, -4.0), w, h) for w, h in sizes]
+    r = BT.BatchedRenderer(cams, torch.zeros(3, device="cuda"), 10, sh_degree=0)
+    loss = BT.BatchedLoss(r, [torch.rand(3, h, w, generator=g).cuda() for w, h in sizes], 0.2)
+    n = r.new_images().numel()
+    buf, out = torch.rand(n + 100, generator=g).cuda(), torch.full((n + 100,), 9.0, device="cuda")
+    want, dwant = loss.forward(buf[7:7 + n].clone()).clone(), r.new_images()
+    loss.backward(buf[7:7 + n].clone(), dwant)
+    assert torch.equal(loss.forward(buf[7:]), want)
+    loss.backward(buf[7:], out[3:])
+    assert torch.equal(out[3:3 + n], dwant) and (out[:3] == 9).all() and (out[3 + n:] == 9).all()
