@@ -257,8 +257,8 @@ struct RenderArgs {
   float* gacc;           // P x DMGS_GACC_STRIDE floats, two planes (gacc_index)
   // optional (multi-view): work-group slot -> tile, heaviest tiles first
   const uint32_t* tile_order;
-  // optional (multi-view): per tile, the largest last
-  // contributor of its pixels (the backward's list length)
+  // optional (multi-view, one work-group a tile and no kept segments): per
+  // tile, the largest last contributor of its pixels (the backward's list length)
   uint32_t* tile_work;
   // optional (forward): the backward accumulator, zeroed by the forward's
   // work-groups in equal shares after their blend work

@@ -824,18 +824,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
       }
     }
   }
-  if (a.tile_work) {  // the backward walks list positions below the tile's largest last contributor
-    __shared__ uint32_t s_max[NT / DMGS_WAVE];
-    uint32_t m = last_contributor;
-    for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
-    if (lane == 0) s_max[wave] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-      if constexpr (SPLIT)
-        atomicMax(&a.tile_work[c.tile], m);  // zero since the tiles were ordered
-      else
-        a.tile_work[c.tile] = m;
+  if constexpr (CELLS && !KEEP && !SPLIT) {
+    if (a.tile_work) {  // the backward walks list positions below the tile's largest last contributor
+      __shared__ uint32_t s_max[NT / DMGS_WAVE];
+      uint32_t m = last_contributor;
+      for (int off = 32; off > 0; off >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, off, 64));
+      if (lane == 0) s_max[wave] = m;
+      __syncthreads();
+      if (threadIdx.x == 0) a.tile_work[c.tile] = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
     }
   }
   if constexpr (SPLIT) {
@@ -1098,7 +1094,6 @@ __global__ __launch_bounds__(256) void tile_bucket_kernel(RenderArgs a, uint8_t*
   if (t < a.num_tiles) {
     const uint32_t b = tile_cost_bucket(a, t, K, use_work != 0);
     bucket[t] = (uint8_t)b;
-    if (!use_work && a.tile_work) a.tile_work[t] = 0u;  // the forward's halves of a tile take the larger of theirs
     atomicAdd(&cnt[b], 1u);
   }
   __syncthreads();
@@ -1132,8 +1127,7 @@ __global__ __launch_bounds__(256) void tile_order_kernel(const uint8_t* __restri
 // The same for few tiles, one work-group and one launch: 5 us where the two passes and the gap between them take 10
 // (400 tiles); with more tiles than its lanes hold in registers the two passes win.
 constexpr int kOrderLanes = 1024, kOrderTiles = 4;  // per lane
-__global__ __launch_bounds__(kOrderLanes) void tile_order_few_kernel(RenderArgs a, int use_work,
-                                                                     uint32_t* __restrict__ order) {
+__global__ __launch_bounds__(kOrderLanes) void tile_order_few_kernel(RenderArgs a, uint32_t* __restrict__ order) {
   __shared__ uint32_t cnt[256], start[256];
   __shared__ uint32_t s_wave[kOrderLanes / 64];
   const int tid = threadIdx.x;
@@ -1144,13 +1138,12 @@ __global__ __launch_bounds__(kOrderLanes) void tile_order_few_kernel(RenderArgs 
   uint32_t b[kOrderTiles], rank[kOrderTiles];
 #pragma unroll
   for (int i = 0; i < kOrderTiles; ++i)  // no load is conditional: they are in flight together
-    b[i] = tile_cost_bucket(a, min(i * kOrderLanes + tid, a.num_tiles - 1), K, use_work != 0);
+    b[i] = tile_cost_bucket(a, min(i * kOrderLanes + tid, a.num_tiles - 1), K, false);
 #pragma unroll
   for (int i = 0; i < kOrderTiles; ++i) {
     const int t = i * kOrderLanes + tid;
     if (t >= a.num_tiles) continue;
     rank[i] = atomicAdd(&cnt[b[i]], 1u);
-    if (!use_work && a.tile_work) a.tile_work[t] = 0u;  // the forward's halves of a tile take the larger of theirs
   }
   __syncthreads();
   uint32_t total;
@@ -1167,10 +1160,6 @@ __global__ __launch_bounds__(kOrderLanes) void tile_order_few_kernel(RenderArgs 
 static void tile_order_impl(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, bool use_work,
                             hipStream_t s, bool hist_zeroed) {
   if (a.num_tiles <= 0 || !a.views) return;
-  if (a.num_tiles <= kOrderLanes * kOrderTiles) {
-    hipLaunchKernelGGL(tile_order_few_kernel, dim3(1), dim3(kOrderLanes), 0, s, a, use_work ? 1 : 0, order);
-    return;
-  }
   const unsigned blocks = (unsigned)((a.num_tiles + 255) / 256);
   if (!hist_zeroed) launch_fill_u32(hist, 512, 0u, s);
   hipLaunchKernelGGL(tile_bucket_kernel, dim3(blocks), dim3(256), 0, s, a, bucket, hist, use_work ? 1 : 0);
@@ -1180,7 +1169,10 @@ static void tile_order_impl(const RenderArgs& a, uint32_t* order, uint8_t* bucke
 
 void launch_tile_order(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, hipStream_t s,
                        bool hist_zeroed) {
-  tile_order_impl(a, order, bucket, hist, false, s, hist_zeroed);
+  if (a.views && a.num_tiles > 0 && a.num_tiles <= kOrderLanes * kOrderTiles)
+    hipLaunchKernelGGL(tile_order_few_kernel, dim3(1), dim3(kOrderLanes), 0, s, a, order);
+  else
+    tile_order_impl(a, order, bucket, hist, false, s, hist_zeroed);
 }
 
 void launch_tile_order_bwd(const RenderArgs& a, uint32_t* order, uint8_t* bucket, uint32_t* hist, hipStream_t s,
