@@ -483,7 +483,8 @@ static void launch_rowscan(uint32_t* hist, uint32_t nb, uint32_t* totals, uint32
     hipLaunchKernelGGL(radix_rowscan_kernel<kScanThreads>, dim3(digits), dim3(kScanThreads), 0, s, hist, nb, totals);
 }
 
-static int sort_items(size_t n) { return n >= ((size_t)4 << 20) ? 16 : 4; }
+constexpr size_t kLongSort = (size_t)4 << 20;  // from here on 4096 keys to a block
+static int sort_items(size_t n) { return n >= kLongSort ? 16 : 4; }
 
 // 512 digits in one pass instead of two passes of 5 and 4 bits: the lists of a view of 257 to 512 cells (1600 x 900,
 // 1920 x 1080) in one trip through memory.  From the size on whose blocks are the duplicate's chunks.  164 M pairs:
@@ -501,14 +502,17 @@ void radix_sort_pairs_wide_digit(const uint32_t* k0, const uint32_t* v0, uint32_
                      (const uint32_t*)scratch, (const uint32_t*)totals, nb, n_dev, (uint32_t*)nullptr);
 }
 
+// The scratch sizes never fall as n grows, though a longer list may need less: memory sized for one capacity serves
+// every smaller one.
 size_t radix_list_scratch_words(size_t n) {
-  return sort_items(n) == 16 ? 512 * ((n + 4095) / 4096) + 512 + 64 : radix_scratch_words(n);
+  const size_t words = radix_scratch_words(n);
+  return sort_items(n) == 16 ? std::max(words, 512 * ((n + 4095) / 4096) + 512 + 64) : words;
 }
 
 size_t radix_scratch_words(size_t n) {
   const size_t tile = (size_t)kSortThreads * sort_items(n);
-  const size_t nb = (n + tile - 1) / tile;
-  return 256 * nb + 256 + 64;
+  const size_t nb = (n + tile - 1) / tile, words = 256 * nb + 256 + 64;
+  return sort_items(n) == 16 ? std::max(words, radix_scratch_words(kLongSort - 1)) : words;
 }
 
 // Entry-key first pass (see radix_sort_entry_keys): when `entry` is set, pass 0
@@ -644,7 +648,8 @@ void launch_gather_u32(const uint32_t* src, const uint32_t* idx, uint32_t* dst, 
 // because a work-group walks its chunk's entries in windows of 256, one memory latency each, and there are few
 // chunks.  With 4096, 1024 and 512 slots, us: 10 k Gaussians at 200 x 200 31, 14 and 9; 491 k face-bound ones at
 // 800 x 800 38, 15 and 11; 1 M at 800 x 800 (2.3 M slots) 25, 18 and 19.
-static uint32_t chunk_slots(uint32_t K) { return sort_items(K) == 16 ? 4096u : K >= (1u << 20) ? 1024u : 512u; }
+constexpr size_t kShortLists = (size_t)1 << 20;
+static uint32_t chunk_slots(uint32_t K) { return sort_items(K) == 16 ? 4096u : K >= kShortLists ? 1024u : 512u; }
 
 __device__ __forceinline__ uint32_t device_count(uint32_t cap, const uint32_t* dev) {
   return dev ? min(cap, *dev) : cap;
@@ -837,9 +842,13 @@ __global__ __launch_bounds__(256) void duplicate_kernel(DupArgs a) {
     for (uint32_t d = threadIdx.x; d <= hmask; d += 256) a.hist[(size_t)d * chunks + chunk] = s_hist[d];
 }
 
-size_t duplicate_scratch_words(size_t K) {
-  const size_t slots = chunk_slots((uint32_t)std::min<size_t>(K, 0xffffffffu));
-  return (K + slots - 1) / slots + 64;
+size_t duplicate_scratch_words(size_t K) {  // does not fall either
+  size_t words = 0;
+  for (const size_t k : {K, std::min(K, kLongSort - 1), std::min(K, kShortLists - 1)}) {
+    const size_t slots = chunk_slots((uint32_t)std::min<size_t>(k, 0xffffffffu));
+    words = std::max(words, (k + slots - 1) / slots + 64);
+  }
+  return words;
 }
 
 void launch_duplicate(const DupArgs& args, hipStream_t s) {

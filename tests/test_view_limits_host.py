@@ -26,3 +26,14 @@ def test_batched_views_refuse_what_a_rectangle_cannot_hold(w, h, ok):
     rc = N.load().dmgs_batched_prepare_views(v, 1, ctypes.byref(tt), ctypes.byref(tc), ctypes.byref(mc), ctypes.byref(tp))
     assert rc == (0 if ok else -1)
     assert ok or "tiles a side" in N.last_error()
+
+
+def test_list_sizes_do_not_fall():
+    """Memory sized for one capacity serves every smaller one, whose blocks and chunks may be smaller."""
+    lib = N.load()
+    at = sorted({e + d for e in (1, 1 << 10, 1 << 20, 4 << 20, 6 << 20, 16 << 20) for d in (-1, 0, 1, 300, 5000)} - {0})
+    for size in (lib.dmgs_batched_lists_size, lib.dmgs_binning_workspace_size):
+        sizes = [size(k) for k in at]
+        assert sizes == sorted(sizes)
+    states = [lib.dmgs_batched_forward_state_size(1, p, 16, 4096) for p in at]
+    assert states == sorted(states)
