@@ -491,7 +491,7 @@ struct MemberList {
 // red and green, the other blue.  16 instructions a splat, in twice as many waves, with the same operations in the
 // same order on every value.  (Eight waves of one work-group share a CU's SIMDs and gain nothing.)
 // Five waves per SIMD where one work-group blends a tile and keeps nothing: the compiler takes 106 registers (four
-// waves) if left alone and 96 if asked (one spilled in the path for odd colours); 16 uneven views 3.34 -> 2.99 ms, 8 views of 800x800 312 -> 294 us,
+// waves) if left alone and 96 without a spill if asked; 16 uneven views 3.34 -> 2.99 ms, 8 views of 800x800 312 -> 294 us,
 // 1920x1080 134 -> 125 us.  Six waves spill 48 bytes (8 views of 800x800 330 us); with kept segments five spill 24
 // (a 10k view 57 -> 59 us, 82k faces 249 -> 255); two work-groups a tile have few waves in flight at any register count.
 template <bool CELLS, bool KEEP, bool SPLIT>
@@ -691,7 +691,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
         }
         continue;
       }
-      if (lane < 12) reach[count + lane] = kPad;
+      int pad = lane;
+      asm volatile("" : "+v"(pad));  // its address is made here: kept over the rounds it would be the register too many
+      if (pad < 12) reach[count + pad] = kPad;
       if constexpr (SPLIT) {
         const bool second = lane >= 32;  // of the pixel's two lanes
         const char* const channels =
