@@ -31,7 +31,7 @@
 // every 64-member segment is a work-group of its own.  Slots (4 KB) come from a counter; a tile that gets
 // none has a longer last segment.  Launches of more than kSegmentTiles tiles fill the GPU without it.
 // Blend backward of one view, us, one wave per tile and with segments (MI355X): 10k Gaussians at 200x200 375
-// and 58, 1M at 800x800 225 and 89, 491k face-bound at 800x800 1385 and 172 (their forwards get 12-43 us longer:
+// and 60, 1M at 800x800 225 and 95, 491k face-bound at 800x800 1385 and 177 (their forwards get 12-43 us longer:
 // the states are written, summed and cleared).
 #include "dmgs_common.h"
 #include "dmgs_kernels.h"
@@ -110,7 +110,7 @@ struct PixelRects {  // four rectangles of w x h pixels, `cols` (1 or 2) to a ro
 // minimiser, which raises the value found by far less than the margins.)  Rectangles side by side share a row's or
 // column's terms, and the logarithm is the hardware's: against four edges of each rectangle behind a branch, 158 vector
 // instructions less per staged splat in the forward's code and 129 in the backward's.  Issued on 8 views of 800x800 of
-// 1M Gaussians 202.5M -> 189.8M and 265.9M -> 259.5M; one 333x251 view of 500k, near, 319 -> 303 us.
+// 1M Gaussians 202.5M -> 189.8M in the forward, 6.4M fewer in the backward; one 333x251 view of 500k, near, 319 -> 303 us.
 template <int NX, int NY>
 __device__ __forceinline__ uint32_t reach_rects(float cx, float cy, float a, float b, float c, float t,
                                                 const PixelRects& rr) {
@@ -865,8 +865,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
 // SIMD (95 registers; six spill, and four take 24 % longer): so a batch is
 // filled before it is walked, what can be decided for 64 staged splats at once
 // (which strips are live) is, one lane per splat, and the ninth sum waits for
-// three others'.  Before and now: sixteen uneven views of 3 M Gaussians 6.96
-// and 5.29 ms, eight 800x800 views of 1 M 462 and 434 us (5.06 ms and 407 us
+// three others'.  Before and now: sixteen uneven views of 3 M Gaussians 6.91
+// and 5.33 ms, eight 800x800 views of 1 M 483 and 438 us (5.06 ms and 424 us
 // with the background in the recursion and the linear forms after the sums,
 // whose gradients differ, see bwd_step).
 //
