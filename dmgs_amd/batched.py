@@ -147,12 +147,12 @@ class BatchedRenderer:
         self.state = self.lists = self.bwd_ws = None
         self.dens = None
         self._offsets = None
-        self._state_backward = False  # the state has room for what a forward keeps for its backward
+        self._state_backward = False  # the state has room for the backward's list segments
 
     # ---- planning ---------------------------------------------------------
     def _alloc_state(self, backward=True):
-        """The state; without ``backward`` without the list segments that a
-        forward keeps for one.  An existing state's contents are kept."""
+        """The state; without ``backward`` without the room for a backward's
+        list segments.  An existing state's contents are kept."""
         size = self.lib.dmgs_batched_state_size if backward else self.lib.dmgs_batched_forward_state_size
         n = size(self.B, self.P, self.total_tiles, self.total_pixels)
         if n == 0:

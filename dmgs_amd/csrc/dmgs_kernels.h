@@ -218,21 +218,23 @@ struct ShSigmoidArgs {
 void launch_sh_sigmoid(const ShSigmoidArgs& a, int coeffs, bool color_major, bool backward, hipStream_t s);
 
 // ---- blend ----
-// List segments that a forward keeps for its backward (render.hip).  At most kSegmentTiles tiles: with 8160
-// tiles (1920x1080) keeping them costs as much as it gives (forward + backward of 1M Gaussians 335 us with,
-// 331 without), with 2500 it saves 60 us of 230.  64 members: shorter ones cost the forward more than the
-// backward gains from 2500 tiles on, 128 lose 15-60 us on the cases with few tiles.
+// List segments of the blend's backward (render.hip).  At most kSegmentTiles tiles: forward and backward blend, us,
+// whole lists and segments: 60k / 300k / 1.5M Gaussians, uniform, at 992x992 (3844 tiles) 217 and 203, 367 and 291,
+// 861 and 651, face-bound 491k 918 and 573, and 300k and 1.5M clustered 502 and 349, 234 and 297 (lists of few
+// members up to where they saturate); at 1920x1080 (8160 tiles, which fill the GPU without) 308 and 397, 389 and 494,
+// 739 and 1026, clustered 449 and 550, 349 and 488.  Only lists of more than 256 members: 64 to 300 us slower with 300k.
 constexpr int kSegmentTiles = 4096;
 constexpr int kSegmentLength = 64;
-constexpr int kTileSegments = 256;  // kept segments of one tile at most
+constexpr int kTileSegments = 256;  // segments of one tile that start from a state, at most
+constexpr int kSegmentParts = 16;   // counters of slots, each with its share of them
+constexpr int kSegmentHeadStride = 32;  // words between two
 constexpr uint32_t kNoSegment = 0xFFFFFFFFu;
-constexpr uint32_t kSegMagic = 0x5E600001u;
 struct Segments {
-  int len, cap;          // members per segment (0: none are kept), slots
-  uint32_t* head;        // [0] slots asked for, [1] kSegMagic once a forward keeps segments
+  int cap;               // slots (0: no segments)
+  uint32_t* head;        // per part: slots asked for
   uint4* rec;            // per slot: tile, first and one past the last list position
-  float4* state;         // per slot: the tile's 256 pixels' T behind the segment and the colour added behind it
-  uint32_t* tile_last;   // per tile: where its last (not kept) segment begins
+  float2* state;         // per slot: the tile's 256 pixels' BwdPixel behind the segment
+  uint32_t* tile_last;   // per tile: where its last segment, which starts from the list's end, begins
 };
 // Single view: W, H, grid_x, grid_y, bg and the image pointers describe the
 // view.  Several views: `views` / `tile_view` map each global tile to its
@@ -257,7 +259,7 @@ struct RenderArgs {
   float* gacc;           // P x DMGS_GACC_STRIDE floats, two planes (gacc_index)
   // optional (multi-view): work-group slot -> tile, heaviest tiles first
   const uint32_t* tile_order;
-  // optional (multi-view, one work-group a tile and no kept segments): per
+  // optional (multi-view, one work-group a tile in the forward): per
   // tile, the largest last contributor of its pixels (the backward's list length)
   uint32_t* tile_work;
   // optional (forward): the backward accumulator, zeroed by the forward's

@@ -9,7 +9,7 @@
 //
 // Forward (render_fwd_quads_kernel): one 256-lane work-group per 16x16 binning tile, each of its four waves
 // owning one 8x8 quadrant, one pixel per lane.  Backward (render_bwd_strips_kernel): one wave per tile, or per
-// kept segment of a tile's list, each lane owning four pixels.
+// segment of a tile's list, each lane owning four pixels.
 //
 // Backward: the list is walked from the back, starting at the largest
 // n_contrib of the tile (entries behind every pixel's last contributor
@@ -21,18 +21,19 @@
 // Several views in one launch: a global tile id indexes the ranges; the view
 // table gives each tile's image size, background and packed output offset.
 //
-// Kept segments.  A lone wave takes 400 ns per (tile, splat) in the backward (a chain of dependent
+// List segments.  A lone wave takes 400 ns per (tile, splat) in the backward (a chain of dependent
 // operations), so a launch of few tiles with long lists (a 200x200 view: 169 tiles, up to 900 entries
-// walked) used to take as long as its longest list: 375 us.  A forward that will be followed by a backward
-// therefore keeps, every 64 members of a tile's list, the pixels' transmittance and the colour added since
-// the last boundary; at the end of the list it turns those colours into "the colour added behind this
-// boundary" (sums from the back, so that each has its own relative precision; the difference of two
-// running totals would lose it).  That is the whole state of the backward recursion at the boundary, so
-// every 64-member segment is a work-group of its own.  Slots (4 KB) come from a counter; a tile that gets
-// none has a longer last segment.  Launches of more than kSegmentTiles tiles fill the GPU without it.
-// Blend backward of one view, us, one wave per tile and with segments (MI355X): 10k Gaussians at 200x200 375
-// and 60, 1M at 800x800 225 and 95, 491k face-bound at 800x800 1385 and 177 (their forwards get 12-43 us longer:
-// the states are written, summed and cleared).
+// walked) takes as long as its longest list: 350 us.  With at most kSegmentTiles tiles a pass of its own
+// (render_bwd_chain_kernel) therefore first walks the lists for the pixels' recursion alone, a quarter of the
+// work a splat and one pixel a lane, and leaves its state at every 64th member, so that every 64-member
+// segment is a work-group of the backward proper.  The pass has the forward's bound and takes as long as it.
+// The recursion is the backward's own, from final_T with the same reciprocals in the same order: each
+// (tile, splat) sum is the same to the last bit with segments, however many slots there are, as without.
+// (States that the forward leaves as it goes by cost no pass, but its transmittances are other roundings of
+// the same products: gradients of scales and rotations, small differences of these sums, moved by up to 2e-3
+// of their rms.)  Slots are 2 KB.
+// Forward, pass and backward of one view, us, whole lists and segments (MI355X): 10k Gaussians at 200x200
+// 36+353 and 36+51+38, 1M at 800x800 53+196 and 53+52+92, 491k face-bound at 800x800 207+1288 and 207+222+178.
 #include "dmgs_common.h"
 #include "dmgs_kernels.h"
 
@@ -389,7 +390,6 @@ __device__ __forceinline__ TileCtx tile_ctx(const RenderArgs& a, int tile, int h
 // A forward work-group's share of clearing the backward accumulator: run
 // after its blend work, so the stores delay no load of the blend.
 __device__ __forceinline__ void clear_share(const RenderArgs& a) {
-  if (a.seg.head && a.seg.len == 0 && blockIdx.x == 0 && threadIdx.x < 2) a.seg.head[threadIdx.x] = 0u;
   if (a.clear_words && blockIdx.x == 0)
     for (int i = threadIdx.x; i < a.clear_words_n; i += blockDim.x) a.clear_words[i] = 0u;
   if (!a.clear) return;
@@ -482,45 +482,39 @@ struct MemberList {
 // latencies overlap) and applies them in order with selects instead of branches.  Against one wave per tile
 // with four pixels per lane: 8 views of 800x800 of 1M Gaussians 400 -> 294 us, 16 uneven views of 3M
 // 5.33 -> 2.99 ms, one 800x800 view 154 -> 48 us, 333x251 of 500k 1377 -> 195 us.  Quadrants because a splat
-// reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on KEEP,
-// CELLS or the launch.
+// reaches fewer 8x8 blocks than 16x4 strips.  The arithmetic of a pixel and its order do not depend on
+// CELLS, SPLIT or the launch.
 // SPLIT: a tile's list is a chain (each pixel's transmittance goes from splat to splat), so a launch of few tiles
 // takes as long as its longest list, however empty the GPU is: 24 instructions a splat in each of four waves.  Two
 // work-groups blend a tile then, 16x8 pixels each with two lanes a pixel: the lanes evaluate the alphas of two
 // consecutive splats side by side, exchange them, and both carry the transmittance over the two in order; one adds
 // red and green, the other blue.  16 instructions a splat, in twice as many waves, with the same operations in the
 // same order on every value.  (Eight waves of one work-group share a CU's SIMDs and gain nothing.)
-// Five waves per SIMD where one work-group blends a tile and keeps nothing: the compiler takes 106 registers (four
+// Five waves per SIMD where one work-group blends a tile: the compiler takes 106 registers (four
 // waves) if left alone and 96 without a spill if asked; 16 uneven views 3.34 -> 2.99 ms, 8 views of 800x800 312 -> 294 us,
-// 1920x1080 134 -> 125 us.  Six waves spill 48 bytes (8 views of 800x800 330 us); with kept segments five spill 24
-// (a 10k view 57 -> 59 us, 82k faces 249 -> 255); two work-groups a tile have few waves in flight at any register count.
-template <bool CELLS, bool KEEP, bool SPLIT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPLIT ? 1 : 5, 8))) void render_fwd_quads_kernel(
+// 1920x1080 134 -> 125 us.  Six waves spill 48 bytes (8 views of 800x800 330 us); two work-groups a tile have
+// few waves in flight at any register count.
+template <bool CELLS, bool SPLIT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SPLIT ? 1 : 5, 8))) void render_fwd_quads_kernel(
     RenderArgs a) {
   constexpr int NT = 256, U = FwdGroup::kN;
-  constexpr int G = KEEP ? 64 : NT;  // staged splats blended per round
   constexpr int kPad = NT * 16;      // offset of the filling splat
   __shared__ FwdSplats<NT + 1> L;    // slot NT: a splat of zero opacity, which fills up groups
   constexpr int C = CELLS ? 4 : 1;   // list positions per lane and chunk
   __shared__ MemberList<C * NT> M;
   __shared__ uint32_t s_wc[2][C][NT / DMGS_WAVE];
-  __shared__ uint32_t s_slot[KEEP ? kTileSegments : 1];
-  __shared__ __align__(16) uint32_t s_reach[NT / DMGS_WAVE][G + 12];
+  __shared__ __align__(16) uint32_t s_reach[NT / DMGS_WAVE][NT + 12];
   const int half = SPLIT ? (int)(blockIdx.x & 1u) : -1;
   const TileCtx c = tile_ctx<true>(a, ordered_tile(a, SPLIT ? (int)(blockIdx.x >> 1) : (int)blockIdx.x), half);
   const float pxf = (float)c.px, pyf = (float)c.py;
   const int len = (int)(c.range.y - c.range.x);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int seg_pixel = ((wave >> 1) * 8 + (lane >> 3)) * 16 + (wave & 1) * 8 + (lane & 7);  // row-major in the tile
   if (threadIdx.x == 0) L.xyq[NT] = L.qorg[NT] = L.bpmi[NT] = make_float4(0.f, 0.f, 0.f, 0.f);
   // T > 0 while the pixel blends; a finished pixel (saturated, or outside the image) keeps -T
   float T = c.inside ? 1.0f : -1.0f;
   float C0 = 0.f, C1 = 0.f, C2 = 0.f;
   uint32_t last_contributor = 0;
-  // kept segments (see Segments): D is the colour added since the last boundary
-  float D0 = 0.f, D1 = 0.f, D2 = 0.f;
-  int seg_begin = 0, seg_members = 0, segs = 0;
 
   // Three overlapping steps: the keys and ids of a chunk of the list are on their way while the records of
   // the next 256 members are, and while the 256 before those are blended.  A chunk of a cell list is four
@@ -611,222 +605,154 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
     __syncthreads();
     n_next = gather();
     ask();
-    if constexpr (KEEP) {
-      // segment boundaries inside this chunk: before a round, once enough members have passed
-      int want = 0, m = seg_members;
-      for (int h = 0; h < n; h += G) {
-        if (m >= a.seg.len) ++want, m = 0;
-        m += min(G, n - h);
-      }
-      want = min(want, kTileSegments - segs);
-      if (want > 0) {
-        if (threadIdx.x == 0) {
-          const uint32_t first = atomicAdd(a.seg.head, (uint32_t)want);
-          for (int k = 0; k < want; ++k) s_slot[segs + k] = first + k < (uint32_t)a.seg.cap ? first + k : kNoSegment;
-        }
-        __syncthreads();
-      }
+    if (__ballot(T > 0.f) == 0) continue;  // wave-uniform: this quadrant is finished
+    // the round's splats that reach this quadrant, as LDS offsets in list order, filled up for whole groups
+    // and for the two groups read ahead
+    uint32_t* const reach = s_reach[wave];
+    int count = 0;
+    uint64_t odd = 0;
+#pragma unroll
+    for (int k = 0; k < NT; k += 64) {
+      const int s = k + lane;
+      const uint32_t mask = L.mask(min(s, NT));
+      const bool reached = s < n && ((mask >> wave) & 1u);
+      const uint64_t bits = __ballot(reached);
+      odd |= __ballot(reached && (mask & kOddColor));
+      if ((bits >> lane) & 1u) reach[count + (int)__popcll(bits & lanemask_lt())] = (uint32_t)s * 16u;
+      count += (int)__popcll(bits);
     }
-    for (int h = 0; h < NT; h += G) {
-      if (h >= n) break;
-      if constexpr (KEEP) {
-        if (seg_members >= a.seg.len && segs < kTileSegments) {
-          const uint32_t slot = s_slot[segs];
-          const int end = (int)L.pos(h) - 1;
-          if (slot != kNoSegment) {
-            a.seg.state[(size_t)slot * 256 + seg_pixel] = make_float4(fabsf(T), D0, D1, D2);
-            D0 = D1 = D2 = 0.f;
-            if (threadIdx.x == 0) a.seg.rec[slot] = make_uint4((uint32_t)c.tile, (uint32_t)seg_begin, (uint32_t)end, 0u);
-            ++segs;
-            seg_begin = end;
-            seg_members = 0;
-          } else {
-            seg_members = -0x40000000;  // no slots left: the rest of the list is one segment
-          }
+    if (count == 0) continue;
+    if (odd != 0) {
+      // The groups below add skipped splats with weight zero, which a colour that is not finite would turn into
+      // NaN in pixels that it does not touch: such a round goes splat by splat, adding only what contributes.
+      for (int i = 0; i < count; ++i) {
+        const uint32_t o = reach[i];
+        const float4 g = lds_at(L.xyq, o), q = lds_at(L.qorg, o), b = lds_at(L.bpmi, o);
+        const float power = power_at(power_dx(g.z, g.w, g.x - pxf), q.x, g.y - pyf);
+        const float alpha = fminf(0.99f, q.y * splat_exp2(power));
+        if (!((power <= 0.0f) & (alpha >= 1.0f / 255.0f) & (T > 0.f))) continue;
+        const float test_T = T * (1.0f - alpha), w = alpha * T;
+        if (test_T >= 0.0001f) {
+          const bool blue = SPLIT && lane >= 32;  // of a pixel's two lanes the one that adds blue, in C0
+          C0 = fmaf(blue ? b.x : q.z, w, C0);
+          C1 = fmaf(q.w, w, C1);
+          C2 = fmaf(b.x, w, C2);
+          T = test_T;
+          last_contributor = __float_as_uint(b.y);
+        } else {
+          T = -T;
         }
-        seg_members += min(G, n - h);
       }
-      if (__ballot(T > 0.f) == 0) continue;  // wave-uniform: this quadrant is finished
-      // the round's splats that reach this quadrant, as LDS offsets in list order, filled up for whole groups
-      // and for the two groups read ahead
-      uint32_t* const reach = s_reach[wave];
-      int count = 0;
-      uint64_t odd = 0;
+      continue;
+    }
+    int pad = lane;
+    asm volatile("" : "+v"(pad));  // its address is made here: kept over the rounds it would be the register too many
+    if (pad < 12) reach[count + pad] = kPad;
+    if constexpr (SPLIT) {
+      const bool second = lane >= 32;  // of the pixel's two lanes
+      const char* const channels =
+          second ? reinterpret_cast<const char*>(L.bpmi) : reinterpret_cast<const char*>(L.qorg) + 8;
+      auto fetch = [&](FwdPairs& g, const uint4& at, int next) {
+        const uint32_t own[2] = {second ? at.y : at.x, second ? at.w : at.z};
+        const uint32_t both[2][2] = {{at.x, at.y}, {at.z, at.w}};
 #pragma unroll
-      for (int k = 0; k < G; k += 64) {
-        const int s = h + k + lane;
-        const uint32_t mask = L.mask(min(s, NT));
-        const bool reached = s < n && ((mask >> wave) & 1u);
-        const uint64_t bits = __ballot(reached);
-        odd |= __ballot(reached && (mask & kOddColor));
-        if ((bits >> lane) & 1u) reach[count + (int)__popcll(bits & lanemask_lt())] = (uint32_t)s * 16u;
-        count += (int)__popcll(bits);
-      }
-      if (count == 0) continue;
-      if (odd != 0) {
-        // The groups below add skipped splats with weight zero, which a colour that is not finite would turn into
-        // NaN in pixels that it does not touch: such a round goes splat by splat, adding only what contributes.
-        for (int i = 0; i < count; ++i) {
-          const uint32_t o = reach[i];
-          const float4 g = lds_at(L.xyq, o), q = lds_at(L.qorg, o), b = lds_at(L.bpmi, o);
-          const float power = power_at(power_dx(g.z, g.w, g.x - pxf), q.x, g.y - pyf);
-          const float alpha = fminf(0.99f, q.y * splat_exp2(power));
-          if (!((power <= 0.0f) & (alpha >= 1.0f / 255.0f) & (T > 0.f))) continue;
-          const float test_T = T * (1.0f - alpha), w = alpha * T;
-          if (test_T >= 0.0001f) {
-            const bool blue = SPLIT && lane >= 32;  // of a pixel's two lanes the one that adds blue, in C0
-            C0 = fmaf(blue ? b.x : q.z, w, C0);
-            C1 = fmaf(q.w, w, C1);
-            C2 = fmaf(b.x, w, C2);
-            if constexpr (KEEP) {
-              D0 = fmaf(q.z, w, D0);
-              D1 = fmaf(q.w, w, D1);
-              D2 = fmaf(b.x, w, D2);
-            }
-            T = test_T;
-            last_contributor = __float_as_uint(b.y);
-          } else {
-            T = -T;
-          }
-        }
-        continue;
-      }
-      int pad = lane;
-      asm volatile("" : "+v"(pad));  // its address is made here: kept over the rounds it would be the register too many
-      if (pad < 12) reach[count + pad] = kPad;
-      if constexpr (SPLIT) {
-        const bool second = lane >= 32;  // of the pixel's two lanes
-        const char* const channels =
-            second ? reinterpret_cast<const char*>(L.bpmi) : reinterpret_cast<const char*>(L.qorg) + 8;
-        auto fetch = [&](FwdPairs& g, const uint4& at, int next) {
-          const uint32_t own[2] = {second ? at.y : at.x, second ? at.w : at.z};
-          const uint32_t both[2][2] = {{at.x, at.y}, {at.z, at.w}};
+        for (int p = 0; p < 2; ++p) {
+          g.xyq[p] = lds_at(L.xyq, own[p]);
+          g.qo[p] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(L.qorg) + own[p]);
+          g.pos[p] = __float_as_uint(lds_at(L.bpmi, own[p]).y);
 #pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            g.xyq[p] = lds_at(L.xyq, own[p]);
-            g.qo[p] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(L.qorg) + own[p]);
-            g.pos[p] = __float_as_uint(lds_at(L.bpmi, own[p]).y);
-#pragma unroll
-            for (int e = 0; e < 2; ++e) g.col[p][e] = *reinterpret_cast<const float2*>(channels + both[p][e]);
-          }
-          g.at = *reinterpret_cast<const uint4*>(reach + next);
-        };
-        // blends `cur` while `next` is on its way; false when nothing is left to do
-        int done = 0;
-        auto step = [&](FwdPairs& cur, FwdPairs& next) {
-          fetch(next, cur.at, done + 8);
-          float alpha[2];
-          bool ok[2];
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const float4 g = cur.xyq[p];
-            const float power = power_at(power_dx(g.z, g.w, g.x - pxf), cur.qo[p].x, g.y - pyf);
-            const float al = fminf(0.99f, cur.qo[p].y * splat_exp2(power));
-            ok[p] = (power <= 0.0f) & (al >= 1.0f / 255.0f);
-            alpha[p] = ok[p] ? al : 0.0f;
-          }
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(alpha[p]), __float_as_uint(alpha[p]), false, false);
-            bool take[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {  // both lanes: the first lane's splat, then the second's
-              const float al = __uint_as_float(x[e]);
-              const float test_T = T * (1.0f - al);
-              take[e] = test_T >= 0.0001f;
-              const float w = take[e] ? al * T : 0.0f;
-              C0 = fmaf(cur.col[p][e].x, w, C0);
-              C1 = fmaf(cur.col[p][e].y, w, C1);  // the blue lane's is not used
-              T = take[e] ? test_T : -fabsf(T);
-            }
-            const bool mine = (second & take[1]) | (!second & take[0]);
-            last_contributor = (mine & ok[p]) ? cur.pos[p] : last_contributor;
-          }
-          done += 4;
-          return done < count && __ballot(T > 0.f) != 0;
-        };
-        FwdPairs g0, g1;
-        fetch(g0, *reinterpret_cast<const uint4*>(reach), 4);
-        while (step(g0, g1) && step(g1, g0)) {
-        }
-        continue;
-      }
-      auto fetch = [&](FwdGroup& g, const uint4& at, int next) {
-        const uint32_t o[U] = {at.x, at.y, at.z, at.w};
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          g.xyq[u] = lds_at(L.xyq, o[u]);
-          g.qorg[u] = lds_at(L.qorg, o[u]);
+          for (int e = 0; e < 2; ++e) g.col[p][e] = *reinterpret_cast<const float2*>(channels + both[p][e]);
         }
         g.at = *reinterpret_cast<const uint4*>(reach + next);
       };
-      // blends `cur` (at the offsets `at`) while `next` is on its way; false when nothing is left to do
+      // blends `cur` while `next` is on its way; false when nothing is left to do
       int done = 0;
-      auto step = [&](FwdGroup& cur, uint4& at, FwdGroup& next) {
-        const uint32_t o[U] = {at.x, at.y, at.z, at.w};
-        float4 bp[U];
+      auto step = [&](FwdPairs& cur, FwdPairs& next) {
+        fetch(next, cur.at, done + 8);
+        float alpha[2];
+        bool ok[2];
 #pragma unroll
-        for (int u = 0; u < U; ++u) bp[u] = lds_at(L.bpmi, o[u]);
-        fetch(next, cur.at, done + 2 * U);
-        at = cur.at;
-        float alpha[U];
-        bool ok[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {  // independent of each other: their latencies overlap
-          const float p = power_at(power_dx(cur.xyq[u].z, cur.xyq[u].w, cur.xyq[u].x - pxf), cur.qorg[u].x, cur.xyq[u].y - pyf);
-          const float al = fminf(0.99f, cur.qorg[u].y * splat_exp2(p));
-          ok[u] = (p <= 0.0f) & (al >= 1.0f / 255.0f);
-          alpha[u] = ok[u] ? al : 0.0f;
+        for (int p = 0; p < 2; ++p) {
+          const float4 g = cur.xyq[p];
+          const float power = power_at(power_dx(g.z, g.w, g.x - pxf), cur.qo[p].x, g.y - pyf);
+          const float al = fminf(0.99f, cur.qo[p].y * splat_exp2(power));
+          ok[p] = (power <= 0.0f) & (al >= 1.0f / 255.0f);
+          alpha[p] = ok[p] ? al : 0.0f;
         }
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const float test_T = T * (1.0f - alpha[u]);  // T itself where the splat is skipped
-          const bool take = test_T >= 0.0001f;         // never for a finished pixel
-          const float w = take ? alpha[u] * T : 0.0f;
-          C0 = fmaf(cur.qorg[u].z, w, C0);
-          C1 = fmaf(cur.qorg[u].w, w, C1);
-          C2 = fmaf(bp[u].x, w, C2);
-          if constexpr (KEEP) {
-            D0 = fmaf(cur.qorg[u].z, w, D0);
-            D1 = fmaf(cur.qorg[u].w, w, D1);
-            D2 = fmaf(bp[u].x, w, D2);
+        for (int p = 0; p < 2; ++p) {
+          const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(alpha[p]), __float_as_uint(alpha[p]), false, false);
+          bool take[2];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {  // both lanes: the first lane's splat, then the second's
+            const float al = __uint_as_float(x[e]);
+            const float test_T = T * (1.0f - al);
+            take[e] = test_T >= 0.0001f;
+            const float w = take[e] ? al * T : 0.0f;
+            C0 = fmaf(cur.col[p][e].x, w, C0);
+            C1 = fmaf(cur.col[p][e].y, w, C1);  // the blue lane's is not used
+            T = take[e] ? test_T : -fabsf(T);
           }
-          T = take ? test_T : -fabsf(T);
-          last_contributor = (take & ok[u]) ? __float_as_uint(bp[u].y) : last_contributor;
+          const bool mine = (second & take[1]) | (!second & take[0]);
+          last_contributor = (mine & ok[p]) ? cur.pos[p] : last_contributor;
         }
-        done += U;
+        done += 4;
         return done < count && __ballot(T > 0.f) != 0;
       };
-      FwdGroup g0, g1;
-      uint4 at_now = *reinterpret_cast<const uint4*>(reach);
-      fetch(g0, at_now, U);
-      while (step(g0, at_now, g1) && step(g1, at_now, g0)) {
+      FwdPairs g0, g1;
+      fetch(g0, *reinterpret_cast<const uint4*>(reach), 4);
+      while (step(g0, g1) && step(g1, g0)) {
       }
+      continue;
+    }
+    auto fetch = [&](FwdGroup& g, const uint4& at, int next) {
+      const uint32_t o[U] = {at.x, at.y, at.z, at.w};
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        g.xyq[u] = lds_at(L.xyq, o[u]);
+        g.qorg[u] = lds_at(L.qorg, o[u]);
+      }
+      g.at = *reinterpret_cast<const uint4*>(reach + next);
+    };
+    // blends `cur` (at the offsets `at`) while `next` is on its way; false when nothing is left to do
+    int done = 0;
+    auto step = [&](FwdGroup& cur, uint4& at, FwdGroup& next) {
+      const uint32_t o[U] = {at.x, at.y, at.z, at.w};
+      float4 bp[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) bp[u] = lds_at(L.bpmi, o[u]);
+      fetch(next, cur.at, done + 2 * U);
+      at = cur.at;
+      float alpha[U];
+      bool ok[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {  // independent of each other: their latencies overlap
+        const float p = power_at(power_dx(cur.xyq[u].z, cur.xyq[u].w, cur.xyq[u].x - pxf), cur.qorg[u].x, cur.xyq[u].y - pyf);
+        const float al = fminf(0.99f, cur.qorg[u].y * splat_exp2(p));
+        ok[u] = (p <= 0.0f) & (al >= 1.0f / 255.0f);
+        alpha[u] = ok[u] ? al : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float test_T = T * (1.0f - alpha[u]);  // T itself where the splat is skipped
+        const bool take = test_T >= 0.0001f;         // never for a finished pixel
+        const float w = take ? alpha[u] * T : 0.0f;
+        C0 = fmaf(cur.qorg[u].z, w, C0);
+        C1 = fmaf(cur.qorg[u].w, w, C1);
+        C2 = fmaf(bp[u].x, w, C2);
+        T = take ? test_T : -fabsf(T);
+        last_contributor = (take & ok[u]) ? __float_as_uint(bp[u].y) : last_contributor;
+      }
+      done += U;
+      return done < count && __ballot(T > 0.f) != 0;
+    };
+    FwdGroup g0, g1;
+    uint4 at_now = *reinterpret_cast<const uint4*>(reach);
+    fetch(g0, at_now, U);
+    while (step(g0, at_now, g1) && step(g1, at_now, g0)) {
     }
   }
-  if constexpr (KEEP) {
-    __syncthreads();
-    if (threadIdx.x == 0) a.seg.tile_last[c.tile] = (uint32_t)seg_begin;
-    // a segment's backward starts from the colour behind it: sum the segments' colours from the back
-    for (int i = segs; i > 0; i -= 8) {
-      float4* at[8];
-      float4 e[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {  // all loads in flight (past the front: the front's, not used)
-        at[k] = a.seg.state + (size_t)s_slot[max(i - 1 - k, 0)] * 256 + seg_pixel;
-        e[k] = *at[k];
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        if (k >= i) break;
-        *at[k] = make_float4(e[k].x, D0, D1, D2);
-        D0 += e[k].y;
-        D1 += e[k].z;
-        D2 += e[k].w;
-      }
-    }
-  }
-  if constexpr (CELLS && !KEEP && !SPLIT) {
+  if constexpr (CELLS && !SPLIT) {
     if (a.tile_work) {  // the backward walks list positions below the tile's largest last contributor
       __shared__ uint32_t s_max[NT / DMGS_WAVE];
       uint32_t m = last_contributor;
@@ -855,6 +781,247 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
   clear_share(a);
 }
 
+// The state of the backward recursion at every 64th member of a tile's list, from the back (see the head of this
+// file): one work-group per tile, the forward's quadrants, one pixel per lane.  First the members are counted and the
+// tile takes as many slots as it has boundaries; then T and S go from splat to splat with the operations of bwd_step
+// on the same values, so that a segment which starts from them goes on exactly as the walk of the whole list would.
+// Bound like the forward by its waves' instructions, and where tiles are few by the longest list's; the same three
+// overlapping steps.  Rounds are whole (256 members, except the last), so that groups of 64 never straddle two: what
+// is left of a packed chunk moves to its front.  Five waves per SIMD instead of four change nothing (1M Gaussians at
+// 800x800 59.5 and 62.8 us).
+__global__ __launch_bounds__(256) void render_bwd_chain_kernel(RenderArgs a) {
+  constexpr int NT = 256, U = FwdGroup::kN, C = 4, G = kSegmentLength;
+  static_assert(G == DMGS_WAVE, "a group is what one wave tests at once");
+  constexpr int kPad = NT * 16;    // offset of the filling splat
+  __shared__ FwdSplats<NT + 1> L;  // slot NT: a splat of zero opacity, which fills up groups
+  __shared__ MemberList<(C + 1) * NT> M;
+  __shared__ uint32_t s_wc[2][C][NT / DMGS_WAVE];
+  __shared__ int s_hi[kTileSegments + 1];  // [i]: one past the position of member 64 i
+  __shared__ uint32_t s_max[NT / DMGS_WAVE], s_first;
+  __shared__ int s_stride;
+  __shared__ __align__(16) uint32_t s_reach[NT / DMGS_WAVE][G + 12];
+  const TileCtx c = tile_ctx<true>(a, ordered_tile(a, (int)blockIdx.x));
+  const float pxf = (float)c.px, pyf = (float)c.py;
+  const int tid = (int)threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pixel = ((wave >> 1) * 8 + (lane >> 3)) * 16 + (wave & 1) * 8 + (lane & 7);  // row-major in the tile
+  if (tid == 0) L.xyq[NT] = L.qorg[NT] = L.bpmi[NT] = make_float4(0.f, 0.f, 0.f, 0.f);
+  float T = 0.f, S = 0.f, g0 = 0.f, g1 = 0.f, g2 = 0.f;
+  uint32_t last = 0;
+  if (c.inside) {
+    const size_t pid = c.pix - c.img / 3;
+    const float* dp = a.dL_dpix + c.img;
+    T = a.final_T[c.pix];
+    last = a.n_contrib[c.pix];
+    g0 = dp[pid];
+    g1 = dp[c.plane + pid];
+    g2 = dp[2 * c.plane + pid];
+  }
+  uint32_t wave_last = last;  // positions at or past it contribute to none of the wave's pixels
+  for (int off = 32; off > 0; off >>= 1) wave_last = max(wave_last, (uint32_t)__shfl_xor((int)wave_last, off, 64));
+  wave_last = __builtin_amdgcn_readfirstlane(wave_last);
+  if (lane == 0) s_max[wave] = wave_last;
+  __syncthreads();
+  const int len = min((int)(c.range.y - c.range.x), (int)max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3])));
+
+  // The visit's k-th position of this lane in the chunk that starts after `at` positions from the back.
+  auto position = [&](int at, int k) { return len - 1 - (at + k * NT + tid); };
+  auto key_of = [&](int pos) { return a.list_keys[c.range.x + (uint32_t)max(pos, 0)]; };
+  // Hands each member of the chunk its number, counted from `first`; returns how many there are.  One barrier.
+  int flip = 0;
+  auto number = [&](int at, const uint32_t(&key)[C], int first, auto&& each) {
+    uint64_t bal[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      bal[k] = __ballot(position(at, k) >= 0 && ((key[k] >> DMGS_CELL_KEY_BITS) & c.bit));
+      if (lane == 0) s_wc[flip][k][wave] = (uint32_t)__popcll(bal[k]);
+    }
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      int before = first + total + (int)__popcll(bal[k] & lanemask_lt());
+#pragma unroll
+      for (int w = 0; w < NT / DMGS_WAVE; ++w) {
+        const int cnt = (int)s_wc[flip][k][w];
+        before += w < wave ? cnt : 0;
+        total += cnt;
+      }
+      if ((bal[k] >> lane) & 1u) each(before, k);
+    }
+    flip ^= 1;
+    return total;
+  };
+
+  int members = 0;
+  if (len > G) {
+    uint32_t key[C], ahead[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) key[k] = key_of(position(0, k));
+    for (int at = 0; at < len; at += C * NT) {
+#pragma unroll
+      for (int k = 0; k < C; ++k) ahead[k] = key_of(position(at + C * NT, k));
+      members += number(at, key, members, [&](int i, int k) {
+        if (i % G == 0 && i / G <= kTileSegments) s_hi[i / G] = position(at, k) + 1;
+      });
+#pragma unroll
+      for (int k = 0; k < C; ++k) key[k] = ahead[k];
+    }
+  }
+  // Slots come from one of kSegmentParts counters (one for all: atomics of 3844 tiles on one address took 100 us).
+  // Segments get longer as its slots are used up (64 members until half of them are gone, then 128 until a quarter is
+  // left, and so on): the longest lists come first, and every tile still finds some.  The backward proper of 1.5M
+  // Gaussians at 800x800 takes 203 us (whole lists 781), 885 with 64 members while slots last.
+  const int boundaries = members > 0 ? min((members - 1) / G, kTileSegments) : 0;
+  const int part = (int)blockIdx.x % kSegmentParts, part_cap = a.seg.cap / kSegmentParts;
+  if (tid == 0) {
+    uint32_t* const head = a.seg.head + part * kSegmentHeadStride;
+    int stride = 1;
+    if (boundaries > 0) {
+      const uint32_t taken = __hip_atomic_load(head, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const int left = part_cap - (int)min(taken, (uint32_t)part_cap);
+      while (stride < kTileSegments && left < part_cap / (2 * stride)) stride *= 2;
+    }
+    s_stride = stride;
+    s_first = boundaries >= stride ? atomicAdd(head, (uint32_t)(boundaries / stride)) : 0u;
+  }
+  __syncthreads();
+  const int stride = s_stride;  // groups of 64 per segment
+  const int usable = min(boundaries / stride, part_cap - (int)min(s_first, (uint32_t)part_cap));
+  const uint32_t first = (uint32_t)(part * part_cap) + s_first;
+  for (int i = tid; i < usable; i += NT)  // the segment in front of boundary i + 1; the last one takes what is left
+    a.seg.rec[first + i] = make_uint4((uint32_t)c.tile, (uint32_t)(i + 1 < usable ? s_hi[(i + 2) * stride] : 0),
+                                      (uint32_t)s_hi[(i + 1) * stride], 0u);
+  if (tid == 0) a.seg.tile_last[c.tile] = usable > 0 ? (uint32_t)s_hi[stride] : 0u;
+  if (usable == 0) return;
+
+  uint32_t key[C], id[C];
+  int next_chunk = 0;  // the first position (from the back) not asked for
+  auto request = [&]() {
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const int pos = position(next_chunk, k);
+      key[k] = key_of(pos);
+      id[k] = a.point_list[c.range.x + (uint32_t)max(pos, 0)];
+    }
+    next_chunk += C * NT;
+  };
+  int used = 0;        // of the packed members those whose records were asked for
+  bool asked = false;  // a chunk is on its way
+  members = 0;         // packed
+  // Packs the chunk on its way, and more until there is a whole round or the list ends; ends with a barrier.
+  auto fill = [&]() {
+    while (asked) {
+      const int left = members - used;  // fewer than a round: where they are and where they go is disjoint
+      if (used > 0 && tid < left) {
+        M.id[tid] = M.id[used + tid];
+        M.pos[tid] = M.pos[used + tid];
+      }
+      const int at = next_chunk - C * NT;
+      used = 0;
+      members = left + number(at, key, left, [&](int i, int k) {
+        M.id[i] = id[k];
+        M.pos[i] = (uint32_t)position(at, k);
+      });
+      asked = members < NT && next_chunk < len;
+      if (asked) request();
+    }
+    __syncthreads();
+  };
+  auto ask = [&]() {
+    if (members - used < NT && next_chunk < len) {
+      request();
+      asked = true;
+    }
+  };
+  float4 r0, r1, r2;  // this lane's record of the next round
+  uint32_t my_id = 0, my_pos = 0;
+  auto gather = [&]() {
+    const int n = min(NT, members - used);
+    const int s = used + min(tid, max(n - 1, 0));  // no lane's loads are conditional
+    my_id = M.id[min(s, (C + 1) * NT - 1)];
+    my_pos = M.pos[min(s, (C + 1) * NT - 1)];
+    const float4* sp = a.splats + (size_t)DMGS_SPLAT_F4 * min(my_id, a.P - 1);
+    r0 = sp[0];
+    r1 = sp[1];
+    r2 = sp[2];
+    used += n;
+    return n;
+  };
+  request();
+  asked = true;
+  fill();
+  int n_next = gather();
+  ask();
+  int next_state = 0, to_state = stride;  // the boundary that comes next, and the groups up to it
+  while (next_state < usable && n_next > 0) {
+    const int n = n_next;
+    __syncthreads();  // the round before has been read
+    if (tid < n) put_splat(L, tid, r0, r1, r2, my_id, a.P, c.rows, my_pos);
+    fill();
+    n_next = gather();
+    ask();
+    for (int h = 0; h < n && next_state < usable; h += G) {
+      uint32_t* const reach = s_reach[wave];
+      const uint64_t bits =
+          __ballot(h + lane < n && ((L.mask(h + lane) >> wave) & 1u) && L.pos(h + lane) < wave_last);
+      const int count = (int)__popcll(bits);
+      if (count > 0) {
+        if ((bits >> lane) & 1u) reach[(int)__popcll(bits & lanemask_lt())] = (uint32_t)(h + lane) * 16u;
+        if (lane < 12) reach[count + lane] = kPad;
+        auto fetch = [&](FwdGroup& g, const uint4& at, int next) {
+          const uint32_t o[U] = {at.x, at.y, at.z, at.w};
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            g.xyq[u] = lds_at(L.xyq, o[u]);
+            g.qorg[u] = lds_at(L.qorg, o[u]);
+          }
+          g.at = *reinterpret_cast<const uint4*>(reach + next);
+        };
+        // walks `cur` (at the offsets `at`) while `next` is on its way; false when nothing is left to do
+        int walked = 0;
+        auto step = [&](FwdGroup& cur, uint4& at, FwdGroup& next) {
+          const uint32_t o[U] = {at.x, at.y, at.z, at.w};
+          float4 bp[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) bp[u] = lds_at(L.bpmi, o[u]);
+          fetch(next, cur.at, walked + 2 * U);
+          at = cur.at;
+          float om[U], inv[U], add[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {  // independent of each other: their latencies overlap
+            const float4 g = cur.xyq[u], q = cur.qorg[u];
+            const float p = power_at(power_dx(g.z, g.w, g.x - pxf), q.x, g.y - pyf);
+            const float alpha = fminf(0.99f, q.y * splat_exp2(p));
+            const bool ok = (p <= 0.0f) & (alpha >= 1.0f / 255.0f) & (__float_as_uint(bp[u].y) < last);
+            om[u] = ok ? 1.f - alpha : 1.f;  // a skipped splat multiplies by one and adds zero
+            inv[u] = __builtin_amdgcn_rcpf(om[u]);
+            const float cg = fmaf(bp[u].x, g2, fmaf(q.w, g1, q.z * g0));
+            add[u] = ok ? __fmul_rn(alpha, cg) : 0.f;
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            T *= inv[u];
+            S = fmaf(om[u], S, add[u]);
+          }
+          walked += U;
+          return walked < count;
+        };
+        FwdGroup e0, e1;
+        uint4 at_now = *reinterpret_cast<const uint4*>(reach);
+        fetch(e0, at_now, U);
+        while (step(e0, at_now, e1) && step(e1, at_now, e0)) {
+        }
+      }
+      if (--to_state == 0) {
+        a.seg.state[(size_t)(first + (uint32_t)next_state) * 256 + pixel] = make_float2(T, S);
+        ++next_state;
+        to_state = stride;
+      }
+    }
+  }
+}
+
 // Backward with one wave per 16x16 tile: lane (lx, ly) owns the pixels
 // (lx, ly + 4k), k = 0..3, i.e. one pixel in each of four 16x4 strips.  The
 // footprint test runs per strip, each pixel is evaluated exactly as in the
@@ -870,26 +1037,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KEEP || SPL
 // with the background in the recursion and the linear forms after the sums,
 // whose gradients differ, see bwd_step).
 //
-// SEGS: the work-groups below a.seg.cap each take one kept segment of a tile's
-// list (see Segments), the others the rest of a tile's list.
+// SEGS: the first a.num_tiles work-groups each take the last segment of a tile's
+// list (or all of it), which starts at the list's end, the others one that
+// starts from a state (see Segments).
 template <bool CELLS, bool SEGS>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void render_bwd_strips_kernel(RenderArgs a) {
   constexpr int NT = 64, BATCH = 64;
   int tile, lo = 0, hi = 0x7fffffff;                   // this work-group's list positions [lo, hi)
   uint32_t seg_end = kNoSegment;                       // the slot of the state at hi (none: the list's end)
   if constexpr (SEGS) {
-    const bool kept = a.seg.head[1] == kSegMagic;
-    if ((int)blockIdx.x < a.seg.cap) {
-      if (!kept || blockIdx.x >= a.seg.head[0]) return;
-      const uint4 r = a.seg.rec[blockIdx.x];
-      if (r.x >= (uint32_t)a.num_tiles) return;  // never used
+    if ((int)blockIdx.x < a.num_tiles) {
+      tile = ordered_tile(a, blockIdx.x);
+      lo = max((int)a.seg.tile_last[tile], 0);
+    } else {  // the parts' used slots in turn, before the unused ones (16k work-groups that only end take 20 us)
+      const uint32_t b = blockIdx.x - (uint32_t)a.num_tiles, part = b % kSegmentParts, i = b / kSegmentParts;
+      if (i >= a.seg.head[part * kSegmentHeadStride]) return;
+      seg_end = part * (uint32_t)(a.seg.cap / kSegmentParts) + i;
+      const uint4 r = a.seg.rec[seg_end];
+      if (r.x >= (uint32_t)a.num_tiles) return;
       tile = (int)r.x;
       lo = max((int)r.y, 0);
       hi = (int)r.z;
-      seg_end = blockIdx.x;
-    } else {
-      tile = (int)blockIdx.x - a.seg.cap;
-      if (kept) lo = max((int)a.seg.tile_last[tile], 0);
     }
   } else {
     tile = ordered_tile(a, blockIdx.x);
@@ -937,10 +1105,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) void
     bg_term[k] = -T_final * (c.bg0 * g0[k] + c.bg1 * g1[k] + c.bg2 * g2[k]);
     st[k] = {T_final, 0.f};
     if constexpr (SEGS) {
-      if (seg_end != kNoSegment) {  // start from the state at hi: T, and the colour behind it
-        const float4 e = a.seg.state[(size_t)seg_end * 256 + threadIdx.x + 64 * k];
-        st[k].T = e.x;
-        st[k].S = (e.y * g0[k] + e.z * g1[k] + e.w * g2[k]) / e.x;
+      if (seg_end != kNoSegment) {  // start from the state at hi
+        const float2 e = a.seg.state[(size_t)seg_end * 256 + threadIdx.x + 64 * k];
+        st[k] = {e.x, e.y};
       }
     }
   }
@@ -1182,11 +1349,6 @@ void launch_tile_order_bwd(const RenderArgs& a, uint32_t* order, uint8_t* bucket
   if (a.tile_work) tile_order_impl(a, order, bucket, hist, true, s, hist_zeroed);
 }
 
-// Kept segments: the header is set before each forward that keeps any.
-__global__ void seg_reset_kernel(uint32_t* head) {
-  if (threadIdx.x < 2) head[threadIdx.x] = threadIdx.x == 0 ? 0u : kSegMagic;
-}
-
 // Two work-groups per tile while they find idle SIMDs, us before and after: 336 tiles of long lists (500k Gaussians,
 // 333x251, near) 196 and 150, 169 tiles (10k, 200x200) 48 and 39, 475 tiles 220 and 171; 512 tiles of 2 views 72 and
 // 59, or 23 and 26 where the lists end after a few splats.  625 tiles of such lists 20 and 28, 1024 24 and 33.
@@ -1194,23 +1356,21 @@ constexpr int kSplitTiles = 512;
 void launch_render_fwd(const RenderArgs& a, hipStream_t s) {
   if (a.num_tiles <= 0) return;
   const dim3 grid(a.num_tiles), block(256);
-  if (a.seg.len > 0) {
-    hipLaunchKernelGGL(seg_reset_kernel, dim3(1), dim3(64), 0, s, a.seg.head);
-    hipLaunchKernelGGL((render_fwd_quads_kernel<true, true, false>), grid, block, 0, s, a);
-  } else if (a.views && a.num_tiles <= kSplitTiles) {
-    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false, true>), dim3(2 * a.num_tiles), block, 0, s, a);
-  } else if (a.views) {
-    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false, false>), grid, block, 0, s, a);
-  } else {
-    hipLaunchKernelGGL((render_fwd_quads_kernel<false, false, false>), grid, block, 0, s, a);
-  }
+  if (a.views && a.num_tiles <= kSplitTiles)
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, true>), dim3(2 * a.num_tiles), block, 0, s, a);
+  else if (a.views)
+    hipLaunchKernelGGL((render_fwd_quads_kernel<true, false>), grid, block, 0, s, a);
+  else
+    hipLaunchKernelGGL((render_fwd_quads_kernel<false, false>), grid, block, 0, s, a);
 }
 
 void launch_render_bwd(const RenderArgs& a, hipStream_t s) {
   if (a.num_tiles <= 0) return;
-  if (a.seg.len > 0)
+  if (a.seg.cap > 0) {
+    launch_fill_u32(a.seg.head, kSegmentParts * kSegmentHeadStride, 0u, s);
+    hipLaunchKernelGGL(render_bwd_chain_kernel, dim3(a.num_tiles), dim3(256), 0, s, a);
     hipLaunchKernelGGL((render_bwd_strips_kernel<true, true>), dim3(a.seg.cap + a.num_tiles), dim3(64), 0, s, a);
-  else if (a.views)
+  } else if (a.views)
     hipLaunchKernelGGL((render_bwd_strips_kernel<true, false>), dim3(a.num_tiles), dim3(64), 0, s, a);
   else
     hipLaunchKernelGGL((render_bwd_strips_kernel<false, false>), dim3(a.num_tiles), dim3(64), 0, s, a);

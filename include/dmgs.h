@@ -310,9 +310,9 @@ int dmgs_batched_tile_view(const dmgs_view* views, int32_t B, int32_t* tile_view
 /* Workspaces of a batch (device memory, caller-owned):
  *   state   K-independent: per (view, Gaussian) splats, keys, radii, scan;
  *           per-tile ranges; per-pixel blend state; up to 4096 tiles, also
- *           list segments a forward with bwd_ws keeps for its backward
- *           (4 to 64 MB; the forward size is without them, for batches whose
- *           bwd_ws is always null; the rest is laid out alike).  Kept until
+ *           the states that a backward starts list segments from (8 to 64
+ *           MB; the forward size is without them, for batches whose bwd_ws
+ *           is always null; the rest is laid out alike).  Kept until
  *           backward.
  *   lists   the (Gaussian, tile) instance lists for up to `capacity`
  *           instances and their sort scratch.  Kept until backward.
