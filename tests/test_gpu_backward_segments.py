@@ -26,7 +26,9 @@ pytestmark = pytest.mark.gpu
     (3000, -1.0, 1.2, (16, 16), -4.0, (0, 0)),      # small splats: quadrants and pixels skip most of them
     (17500, -4.6, 1.2, (16, 16), -4.0, (0, 0)),     # more boundaries than a tile keeps
     (9000, -1.0, 1.2, (70, 64), -4.5, (1, 2)),      # a few members in each chunk
-    (9000, -1.0, 1.2, (70, 64), -4.5, (4, 1))])     # partly outside the image
+    (9000, -1.0, 1.2, (70, 64), -4.5, (4, 1)),      # partly outside the image
+    (2000, -5.2, 4.0, (320, 320), 0.5, (3, 7)),     # 400 tiles share 4096 slots: longer segments
+    (2000, -5.2, 4.0, (320, 320), 0.5, (10, 10))])
 def test_segments_equal_whole_lists(n, logit, dist, size, scale, tile):
     print(f"case: segments n={n} logit={logit} dist={dist} size={size} scale={scale} tile={tile}", flush=True)
     g = torch.Generator().manual_seed(n)
