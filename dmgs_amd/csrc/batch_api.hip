@@ -211,7 +211,8 @@ dmgs::RenderArgs render_args(const dmgs_batch* b, const Ctx& c) {
   r.n_contrib = at<uint32_t>(b->state, c.S.n_contrib);
   r.gacc = static_cast<float*>(b->bwd_ws);
   r.tile_order = at<uint32_t>(b->state, c.S.tile_order);
-  r.tile_work = at<uint32_t>(b->state, c.S.tile_work);  // the forward measures each tile's backward list length
+  // the forward measures each tile's backward list length, for the order of a backward of whole lists
+  if (b->total_tiles > dmgs::kSegmentTiles) r.tile_work = at<uint32_t>(b->state, c.S.tile_work);
   if (b->bwd_ws && c.S.seg_cap) {
     r.seg.head = at<uint32_t>(b->state, c.S.seg_head);
     r.seg.cap = c.S.seg_cap;
@@ -309,13 +310,12 @@ int blend_views(const dmgs_batch* b, const Ctx& c, float* images, hipStream_t st
 int blend_views_backward(const dmgs_batch* b, const Ctx& c, const float* dL_dimages, hipStream_t st) {
   dmgs::RenderArgs r = render_args(b, c);
   r.dL_dpix = dL_dimages;
-  // re-order the tiles by the list lengths the forward measured (the
+  // re-order the tiles by the list lengths, if the forward measured them (the
   // forward blend, and then each backward blend, zero the histogram)
   r.clear_words = at<uint32_t>(b->state, c.S.bucket_hist);
   r.clear_words_n = 512;
-  if (r.seg.cap == 0)
-    dmgs::launch_tile_order_bwd(r, at<uint32_t>(b->state, c.S.tile_order), at<uint8_t>(b->state, c.S.tile_bucket),
-                                at<uint32_t>(b->state, c.S.bucket_hist), st, true);
+  dmgs::launch_tile_order_bwd(r, at<uint32_t>(b->state, c.S.tile_order), at<uint8_t>(b->state, c.S.tile_bucket),
+                              at<uint32_t>(b->state, c.S.bucket_hist), st, true);
   dmgs::launch_render_bwd(r, st);
   return bcheck("batch render backward", st);
 }
